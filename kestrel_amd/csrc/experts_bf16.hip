@@ -1,6 +1,6 @@
 // The linears of routed experts on the matrix cores (bf16): the pairs (token, choice) of a step come listed by expert, in
-// runs that start on multiples of 128 rows of the list (ka_experts_sort), and a workgroup multiplies one tile of 128 list
-// rows by 256 rows of its expert's weights (ka_listed_tiles.h): out[row] = act(a[row'] W_e^T).
+// runs that start on multiples of a tile's rows (ka_experts_sort, ka_experts_gemm_tile), and a workgroup multiplies one
+// tile of list rows by 256 rows of its expert's weights: out[row] = act(a[row'] W_e^T).
 //
 //  * the first linear gathers: list row i holds pair p = sorted[i] (-1: an unused row), whose input is row p / gather_div
 //    of `a`; its output goes to row i of `out` (the hidden rows stay in list order);
@@ -11,7 +11,12 @@
 // The weights are the row operand: a lane ends with outputs of ONE list row, four neighbours at a time, so the pair of a
 // gated output meets in a lane's registers.
 #include "ka_common.h"
+#include "ka_dma_tiles.h"
 #include "ka_listed_tiles.h"
+
+#include <math.h>
+
+#include <utility>
 
 typedef __attribute__((ext_vector_type(2))) __bf16 eb_bf16x2;
 
@@ -87,17 +92,189 @@ experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, cons
     }
 }
 
-KA_API int ka_experts_gemm_tile() { return KL_ROWS; }
+// ----------------------------------------------------------------------------
+// The same linears where K is a multiple of 64: operands go from memory straight into LDS (ka_dma_tiles.h), the list's rows
+// gathered by the addresses of the loads. Eight waves and 256 weight rows a workgroup; a tile has 64, 128 or 256 list rows, as
+// many as the list was made for.
+//
+// What bounds it: an expert sees a few hundred rows of a step, so its weights come from HBM for little more work than they cost
+// to read (62 experts of 2 x 896 x 4,096 at 198 rows each: 910 MB and 180 GFLOP, 160 us of either). The tiles that share an
+// expert therefore run side by side on one XCD (workgroups go to the XCDs in turn; each XCD gets one stretch of the list, all
+// columns of a list tile before the next), so that its L2 passes weights between list tiles and rows between column
+// tiles. For that the used part of the list has to be known, or the XCD with its unused end would idle: every workgroup counts
+// the tiles that have an expert, in one read of the list of tiles.
+//
+// Measured, us of the gated first and the fp32 second linear, before (the kernel above, which staged through registers, one wave
+// a SIMD, with sums that went through scratch memory) -> now: 62 experts of 4,096 x 896, 2,048 tokens of 6 choices 542 + 372 ->
+// 261 + 187; 512 tokens 302 + 175 -> 163 + 114; 30 experts of 2,048 x 704, 2,048 tokens of 4 choices 147 + 119 -> 81 + 60.
+// ----------------------------------------------------------------------------
+struct ExpertsDmaArgs {
+    const bf16_t* a;
+    long lda;
+    int gather_div;             // as above
+    const bf16_t* W;
+    const int* sorted;
+    const int* tile_expert;
+    int n_tiles, tiles_n, N, K, act;
+    KaGateClamp clamp;
+    void* out;
+    long ldo;
+    int scatter;
+};
 
-// Whether the kernel covers these sizes and this alignment.
+template <int WN, int WM, int GN, int GM, int NS, int SL, bool GATED, bool F32>
+__global__ void __launch_bounds__(KA_WAVE * GN * GM)
+    __attribute__((amdgpu_waves_per_eu(GN * GM / 4, (WN * WM > 8 ? 1 : 2) * (GN * GM / 4))))
+experts_dma_kernel(ExpertsDmaArgs g) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS>;
+    constexpr int BN = T::BN, BM = T::BM, CPR = T::CPR;
+    extern __shared__ __attribute__((aligned(16))) unsigned char eb_dma_lds[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KA_WAVE), lane = tid % KA_WAVE;
+    int used = 0;
+    for (int t0 = 0; t0 < g.n_tiles; t0 += T::WAVES * KA_WAVE)
+        used += __syncthreads_count(t0 + tid < g.n_tiles && g.tile_expert[min(t0 + tid, g.n_tiles - 1)] >= 0);
+    const int total = used * g.tiles_n, per_xcd = (total + 7) / 8;
+    const int at = blockIdx.x / 8, logical = blockIdx.x % 8 * per_xcd + at;
+    if (at >= per_xcd || logical >= total) return;
+    const int tile = logical / g.tiles_n, n0 = (logical - tile * g.tiles_n) * BN;
+    const int e = g.tile_expert[tile], i0 = tile * BM;
+    const int wn = wave / GM, wm = wave % GM, li = lane % 32, lg = lane / 32;
+    const bf16_t* wsrc[T::W_LOADS];
+    const bf16_t* xsrc[T::X_LOADS];
+#pragma unroll
+    for (int i = 0; i < T::X_LOADS; ++i) {
+        const int r = kd_load_row<CPR>(wave * T::X_LOADS + i, lane);
+        const long row = g.gather_div > 0 ? (long)(max(g.sorted[i0 + r], 0) / g.gather_div) : (long)i0 + r;
+        xsrc[i] = g.a + row * g.lda + kd_load_channel<CPR>(r, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < T::W_LOADS; ++i) {
+        const int r = kd_load_row<CPR>(wave * T::W_LOADS + i, lane);
+        wsrc[i] = g.W + ((size_t)e * g.N + min(n0 + r, g.N - 1)) * g.K + kd_load_channel<CPR>(r, lane);
+    }
+    floatx16 acc[WN][WM];
+#pragma unroll
+    for (int a = 0; a < WN; ++a)
+#pragma unroll
+        for (int b = 0; b < WM; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+    kd_product<WN, WM, GN, GM, 64, NS, SL>(eb_dma_lds, wave, lane, g.K, wsrc, xsrc, acc);
+
+    // A lane ends with four neighbouring weight rows of one list row, a store instruction would touch 32 rows with 8 or 16
+    // bytes each: a wave passes 32 list rows at a time through its share of LDS and stores its piece of every row whole.
+    using E = std::conditional_t<F32, float, bf16_t>;
+    constexpr int OUTS = GATED ? 16 * WN : 32 * WN;      // outputs of a row of the wave's tile
+    constexpr int RB = OUTS * (int)sizeof(E), RS = RB + (F32 ? 16 : 8), CH = RB / 16, PER = 16 / (int)sizeof(E), RPI = KA_WAVE / CH;
+    static_assert(32 * RS <= T::SMEM / T::WAVES, "a wave's share of LDS does not hold 32 rows of its tile");
+    const int n_out = GATED ? g.N / 2 : g.N, o_wave = (n0 + wn * 32 * WN) / (GATED ? 2 : 1);
+    unsigned char* mine = eb_dma_lds + wave * (T::SMEM / T::WAVES);
+    gd_barrier();                                        // the last stage has been read by everybody
+    gd_static_for<0, WM>([&](auto bc) {
+        constexpr int b = decltype(bc)::value;
+        gd_static_for<0, WN>([&](auto ac) {
+            constexpr int a = decltype(ac)::value;
+            gd_static_for<0, 4>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                const floatx4 v = {acc[a][b][q * 4], acc[a][b][q * 4 + 1], acc[a][b][q * 4 + 2], acc[a][b][q * 4 + 3]};
+                const int nl = a * 32 + q * 8 + lg * 4;
+                if constexpr (GATED) {
+                    eb_bf16x2 y;
+                    y[0] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, v[0], v[1]);
+                    y[1] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, v[2], v[3]);
+                    *reinterpret_cast<eb_bf16x2*>(mine + li * RS + nl) = y;
+                } else if constexpr (F32) {
+                    *reinterpret_cast<floatx4*>(mine + li * RS + nl * 4) = v;
+                } else {
+                    bf16x4 y;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) y[x] = (bf16_t)ka_activate_fast(g.act, v[x]);
+                    *reinterpret_cast<bf16x4*>(mine + li * RS + nl * 2) = y;
+                }
+            });
+        });
+        at_epilogue_wave_sync();
+#pragma unroll
+        for (int r0 = 0; r0 < 32; r0 += RPI) {
+            const int rl = r0 + lane / CH, c = lane % CH, i = i0 + wm * 32 * WM + b * 32 + rl, o = o_wave + c * PER;
+            const int p = g.sorted[i];
+            if (p >= 0 && o < n_out) {
+                const unsigned char* from = mine + rl * RS + c * 16;
+                E* op = reinterpret_cast<E*>(g.out) + (g.scatter ? (long)p : (long)i) * g.ldo + o;
+                if (o + PER <= n_out) {
+                    *reinterpret_cast<floatx4*>(op) = *reinterpret_cast<const floatx4*>(from);
+                } else {
+                    for (int x = 0; x < PER && o + x < n_out; ++x) op[x] = reinterpret_cast<const E*>(from)[x];
+                }
+            }
+        }
+        at_epilogue_wave_sync();                         // the next pass writes over what was just read
+    });
+}
+
+template <int WN, int WM, int GN, int GM, int NS, int SL, bool GATED, bool F32>
+static int experts_dma_launch(const ExpertsDmaArgs& g, hipStream_t stream) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS>;
+    static bool configured = false;
+    auto kernel = experts_dma_kernel<WN, WM, GN, GM, NS, SL, GATED, F32>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM);
+        KA_CHECK(e == hipSuccess, "ka_experts_gemm_bf16: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
+        configured = true;
+    }
+    static_assert(T::BN == 256, "the caller counts columns of 256");
+    const long blocks = ((long)g.n_tiles * g.tiles_n + 7) / 8 * 8;
+    KA_CHECK(blocks < (1L << 31), "ka_experts_gemm_bf16: too many tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * GN * GM), T::SMEM, stream, g);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+template <int WN, int WM, int GN, int GM, int NS, int SL>
+static int experts_dma(const ExpertsDmaArgs& g, int out_f32, hipStream_t stream) {
+    if (ka_act_gated(g.act)) return experts_dma_launch<WN, WM, GN, GM, NS, SL, true, false>(g, stream);
+    if (out_f32) return experts_dma_launch<WN, WM, GN, GM, NS, SL, false, true>(g, stream);
+    return experts_dma_launch<WN, WM, GN, GM, NS, SL, false, false>(g, stream);
+}
+
+// Whether the kernels cover these sizes and this alignment.
 KA_API int ka_experts_gemm_supported(long lda, int N, int K, long ldo, int act, int out_f32) {
     const int n_out = ka_act_outputs(act, N);
     return K > 0 && K % 16 == 0 && lda % 8 == 0 && N > 0 && (!ka_act_gated(act) || (N % 4 == 0 && ldo % 2 == 0 && !out_f32)) &&
            (!out_f32 || ldo % 4 == 0) && ldo >= n_out ? 1 : 0;
 }
 
+static bool experts_dma_covers(int N, int K, long ldo, int act, int out_f32) {
+    return K % 64 == 0 && ldo * (out_f32 ? 4 : 2) % 16 == 0 && !(out_f32 && act) && (!ka_act_gated(act) || N % 4 == 0);
+}
+
+// List rows of a tile for `n_pairs` pairs of `E` experts whose linears have N1 x K1 and N2 x K2 weights (the second K is the
+// first's output): the list has to be made for it. The kernel that stages through registers has tiles of KL_ROWS; for the other
+// one the choice goes by the rows an expert can expect, with a quarter on top for routers that do not spread evenly:
+//  * where these fit 64, a tile holds an expert and there is nothing to gain from a larger one (50 rows: 277 us both linears
+//    of 62 x 4,096 x 896, against 300 with 128 and 402 with 256);
+//  * else by the rounds that the tiles make on the chip, one workgroup a CU. A row of a tile of 128 costs 1.2 times one of a tile
+//    of 256, which asks LDS for less per product (198 rows of the same experts: 525 against 448 us); where an expert's
+//    last tile is half empty or the tiles just miss a round, 128 is ahead (256 rows of 30 experts of 2,048 x 704: 141
+//    against 183 us; 150 rows: 119 against 105).
+KA_API int ka_experts_gemm_tile(int n_pairs, int E, int N1, int K1, int act, int N2) {
+    const int ff = ka_act_outputs(act, N1);
+    if (n_pairs <= 0 || E <= 0 || !experts_dma_covers(N1, K1, ff, act, 0) || !experts_dma_covers(N2, ff, N2, 0, 1)) return KL_ROWS;
+    const double rows = (double)n_pairs / E, most = 1.25 * rows;
+    if (most <= 64) return 64;
+    const int cus = ka_compute_units();
+    auto cost = [&](int tile) {
+        const double tiles = E * (most <= tile ? 1.0 : rows / tile + 0.5);
+        double sum = 0;
+        for (const auto& [n, k] : {std::pair<int, int>{N1, K1}, {N2, ff}})
+            sum += ceil(tiles * ka_cdiv(n, 256) / cus) * tile * k;
+        return sum;
+    };
+    return cost(256) < 1.2 * cost(128) ? 256 : 128;
+}
+
 KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const void* W, const int* sorted, const int* tile_expert,
-                                int n_tiles, int N, int K, int act, int clamped, float limit, float slope, float shift, void* out,
+                                int n_tiles, int tile, int N, int K, int act, int clamped, float limit, float slope, float shift, void* out,
                                 long ldo, int scatter, int out_f32, hipStream_t stream) {
     const char* who = "ka_experts_gemm_bf16";
     KA_CHECK(!clamped || ka_act_gated(act), "%s: clamps are a gated linear's", who);
@@ -106,6 +283,13 @@ KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const v
     KA_CHECK(ka_act_known(act) && ka_experts_gemm_supported(lda, N, K, ldo, act, out_f32), "%s: sizes N=%d K=%d not covered", who, N, K);
     KA_CHECK((uintptr_t)a % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)out % 16 == 0, "%s: operands must be 16-byte aligned", who);
     if (n_tiles == 0) return 0;
+    if (experts_dma_covers(N, K, ldo, act, out_f32)) {
+        const ExpertsDmaArgs g{(const bf16_t*)a, lda, gather_div, (const bf16_t*)W, sorted, tile_expert, n_tiles, ka_cdiv(N, 256), N, K, act, clamp, out, ldo, scatter};
+        if (tile == 64) return experts_dma<2, 1, 4, 2, 3, 2>(g, out_f32, stream);
+        if (tile == 128) return experts_dma<2, 2, 4, 2, 3, 2>(g, out_f32, stream);
+        if (tile == 256) return experts_dma<2, 4, 4, 2, 2, 1>(g, out_f32, stream);
+    }
+    KA_CHECK(tile == KL_ROWS, "%s: no kernel for tiles of %d list rows at these sizes", who, tile);
     const dim3 grid((N + KL_COLS - 1) / KL_COLS, n_tiles);
     static bool sized = false;
     if (!sized) {

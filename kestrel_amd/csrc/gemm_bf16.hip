@@ -12,16 +12,12 @@
 // That kernel takes any K (in steps of 8); where K is a multiple of 64 the large-tile kernel
 // further down, which loads straight into LDS, is used instead.
 #include "ka_common.h"
+#include "ka_dma_tiles.h"
 #include "ka_partials.h"
 
 #include <stdlib.h>
 
 #include <type_traits>
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((ext_vector_type(16))) float floatx16;
-typedef __attribute__((ext_vector_type(4))) float floatx4;
 
 constexpr int GB_THREADS = 256;
 constexpr int GB_PAD = 8;          // bf16 of padding per LDS row
@@ -172,75 +168,15 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restric
 }
 
 // ----------------------------------------------------------------------------
-// The large-tile kernel. Four (2 x 2) or eight (4 x 2) waves, each with WN x WM MFMA tiles of
-// 32 x 32. K-steps of BK go from global memory straight into LDS (global_load_lds_dwordx4: no
-// registers, no ds_write), NS stages, one barrier per step. Chunk c (16 bytes) of tile row r
-// lies at place c ^ swizzle(r) of its row, chosen by which chunk each lane of the load asks
-// for, so that the rows that one pass of a 16-byte LDS read touches fall on different banks
-// without padding. Rows past the end of a matrix are read from its last row (and never stored);
-// K must be a multiple of BK.
+// The large-tile kernel: four (2 x 2) or eight (4 x 2) waves over the loop of ka_dma_tiles.h. Rows past the end of a matrix are
+// read from its last row (and never stored); K must be a multiple of BK.
 // ----------------------------------------------------------------------------
-constexpr int gd_smem(int bn, int bm, int bk, int ns) { return ns * (bn + bm) * bk * 2; }
-
-// A loop whose index is a compile-time constant in every round (the accumulators are up to 256
-// registers: an index the compiler does not resolve would put them in memory).
-template <int I, int N, typename F>
-__device__ __forceinline__ void gd_static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        gd_static_for<I + 1, N>(f);
-    }
-}
-
-#define GD_GLOBAL __attribute__((address_space(1)))
-#define GD_LDS __attribute__((address_space(3)))
-
-// s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, the other counters at their maximum)
-template <int N>
-__device__ __forceinline__ void gd_wait_loads() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-}
-
-// Waits until at most `younger` x LPW of this wave's loads are still in flight (the count of an
-// s_waitcnt is an immediate: one instruction per value that can occur, at most MAX).
-template <int LPW, int MAX>
-__device__ __forceinline__ void gd_wait_younger(int younger) {
-    static_assert(LPW * (MAX > 0 ? MAX : 0) <= 63, "more loads in flight than the counter holds");
-    if constexpr (MAX <= 0) {
-        gd_wait_loads<0>();
-    } else {
-        if (younger >= MAX) gd_wait_loads<LPW * MAX>();
-        else gd_wait_younger<LPW, MAX - 1>(younger);
-    }
-}
-
-// s_waitcnt lgkmcnt(0) alone: this wave's LDS reads have all arrived in its registers
-__device__ __forceinline__ void gd_wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
-
-// The barrier alone, without the fence that __syncthreads() puts before it: that fence waits
-// for every load in flight, the younger stages' too. What must be ordered here is ordered by
-// hand: a wave has waited for its own loads of the stage (vmcnt) and for its LDS reads of the
-// stage before (their values were used) when it arrives.
-__device__ __forceinline__ void gd_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// Orders the LDS traffic of one wave: what its lanes wrote before is seen by its lanes after.
-__device__ __forceinline__ void at_epilogue_wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <int WN, int WM, int GN, int GM, int BK, int NS, int SL>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM)
     __attribute__((amdgpu_waves_per_eu(GN * GM / 4, (WN * WM > 8 ? 1 : 2) * (GN * GM / 4))))
 gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, long ldw,
                 const float* __restrict__ bias, void* __restrict__ out, int out_dtype, long ldo, int M,
                 int N, int K, int act, int accumulate, int tiles_n, int tiles_m, int k_per) {
-    static_assert(BK == 32 || BK == 64, "K-steps of 32 or 64");
     // K cut into parts (grid y): part p multiplies the k_per columns from p * k_per on and writes
     // its sums as fp32 [M, N] of its own (the host passes the partial buffer as `out`, no bias,
     // no activation; a finishing kernel adds the parts up)
@@ -251,17 +187,8 @@ gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict
         K = min(k_per, K - part * k_per);
         out = reinterpret_cast<float*>(out) + (size_t)part * M * ldo;
     }
-    static_assert(NS >= 2 && NS <= 8, "two to eight stages");
-    static_assert(GN * GM == 4 || GN * GM == 8, "four or eight waves");
-    constexpr int WAVES = GN * GM;
-    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM;
-    constexpr int ROW = BK * 2;                          // bytes of a tile row
-    constexpr int CPR = BK / 8;                          // 16-byte chunks of a tile row
-    constexpr int RPL = KA_WAVE / CPR;                   // rows that one load of 1 KB brings
-    constexpr int STAGE = (BN + BM) * ROW;               // bytes of one stage: W rows, then X rows
-    constexpr int W_LOADS = BN / RPL / WAVES, X_LOADS = BM / RPL / WAVES;   // loads per wave and stage
-    static_assert(W_LOADS * RPL * WAVES == BN && X_LOADS * RPL * WAVES == BM, "the tile does not divide over the waves' loads");
-    constexpr int LPW = W_LOADS + X_LOADS;
+    using T = KdTile<WN, WM, GN, GM, BK, NS>;
+    constexpr int WAVES = T::WAVES, BN = T::BN, BM = T::BM, CPR = T::CPR, W_LOADS = T::W_LOADS, X_LOADS = T::X_LOADS;
     extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
     int pid = blockIdx.x;
     int total = tiles_n * tiles_m;
@@ -282,131 +209,23 @@ gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
 
-    // Chunk c of row r lies at place c ^ swizzle(r) of its row. One pass of a 16-byte LDS read
-    // serves 16 lanes, which here read the same chunk of 16 consecutive rows, and the 64 banks
-    // hold 256 bytes: two rows of 128 bytes, so rows of the same parity must differ in their
-    // place ((r >> 1) & 7), or four rows of 64 bytes ((r >> 2) & 3). (Measured with r & 7: half
-    // of the LDS cycles were bank conflicts, rows r and r + 8 meeting in one pass.)
-    auto swizzle = [](int r) { return CPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
-    // What this lane asks for in a load of RPL rows: row lane / CPR of them, and the chunk that
-    // belongs at place lane % CPR of that row.
-    const int lrow = lane / CPR;
+    // What this lane asks for in the wave's loads. Rows past the end of a matrix are read from its last row (and never stored).
     const bf16_t* wsrc[W_LOADS];
     const bf16_t* xsrc[X_LOADS];
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
-        int r = (wave * W_LOADS + i) * RPL + lrow;
-        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + ((lane % CPR) ^ swizzle(r)) * 8;
+        const int r = kd_load_row<CPR>(wave * W_LOADS + i, lane);
+        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + kd_load_channel<CPR>(r, lane);
     }
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) {
-        int r = (wave * X_LOADS + i) * RPL + lrow;
-        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + ((lane % CPR) ^ swizzle(r)) * 8;
+        const int r = kd_load_row<CPR>(wave * X_LOADS + i, lane);
+        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane);
     }
-    auto fetch = [&](int stage, int k0) {
-        unsigned char* base = gb_lds + stage * STAGE;
-#pragma unroll
-        for (int i = 0; i < W_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + k0),
-                                             (GD_LDS void*)(base + (wave * W_LOADS + i) * RPL * ROW), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < X_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + k0),
-                                             (GD_LDS void*)(base + BN * ROW + (wave * X_LOADS + i) * RPL * ROW), 16, 0, 0);
-    };
-
-    // operand addresses inside a stage: tile row li of each of this wave's tiles; the k-chunk
-    // of k-step ks is ks * 2 + lg
-    int wrow_off[WN], xrow_off[WM];
-#pragma unroll
-    for (int a = 0; a < WN; ++a) wrow_off[a] = (wn * 32 * WN + a * 32 + li) * ROW;
-#pragma unroll
-    for (int b = 0; b < WM; ++b) xrow_off[b] = BN * ROW + (wm * 32 * WM + b * 32 + li) * ROW;
-    const int swz = swizzle(li);
-
-    // The K-steps' operands are read from LDS a group of SL k-slices (of 16) at a time, one group
-    // ahead of the group that is being multiplied, also across the edge of a K-step: the MFMAs of a
-    // stage's last group run while the first group of the next stage is on its way from LDS, so the
-    // matrix pipes do not stand still at every K-step while both waves of a SIMD wait for LDS
-    // together. For that the barrier of a K-step stands before the last group's MFMAs: a wave
-    // arrives when its own loads of the next stage have landed and its own reads of this stage are
-    // in its registers. After the barrier everybody's have, so the next stage may be read and this
-    // stage's memory may be written: the load of stage s + NS goes out, and has NS - 1 K-steps to land.
-    constexpr int G = BK / 16 / SL;                      // groups per K-step
-    static_assert(G * SL * 16 == BK, "the groups of slices do not divide a K-step");
-    const int steps = K / BK;
-    // NS stages go out at once; the first has to be there before anything can be read
-#pragma unroll
-    for (int st = 0; st < NS; ++st)
-        if (st < steps) fetch(st, st * BK);
-    {
-        const int younger = min(NS - 1, steps - 1);
-        gd_wait_younger<LPW, NS - 1>(younger);
-        gd_barrier();
-    }
-    bf16x8 wa[2][SL][WN], xb[2][SL][WM];
-    auto operands = [&](auto slot_c, int stage, int g) {
-        constexpr int slot = decltype(slot_c)::value;
-        const unsigned char* base = gb_lds + (stage % NS) * STAGE;
-#pragma unroll
-        for (int i = 0; i < SL; ++i) {
-            const int place = (((g * SL + i) * 2 + lg) ^ swz) * 16;
-#pragma unroll
-            for (int a = 0; a < WN; ++a) wa[slot][i][a] = *reinterpret_cast<const bf16x8*>(base + wrow_off[a] + place);
-#pragma unroll
-            for (int b = 0; b < WM; ++b) xb[slot][i][b] = *reinterpret_cast<const bf16x8*>(base + xrow_off[b] + place);
-        }
-    };
-    const int groups = steps * G;
-    // group t (stage t / G, its group t % G) is multiplied from the registers of slot t & 1
-    auto group = [&](auto slot_c, int t) {
-        constexpr int slot = decltype(slot_c)::value;
-        const int st = t / G, g = t % G;
-        if (g == G - 1 && st + 1 < steps) {
-            // own loads of stage st + 1 landed (the stages after it may stay in flight), own reads of
-            // stage st done (they are the operands of this group, needed below in any case)
-            const int younger = min(NS - 2, steps - 2 - st);
-            gd_wait_younger<LPW, NS - 2>(younger);
-            gd_wait_lds();
-            gd_barrier();
-            if (st + NS < steps) fetch(st % NS, (st + NS) * BK);
-        }
-        // (always, also after the last group, whose "next" is read from memory nobody needs: a read
-        // under a condition makes the compiler wait for every read in flight before the MFMAs,
-        // the ones just asked for included)
-        operands(std::integral_constant<int, slot ^ 1>{}, (t + 1) / G, (t + 1) % G);
-#pragma unroll
-        for (int i = 0; i < SL; ++i)
-#pragma unroll
-            for (int a = 0; a < WN; ++a)
-#pragma unroll
-                for (int b = 0; b < WM; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[slot][i][a], xb[slot][i][b], acc[a][b], 0, 0, 0);
-        // The reads of the next group go out behind this group's second MFMA, into registers of
-        // their own, and have the rest of the group's MFMAs to arrive. (Left to itself the compiler
-        // gives both groups the same registers and asks for the next operands only after the
-        // MFMAs that use the present ones, three MFMAs before they are needed. Asked for ahead of
-        // the group's first MFMA they would be waited for at once: the compiler waits for every
-        // read in flight where this loop needs the older ones only.)
-        constexpr int FIRST = SL * WN * WM > 2 ? 2 : 1;
-        __builtin_amdgcn_sched_group_barrier(0x008, FIRST, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, SL * (WN + WM), 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, SL * WN * WM - FIRST, 0);
-    };
-    // (Nothing but LDS reads may be in flight on the counter they share with scalar loads when the
-    // loop is entered: with a scalar load among them the compiler can no longer count on arrival
-    // in order and waits, in every round, for all reads, the ones just asked for included.)
-    // (The arguments that only the epilogue uses are asked for here for the same reason: the
-    // compiler otherwise fetches them, with scalar loads, as late as it can.)
+    // (The arguments that only the epilogue uses are asked for here: the compiler otherwise fetches them, with scalar loads, as
+    // late as it can, and a scalar load in flight on the counter that LDS reads share makes the loop wait for all of them.)
     asm volatile("" ::"s"(bias), "s"(out), "s"(ldo), "s"(act), "s"(accumulate), "s"(out_dtype), "s"(M), "s"(N));
-    gd_wait_lds();
-    operands(std::integral_constant<int, 0>{}, 0, 0);
-    int t = 0;
-    for (; t + 1 < groups; t += 2) {
-        group(std::integral_constant<int, 0>{}, t);
-        group(std::integral_constant<int, 1>{}, t + 1);
-    }
-    if (t < groups) group(std::integral_constant<int, 0>{}, t);
+    kd_product<WN, WM, GN, GM, BK, NS, SL>(gb_lds, wave, lane, K, wsrc, xsrc, acc);
 
     // Epilogue. acc[a][b][v] is out[m][n] with n = n0 + wn*32*WN + a*32 + (v/4)*8 + lg*4 + v%4 and
     // m = m0 + wm*32*WM + b*32 + li: a lane holds four neighbouring outputs of one row, and one
@@ -419,8 +238,8 @@ gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict
     gd_barrier();                                        // the last stage has been read by everybody
     const bool bias_vec = (N % 4 == 0) && (reinterpret_cast<uintptr_t>(bias) % 16 == 0);
     auto staged = [&](auto* typed_out) {
-        using T = std::remove_pointer_t<decltype(typed_out)>;
-        constexpr int ES = sizeof(T);                    // 2 or 4
+        using E = std::remove_pointer_t<decltype(typed_out)>;
+        constexpr int ES = sizeof(E);                    // 2 or 4
         constexpr int PER = 16 / ES;                     // outputs per 16-byte store
         constexpr int RB = 32 * WN * ES;                 // bytes of a row of the wave's tile
         constexpr int RS = RB + (ES == 2 ? 8 : 16);      // its place in LDS: padded so that the lanes' writes spread over the banks
@@ -469,7 +288,7 @@ gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict
                 const int m = m_wave + b0 * 32 + rl, n = n_wave + c * PER;
                 if (lane < RPI * CH && rl < nb * 32 && m < M && n < N) {      // (a row's chunks need not divide 64 lanes)
                     const unsigned char* from = mine + rl * RS + c * 16;
-                    T* op = typed_out + (size_t)m * ldo + n;
+                    E* op = typed_out + (size_t)m * ldo + n;
                     if (wide && n + PER <= N) {
                         if constexpr (ES == 2) {
                             *reinterpret_cast<bf16x8*>(op) = *reinterpret_cast<const bf16x8*>(from);
@@ -482,7 +301,7 @@ gemm_dma_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict
                             *reinterpret_cast<floatx4*>(op) = x;
                         }
                     } else {
-                        const T* src = reinterpret_cast<const T*>(from);
+                        const E* src = reinterpret_cast<const E*>(from);
                         for (int i = 0; i < PER && n + i < N; ++i) {
                             if constexpr (ES == 2) op[i] = src[i];
                             else op[i] = accumulate ? op[i] + src[i] : src[i];

@@ -69,7 +69,8 @@ _SIGNATURES = {
                              _c_long, _c_void_p, _c_void_p],
     "ka_heads_linear_supported": [_c_long, _c_int, _c_long, _c_int, _c_int, _c_int],
     "ka_experts_gemm_supported": [_c_long, _c_int, _c_int, _c_long, _c_int, _c_int],
-    "ka_experts_gemm_bf16": [_c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
+    "ka_experts_gemm_tile": [_c_int] * 6,
+    "ka_experts_gemm_bf16": [_c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                              _c_float, _c_float, _c_void_p, _c_long, _c_int, _c_int, _c_void_p],
     "ka_experts_few_supported": [_c_int, _c_long, _c_int, _c_int, _c_int],
     "ka_experts_few_bf16": [_c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float,
@@ -164,6 +165,7 @@ def chip_sizes(device=None) -> ChipSizes:
 
 
 ACT_GATED = 0x100                  # (ops.linear.ACT_GATED)
+EXPERTS_LARGEST_TILE = 256         # list rows of the largest tile of the experts' linears
 
 _lib = None
 _scratch: Dict[int, torch.Tensor] = {}
@@ -192,8 +194,6 @@ def lib():
             getattr(handle, name).restype = _c_int
         handle.ka_attention_biased_supported.argtypes = [_c_int] * 3
         handle.ka_attention_biased_supported.restype = _c_int
-        handle.ka_experts_gemm_tile.argtypes = []
-        handle.ka_experts_gemm_tile.restype = _c_int
         handle.ka_attention_biased_query_block.argtypes = []
         handle.ka_attention_biased_query_block.restype = _c_int
         handle.ka_attention_decode_beside_supported.argtypes = [_c_int] * 6
@@ -978,12 +978,13 @@ def experts_few_bf16(h, pairs, down, chosen, hidden, y, act, clamp=None) -> bool
     return True
 
 
-def experts_feed_forward_bf16(h, pairs, down, chosen, hidden, y, act, workspace, clamp=None) -> bool:
+def experts_feed_forward_bf16(h, pairs, down, chosen, hidden, y, act, workspace, clamp=None, tile=None) -> bool:
     """Both linears of the chosen experts for all pairs of a step on the matrix cores, an expert's pairs together: the pairs
     are listed by expert (``ops.core.experts_sort``), the first linear (gated or not, as ``act`` says) gathers every pair's token from ``h`` ``[n, dim]`` and
     leaves the hidden rows in list order, the second writes fp32 ``y`` ``[n top, dim]`` at the pairs' own rows. ``pairs``
     ``[E, 2 hidden, dim]`` (not gated: ``[E, hidden, dim]``), ``down`` ``[E, dim, hidden]``, ``chosen`` int32 ``[n, top]``; ``hidden`` is not used (the list's hidden rows
-    live in the workspace). ``clamp`` (a ``GateClamp``): the pair's product is the clamped one. False: not covered (sizes that are no multiple of 16, alignment), nothing was run."""
+    live in the workspace). ``clamp`` (a ``GateClamp``): the pair's product is the clamped one. ``tile``: list rows of a tile (for tests; else
+    chosen by the sizes). False: not covered (sizes that are no multiple of 16, alignment), nothing was run."""
     n, top = chosen.shape
     n_experts, n_pair_rows, dim = pairs.shape
     ff = down.shape[2]
@@ -998,17 +999,19 @@ def experts_feed_forward_bf16(h, pairs, down, chosen, hidden, y, act, workspace,
         raise KernelError("experts: the first linear's rows do not fit the hidden size")
     if not handle.ka_experts_gemm_supported(lda, n_pair_rows, dim, ff, act, 0) or not handle.ka_experts_gemm_supported(ff, dim, ff, dim, 0, 1):
         return False
-    tile = int(handle.ka_experts_gemm_tile())
-    # (sized by the step's tokens alone: the same for every replay of a captured step)
+    tile = int(tile or handle.ka_experts_gemm_tile(n * top, n_experts, n_pair_rows, dim, act, dim))
+    # (sized by the step's tokens alone: the same for every replay of a captured step; the scratch tensors for the largest tile, so
+    # that a step of fewer tokens never asks for more)
     capacity = -(-(n * top + n_experts * (tile - 1)) // tile) * tile
     if capacity // tile > 65535:
         return False
-    listed = workspace.get("experts.sorted", (capacity,), torch.int32)
-    tile_expert = workspace.get("experts.tile_expert", (capacity // tile,), torch.int32)
-    rows = workspace.get("experts.hidden_listed", (capacity, ff), torch.bfloat16)
+    room = max(n * top + n_experts * (EXPERTS_LARGEST_TILE - 1), capacity)
+    listed = workspace.get("experts.sorted", (room,), torch.int32)[:capacity]
+    tile_expert = workspace.get("experts.tile_expert", (room,), torch.int32)[:capacity // tile]
+    rows = workspace.get("experts.hidden_listed", (room, ff), torch.bfloat16)
     core.experts_sort(chosen.view(-1), n_experts, tile, listed, tile_expert)
     _check(handle.ka_experts_gemm_bf16(h.data_ptr(), lda, top, pairs.data_ptr(), listed.data_ptr(), tile_expert.data_ptr(), capacity // tile,
-                                       n_pair_rows, dim, act, *core._clamp_args(clamp, act), rows.data_ptr(), ff, 0, 0, stream_ptr()))
+                                       tile, n_pair_rows, dim, act, *core._clamp_args(clamp, act), rows.data_ptr(), ff, 0, 0, stream_ptr()))
     _check(handle.ka_experts_gemm_bf16(rows.data_ptr(), ff, 0, down.data_ptr(), listed.data_ptr(), tile_expert.data_ptr(), capacity // tile,
-                                       dim, ff, 0, *core._clamp_args(None, 0), y.data_ptr(), dim, 1, 1, stream_ptr()))
+                                       tile, dim, ff, 0, *core._clamp_args(None, 0), y.data_ptr(), dim, 1, 1, stream_ptr()))
     return True
