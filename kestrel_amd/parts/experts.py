@@ -29,13 +29,16 @@ class RoutedExperts(FeedForward):
     step of up to ``PAIR_BY_PAIR_TO`` computes every pair by itself, its expert's weights streamed for it
     (``ops.core.experts_linear``; fp32 always does); up to ``FEW_PAIRS_TO`` every chosen expert's weights are streamed once past its pairs
     (``ops.fast.experts_few_bf16``); beyond, the pairs are listed by expert first and each expert's go through the matrix cores in
-    tiles (``ops.fast.experts_feed_forward_bf16``). Measured, both linears, 31 experts of 2,048 x 704: 4 tokens of 5 pairs 38, 38 and 94
-    us in this order, 8 tokens 62, 52 and 98, 32 tokens 201, 72 and 106, 96 tokens (480 pairs) -, 118 and 119. Either way a
+    tiles (``ops.fast.experts_feed_forward_bf16``); where width or hidden size is no multiple of 64 the tiles are the slower ones
+    and their turn comes at ``FEW_PAIRS_TO_UNALIGNED``. Measured, both linears, 31 experts of 2,048 x 704, choices of 5: 4 tokens 38 us pair
+    by pair, 38 streamed once, 8 tokens 62 and 56 (lists 61), 16 tokens 60 and 60 by lists, 32 tokens 69 and 66, 96 tokens 95 and 68; 62
+    experts of 4,096 x 896, choices of 6: 16 tokens 232 and 235, 24 tokens 268 and 251, 40 tokens 290 and 257 (5.3 TB/s). Either way a
     pair's result depends on its own row alone."""
 
     replays_every_step = True
     PAIR_BY_PAIR_TO = 20
-    FEW_PAIRS_TO = 512
+    FEW_PAIRS_TO = 128
+    FEW_PAIRS_TO_UNALIGNED = 512
 
     def __init__(self, spec: RoutedExpertsSpec) -> None:
         super().__init__(spec)
@@ -138,7 +141,8 @@ class RoutedExperts(FeedForward):
         if self.dtype == torch.bfloat16 and n * top > self.PAIR_BY_PAIR_TO:
             from ..ops import fast
             operands = (h, self.pairs, self.down, chosen, hidden, y, self.up_act)
-            done = n * top <= self.FEW_PAIRS_TO and fast.experts_few_bf16(*operands, clamp=self.clamp)
+            few_to = self.FEW_PAIRS_TO if spec.dim % 64 == 0 and spec.hidden_dim % 64 == 0 else self.FEW_PAIRS_TO_UNALIGNED
+            done = n * top <= few_to and fast.experts_few_bf16(*operands, clamp=self.clamp)
             done = done or fast.experts_feed_forward_bf16(*operands, ws, clamp=self.clamp)
         if not done:
             flat = chosen.view(-1)
