@@ -3,8 +3,10 @@
 // Plain FMA in fp32 with an LDS-tiled 64x64x16 block, any M, N, K, any mix of fp32
 // and bf16 operands. Every output element is the sum over k = 0..K-1 in that order,
 // whatever M and N are, so a row's result does not depend on what else is in the
-// batch. This is the true 32-bit path and the fallback of the bf16 path.
+// batch. This is the true 32-bit path and the fallback of the bf16 path. (Many rows, and few rows, of
+// aligned fp32 operands have kernels of their own below, each with its own fixed order of the sum.)
 #include "ka_common.h"
+#include "ka_dma_tiles.h"
 
 constexpr int GT = 64;   // tile edge in M and N
 constexpr int GK = 16;   // tile depth
@@ -66,6 +68,207 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
             out[o] = ka_from_float<TOut>(v);
         }
     }
+}
+
+// Many rows in fp32 where K is a multiple of 32: true fp32 products and sums on the matrix pipes (v_mfma_f32_32x32x2_f32, twice
+// the rate of the vector unit without packed FMAs), operands straight from memory into swizzled LDS as in ka_dma_tiles.h (a
+// K-step of 32 numbers is the same 128 bytes a row), two stages.
+//
+// The order of a sum is fixed by K alone: K is cut into F32_PARTS parts, each summed from zero in the order of its products
+// (of every eight k the order 0 4 1 5 2 6 3 7: a lane holds four neighbours), and the parts' sums are added in their order.
+// A part may therefore be anybody's: KG = 1, the waves walk over the parts one after the other; KG = 4, a workgroup has four
+// times the waves, each quarter multiplies its own part and the sums meet in LDS. The second fills the chip where tiles are few
+// (a prompt of some hundred rows), and its bits are those of the first.
+//
+// Measured, us, in the vector unit's kernel below -> here: 303 rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x 8,192 and 8,192 x
+// 2,048 254, 262, 276 and 1,006 -> 82, 41, 120 and 145; 2,048 rows 813, 267, 1,017 and 1,041 -> 459, 154, 623 and 604 (114 TFLOP/s of
+// the 157 that the pipes have). Error against 64 bits of such sums: 8.1e-7 -> 4.1e-7 (K = 8,192: 1.6e-6 -> 8.1e-7).
+constexpr int F32_PARTS = 4;
+constexpr int F32_STEP = 32;
+
+template <int WN, int WM, int GN, int GM, int KG>
+__global__ void __launch_bounds__(KA_WAVE * GN * GM * KG)
+gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
+                     float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
+    static_assert(KG == 1 || KG == F32_PARTS, "the parts one after the other, or one a group of waves");
+    constexpr int WAVES = GN * GM, BN = 32 * WN * GN, BM = 32 * WM * GM;
+    constexpr int ROW = F32_STEP * 4, CPR = 8, RPL = KA_WAVE / CPR, STAGE = (BN + BM) * ROW;
+    constexpr int W_LOADS = BN / RPL / WAVES, X_LOADS = BM / RPL / WAVES;
+    extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
+    const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8;
+    const int logical = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
+    if (logical >= total || (int)blockIdx.x / 8 >= per_xcd) return;
+    const int n0 = logical / tiles_m * BN, m0 = logical % tiles_m * BM;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    const int group = wave / WAVES, part_wave = wave % WAVES;
+    const int wn = part_wave / GM, wm = part_wave % GM, li = lane % 32, lg = lane / 32;
+    const float* wsrc[W_LOADS];
+    const float* xsrc[X_LOADS];
+#pragma unroll
+    for (int i = 0; i < W_LOADS; ++i) {
+        const int r = kd_load_row<CPR>(part_wave * W_LOADS + i, lane);
+        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + kd_load_channel<CPR>(r, lane) / 2;      // (four numbers a piece)
+    }
+#pragma unroll
+    for (int i = 0; i < X_LOADS; ++i) {
+        const int r = kd_load_row<CPR>(part_wave * X_LOADS + i, lane);
+        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2;
+    }
+    unsigned char* mine = gf_lds + group * 2 * STAGE;
+    auto fetch = [&](int stage, int k) {
+        unsigned char* base = mine + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < W_LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + k), (GD_LDS void*)(base + (part_wave * W_LOADS + i) * RPL * ROW), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < X_LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + k), (GD_LDS void*)(base + BN * ROW + (part_wave * X_LOADS + i) * RPL * ROW), 16, 0, 0);
+    };
+    const int swz = kd_swizzle<CPR>(li);
+    floatx16 acc[WN][WM], sum[WN][WM];
+    auto clear = [](floatx16 (&x)[WN][WM]) {
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) x[a][b][v] = 0.f;
+    };
+    clear(acc);
+    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP, k_steps = K / F32_STEP;
+    // this wave's steps: all of K, or its group's part
+    const int first = KG == 1 ? 0 : group * part_steps;
+    const int steps = max(0, min(KG == 1 ? k_steps : part_steps, k_steps - first));
+    const int rounds = KG == 1 ? k_steps : min(part_steps, k_steps);           // (the same for every wave: barriers)
+    if (steps > 0) fetch(0, first * F32_STEP);
+    int done = 0;                                                              // KG == 1: parts added into `sum`
+    for (int s = 0; s < rounds; ++s) {
+        gd_wait_loads<0>();                                                    // own loads of this step have landed
+        gd_wait_lds();                                                         // own reads of the step before are in registers
+        gd_barrier();
+        if (s + 1 < steps) fetch((s + 1) & 1, (first + s + 1) * F32_STEP);
+        if (s < steps) {
+            const unsigned char* base = mine + (s & 1) * STAGE;
+#pragma unroll
+            for (int g = 0; g < F32_STEP / 8; ++g) {
+                const int place = ((g * 2 + lg) ^ swz) * 16;
+                floatx4 w[WN], x[WM];
+#pragma unroll
+                for (int a = 0; a < WN; ++a) w[a] = *reinterpret_cast<const floatx4*>(base + ((wn * WN + a) * 32 + li) * ROW + place);
+#pragma unroll
+                for (int b = 0; b < WM; ++b) x[b] = *reinterpret_cast<const floatx4*>(base + (BN + (wm * WM + b) * 32 + li) * ROW + place);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int a = 0; a < WN; ++a)
+#pragma unroll
+                        for (int b = 0; b < WM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[a][j], x[b][j], acc[a][b], 0, 0, 0);
+            }
+        }
+        if (KG == 1 && (s + 1) % part_steps == 0 && s + 1 < rounds) {          // a part ends
+#pragma unroll
+            for (int a = 0; a < WN; ++a)
+#pragma unroll
+                for (int b = 0; b < WM; ++b)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sum[a][b][v] = done ? sum[a][b][v] + acc[a][b][v] : acc[a][b][v];
+            clear(acc);
+            ++done;
+        }
+    }
+    // acc[a][b][v] is out[m][n] with n = n0 + (wn WN + a) 32 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + (wm WM + b) 32 + li
+    const bool vectors = N % 4 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    auto store = [&](int a, int b, int q, const float (&y)[4]) {
+        const int m = m0 + (wm * WM + b) * 32 + li, n = n0 + (wn * WN + a) * 32 + q * 8 + lg * 4;
+        if (m >= M || n >= N) return;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = y[j] + (bias && n + j < N ? bias[n + j] : 0.f);
+        if (ka_act_gated(act)) {
+            ka_gated_store<false, 4>(out, KA_F32, ldo, m, n, N, v, act);
+            return;
+        }
+        if (act)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = ka_activate(act, v[j]);
+        float* op = out + (size_t)m * ldo + n;
+        if (vectors) {
+            floatx4 r = {v[0], v[1], v[2], v[3]};
+            if (accumulate) r = *reinterpret_cast<const floatx4*>(op) + r;
+            *reinterpret_cast<floatx4*>(op) = r;
+        } else {
+            for (int j = 0; j < 4 && n + j < N; ++j) op[j] = accumulate ? op[j] + v[j] : v[j];
+        }
+    };
+    if constexpr (KG == 1) {
+        gd_static_for<0, WN * WM * 4>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
+            float y[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = done ? sum[a][b][q * 4 + j] + acc[a][b][q * 4 + j] : acc[a][b][q * 4 + j];
+            store(a, b, q, y);
+        });
+    } else {
+        // the parts' sums through LDS; every group of waves finishes a quarter of the tile's numbers
+        gd_wait_lds();
+        gd_barrier();
+        float* sums = reinterpret_cast<float*>(gf_lds);
+        gd_static_for<0, WN * WM * 4>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
+            *reinterpret_cast<floatx4*>(sums + (((group * WAVES + part_wave) * WN * WM * 4 + i) * KA_WAVE + lane) * 4) =
+                floatx4{acc[a][b][q * 4], acc[a][b][q * 4 + 1], acc[a][b][q * 4 + 2], acc[a][b][q * 4 + 3]};
+        });
+        gd_wait_lds();
+        gd_barrier();
+        const int parts = (k_steps + part_steps - 1) / part_steps;             // (those that hold anything)
+        gd_static_for<0, WN * WM>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const int at = i * 4 + group;
+            floatx4 y = *reinterpret_cast<const floatx4*>(sums + ((part_wave * WN * WM * 4 + at) * KA_WAVE + lane) * 4);
+            for (int p = 1; p < parts; ++p) y += *reinterpret_cast<const floatx4*>(sums + (((p * WAVES + part_wave) * WN * WM * 4 + at) * KA_WAVE + lane) * 4);
+            const float v[4] = {y[0], y[1], y[2], y[3]};
+            store(i / WM, i % WM, group, v);
+        });
+    }
+}
+
+template <int WN, int WM, int GN, int GM, int KG>
+static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+                           int act, int accumulate, hipStream_t stream) {
+    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * 2 * (BN + BM) * F32_STEP * 4;
+    static bool configured = false;
+    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        KA_CHECK(e == hipSuccess, "ka_linear_generic: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+        configured = true;
+    }
+    const int tiles_n = ka_cdiv(N, BN), tiles_m = ka_cdiv(M, BM);
+    const long blocks = ((long)tiles_n * tiles_m + 7) / 8 * 8;
+    KA_CHECK(blocks < (1L << 31), "ka_linear_generic: too many tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * GN * GM * KG), smem, stream, A, lda, W, ldw, bias, out, ldo, M, N, K, act,
+                       accumulate, tiles_n, tiles_m);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// The tile: the one that takes the fewest blocks of 32 x 32 x K one after the other on the fullest CU, weighed by the rate the
+// tile reaches where CUs are full (TFLOP/s: smaller tiles read L2 and LDS more often per product). All give the same bits.
+//   303 rows of 2,048 x 6,144: 150 us with 64 x 128, 82 with 64 x 64, 94 with 64 x 32, 96 with 32 x 32;
+//   157 rows of 2,048 x 6,144: 93, 82, 50, 54;  17 rows of 2,048 x 2,048: 88, 40, 24, 19;
+//   2,048 rows of 8,192 x 2,048: 604, 630, 683, 766 (128 x 128: 641).
+static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+                           int act, int accumulate, hipStream_t stream) {
+    const int cus = ka_compute_units();
+    auto cost = [&](int bn, int bm, float rate) { return ka_cdiv((long)ka_cdiv(N, bn) * ka_cdiv(M, bm), cus) * (float)(bn * bm) / rate; };
+    const float t128 = cost(64, 128, 112.f), t64 = cost(64, 64, 104.f), t32 = cost(64, 32, 90.f), t1 = cost(32, 32, 85.f);
+    const float best = fminf(fminf(t128, t64), fminf(t32, t1));
+#define KA_F32(...) return launch_f32_mfma<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
+    if (t128 <= best) KA_F32(1, 2, 2, 2, 1);
+    if (t64 <= best) KA_F32(1, 2, 2, 1, F32_PARTS);
+    if (t32 <= best) KA_F32(1, 1, 2, 1, F32_PARTS);
+    KA_F32(1, 1, 1, 1, F32_PARTS);
+#undef KA_F32
 }
 
 // Many rows in fp32 (prompts on the 32-bit path): the same sums, k in ascending order for every
@@ -156,48 +359,109 @@ gemm_f32_kernel(const float* __restrict__ A, long lda, const float* __restrict__
     }
 }
 
-// Few rows in fp32 (decoding on the 32-bit path): the tile above would put a sixteenth of its
-// threads to work and read every weight through LDS. Here a wave owns one output column: its
-// lanes walk over K with 16-byte loads of the weight row and of each activation row, every lane
-// adds up its own k in their order, and the lanes' sums meet in a fixed tree. Plain fp32 FMA as
-// above; the order of a sum is another than the tile's, the same for every M and N.
+// Few rows in fp32 (decoding on the 32-bit path): the tiles above would put a sixteenth of their threads to work and read every
+// weight through LDS. Here a wave owns C output columns: its lanes walk over K with 16-byte loads of the weight rows and of each
+// activation row, every lane adds up its own k in their order, and the lanes' sums meet in a fixed tree. The order of a sum
+// is the same for every M and N.
+//
+// What bounds it is the stream of weights. Four steps of it are asked for at once (without a branch between them: the loads of a
+// loop over the rows that are there are not hoisted over each other), and a step's activations, which come from the CU's cache,
+// serve all C columns. Measured, us, before -> now, three rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x 8,192, 8,192 x 2,048 and the
+// head of 2,048 x 51,200: 14.3, 11.0, 23.5, 35.8 and 124 -> 12.7, 6.7, 16.5, 19.6 and 79; one row 11.1, 8.9, 15.7, 22.4 and 78 -> 10.1,
+// 4.6, 12.6, 12.5 (5.4 TB/s) and 64.
 constexpr int GV_ROWS = 16;      // most rows
-constexpr int GV_WAVES = 4;      // output columns per workgroup
+constexpr int GV_WAVES = 4;      // waves per workgroup
 
 typedef __attribute__((ext_vector_type(4))) float gv_float4;
 
+template <int MB, int C>
 __global__ void __launch_bounds__(GV_WAVES * KA_WAVE)
 gemv_f32_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
                 const float* __restrict__ bias, float* __restrict__ out, long ldo, int M, int N, int K, int act,
                 int accumulate) {
+    constexpr int STEP = KA_WAVE * 4, U = 4;
+    constexpr int UA = MB <= 4 ? U : MB <= 8 ? 2 : 1;        // steps whose activations are asked for at once
     const int wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
-    const int n = blockIdx.x * GV_WAVES + wave;
-    if (n >= N) return;
-    const float* wrow = W + (size_t)n * ldw;
-    float acc[GV_ROWS];
+    const int n0 = (blockIdx.x * GV_WAVES + wave) * C;
+    if (n0 >= N) return;
+    const float* w[C];
 #pragma unroll
-    for (int m = 0; m < GV_ROWS; ++m) acc[m] = 0.f;
-    for (int k = lane * 4; k < K; k += KA_WAVE * 4) {
-        const gv_float4 w = *reinterpret_cast<const gv_float4*>(wrow + k);
+    for (int c = 0; c < C; ++c) w[c] = W + (size_t)min(n0 + c, N - 1) * ldw + lane * 4;       // (columns past the end: not stored)
+    const float* a[MB];
 #pragma unroll
-        for (int m = 0; m < GV_ROWS; ++m) {
-            if (m < M) {
-                const gv_float4 a = *reinterpret_cast<const gv_float4*>(A + (size_t)m * lda + k);
-                acc[m] = fmaf(a[3], w[3], fmaf(a[2], w[2], fmaf(a[1], w[1], fmaf(a[0], w[0], acc[m]))));
+    for (int m = 0; m < MB; ++m) a[m] = A + (size_t)min(m, M - 1) * lda + lane * 4;           // (rows past the end: not stored)
+    float acc[C][MB];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int m = 0; m < MB; ++m) acc[c][m] = 0.f;
+    auto add = [&](const gv_float4 (&x)[C], const gv_float4 (&y)[MB]) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+                acc[c][m] = fmaf(y[m][3], x[c][3], fmaf(y[m][2], x[c][2], fmaf(y[m][1], x[c][1], fmaf(y[m][0], x[c][0], acc[c][m]))));
+    };
+    int k = 0;
+    for (; k + U * STEP <= K; k += U * STEP) {
+        gv_float4 x[U][C];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int c = 0; c < C; ++c) x[u][c] = __builtin_nontemporal_load(reinterpret_cast<const gv_float4*>(w[c] + k + u * STEP));
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += UA) {
+            gv_float4 y[UA][MB];
+#pragma unroll
+            for (int u = 0; u < UA; ++u)
+#pragma unroll
+                for (int m = 0; m < MB; ++m) y[u][m] = *reinterpret_cast<const gv_float4*>(a[m] + k + (u0 + u) * STEP);
+#pragma unroll
+            for (int u = 0; u < UA; ++u) add(x[u0 + u], y[u]);
+        }
+    }
+    for (; k + lane * 4 < K; k += STEP) {
+        gv_float4 x[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) x[c] = *reinterpret_cast<const gv_float4*>(w[c] + k);
+        gv_float4 y[MB];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) y[m] = *reinterpret_cast<const gv_float4*>(a[m] + k);
+        add(x, y);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            float v = ka_wave_sum(acc[c][m]);
+            if (lane == 0 && m < M && n0 + c < N) {
+                v += bias ? bias[n0 + c] : 0.f;
+                if (act) v = ka_activate(act, v);
+                const size_t o = (size_t)m * ldo + n0 + c;
+                out[o] = accumulate ? out[o] + v : v;
             }
         }
     }
-#pragma unroll
-    for (int m = 0; m < GV_ROWS; ++m) {
-        if (m >= M) break;
-        float v = ka_wave_sum(acc[m]);
-        if (lane == 0) {
-            v += bias ? bias[n] : 0.f;
-            if (act) v = ka_activate(act, v);
-            const size_t o = (size_t)m * ldo + n;
-            out[o] = accumulate ? out[o] + v : v;
-        }
-    }
+}
+
+template <int MB, int C>
+static void launch_gemv_form(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+                             int act, int accumulate, hipStream_t stream) {
+    hipLaunchKernelGGL((gemv_f32_kernel<MB, C>), dim3(ka_cdiv(N, C * GV_WAVES)), dim3(GV_WAVES * KA_WAVE), 0, stream, A, lda, W, ldw, bias, out,
+                       ldo, M, N, K, act, accumulate);
+}
+
+// Columns a wave: more of them ask the cache for fewer activations, fewer of them leave more waves to wait for memory. Two are
+// best over most of the range; one where there are less than 16 waves a CU and at most four rows (2,048 columns of 8,192 at three
+// rows: 19.6 us, 22.5 with two, 22.8 with four), four from eight rows and 32 waves a CU on (51,200 x 2,048 at sixteen rows:
+// 210, 228 with two, 306 with one).
+template <int MB>
+static void launch_gemv(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K, int act,
+                        int accumulate, hipStream_t stream) {
+    const int cus = ka_compute_units();
+    if (MB <= 4 && N < 16 * cus) launch_gemv_form<MB, 1>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
+    else if (MB >= 8 && N >= 32 * cus) launch_gemv_form<MB, 4>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
+    else launch_gemv_form<MB, 2>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
 }
 
 template <typename TA, typename TW, typename TOut>
@@ -224,6 +488,9 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
     int key = a_dtype * 4 + w_dtype * 2 + out_dtype;
     const bool vectors = key == 0 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 &&
                          (uintptr_t)W % 16 == 0;
+    if (vectors && M > GV_ROWS && K % F32_STEP == 0) {
+        return launch_f32_best((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream);
+    }
     if (vectors && M > GV_ROWS && ka_cdiv(M, 64) <= 65535) {
         if ((long)ka_cdiv(N, GF) * ka_cdiv(M, GF) >= 512)
             hipLaunchKernelGGL(gemm_f32_kernel<8>, dim3(ka_cdiv(N, GF), ka_cdiv(M, GF)), dim3(256), 0, stream, (const float*)A, lda,
@@ -235,8 +502,13 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
         return 0;
     }
     if (vectors && M <= GV_ROWS && !ka_act_gated(act)) {      // (a wave per column there: the pair of a gate would meet nowhere)
-        hipLaunchKernelGGL(gemv_f32_kernel, dim3(ka_cdiv(N, GV_WAVES)), dim3(GV_WAVES * KA_WAVE), 0, stream,
-                           (const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate);
+#define KA_GEMV(MB) launch_gemv<MB>((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream)
+        if (M <= 1) KA_GEMV(1);
+        else if (M <= 2) KA_GEMV(2);
+        else if (M <= 4) KA_GEMV(4);
+        else if (M <= 8) KA_GEMV(8);
+        else KA_GEMV(16);
+#undef KA_GEMV
         KA_LAUNCH_CHECK();
         return 0;
     }
