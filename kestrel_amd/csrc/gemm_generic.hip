@@ -74,15 +74,17 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 // the rate of the vector unit without packed FMAs), operands straight from memory into swizzled LDS as in ka_dma_tiles.h (a
 // K-step of 32 numbers is the same 128 bytes a row), two stages.
 //
-// The order of a sum is fixed by K alone: K is cut into F32_PARTS parts, each summed from zero in the order of its products
-// (of every eight k the order 0 4 1 5 2 6 3 7: a lane holds four neighbours), and the parts' sums are added in their order.
-// A part may therefore be anybody's: KG = 1, the waves walk over the parts one after the other; KG = 4, a workgroup has four
-// times the waves, each quarter multiplies its own part and the sums meet in LDS. The second fills the chip where tiles are few
-// (a prompt of some hundred rows), and its bits are those of the first.
+// The order of a sum is fixed by K alone. Every sixteen k are summed from zero (of every eight in the order 0 4 1 5 2 6 3 7: a lane
+// holds four neighbours), these sums are added in order within a part, K being cut into F32_PARTS parts, and the parts' sums
+// are added in their order. The short chains cost 5 to 8 % (an addition on the vector unit per eight products) and take the
+// error of a sum from that of a chain of K / 4 terms to that of one of K / 64.
+// A part may be anybody's: KG = 1, the waves walk over the parts one after the other; KG = 4, a workgroup has four times the waves,
+// each quarter multiplies its own part and the sums meet in LDS. The second fills the chip where tiles are few (a prompt of some
+// hundred rows), and its bits are those of the first.
 //
 // Measured, us, in the vector unit's kernel below -> here: 303 rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x 8,192 and 8,192 x
-// 2,048 254, 262, 276 and 1,006 -> 82, 41, 120 and 145; 2,048 rows 813, 267, 1,017 and 1,041 -> 459, 154, 623 and 604 (114 TFLOP/s of
-// the 157 that the pipes have). Error against 64 bits of such sums: 8.1e-7 -> 4.1e-7 (K = 8,192: 1.6e-6 -> 8.1e-7).
+// 2,048 254, 262, 276 and 1,006 -> 95, 43, 138 and 152; 2,048 rows 813, 267, 1,017 and 1,041 -> 484, 164, 666 and 649 (107 TFLOP/s of
+// the 157 that the pipes have). Error against 64 bits of such sums: 8.1e-7 -> 1.4e-7 (K = 8,192: 1.6e-6 -> 2.2e-7).
 constexpr int F32_PARTS = 4;
 constexpr int F32_STEP = 32;
 
@@ -150,19 +152,25 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
         if (s < steps) {
             const unsigned char* base = mine + (s & 1) * STAGE;
 #pragma unroll
-            for (int g = 0; g < F32_STEP / 8; ++g) {
-                const int place = ((g * 2 + lg) ^ swz) * 16;
-                floatx4 w[WN], x[WM];
+            for (int g = 0; g < F32_STEP / 16; ++g) {
+                floatx4 w[2][WN], x[2][WM];
 #pragma unroll
-                for (int a = 0; a < WN; ++a) w[a] = *reinterpret_cast<const floatx4*>(base + ((wn * WN + a) * 32 + li) * ROW + place);
+                for (int h = 0; h < 2; ++h) {
+                    const int place = (((g * 2 + h) * 2 + lg) ^ swz) * 16;
 #pragma unroll
-                for (int b = 0; b < WM; ++b) x[b] = *reinterpret_cast<const floatx4*>(base + (BN + (wm * WM + b) * 32 + li) * ROW + place);
+                    for (int a = 0; a < WN; ++a) w[h][a] = *reinterpret_cast<const floatx4*>(base + ((wn * WN + a) * 32 + li) * ROW + place);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                    for (int b = 0; b < WM; ++b) x[h][b] = *reinterpret_cast<const floatx4*>(base + (BN + (wm * WM + b) * 32 + li) * ROW + place);
+                }
 #pragma unroll
-                    for (int a = 0; a < WN; ++a)
+                for (int a = 0; a < WN; ++a)
 #pragma unroll
-                        for (int b = 0; b < WM; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[a][j], x[b][j], acc[a][b], 0, 0, 0);
+                    for (int b = 0; b < WM; ++b) {
+                        floatx16 few = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) few = __builtin_amdgcn_mfma_f32_32x32x2f32(w[j / 4][a][j % 4], x[j / 4][b][j % 4], few, 0, 0, 0);
+                        acc[a][b] += few;
+                    }
             }
         }
         if (KG == 1 && (s + 1) % part_steps == 0 && s + 1 < rounds) {          // a part ends
@@ -254,9 +262,8 @@ static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, c
 
 // The tile: the one that takes the fewest blocks of 32 x 32 x K one after the other on the fullest CU, weighed by the rate the
 // tile reaches where CUs are full (TFLOP/s: smaller tiles read L2 and LDS more often per product). All give the same bits.
-//   303 rows of 2,048 x 6,144: 150 us with 64 x 128, 82 with 64 x 64, 94 with 64 x 32, 96 with 32 x 32;
-//   157 rows of 2,048 x 6,144: 93, 82, 50, 54;  17 rows of 2,048 x 2,048: 88, 40, 24, 19;
-//   2,048 rows of 8,192 x 2,048: 604, 630, 683, 766 (128 x 128: 641).
+// (us with 64 x 128, 64 x 64, 64 x 32 and 32 x 32 before the sums were cut into sixteens: 303 rows of 2,048 x 6,144 150, 82, 94,
+// 96; 157 rows 93, 82, 50, 54; 17 rows of 2,048 x 2,048 88, 40, 24, 19; 2,048 rows of 8,192 x 2,048 604, 630, 683, 766.)
 static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
     const int cus = ka_compute_units();
