@@ -337,6 +337,22 @@ KA_API int ka_decayed_memory_supported(int d) {
     return decay_shape(d, &ni, &parts) ? 1 : 0;
 }
 
+// The read-outs of ka_decayed_memory from fp32 `raw` [n, H d]: norm, gain and gate.
+KA_API int ka_decayed_readout(const float* raw, const void* gate, long stride, int dtype, const float* gain, void* out, long out_stride, int n,
+                              int H, int d, float eps, hipStream_t stream) {
+    KA_CHECK(n >= 0 && H > 0 && d > 0 && eps >= 0.f && (dtype == KA_F32 || dtype == KA_BF16), "ka_decayed_readout: bad sizes or dtype %d", dtype);
+    if (n == 0) return 0;
+    const int pairs = n * H;
+    if (dtype == KA_F32)
+        hipLaunchKernelGGL(decayed_readout_kernel<float>, dim3((pairs + 3) / 4), dim3(256), 0, stream, raw, gain, (const float*)gate, stride,
+                           (float*)out, out_stride, n, H, d, eps);
+    else
+        hipLaunchKernelGGL(decayed_readout_kernel<bf16_t>, dim3((pairs + 3) / 4), dim3(256), 0, stream, raw, gain, (const bf16_t*)gate, stride,
+                           (bf16_t*)out, out_stride, n, H, d, eps);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
 // raw: fp32 scratch [n, H d] of the caller's.
 KA_API int ka_decayed_memory(const void* r, const void* k, const void* v, const void* gate, long stride, int dtype, const float* pre,
                              const float* u, const float* gain, float* state, long state_stride, const float* x, int dim,
@@ -376,13 +392,5 @@ KA_API int ka_decayed_memory(const void* r, const void* k, const void* v, const 
 #undef RP_LAUNCH_ALL
 #undef RP_LAUNCH
     KA_LAUNCH_CHECK();
-    const int pairs = n * H;
-    if (dtype == KA_F32)
-        hipLaunchKernelGGL(decayed_readout_kernel<float>, dim3((pairs + 3) / 4), dim3(256), 0, stream, raw, gain, (const float*)gate, stride,
-                           (float*)out, out_stride, n, H, d, eps);
-    else
-        hipLaunchKernelGGL(decayed_readout_kernel<bf16_t>, dim3((pairs + 3) / 4), dim3(256), 0, stream, raw, gain, (const bf16_t*)gate, stride,
-                           (bf16_t*)out, out_stride, n, H, d, eps);
-    KA_LAUNCH_CHECK();
-    return 0;
+    return ka_decayed_readout(raw, gate, stride, dtype, gain, out, out_stride, n, H, d, eps, stream);
 }

@@ -68,6 +68,7 @@ _SIGNATURES = {
     "ka_decayed_memory": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                           _c_long, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_float,
                           _c_void_p, _c_void_p],
+    "ka_decayed_readout": [_c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     "ka_route": [_c_void_p, _c_long, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p, _c_void_p,
                  _c_void_p],
     "ka_experts_linear": [_c_void_p, _c_long, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
@@ -908,16 +909,8 @@ def decayed_memory_supported(head_dim: int) -> bool:
     return bool(lib().ka_decayed_memory_supported(int(head_dim)))
 
 
-def decayed_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, pre: torch.Tensor, u: torch.Tensor,
-                   gain: torch.Tensor, state: torch.Tensor, x: Optional[torch.Tensor], cu_q: torch.Tensor, row_slot: torch.Tensor,
-                   out: torch.Tensor, n_heads: int, head_dim: int, eps: float, raw: Optional[torch.Tensor] = None) -> None:
-    """A decaying matrix memory over the packed tokens of a step. Per head a state ``S`` ``[d, d]``; for every token of a row, in
-    order: ``o_j = sum_i r_i (S_ij + u_i k_i v_j)``, then ``S_ij <- exp(-exp(pre_i)) S_ij + k_i v_j``; ``o`` divided by its root mean
-    square over the head (``eps``), times ``gain``, times ``gate``. ``r, k, v, gate``: ``[n, H d]`` views of one type with one
-    row stride; ``pre`` fp32 ``[n, H d]``; ``u``, ``gain`` fp32 ``[H d]``; ``state`` fp32 ``[slots + 1, H d d + dim]``, a row per
-    request slot: the matrices, then the stream's last row (``x`` fp32 ``[n, dim]``, kept for the next step's token shift;
-    ``None``: the rows hold the matrices alone). A row of the step without a request writes zeros and touches no state.
-    ``raw``: fp32 scratch ``[n, H d]`` for the read-outs before their norm (a captured step passes its workspace's)."""
+def check_decayed_memory(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, out, n_heads: int, head_dim: int):
+    """Refuses operands that do not fit the decaying memory's kernels; ``(tokens, rows, dim of x)``."""
     _dev(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, out)
     n = r.shape[0]
     width = n_heads * head_dim
@@ -934,6 +927,21 @@ def decayed_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torc
     n_rows = row_slot.numel()
     _need(cu_q.dtype == torch.int32 and cu_q.numel() == n_rows + 1 and row_slot.dtype == torch.int32, "decayed_memory: cu_q int32 [rows + 1]")
     _need(out.dtype == r.dtype and out.dim() == 2 and out.stride(1) == 1 and tuple(out.shape) == (n, width), "decayed_memory: out [n, H d]")
+    return n, n_rows, dim
+
+
+def decayed_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, pre: torch.Tensor, u: torch.Tensor,
+                   gain: torch.Tensor, state: torch.Tensor, x: Optional[torch.Tensor], cu_q: torch.Tensor, row_slot: torch.Tensor,
+                   out: torch.Tensor, n_heads: int, head_dim: int, eps: float, raw: Optional[torch.Tensor] = None) -> None:
+    """A decaying matrix memory over the packed tokens of a step. Per head a state ``S`` ``[d, d]``; for every token of a row, in
+    order: ``o_j = sum_i r_i (S_ij + u_i k_i v_j)``, then ``S_ij <- exp(-exp(pre_i)) S_ij + k_i v_j``; ``o`` divided by its root mean
+    square over the head (``eps``), times ``gain``, times ``gate``. ``r, k, v, gate``: ``[n, H d]`` views of one type with one
+    row stride; ``pre`` fp32 ``[n, H d]``; ``u``, ``gain`` fp32 ``[H d]``; ``state`` fp32 ``[slots + 1, H d d + dim]``, a row per
+    request slot: the matrices, then the stream's last row (``x`` fp32 ``[n, dim]``, kept for the next step's token shift;
+    ``None``: the rows hold the matrices alone). A row of the step without a request writes zeros and touches no state.
+    ``raw``: fp32 scratch ``[n, H d]`` for the read-outs before their norm (a captured step passes its workspace's)."""
+    n, n_rows, dim = check_decayed_memory(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, out, n_heads, head_dim)
+    width = n_heads * head_dim
     if raw is None:
         raw = torch.empty((n, width), dtype=torch.float32, device=r.device)
     _need(raw.dtype == torch.float32 and raw.is_contiguous() and raw.numel() >= n * width and raw.is_cuda, "decayed_memory: raw fp32 [n, H d]")
@@ -941,6 +949,17 @@ def decayed_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torc
                                    code_of(r.dtype), pre.data_ptr(), u.data_ptr(), gain.data_ptr(), state.data_ptr(), state.stride(0),
                                    _ptr(x), dim, cu_q.data_ptr(), row_slot.data_ptr(), out.data_ptr(),
                                    out.stride(0) if n > 1 else width, n, n_rows, n_heads, head_dim, float(eps), raw.data_ptr(), stream_ptr()))
+
+
+def decayed_readout(raw: torch.Tensor, gate: torch.Tensor, gain: torch.Tensor, out: torch.Tensor, n_heads: int, head_dim: int, eps: float) -> None:
+    """The read-outs of ``decayed_memory`` from fp32 ``raw`` ``[n, H d]``: every head over its root mean square, times gain and gate."""
+    _dev(raw, gate, gain, out)
+    n, width = out.shape[0], n_heads * head_dim
+    _need(raw.dtype == torch.float32 and raw.is_contiguous() and tuple(raw.shape) == (n, width) and tuple(out.shape) == (n, width) and out.stride(1) == 1
+          and gate.dtype == out.dtype and tuple(gate.shape) == (n, width) and gate.stride(1) == 1 and gain.dtype == torch.float32
+          and gain.is_contiguous() and gain.numel() == width, "decayed_readout: raw fp32, gate and out [n, H d], gain fp32 [H d]")
+    _check(lib().ka_decayed_readout(raw.data_ptr(), gate.data_ptr(), gate.stride(0) if n > 1 else width, code_of(out.dtype), gain.data_ptr(),
+                                    out.data_ptr(), out.stride(0) if n > 1 else width, n, n_heads, head_dim, float(eps), stream_ptr()))
 
 
 ROUTER_SCORES = {"softmax": 0, "sigmoid": 2}

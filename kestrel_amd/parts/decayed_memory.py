@@ -33,10 +33,12 @@ class DecayedMemory(Mixer):
     activation type. The five projections are linears of that type; the second linear of the decay writes fp32 (with
     ``w0`` as its bias) and the exponentials are taken in the recurrence kernel, so that everything that enters the
     recurrence besides the projections is fp32. One kernel walks over every row's tokens in order and a second normalises the read-outs
-    (``ops.core.decayed_memory``), whatever the step holds: a prompt, a portion, single tokens. Rows without a request
+    (``ops.core.decayed_memory``): single tokens, every step in float32, heads that the chunks do not take. Prompts and portions in
+    bfloat16 go by chunks of 64 tokens over the matrix cores (``ops.fast.decayed_chunks_bf16``). Rows without a request
     (the padding of a replayed step) write zeros and touch no state."""
 
     replays_every_step = True
+    CHUNKS_FROM_TOKENS = 65      # (64 tokens of one row: 27 us one by one, 34 by chunks; 512: 157 and 36)
     reads_stream = True
 
     def __init__(self, spec: DecayedMemorySpec) -> None:
@@ -100,8 +102,14 @@ class DecayedMemory(Mixer):
         out = ws.get("decay.out", (n, self.width), self.dtype)
         r, k, v, g = (rkvg[:, i * self.width:(i + 1) * self.width] for i in range(4))
         raw = ws.get("decay.raw", (n, self.width), torch.float32)
-        core.decayed_memory(r, k, v, g, pre, self.u, self.gain, state, x, batch.cu_q, batch.row_slot, out, spec.n_heads,
-                            spec.head_dim, spec.eps, raw=raw)
+        operands = (r, k, v, g, pre, self.u, self.gain, state, x, batch.cu_q, batch.row_slot, out, spec.n_heads, spec.head_dim, spec.eps)
+        if self.dtype == torch.bfloat16 and not batch.decode_only and n >= self.CHUNKS_FROM_TOKENS:
+            # (sized by the host side of the batch alone: the same for every replay of a captured step)
+            from ..ops import fast
+            need = fast.gated_chunks_scratch(n, batch.n_rows, spec.n_heads, spec.head_dim, spec.head_dim)
+            if need and fast.decayed_chunks_bf16(*operands, raw, ws.get("decay.chunks", (need,), torch.float32)):
+                return out
+        core.decayed_memory(*operands, raw=raw)
         return out
 
     def output_projection(self):
