@@ -314,12 +314,12 @@ KA_API int ka_experts_combine(const float* y, const void* h, long h_stride, int 
 // added into the fp32 stream x, and the norm of the new rows is computed, in the same launch (ka_rows.h). A workgroup
 // per token; the sums are those of ka_experts_combine, in its order.
 // ----------------------------------------------------------------------------
-template <typename T, int PIECES>
-__global__ void __launch_bounds__(KA_ROW_THREADS)
+template <typename T, int PIECES, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 experts_combine_normed_kernel(const float* __restrict__ y, const T* __restrict__ h_in, long h_stride, const int* __restrict__ chosen,
                               const float* __restrict__ weights, int top, int E, const float* __restrict__ shared,
                               const float* __restrict__ shared_gate, long gate_stride, float* __restrict__ x, int dim, KaRowNorms a) {
-    __shared__ float smem[KA_ROW_WAVES];
+    __shared__ float smem[THREADS / KA_WAVE];
     const int t = blockIdx.x;
     const float sg = shared ? (shared_gate ? 1.0f / (1.0f + expf(-shared_gate[(size_t)t * gate_stride])) : 1.f) : 0.f;
     auto one = [&](int c) {
@@ -331,33 +331,44 @@ experts_combine_normed_kernel(const float* __restrict__ y, const T* __restrict__
         }
         return shared ? fmaf(sg, shared[(size_t)t * dim + c], acc) : acc;
     };
+    // (everything a piece needs is asked for at once, eight choices at a time and nothing behind a branch; an identity expert has a
+    // row in `y` too, which is not used)
     auto piece = [&](int c) {
+        const T* hp = h_in + (size_t)t * h_stride + c;
+        const float4 own = make_float4(ka_to_float(hp[0]), ka_to_float(hp[1]), ka_to_float(hp[2]), ka_to_float(hp[3]));
+        const float4 common = shared ? *reinterpret_cast<const float4*>(shared + (size_t)t * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        constexpr int AHEAD = PIECES == 1 ? 8 : 4;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k = 0; k < top; ++k) {
-            const int e = chosen[(size_t)t * top + k];
-            const float w = weights[(size_t)t * top + k];
-            float4 v;
-            if (e < E) {
-                v = *reinterpret_cast<const float4*>(y + ((size_t)t * top + k) * dim + c);
-            } else {
-                const T* hp = h_in + (size_t)t * h_stride + c;
-                v = make_float4(ka_to_float(hp[0]), ka_to_float(hp[1]), ka_to_float(hp[2]), ka_to_float(hp[3]));
+        for (int k0 = 0; k0 < top; k0 += AHEAD) {
+            float4 v[AHEAD];
+            float w[AHEAD];
+            bool has[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const size_t at = (size_t)t * top + min(k0 + k, top - 1);
+                w[k] = weights[at];
+                has[k] = chosen[at] < E;
+                v[k] = *reinterpret_cast<const float4*>(y + at * dim + c);
             }
-            acc.x = fmaf(w, v.x, acc.x);
-            acc.y = fmaf(w, v.y, acc.y);
-            acc.z = fmaf(w, v.z, acc.z);
-            acc.w = fmaf(w, v.w, acc.w);
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                if (k0 + k >= top) continue;
+                const float4 z = has[k] ? v[k] : own;
+                acc.x = fmaf(w[k], z.x, acc.x);
+                acc.y = fmaf(w[k], z.y, acc.y);
+                acc.z = fmaf(w[k], z.z, acc.z);
+                acc.w = fmaf(w[k], z.w, acc.w);
+            }
         }
         if (shared) {
-            const float4 v = *reinterpret_cast<const float4*>(shared + (size_t)t * dim + c);
-            acc.x = fmaf(sg, v.x, acc.x);
-            acc.y = fmaf(sg, v.y, acc.y);
-            acc.z = fmaf(sg, v.z, acc.z);
-            acc.w = fmaf(sg, v.w, acc.w);
+            acc.x = fmaf(sg, common.x, acc.x);
+            acc.y = fmaf(sg, common.y, acc.y);
+            acc.z = fmaf(sg, common.z, acc.z);
+            acc.w = fmaf(sg, common.w, acc.w);
         }
         return acc;
     };
-    ka_finish_row<PIECES>(x, t, dim, a, piece, one, smem);
+    ka_finish_row<PIECES, THREADS>(x, t, dim, a, piece, one, smem);
 }
 
 KA_API int ka_experts_combine_normed(const float* y, const void* h_in, long h_stride, int dtype, const int* chosen, const float* weights,
@@ -366,24 +377,18 @@ KA_API int ka_experts_combine_normed(const float* y, const void* h_in, long h_st
     const char* who = "ka_experts_combine_normed";
     KA_CHECK(n >= 0 && top > 0 && dim > 0 && h_stride >= dim && eps >= 0.f && eps2 >= 0.f && gain != nullptr, "%s: bad sizes", who);
     KA_CHECK(dtype == KA_F32 || dtype == KA_BF16, "%s: unsupported dtype %d", who, dtype);
-    KA_CHECK((gain2 == nullptr) == (h == nullptr), "%s: the second norm needs gains and rows", who);
+    KA_CHECK(gain2 == nullptr || h != nullptr, "%s: the second norm needs its rows", who);
     if (n == 0) return 0;
     const KaRowNorms a{gain, eps, gain2, eps2, h, dtype == KA_BF16};
-    const dim3 grid(n), block(KA_ROW_THREADS);
-    const int pieces = (uintptr_t)shared % 16 == 0 ? ka_row_pieces(dim, x, y, a) : 0;
-#define EX_COMBINE(T, P)                                                                                                            \
-    hipLaunchKernelGGL((experts_combine_normed_kernel<T, P>), grid, block, 0, stream, y, (const T*)h_in, h_stride, chosen, weights, top, E, \
-                       shared, shared_gate, gate_stride, x, dim, a)
-#define EX_COMBINE_ALL(T)                   \
-    switch (pieces) {                       \
-        case 1: EX_COMBINE(T, 1); break;    \
-        case 2: EX_COMBINE(T, 2); break;    \
-        case 4: EX_COMBINE(T, 4); break;    \
-        case 8: EX_COMBINE(T, 8); break;    \
-        default: EX_COMBINE(T, 0); break;   \
-    }
-    if (dtype == KA_F32) { EX_COMBINE_ALL(float) } else { EX_COMBINE_ALL(bf16_t) }
-#undef EX_COMBINE_ALL
+    const int pieces = (uintptr_t)shared % 16 == 0 ? ka_row_pieces(n, dim, x, y, a) : 0;
+#define EX_COMBINE(T, P, THREADS)                                                                                                  \
+    hipLaunchKernelGGL((experts_combine_normed_kernel<T, P, THREADS>), dim3(n), dim3(THREADS), 0, stream, y, (const T*)h_in, h_stride, chosen, \
+                       weights, top, E, shared, shared_gate, gate_stride, x, dim, a)
+#define EX_COMBINE_F32(P, THREADS) EX_COMBINE(float, P, THREADS)
+#define EX_COMBINE_BF16(P, THREADS) EX_COMBINE(bf16_t, P, THREADS)
+    if (dtype == KA_F32) { KA_ROW_CASES(pieces, EX_COMBINE_F32) } else { KA_ROW_CASES(pieces, EX_COMBINE_BF16) }
+#undef EX_COMBINE_F32
+#undef EX_COMBINE_BF16
 #undef EX_COMBINE
     KA_LAUNCH_CHECK();
     return 0;

@@ -1,24 +1,26 @@
 // Finishing a row of the fp32 residual stream: a sublayer's output d is normalised and added, x += d / rms(d) * gain with
 // rms(d) = sqrt(mean(d^2) + eps), and the norm that the next reader of the stream begins with is computed from the new
-// row, h = x / rms(x) * gain2, in the same pass. A workgroup of KA_ROW_THREADS threads takes a row; what computes d is the
-// caller's business (a load, a weighted sum). All arithmetic is fp32.
+// row, h = x / rms(x) * gain2, in the same pass (without gain2 the new row itself is left there, rounded). A workgroup takes a row, of
+// KA_ROW_THREADS threads where there are many rows, of a thread per four channels, up to 1,024, where there are few; what
+// computes d is the caller's business (a load, a weighted sum). All arithmetic is fp32. Eight rows of 2,048 behind four experts: 4.5 us, where
+// the sum, its norm into the stream and the rounding for the next reader were three launches of 13.4, 6.2 and 4.5.
 #pragma once
 
 #include "ka_common.h"
 
 constexpr int KA_ROW_THREADS = 256;
-constexpr int KA_ROW_WAVES = KA_ROW_THREADS / KA_WAVE;
 constexpr int KA_ROW_MAX_PIECES = 8;        // pieces of four channels a thread keeps in registers: rows of up to 8192 channels
 
 struct KaRowNorms {
     const float* gain;      // of the norm of d
     float eps;
-    const float* gain2;     // of the norm of the new row; null: there is none
+    const float* gain2;     // of the norm of the new row; null: the row as it is
     float eps2;
-    void* h;                // where that norm goes, rows of dim numbers
+    void* h;                // where that goes, rows of dim numbers; null: nowhere
     int h_bf16;
 };
 
+template <int THREADS>
 __device__ __forceinline__ float ka_row_sum(float v, float* smem) {
     v = ka_wave_sum(v);
     __syncthreads();
@@ -26,7 +28,7 @@ __device__ __forceinline__ float ka_row_sum(float v, float* smem) {
     __syncthreads();
     float total = 0.f;
 #pragma unroll
-    for (int w = 0; w < KA_ROW_WAVES; ++w) total += smem[w];
+    for (int w = 0; w < THREADS / KA_WAVE; ++w) total += smem[w];
     return total;
 }
 
@@ -35,9 +37,9 @@ __device__ __forceinline__ void ka_row_store_h(const KaRowNorms& a, size_t at, f
     else reinterpret_cast<float*>(a.h)[at] = v;
 }
 
-// PIECES > 0: dim is a multiple of 4 and at most 4 PIECES KA_ROW_THREADS, rows are 16-byte aligned; `piece(c)` gives d of the
+// PIECES > 0: dim is a multiple of 4 and at most 4 PIECES THREADS, rows are 16-byte aligned; `piece(c)` gives d of the
 // channels c .. c + 3. PIECES = 0: any dim; `one(c)` gives d of channel c (asked for twice).
-template <int PIECES, typename Piece, typename One>
+template <int PIECES, int THREADS, typename Piece, typename One>
 __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, int dim, const KaRowNorms& a, Piece piece, One one,
                                               float* smem) {
     const int tid = threadIdx.x;
@@ -48,18 +50,18 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
         float s = 0.f;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * KA_ROW_THREADS + tid) * 4;
+            const int c = (p * THREADS + tid) * 4;
             if (c < dim) {
                 d[p] = piece(c);
                 y[p] = *reinterpret_cast<const float4*>(x + at + c);
                 s += d[p].x * d[p].x + d[p].y * d[p].y + d[p].z * d[p].z + d[p].w * d[p].w;
             }
         }
-        const float r = 1.0f / sqrtf(ka_row_sum(s, smem) / (float)dim + a.eps);
+        const float r = 1.0f / sqrtf(ka_row_sum<THREADS>(s, smem) / (float)dim + a.eps);
         float s2 = 0.f;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * KA_ROW_THREADS + tid) * 4;
+            const int c = (p * THREADS + tid) * 4;
             if (c < dim) {
                 const float4 g = *reinterpret_cast<const float4*>(a.gain + c);
                 y[p].x += d[p].x * r * g.x;
@@ -70,14 +72,17 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
                 s2 += y[p].x * y[p].x + y[p].y * y[p].y + y[p].z * y[p].z + y[p].w * y[p].w;
             }
         }
-        if (a.gain2 == nullptr) return;
-        const float r2 = 1.0f / sqrtf(ka_row_sum(s2, smem) / (float)dim + a.eps2);
+        if (a.h == nullptr) return;
+        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_row_sum<THREADS>(s2, smem) / (float)dim + a.eps2) : 1.f;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * KA_ROW_THREADS + tid) * 4;
+            const int c = (p * THREADS + tid) * 4;
             if (c < dim) {
-                const float4 g = *reinterpret_cast<const float4*>(a.gain2 + c);
-                const float4 v = make_float4(y[p].x * r2 * g.x, y[p].y * r2 * g.y, y[p].z * r2 * g.z, y[p].w * r2 * g.w);
+                float4 v = y[p];
+                if (a.gain2) {
+                    const float4 g = *reinterpret_cast<const float4*>(a.gain2 + c);
+                    v = make_float4(v.x * r2 * g.x, v.y * r2 * g.y, v.z * r2 * g.z, v.w * r2 * g.w);
+                }
                 if (a.h_bf16) {
                     row_bf16x4 b;
                     b[0] = (bf16_t)v.x;
@@ -92,29 +97,48 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
         }
     } else {
         float s = 0.f;
-        for (int c = tid; c < dim; c += KA_ROW_THREADS) {
+        for (int c = tid; c < dim; c += THREADS) {
             const float d = one(c);
             s += d * d;
         }
-        const float r = 1.0f / sqrtf(ka_row_sum(s, smem) / (float)dim + a.eps);
+        const float r = 1.0f / sqrtf(ka_row_sum<THREADS>(s, smem) / (float)dim + a.eps);
         float s2 = 0.f;
-        for (int c = tid; c < dim; c += KA_ROW_THREADS) {
+        for (int c = tid; c < dim; c += THREADS) {
             const float y = x[at + c] + one(c) * r * a.gain[c];
             x[at + c] = y;
             s2 += y * y;
         }
-        if (a.gain2 == nullptr) return;
-        const float r2 = 1.0f / sqrtf(ka_row_sum(s2, smem) / (float)dim + a.eps2);
-        for (int c = tid; c < dim; c += KA_ROW_THREADS) ka_row_store_h(a, at + c, x[at + c] * r2 * a.gain2[c]);      // (its own writes)
+        if (a.h == nullptr) return;
+        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_row_sum<THREADS>(s2, smem) / (float)dim + a.eps2) : 1.f;
+        for (int c = tid; c < dim; c += THREADS) ka_row_store_h(a, at + c, x[at + c] * r2 * (a.gain2 ? a.gain2[c] : 1.f));      // (its own writes)
     }
 }
 
-// Pieces of four channels a thread holds of rows of `dim` channels in the form with registers; 0: the general form.
-static inline int ka_row_pieces(int dim, const void* x, const void* d, const KaRowNorms& a) {
+// Pieces of four channels a thread holds of rows of `dim` channels in the form with registers, times ten, with 1 or 2 added where a
+// row gets 512 or 1,024 threads (fewer rows than two a CU); 0: the general form.
+static inline int ka_row_pieces(int n, int dim, const void* x, const void* d, const KaRowNorms& a) {
     const uintptr_t all = (uintptr_t)x | (uintptr_t)d | (uintptr_t)a.gain | (uintptr_t)a.gain2;
     if (dim % 4 != 0 || all % 16 != 0 || (uintptr_t)a.h % (a.h_bf16 ? 8 : 16) != 0) return 0;
     const int need = (dim + 4 * KA_ROW_THREADS - 1) / (4 * KA_ROW_THREADS);
+    if (n < 2 * ka_compute_units()) {
+        if (need == 2) return 11;
+        if (need > 2 && need <= 4) return 12;
+        if (need > 4 && need <= 8) return 22;
+    }
     for (int p : {1, 2, 4, 8})
-        if (need <= p) return p;
+        if (need <= p) return p * 10;
     return 0;
 }
+
+// LAUNCH(pieces, threads) of the form that ka_row_pieces named.
+#define KA_ROW_CASES(PIECES, LAUNCH)   \
+    switch (PIECES) {                  \
+        case 10: LAUNCH(1, 256); break; \
+        case 20: LAUNCH(2, 256); break; \
+        case 40: LAUNCH(4, 256); break; \
+        case 80: LAUNCH(8, 256); break; \
+        case 11: LAUNCH(1, 512); break; \
+        case 12: LAUNCH(1, 1024); break;\
+        case 22: LAUNCH(2, 1024); break;\
+        default: LAUNCH(0, 256); break; \
+    }

@@ -448,31 +448,26 @@ KA_API int ka_branches_sum(float* x, const float* a, const float* gain_a, float 
 }
 
 // ----------------------------------------------------------------------------
-// x += d / rms(d) * gain for fp32 rows d and, of the new rows, h = x / rms(x) * gain2 (h optional): ka_rows.h.
+// x += d / rms(d) * gain for fp32 rows d and, of the new rows, h = x / rms(x) * gain2, or their rounding (h optional): ka_rows.h.
 // ----------------------------------------------------------------------------
-template <int PIECES>
-__global__ void __launch_bounds__(KA_ROW_THREADS)
+template <int PIECES, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 add_normed_kernel(float* __restrict__ x, const float* __restrict__ d, KaRowNorms a, int dim) {
-    __shared__ float smem[KA_ROW_WAVES];
+    __shared__ float smem[THREADS / KA_WAVE];
     const float* row = d + (size_t)blockIdx.x * dim;
-    ka_finish_row<PIECES>(x, blockIdx.x, dim, a, [&](int c) { return *reinterpret_cast<const float4*>(row + c); },
+    ka_finish_row<PIECES, THREADS>(x, blockIdx.x, dim, a, [&](int c) { return *reinterpret_cast<const float4*>(row + c); },
                           [&](int c) { return row[c]; }, smem);
 }
 
 KA_API int ka_add_normed(float* x, const float* d, const float* gain, float eps, const float* gain2, float eps2, void* h, int h_dtype,
                          int n, int dim, hipStream_t stream) {
     KA_CHECK(n >= 0 && dim > 0 && eps >= 0.f && eps2 >= 0.f && gain != nullptr, "ka_add_normed: bad sizes or no gain");
-    KA_CHECK((gain2 == nullptr) == (h == nullptr) && (h_dtype == KA_F32 || h_dtype == KA_BF16), "ka_add_normed: the second norm needs gains and rows");
+    KA_CHECK((gain2 == nullptr || h != nullptr) && (h_dtype == KA_F32 || h_dtype == KA_BF16), "ka_add_normed: the second norm needs its rows");
     if (n == 0) return 0;
     const KaRowNorms a{gain, eps, gain2, eps2, h, h_dtype == KA_BF16};
-    const dim3 grid(n), block(KA_ROW_THREADS);
-    switch (ka_row_pieces(dim, x, d, a)) {
-        case 1: hipLaunchKernelGGL(add_normed_kernel<1>, grid, block, 0, stream, x, d, a, dim); break;
-        case 2: hipLaunchKernelGGL(add_normed_kernel<2>, grid, block, 0, stream, x, d, a, dim); break;
-        case 4: hipLaunchKernelGGL(add_normed_kernel<4>, grid, block, 0, stream, x, d, a, dim); break;
-        case 8: hipLaunchKernelGGL(add_normed_kernel<8>, grid, block, 0, stream, x, d, a, dim); break;
-        default: hipLaunchKernelGGL(add_normed_kernel<0>, grid, block, 0, stream, x, d, a, dim); break;
-    }
+#define MP_ADD_NORMED(P, THREADS) hipLaunchKernelGGL((add_normed_kernel<P, THREADS>), dim3(n), dim3(THREADS), 0, stream, x, d, a, dim)
+    KA_ROW_CASES(ka_row_pieces(n, dim, x, d, a), MP_ADD_NORMED)
+#undef MP_ADD_NORMED
     KA_LAUNCH_CHECK();
     return 0;
 }

@@ -5,8 +5,10 @@
 // What computes y is the caller's business: a load, or the weighted sum of a routed mixture's experts.
 #include "ka_common.h"
 
+// A workgroup has a row. Of many rows each gets 256 threads and a thread several pieces of it; where there are fewer rows than two a
+// CU (a decode step) a row gets a thread per piece, up to 1,024: it then waits for memory once (48 rows of four streams of
+// 4,096: 11 -> 5.1 us between sublayers and 24 -> 8.3 behind six experts).
 constexpr int ST_THREADS = 256;
-constexpr int ST_WAVES = ST_THREADS / KA_WAVE;
 constexpr int ST_MAX_STREAMS = 16;
 
 struct StreamArgs {
@@ -25,6 +27,7 @@ struct StreamArgs {
     int S, dim;
 };
 
+template <int THREADS>
 __device__ __forceinline__ float st_block_sum(float v, float* smem) {
     v = ka_wave_sum(v);
     __syncthreads();
@@ -32,7 +35,7 @@ __device__ __forceinline__ float st_block_sum(float v, float* smem) {
     __syncthreads();
     float total = 0.f;
 #pragma unroll
-    for (int w = 0; w < ST_WAVES; ++w) total += smem[w];
+    for (int w = 0; w < THREADS / KA_WAVE; ++w) total += smem[w];
     return total;
 }
 
@@ -40,9 +43,9 @@ __device__ __forceinline__ float4 st_fma4(float a, const float4& b, const float4
     return make_float4(fmaf(a, b.x, c.x), fmaf(a, b.y, c.y), fmaf(a, b.z, c.z), fmaf(a, b.w, c.w));
 }
 
-// S streams in registers, PIECES pieces of four channels a thread (dim a multiple of 4 and at most 4 PIECES ST_THREADS, rows
+// S streams in registers, PIECES pieces of four channels a thread (dim a multiple of 4 and at most 4 PIECES THREADS, rows
 // 16-byte aligned). `piece(c)` gives y of the channels c .. c + 3.
-template <int S, int PIECES, typename Piece>
+template <int S, int PIECES, int THREADS, typename Piece>
 __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, float* smem) {
     typedef __attribute__((ext_vector_type(4))) __bf16 st_bf16x4;
     const int i = blockIdx.x, tid = threadIdx.x, dim = a.dim;
@@ -68,7 +71,7 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
         float4 v[AT_ONCE][S], y[AT_ONCE];
 #pragma unroll
         for (int p = 0; p < AT_ONCE; ++p) {
-            const int c = ((p0 + p) * ST_THREADS + tid) * 4;
+            const int c = ((p0 + p) * THREADS + tid) * 4;
             if (c >= dim) continue;
             if (a.embedded) {
                 v[p][0] = *reinterpret_cast<const float4*>(a.embedded + (size_t)i * dim + c);
@@ -80,7 +83,7 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
         }
 #pragma unroll
         for (int p = 0; p < AT_ONCE; ++p) {
-            const int c = ((p0 + p) * ST_THREADS + tid) * 4;
+            const int c = ((p0 + p) * THREADS + tid) * 4;
             float4& sums = u[p0 + p];
             sums = make_float4(0.f, 0.f, 0.f, 0.f);
             if (c >= dim) continue;
@@ -108,19 +111,19 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
         }
     }
     if (a.h == nullptr) return;
-    const float mean = a.rms ? 0.f : st_block_sum(sum, smem) / (float)dim;
+    const float mean = a.rms ? 0.f : st_block_sum<THREADS>(sum, smem) / (float)dim;
     float ss = 0.f;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-        if ((p * ST_THREADS + tid) * 4 < dim) {
+        if ((p * THREADS + tid) * 4 < dim) {
             u[p] = make_float4(u[p].x - mean, u[p].y - mean, u[p].z - mean, u[p].w - mean);
             ss += u[p].x * u[p].x + u[p].y * u[p].y + u[p].z * u[p].z + u[p].w * u[p].w;
         }
     }
-    const float r = 1.0f / sqrtf(st_block_sum(ss, smem) / (float)dim + a.eps);
+    const float r = 1.0f / sqrtf(st_block_sum<THREADS>(ss, smem) / (float)dim + a.eps);
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-        const int c = (p * ST_THREADS + tid) * 4;
+        const int c = (p * THREADS + tid) * 4;
         if (c < dim) {
             const float4 g = *reinterpret_cast<const float4*>(a.gain + c);
             float4 v = make_float4(u[p].x * r * g.x, u[p].y * r * g.y, u[p].z * r * g.z, u[p].w * r * g.w);
@@ -175,13 +178,13 @@ __device__ __forceinline__ void st_step_any(const StreamArgs& a, One one, float*
         if (a.h) sum += read(c);              // (a thread reads its own writes)
     }
     if (a.h == nullptr) return;
-    const float mean = a.rms ? 0.f : st_block_sum(sum, smem) / (float)dim;
+    const float mean = a.rms ? 0.f : st_block_sum<ST_THREADS>(sum, smem) / (float)dim;
     float ss = 0.f;
     for (int c = tid; c < dim; c += ST_THREADS) {
         const float u = read(c) - mean;
         ss += u * u;
     }
-    const float r = 1.0f / sqrtf(st_block_sum(ss, smem) / (float)dim + a.eps);
+    const float r = 1.0f / sqrtf(st_block_sum<ST_THREADS>(ss, smem) / (float)dim + a.eps);
     for (int c = tid; c < dim; c += ST_THREADS) {
         float v = (read(c) - mean) * r * a.gain[c];
         if (a.bias) v += a.bias[c];
@@ -190,12 +193,12 @@ __device__ __forceinline__ void st_step_any(const StreamArgs& a, One one, float*
     }
 }
 
-template <int S, int PIECES>
-__global__ void __launch_bounds__(ST_THREADS) streams_step_kernel(StreamArgs a, const float* __restrict__ y) {
-    __shared__ float smem[ST_WAVES];
+template <int S, int PIECES, int THREADS>
+__global__ void __launch_bounds__(THREADS) streams_step_kernel(StreamArgs a, const float* __restrict__ y) {
+    __shared__ float smem[THREADS / KA_WAVE];
     const float* yr = y ? y + (size_t)blockIdx.x * a.dim : nullptr;
     if constexpr (S > 0)
-        st_step_regs<S, PIECES>(a, [&](int c) { return *reinterpret_cast<const float4*>(yr + c); }, smem);
+        st_step_regs<S, PIECES, THREADS>(a, [&](int c) { return *reinterpret_cast<const float4*>(yr + c); }, smem);
     else
         st_step_any(a, [&](int c) { return yr[c]; }, smem);
 }
@@ -214,32 +217,36 @@ struct StreamExperts {
     long gate_stride;
 };
 
-template <typename T, int S, int PIECES>
-__global__ void __launch_bounds__(ST_THREADS) streams_experts_kernel(StreamArgs a, StreamExperts e) {
-    __shared__ float smem[ST_WAVES];
+template <typename T, int S, int PIECES, int THREADS>
+__global__ void __launch_bounds__(THREADS) streams_experts_kernel(StreamArgs a, StreamExperts e) {
+    __shared__ float smem[THREADS / KA_WAVE];
     const int t = blockIdx.x, dim = a.dim;
     const T* hp = reinterpret_cast<const T*>(e.h_in) + (size_t)t * e.h_stride;
     const float sg = e.shared ? (e.shared_gate ? 1.0f / (1.0f + expf(-e.shared_gate[(size_t)t * e.gate_stride])) : 1.f) : 0.f;
     if constexpr (S > 0) {
-        st_step_regs<S, PIECES>(a, [&](int c) {
+        st_step_regs<S, PIECES, THREADS>(a, [&](int c) {
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-            // (four choices in flight; a choice without weights of its own has a row in `pairs` too, which is not used)
-            for (int k0 = 0; k0 < e.top; k0 += 4) {
-                float4 v[4];
-                float w[4];
+            // (everything is asked for at once, eight choices at a time and nothing behind a branch; a choice without weights of
+            // its own has a row in `pairs` too, which is not used)
+            const float4 own = make_float4(ka_to_float(hp[c]), ka_to_float(hp[c + 1]), ka_to_float(hp[c + 2]), ka_to_float(hp[c + 3]));
+            const float4 common = e.shared ? *reinterpret_cast<const float4*>(e.shared + (size_t)t * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            constexpr int AHEAD = PIECES == 1 ? 8 : 4;
+            for (int k0 = 0; k0 < e.top; k0 += AHEAD) {
+                float4 v[AHEAD];
+                float w[AHEAD];
+                bool has[AHEAD];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
+                for (int k = 0; k < AHEAD; ++k) {
                     const size_t at = (size_t)t * e.top + min(k0 + k, e.top - 1);
                     w[k] = e.weights[at];
+                    has[k] = e.chosen[at] < e.E;
                     v[k] = *reinterpret_cast<const float4*>(e.pairs + at * dim + c);
-                    if (e.chosen[at] >= e.E) v[k] = make_float4(ka_to_float(hp[c]), ka_to_float(hp[c + 1]), ka_to_float(hp[c + 2]), ka_to_float(hp[c + 3]));
                 }
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k0 + k < e.top) acc = st_fma4(w[k], v[k], acc);
+                for (int k = 0; k < AHEAD; ++k)
+                    if (k0 + k < e.top) acc = st_fma4(w[k], has[k] ? v[k] : own, acc);
             }
-            if (e.shared) acc = st_fma4(sg, *reinterpret_cast<const float4*>(e.shared + (size_t)t * dim + c), acc);
-            return acc;
+            return e.shared ? st_fma4(sg, common, acc) : acc;
         }, smem);
     } else {
         st_step_any(a, [&](int c) {
@@ -253,25 +260,34 @@ __global__ void __launch_bounds__(ST_THREADS) streams_experts_kernel(StreamArgs 
     }
 }
 
-// Pieces of four channels a thread holds in the form with registers; 0: the general form.
-static int st_pieces(const StreamArgs& a, const void* y, const void* shared) {
+// Pieces of four channels a thread holds in the form with registers, times ten, with 1 or 2 added where a row gets 512 or 1,024 threads
+// (few rows); 0: the general form.
+static int st_pieces(const StreamArgs& a, int n, const void* y, const void* shared) {
     const uintptr_t all = (uintptr_t)a.x | (uintptr_t)a.embedded | (uintptr_t)a.gain | (uintptr_t)a.bias | (uintptr_t)y | (uintptr_t)shared;
     if (a.S > 4 || a.dim % 4 != 0 || all % 16 != 0 || (uintptr_t)a.h % (a.h_bf16 ? 8 : 16) != 0) return 0;
     const int need = ka_cdiv(a.dim, 4 * ST_THREADS);
+    if (n < 2 * ka_compute_units()) {
+        if (need == 2) return 11;
+        if (need > 2 && need <= 4) return 12;
+        if (need > 4 && need <= 8) return 22;
+    }
     for (int p : {1, 2, 4, 8})
-        if (need <= p) return p;
+        if (need <= p) return p * 10;
     return 0;
 }
 
-#define ST_CASES(LAUNCH, S)          \
-    switch (pieces) {                \
-        case 1: LAUNCH(S, 1); break; \
-        case 2: LAUNCH(S, 2); break; \
-        case 4: LAUNCH(S, 4); break; \
-        default: LAUNCH(S, 8); break;\
+#define ST_CASES(LAUNCH, S)                \
+    switch (pieces) {                      \
+        case 10: LAUNCH(S, 1, 256); break; \
+        case 20: LAUNCH(S, 2, 256); break; \
+        case 40: LAUNCH(S, 4, 256); break; \
+        case 11: LAUNCH(S, 1, 512); break; \
+        case 12: LAUNCH(S, 1, 1024); break;\
+        case 22: LAUNCH(S, 2, 1024); break;\
+        default: LAUNCH(S, 8, 256); break; \
     }
 #define ST_DISPATCH(LAUNCH)                       \
-    if (pieces == 0) { LAUNCH(0, 0); }            \
+    if (pieces == 0) { LAUNCH(0, 0, 256); }       \
     else if (a.S == 1) { ST_CASES(LAUNCH, 1) }    \
     else if (a.S == 2) { ST_CASES(LAUNCH, 2) }    \
     else if (a.S == 3) { ST_CASES(LAUNCH, 3) }    \
@@ -294,8 +310,8 @@ KA_API int ka_streams_step(float* x, const float* embedded, const float* y, cons
     if (const int status = st_check(who, a, n, h_dtype)) return status;
     KA_CHECK((mix == nullptr) == (y == nullptr), "%s: writing needs a sublayer's output", who);
     if (n == 0) return 0;
-    const int pieces = st_pieces(a, y, nullptr);
-#define ST_LAUNCH(S_, P_) hipLaunchKernelGGL((streams_step_kernel<S_, P_>), dim3(n), dim3(ST_THREADS), 0, stream, a, y)
+    const int pieces = st_pieces(a, n, y, nullptr);
+#define ST_LAUNCH(S_, P_, T_) hipLaunchKernelGGL((streams_step_kernel<S_, P_, T_>), dim3(n), dim3(T_), 0, stream, a, y)
     ST_DISPATCH(ST_LAUNCH)
 #undef ST_LAUNCH
     KA_LAUNCH_CHECK();
@@ -313,9 +329,9 @@ KA_API int ka_streams_experts(float* x, const float* pairs, const void* h_in, lo
     KA_CHECK(dtype == KA_F32 || dtype == KA_BF16, "%s: unsupported dtype %d", who, dtype);
     if (n == 0) return 0;
     const StreamExperts e{pairs, h_in, h_stride, chosen, weights, top, E, shared, shared_gate, gate_stride};
-    const int pieces = st_pieces(a, pairs, shared);
-#define ST_LAUNCH_F32(S_, P_) hipLaunchKernelGGL((streams_experts_kernel<float, S_, P_>), dim3(n), dim3(ST_THREADS), 0, stream, a, e)
-#define ST_LAUNCH_BF16(S_, P_) hipLaunchKernelGGL((streams_experts_kernel<bf16_t, S_, P_>), dim3(n), dim3(ST_THREADS), 0, stream, a, e)
+    const int pieces = st_pieces(a, n, pairs, shared);
+#define ST_LAUNCH_F32(S_, P_, T_) hipLaunchKernelGGL((streams_experts_kernel<float, S_, P_, T_>), dim3(n), dim3(T_), 0, stream, a, e)
+#define ST_LAUNCH_BF16(S_, P_, T_) hipLaunchKernelGGL((streams_experts_kernel<bf16_t, S_, P_, T_>), dim3(n), dim3(T_), 0, stream, a, e)
     if (dtype == KA_F32) { ST_DISPATCH(ST_LAUNCH_F32) } else { ST_DISPATCH(ST_LAUNCH_BF16) }
 #undef ST_LAUNCH_F32
 #undef ST_LAUNCH_BF16

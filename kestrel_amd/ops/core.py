@@ -490,7 +490,7 @@ def _norm_pair(who: str, x, norm, then, rows):
     for pair in (norm,) + ((then,) if then is not None else ()):
         gain = pair[0]
         _need(gain.is_cuda and gain.dtype == torch.float32 and gain.is_contiguous() and gain.numel() == dim, f"{who}: gains fp32 [dim]")
-    _need((then is None) == (rows is None), f"{who}: the second norm needs its rows")
+    _need(then is None or rows is not None, f"{who}: the second norm needs its rows")
     _need(rows is None or (rows.is_cuda and rows.is_contiguous() and tuple(rows.shape) == (n, dim)), f"{who}: rows must be [n, dim]")
     return (norm[0].data_ptr(), float(norm[1]), None if then is None else then[0].data_ptr(), 0.0 if then is None else float(then[1]),
             _ptr(rows))
@@ -498,7 +498,8 @@ def _norm_pair(who: str, x, norm, then, rows):
 
 def add_normed(x: torch.Tensor, delta: torch.Tensor, norm, then=None, rows: Optional[torch.Tensor] = None) -> None:
     """``x += delta / rms(delta) * gain`` for fp32 rows ``delta`` into the fp32 stream ``x``, with ``norm = (gain, eps)`` and
-    ``rms(y) = sqrt(mean(y^2) + eps)``; with ``then`` (the same form) also ``rows = x / rms(x) * gain`` of the new rows."""
+    ``rms(y) = sqrt(mean(y^2) + eps)``; with ``then`` (the same form) also ``rows = x / rms(x) * gain`` of the new rows, with ``rows``
+    alone the new rows themselves, in that tensor's type."""
     _dev(x, delta, rows)
     n, dim = x.shape
     _need(delta.dtype == torch.float32 and delta.is_contiguous() and delta.shape == x.shape, "add_normed: delta must be fp32 of the shape of x")
@@ -1038,7 +1039,7 @@ def experts_combine_normed(y: torch.Tensor, h: torch.Tensor, chosen: torch.Tenso
                            shared: Optional[torch.Tensor], shared_gate: Optional[torch.Tensor], x: torch.Tensor, norm, then=None,
                            rows: Optional[torch.Tensor] = None) -> None:
     """The weighted sum of ``experts_combine`` as a ``delta`` of ``add_normed``: normalised and added into the fp32 stream ``x``, with
-    the norm ``then`` of the new rows into ``rows`` (of ``h``'s type), in one launch."""
+    the norm ``then`` of the new rows (without it: the rows themselves) into ``rows`` (of ``h``'s type), in one launch."""
     _dev(y, h, chosen, weights, shared, shared_gate, x, rows)
     n, dim = x.shape
     top = chosen.shape[1]

@@ -237,55 +237,82 @@ def _parallel_two_norms(block: "Block", x, batch, cache) -> None:
 _parallel_two_norms.defers = True
 
 
-def _output_norms(block: "Block", x, batch, cache) -> None:
+class StreamRounding:
+    """What a block of the arrangement ``output_norms`` reads first: the stream itself, rounded to the activation type (``wanted``) or, for a
+    mixer that says ``reads_stream``, as it is. No norm: it offers no operands of one."""
+
+    def __init__(self, wanted: bool) -> None:
+        self.wanted = wanted
+
+    def layernorm_operands(self):
+        return None
+
+    def rms_operands(self):
+        return None
+
+
+def _output_norms(block: "Block", x, batch, cache, normed=None, then=None):
     """``x += norm(mixer(x)); x += norm2(ff(x))``: the parts read the stream itself (rounded to the activation type, or,
     for a mixer that says ``reads_stream``, as it is) and the norms stand behind them. Each part writes its output into
-    an fp32 buffer (``mix``; a part without it adds into a cleared buffer through ``forward``), and the norm's kernel adds
-    the normalised rows into the stream (``Norm.add_normed``)."""
+    an fp32 buffer (``mix``; a part without it adds into a cleared buffer through ``forward``); one launch normalises it, adds it
+    into the stream and leaves the rounding that the next reader begins with (``normed``, from the block before). A feed-forward
+    that offers ``mix_normed`` takes that launch's work into its own last one."""
     from ..ops import core
 
     ws = batch.workspace
     delta = ws.get("block.delta", tuple(x.shape), torch.float32)
+    rounds = block.dtype != torch.float32
 
-    def rounded():
-        if block.dtype == torch.float32:
-            return x
-        h = ws.get("block.h", tuple(x.shape), block.dtype)
+    def rounded(name: str):
+        h = ws.get(name, tuple(x.shape), block.dtype)
         core.cast_columns(x, h)
         return h
 
-    def add(norm, also_rounded: bool = False) -> bool:
-        """``x += norm(delta)``; with ``also_rounded`` the stream's rounding is left in ``block.h`` by the same launch where
-        the norm offers that (returns whether it did)."""
+    def add(norm, rows) -> bool:
+        """``x += norm(delta)``, the stream's rounding into ``rows`` (``None``: not wanted); returns whether ``rows`` was written."""
+        first = norm.rms_operands() if callable(getattr(norm, "rms_operands", None)) else None
+        if first is not None:
+            core.add_normed(x, delta, first, None, rows)
+            return rows is not None
         if callable(getattr(norm, "add_normed", None)):
-            if also_rounded and block.dtype != torch.float32:
-                norm.add_normed(delta, x, rounded=ws.get("block.h", tuple(x.shape), block.dtype))
-                return True
             norm.add_normed(delta, x)
-            return False
-        normed = ws.get("block.normed", tuple(x.shape), torch.float32)
-        norm.forward(delta, normed)
-        core.add_scaled(x, normed, 1.0)
+        else:
+            summed = ws.get("block.normed", tuple(x.shape), torch.float32)
+            norm.forward(delta, summed)
+            core.add_scaled(x, summed, 1.0)
         return False
 
     mixer = block.mixer
-    source = x if getattr(mixer, "reads_stream", False) else rounded()
+    source = x
+    if rounds and not getattr(mixer, "reads_stream", False):
+        source = normed if normed is not None else rounded("block.h")
     if callable(getattr(mixer, "mix", None)):
         mixer.mix(source, batch, cache, delta, False)
     else:
         delta.zero_()
         mixer.forward(source, batch, cache, delta)
+    handed = ws.get("block.handed", tuple(x.shape), block.dtype) if rounds and isinstance(then, StreamRounding) and then.wanted else None
     ff = block.feed_forward
-    left = add(block.norm, also_rounded=ff is not None)
-    if ff is not None:
-        # (the feed-forward reads the stream's rounding, which the launch before has left where the norm could)
-        h = ws.get("block.h", tuple(x.shape), block.dtype) if left else rounded()
-        if callable(getattr(ff, "mix", None)):
-            ff.mix(h, batch, delta, False)
-        else:
-            delta.zero_()
-            ff.forward(h, batch, delta)
-        add(block.norm2)
+    if ff is None:
+        return handed if add(block.norm, handed) else None
+    h = x
+    if rounds:
+        h = ws.get("block.h2", tuple(x.shape), block.dtype)
+    if not add(block.norm, h if rounds else None) and rounds:
+        core.cast_columns(x, h)
+    second = block.norm2.rms_operands() if callable(getattr(block.norm2, "rms_operands", None)) else None
+    if callable(getattr(ff, "mix_normed", None)) and second is not None:
+        ff.mix_normed(h, batch, x, second, None, handed)
+        return handed
+    if callable(getattr(ff, "mix", None)):
+        ff.mix(h, batch, delta, False)
+    else:
+        delta.zero_()
+        ff.forward(h, batch, delta)
+    return handed if add(block.norm2, handed) else None
+
+
+_output_norms.hands_over = True
 
 
 def _add_normed(norm, delta, x, then, rows, ws) -> bool:
@@ -440,6 +467,8 @@ class Block:
         if spec.arrangement == "parallel_two_norms" and spec.feed_forward is not None and self.norm2 is None:
             raise ValueError("the parallel_two_norms arrangement needs norm2 for its feed-forward")
         self.feed_forward = build_part("feed_forward", spec.feed_forward) if spec.feed_forward is not None else None
+        if spec.arrangement == "output_norms":
+            self.reader = StreamRounding(not getattr(self.mixer, "reads_stream", False))
         self.dtype: Optional[torch.dtype] = None
         self._run = ARRANGEMENTS[spec.arrangement]
 

@@ -175,7 +175,8 @@ class RoutedExperts(FeedForward):
 
     def mix_normed(self, h, batch, x, norm, then, rows) -> None:
         """The feed-forward of ``h``, normalised (``norm``: ``(gain, eps)`` of a root-mean-square norm) and added into fp32 ``x``
-        by the launch that takes the weighted sum; ``then`` (the same form) of the new rows of ``x`` goes into ``rows``."""
+        by the launch that takes the weighted sum; ``then`` (the same form) of the new rows of ``x``, or without it their rounding, goes
+        into ``rows``."""
         y, chosen, weights, shared_out, gate = self._outputs(h, batch)
         core.experts_combine_normed(y, h, chosen, weights, self.pairs.shape[0], shared_out, gate, x, norm, then, rows)
 
