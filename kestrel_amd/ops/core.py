@@ -68,6 +68,9 @@ _SIGNATURES = {
     "ka_decayed_memory": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                           _c_long, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_float,
                           _c_void_p, _c_void_p],
+    "ka_decayed_step_supported": [_c_int, _c_int],
+    "ka_decayed_step": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_void_p,
+                        _c_void_p, _c_void_p, _c_long, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     "ka_decayed_readout": [_c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     "ka_route": [_c_void_p, _c_long, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p, _c_void_p,
                  _c_void_p],
@@ -950,6 +953,33 @@ def decayed_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torc
                                    code_of(r.dtype), pre.data_ptr(), u.data_ptr(), gain.data_ptr(), state.data_ptr(), state.stride(0),
                                    _ptr(x), dim, cu_q.data_ptr(), row_slot.data_ptr(), out.data_ptr(),
                                    out.stride(0) if n > 1 else width, n, n_rows, n_heads, head_dim, float(eps), raw.data_ptr(), stream_ptr()))
+
+
+def decayed_step(r, k, v, gate, low, w2, w0, u, gain, state, x, row_slot, out, n_heads: int, head_dim: int, eps: float) -> bool:
+    """A step of single tokens (row ``i`` brings token ``i``) of ``decayed_memory`` in one launch, with ``pre = w2 low + w0``: ``low`` ``[n, rank]``
+    and ``w2`` ``[H d, rank]`` of the type of ``r``, ``w0`` fp32 ``[H d]``, the other operands as there. False: sizes or alignment not
+    covered, nothing was run."""
+    _dev(r, k, v, gate, low, w2, w0, u, gain, state, x, row_slot, out)
+    n, rank = low.shape
+    who, width = "decayed_step", n_heads * head_dim
+    dim = 0 if x is None else x.shape[1]
+    if not lib().ka_decayed_step_supported(int(head_dim), int(rank)) or state.stride(0) % 4 or state.data_ptr() % 16:
+        return False
+    for t in (r, k, v, gate):
+        _need(t.dtype == r.dtype and tuple(t.shape) == (n, width) and t.stride(1) == 1 and (n <= 1 or t.stride(0) == r.stride(0)),
+              f"{who}: r, k, v and gate must be [n, H d] of one type and row stride")
+    _need(low.dtype == r.dtype and low.stride(1) == 1 and w2.dtype == r.dtype and w2.is_contiguous() and tuple(w2.shape) == (width, rank), f"{who}: low [n, rank], w2 [H d, rank]")
+    for t in (w0, u, gain):
+        _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == width, f"{who}: w0, u and gain fp32 [H d]")
+    _need(x is None or (x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == n), f"{who}: x fp32 [n, dim]")
+    _need(state.dtype == torch.float32 and state.is_contiguous() and state.dim() == 2 and state.shape[1] == width * head_dim + dim, f"{who}: state fp32 [slots, H d d + dim]")
+    _need(row_slot.dtype == torch.int32 and row_slot.numel() == n, f"{who}: as many rows as tokens")
+    _need(out.dtype == r.dtype and out.stride(1) == 1 and tuple(out.shape) == (n, width), f"{who}: out [n, H d]")
+    _check(lib().ka_decayed_step(r.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), r.stride(0) if n > 1 else max(r.stride(0), width), code_of(r.dtype),
+                                 low.data_ptr(), low.stride(0) if n > 1 else max(low.stride(0), rank), w2.data_ptr(), w0.data_ptr(), rank, u.data_ptr(),
+                                 gain.data_ptr(), state.data_ptr(), state.stride(0), _ptr(x), dim, row_slot.data_ptr(), out.data_ptr(),
+                                 out.stride(0) if n > 1 else max(out.stride(0), width), n, n_heads, head_dim, float(eps), stream_ptr()))
+    return True
 
 
 def decayed_readout(raw: torch.Tensor, gate: torch.Tensor, gain: torch.Tensor, out: torch.Tensor, n_heads: int, head_dim: int, eps: float) -> None:

@@ -75,6 +75,7 @@ _SIGNATURES = {
     "ka_experts_few_supported": [_c_int, _c_long, _c_int, _c_int, _c_int],
     "ka_experts_few_bf16": [_c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float,
                             _c_float, _c_void_p, _c_long, _c_int, _c_void_p],
+    "ka_linears_few_bf16": [_c_int, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p],
     "ka_matrix_memory_chunks_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                      _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float,
                                      _c_void_p, _c_int, _c_void_p],
@@ -168,6 +169,8 @@ def chip_sizes(device=None) -> ChipSizes:
 
 ACT_GATED = 0x100                  # (ops.linear.ACT_GATED)
 EXPERTS_LARGEST_TILE = 256         # list rows of the largest tile of the experts' linears
+LINEARS_FEW_ROWS = 32              # most rows, and most linears, of a launch of several linears
+LINEARS_FEW_COUNT = 8
 
 _lib = None
 _scratch: Dict[int, torch.Tensor] = {}
@@ -980,6 +983,28 @@ def decayed_chunks_bf16(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, o
         core.decayed_readout(raw.view(-1)[:n * width].view(n, width), gate, gain, out, n_heads, head_dim, eps)
         return True
     _check(status)
+    return True
+
+
+def linears_few_bf16(inputs, weights, outs, acts) -> bool:
+    """``out = act(a @ w.T)`` of several linears of one input size in one launch for few bf16 rows: ``inputs`` ``[n, K]`` of one row stride, ``weights``
+    ``[N, K]``, ``outs`` ``[n, N]`` (each with a row stride of its own). False: not covered, nothing was run."""
+    n, k = inputs[0].shape
+    count = len(weights)
+    lda = inputs[0].stride(0) if n > 1 else k
+    core._dev(*inputs, *weights, *outs)
+    if not 0 < n <= LINEARS_FEW_ROWS or not 0 < count <= LINEARS_FEW_COUNT or k % 8 or lda % 8:
+        return False
+    for a, w, o, act in zip(inputs, weights, outs, acts):
+        if tuple(a.shape) != (n, k) or w.dim() != 2 or w.shape[1] != k or tuple(o.shape) != (n, w.shape[0]):
+            raise KernelError("linears: inputs, weights and outputs do not belong together")
+        if any(t.dtype != torch.bfloat16 or t.stride(1) != 1 for t in (a, w, o)) or not w.is_contiguous() or (n > 1 and a.stride(0) != lda) \
+                or a.data_ptr() % 16 or w.data_ptr() % 16 or act & ACT_GATED:
+            return False
+    pointers = lambda ts: (ctypes.c_void_p * count)(*(t.data_ptr() for t in ts))  # noqa: E731
+    _check(lib().ka_linears_few_bf16(count, pointers(inputs), lda, pointers(weights), (ctypes.c_int * count)(*(w.shape[0] for w in weights)),
+                                     (ctypes.c_int * count)(*(int(a) for a in acts)), pointers(outs),
+                                     (ctypes.c_long * count)(*(o.stride(0) if n > 1 else o.shape[1] for o in outs)), n, k, stream_ptr()))
     return True
 
 

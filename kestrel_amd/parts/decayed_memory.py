@@ -33,8 +33,10 @@ class DecayedMemory(Mixer):
     activation type. The five projections are linears of that type; the second linear of the decay writes fp32 (with
     ``w0`` as its bias) and the exponentials are taken in the recurrence kernel, so that everything that enters the
     recurrence besides the projections is fp32. One kernel walks over every row's tokens in order and a second normalises the read-outs
-    (``ops.core.decayed_memory``): single tokens, every step in float32, heads that the chunks do not take. Prompts and portions in
-    bfloat16 go by chunks of 64 tokens over the matrix cores (``ops.fast.decayed_chunks_bf16``). Rows without a request
+    (``ops.core.decayed_memory``): prompts in float32, short portions, heads that the other kernels do not take. Prompts and portions in
+    bfloat16 go by chunks of 64 tokens over the matrix cores (``ops.fast.decayed_chunks_bf16``); a step of single tokens takes one launch
+    for the decay's second linear, the recurrence, norm and gate (``ops.core.decayed_step``), behind one launch for the five
+    projections in bfloat16 (``ops.fast.linears_few_bf16``). Rows without a request
     (the padding of a replayed step) write zeros and touch no state."""
 
     replays_every_step = True
@@ -93,14 +95,23 @@ class DecayedMemory(Mixer):
         mixes = ws.get("decay.mixes", (len(MIXES), n, spec.dim), self.dtype)
         core.token_shift(x, kept, self.mu, batch.token_row, batch.cu_q, batch.row_slot, mixes)
         rkvg = ws.get("decay.rkvg", (n, 4 * self.width), self.dtype)
-        for i, (weight, act) in enumerate(((self.w_r, 0), (self.w_k, 0), (self.w_v, 0), (self.w_g, self._silu))):
-            linear(mixes[i], weight, None, rkvg[:, i * self.width:(i + 1) * self.width], act=act)
         low = ws.get("decay.low", (n, self.w_1.shape[0]), self.dtype)
-        linear(mixes[4], self.w_1, None, low, act=self._tanh)
+        r, k, v, g = (rkvg[:, i * self.width:(i + 1) * self.width] for i in range(4))
+        weights, outs = (self.w_r, self.w_k, self.w_v, self.w_g, self.w_1), (r, k, v, g, low)
+        acts = (0, 0, 0, self._silu, self._tanh)
+        done = False
+        if self.dtype == torch.bfloat16:
+            from ..ops import fast
+            done = fast.linears_few_bf16(list(mixes), weights, outs, acts)
+        if not done:
+            for mix, weight, projected, act in zip(mixes, weights, outs, acts):
+                linear(mix, weight, None, projected, act=act)
+        out = ws.get("decay.out", (n, self.width), self.dtype)
+        if batch.decode_only and core.decayed_step(r, k, v, g, low, self.w_2, self.w_0, self.u, self.gain, state, x, batch.row_slot, out,
+                                                   spec.n_heads, spec.head_dim, spec.eps):
+            return out
         pre = ws.get("decay.pre", (n, self.width), torch.float32)
         linear(low, self.w_2, self.w_0, pre)
-        out = ws.get("decay.out", (n, self.width), self.dtype)
-        r, k, v, g = (rkvg[:, i * self.width:(i + 1) * self.width] for i in range(4))
         raw = ws.get("decay.raw", (n, self.width), torch.float32)
         operands = (r, k, v, g, pre, self.u, self.gain, state, x, batch.cu_q, batch.row_slot, out, spec.n_heads, spec.head_dim, spec.eps)
         if self.dtype == torch.bfloat16 and not batch.decode_only and n >= self.CHUNKS_FROM_TOKENS:
