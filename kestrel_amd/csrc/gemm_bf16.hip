@@ -339,6 +339,157 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
     return 0;
 }
 
+// The two last linears of a block whose branches run side by side, out += A1 W1^T + A2 W2^T, for more rows than the
+// weight-streaming kernels take and fewer than fill the chip with tiles of the output: K of both, one behind the other, is cut
+// into `parts` parts of `per` K-steps (grid y), and a part's sums go out as fp32 [M, N] of its own, which the kernel that
+// finishes the rows adds up (with both biases, the residual and the next block's norm).
+struct PairTilesArgs {
+    const bf16_t* A[2];     // [M, K[s]]
+    const bf16_t* W[2];     // [N, K[s]]
+    long lda[2], ldw[2];
+    int steps[2];           // K[s] / BK
+    int M, N, tiles_n, tiles_m, per;
+    float* partial;         // [parts, M, N]
+};
+
+// The rows of A are the product's first operand here: a lane then holds one column of 16 rows, and a store of the wave covers
+// two rows of 128 bytes, whole lines of the memory, without a pass through LDS.
+template <int WN, int WM, int GN, int GM, int BK, int NS, int SL>
+__global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(GN * GM / 4, GN * GM / 4)))
+pair_tiles_kernel(PairTilesArgs p) {
+    using T = KdTile<WN, WM, GN, GM, BK, NS>;
+    constexpr int CPR = T::CPR;
+    extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
+    const int total = p.tiles_n * p.tiles_m, per_xcd = (total + 7) / 8;
+    const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;        // an XCD's tiles: neighbours in N, whose rows of W they share
+    if (logical >= total) return;
+    const int m0 = (logical % p.tiles_m) * T::BN, n0 = (logical / p.tiles_m) * T::BM;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KA_WAVE), lane = tid % KA_WAVE;
+    const int lo = blockIdx.y * p.per, hi = min(lo + p.per, p.steps[0] + p.steps[1]);
+
+    floatx16 acc[WN][WM];
+#pragma unroll
+    for (int a = 0; a < WN; ++a)
+#pragma unroll
+        for (int b = 0; b < WM; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+#pragma unroll 1
+    for (int s = 0; s < 2; ++s) {
+        const int before = s ? p.steps[0] : 0;
+        const int first = max(lo - before, 0), last = min(hi - before, p.steps[s]);
+        if (first >= last) continue;                     // (the same for the whole workgroup)
+        const bf16_t* const A = p.A[s] + (size_t)first * BK;
+        const bf16_t* const W = p.W[s] + (size_t)first * BK;
+        const bf16_t* asrc[T::W_LOADS];
+        const bf16_t* wsrc[T::X_LOADS];
+#pragma unroll
+        for (int i = 0; i < T::W_LOADS; ++i) {
+            const int r = kd_load_row<CPR>(wave * T::W_LOADS + i, lane);
+            asrc[i] = A + (size_t)min(m0 + r, p.M - 1) * p.lda[s] + kd_load_channel<CPR>(r, lane);
+        }
+#pragma unroll
+        for (int i = 0; i < T::X_LOADS; ++i) {
+            const int r = kd_load_row<CPR>(wave * T::X_LOADS + i, lane);
+            wsrc[i] = W + (size_t)min(n0 + r, p.N - 1) * p.ldw[s] + kd_load_channel<CPR>(r, lane);
+        }
+        // everybody has read the last stage of the segment before
+        gd_wait_lds();
+        gd_barrier();
+        kd_product<WN, WM, GN, GM, BK, NS, SL>(gb_lds, wave, lane, (last - first) * BK, asrc, wsrc, acc);
+    }
+
+    float* const mine = p.partial + (size_t)blockIdx.y * p.M * p.N;
+    const int wn = wave / GM, wm = wave % GM, li = lane % 32, lg = lane / 32;
+#pragma unroll
+    for (int b = 0; b < WM; ++b) {
+        const int n = n0 + wm * 32 * WM + b * 32 + li;
+        if (n >= p.N) continue;
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = m0 + wn * 32 * WN + a * 32 + (v / 4) * 8 + lg * 4 + v % 4;
+                if (m < p.M) mine[(size_t)m * p.N + n] = acc[a][b][v];
+            }
+    }
+}
+
+// Bound by the K-steps that follow one another on a CU, 0.5 to 0.6 us each whatever the stages in flight (three to five: 73 to
+// 71 us for K = 8,192 alone on 64 CUs): parts of K spread them over all CUs. Measured with the norm that follows, against the
+// vendor library's two products and the norm's launch (us; K = 2,560 + 10,240, N = 2,560): 128 rows 31 against 78, 512 rows
+// 57 (three parts) against 83, 1,024 rows 106 against 117.
+constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5;
+
+// Parts of K for `ka_linear_pair_tiles_bf16`: as many as leave the fewest K-steps to a CU, a part more than another costing
+// the finishing kernel one more read of the output.
+static int pair_tiles_parts(int M, int N, int steps, long partial_floats) {
+    const int cus = ka_compute_units();
+    const long tiles = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
+    int best = 0;
+    double best_cost = 0;
+    for (int parts = 1; parts <= 8 && (long)parts * M * N <= partial_floats; ++parts) {
+        const int per = ka_cdiv(steps, parts);
+        if ((parts > 1 && per < 4) || ka_cdiv(steps, per) != parts) continue;
+        const double rounds = (double)((tiles * parts + cus - 1) / cus);
+        const double cost = rounds * (per + 8) * 0.55 + parts * (double)M * N * 8.0 / 4.0e6;     // us
+        if (best == 0 || cost < best_cost) { best = parts; best_cost = cost; }
+    }
+    return best;
+}
+
+KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats) {
+    if (M < 1 || N < 1 || N % 4 || K1 % PT_BK || K2 % PT_BK || K1 < PT_BK || K2 < PT_BK) return 0;
+    return pair_tiles_parts(M, N, (K1 + K2) / PT_BK, partial_floats);
+}
+
+KA_API int ka_linear_pair_tiles_bf16(const void* A1, long lda1, int K1, const void* A2, long lda2, int K2, const void* W1, long ldw1,
+                                     const float* bias1, const void* W2, long ldw2, const float* bias2, float* out, long ldo, int N,
+                                     int accumulate, int M, int parts, float* partials, long partial_floats, const float* gamma,
+                                     const float* beta, float eps, void* normed, int normed_dtype, long ldn, hipStream_t stream) {
+    const char* who = "ka_linear_pair_tiles_bf16";
+    KA_CHECK(M > 0 && N > 0 && N % 4 == 0, "%s: M=%d N=%d (N must be a multiple of 4)", who, M, N);
+    KA_CHECK(K1 >= PT_BK && K2 >= PT_BK && K1 % PT_BK == 0 && K2 % PT_BK == 0, "%s: K must be multiples of %d, got %d and %d", who, PT_BK, K1, K2);
+    KA_CHECK(lda1 % 8 == 0 && ldw1 % 8 == 0 && lda2 % 8 == 0 && ldw2 % 8 == 0 && lda1 >= K1 && ldw1 >= K1 && lda2 >= K2 && ldw2 >= K2,
+             "%s: row strides must be multiples of 8 and >= K", who);
+    KA_CHECK(((uintptr_t)A1 | (uintptr_t)A2 | (uintptr_t)W1 | (uintptr_t)W2 | (uintptr_t)out | (uintptr_t)partials) % 16 == 0,
+             "%s: operands must be 16-byte aligned", who);
+    KA_CHECK(((uintptr_t)bias1 | (uintptr_t)bias2) % 16 == 0 || !gamma, "%s: biases must be 16-byte aligned beside a norm", who);
+    KA_CHECK(ldo >= N && ldo % 4 == 0, "%s: output stride %ld for N=%d", who, ldo, N);
+    const int steps = (K1 + K2) / PT_BK;
+    KA_CHECK(parts >= 1 && parts <= steps && partials && (long)parts * M * N <= partial_floats, "%s: %d parts of %d steps, %ld floats", who, parts, steps,
+             partial_floats);
+    PairTilesArgs p;
+    p.A[0] = (const bf16_t*)A1; p.lda[0] = lda1; p.W[0] = (const bf16_t*)W1; p.ldw[0] = ldw1; p.steps[0] = K1 / PT_BK;
+    p.A[1] = (const bf16_t*)A2; p.lda[1] = lda2; p.W[1] = (const bf16_t*)W2; p.ldw[1] = ldw2; p.steps[1] = K2 / PT_BK;
+    p.M = M; p.N = N; p.tiles_n = ka_cdiv(N, PT_TILE); p.tiles_m = ka_cdiv(M, PT_TILE);
+    p.per = ka_cdiv(steps, parts);
+    parts = ka_cdiv(steps, p.per);
+    p.partial = partials;
+    const long total = (long)p.tiles_n * p.tiles_m, launched = ((total + 7) / 8) * 8;
+    KA_CHECK(launched < (1L << 31), "%s: too many tiles", who);
+    auto kernel = pair_tiles_kernel<1, 2, 4, 2, PT_BK, PT_STAGES, 2>;
+    constexpr int smem = KdTile<1, 2, 4, 2, PT_BK, PT_STAGES>::SMEM;
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        KA_CHECK(e == hipSuccess, "%s: cannot reserve %d bytes of LDS: %s", who, smem, hipGetErrorString(e));
+        configured = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)launched, parts), dim3(512), smem, stream, p);
+    KA_LAUNCH_CHECK();
+    if (gamma) {
+        const KaThenNorm then = {gamma, beta, eps, normed, normed_dtype, ldn};
+        KA_CHECK(ka_then_norm_fits(N) && normed && ldn >= N && ldn % 4 == 0, "%s: cannot normalise rows of %d", who, N);
+        ka_launch_finish_norm(M, N, stream, partials, parts, bias1, bias2, out, ldo, accumulate, then);
+    } else {
+        hipLaunchKernelGGL(ka_partials_finish_kernel, dim3(ka_cdiv((long)M * (N / 4), 256)), dim3(256), 0, stream, partials, parts, bias1, bias2,
+                           out, KA_F32, ldo, M, N, KA_ACT_NONE, accumulate);
+    }
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
 template <int NT, int MT, int BK>
 static int launch_config(const bf16_t* A, long lda, const bf16_t* W, long ldw, const float* bias, void* out,
                          int out_dtype, long ldo, int M, int N, int K, int act, int accumulate,

@@ -82,7 +82,8 @@ static inline bool ka_then_norm_fits(int N) { return N % 4 == 0 && N <= KA_ROW_T
 // thread needs is asked for at once, from places moved inside the row where the thread has nothing
 // there: one trip to memory whatever the width (a row of 2560, whose second four only a quarter of
 // the threads have, took two: 6.6 us against 5.1 for a row of 2048).
-template <int JN>
+// U: parts asked for at once, four or eight (a part past the last is the last again, asked for in vain).
+template <int JN, int U>
 static __global__ void __launch_bounds__(KA_ROW_THREADS)
 ka_partials_finish_norm_kernel(const float* __restrict__ partial, int splits, const float* __restrict__ bias,
                                const float* __restrict__ bias2, float* __restrict__ out, long ldo, int M, int N,
@@ -92,7 +93,7 @@ ka_partials_finish_norm_kernel(const float* __restrict__ partial, int splits, co
     __shared__ float red[2][WAVES];
     const int m = blockIdx.x, quads = N / 4;
     const int wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
-    ka_floatx4 x[JN], g[JN], b[JN], first[JN][8], extra[JN][2];
+    ka_floatx4 x[JN], g[JN], b[JN], first[JN][U], extra[JN][2];
     const ka_floatx4 zero = ka_floatx4{0.f, 0.f, 0.f, 0.f};
     float sum = 0.f;
 #pragma unroll
@@ -103,7 +104,7 @@ ka_partials_finish_norm_kernel(const float* __restrict__ partial, int splits, co
         x[j] = *reinterpret_cast<const ka_floatx4*>(out + (size_t)m * ldo + n);
         if (splits > 0) {                                      // (the same for all threads)
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < U; ++u)
                 first[j][u] = *reinterpret_cast<const ka_floatx4*>(partial + ((size_t)min(u, splits - 1) * M + m) * N + n);
             extra[j][0] = bias ? *reinterpret_cast<const ka_floatx4*>(bias + n) : zero;
             extra[j][1] = bias2 ? *reinterpret_cast<const ka_floatx4*>(bias2 + n) : zero;
@@ -118,15 +119,15 @@ ka_partials_finish_norm_kernel(const float* __restrict__ partial, int splits, co
         if (splits > 0) {
             ka_floatx4 s = zero;
 #pragma unroll
-            for (int u = 0; u < 8; ++u)                        // the parts in their order
+            for (int u = 0; u < U; ++u)                        // the parts in their order
                 if (u < splits) s += first[j][u];
-            for (int sp0 = 8; sp0 < splits; sp0 += 8) {        // more than eight parts: eight more at a time
-                ka_floatx4 p[8];
+            for (int sp0 = U; sp0 < splits; sp0 += U) {        // more parts: as many more at a time
+                ka_floatx4 p[U];
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
+                for (int u = 0; u < U; ++u)
                     p[u] = *reinterpret_cast<const ka_floatx4*>(partial + ((size_t)min(sp0 + u, splits - 1) * M + m) * N + n);
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
+                for (int u = 0; u < U; ++u)
                     if (sp0 + u < splits) s += p[u];
             }
             s += extra[j][0];
@@ -184,10 +185,22 @@ ka_partials_finish_norm_kernel(const float* __restrict__ partial, int splits, co
 static inline void ka_launch_finish_norm(int M, int N, hipStream_t stream, const float* partial, int splits, const float* bias,
                                          const float* bias2, float* out, long ldo, int accumulate, const KaThenNorm& then) {
     const int fours = (N / 4 + KA_ROW_THREADS - 1) / KA_ROW_THREADS;
-    switch (fours) {
-        case 1: hipLaunchKernelGGL(ka_partials_finish_norm_kernel<1>, dim3(M), dim3(KA_ROW_THREADS), 0, stream, partial, splits, bias, bias2, out, ldo, M, N, accumulate, then); break;
-        case 2: hipLaunchKernelGGL(ka_partials_finish_norm_kernel<2>, dim3(M), dim3(KA_ROW_THREADS), 0, stream, partial, splits, bias, bias2, out, ldo, M, N, accumulate, then); break;
-        case 3: hipLaunchKernelGGL(ka_partials_finish_norm_kernel<3>, dim3(M), dim3(KA_ROW_THREADS), 0, stream, partial, splits, bias, bias2, out, ldo, M, N, accumulate, then); break;
-        default: hipLaunchKernelGGL(ka_partials_finish_norm_kernel<4>, dim3(M), dim3(KA_ROW_THREADS), 0, stream, partial, splits, bias, bias2, out, ldo, M, N, accumulate, then); break;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(M), dim3(KA_ROW_THREADS), 0, stream, partial, splits, bias, bias2, out, ldo, M, N, accumulate, then);
+    };
+    if (splits <= 4) {
+        switch (fours) {
+            case 1: launch(ka_partials_finish_norm_kernel<1, 4>); break;
+            case 2: launch(ka_partials_finish_norm_kernel<2, 4>); break;
+            case 3: launch(ka_partials_finish_norm_kernel<3, 4>); break;
+            default: launch(ka_partials_finish_norm_kernel<4, 4>); break;
+        }
+    } else {
+        switch (fours) {
+            case 1: launch(ka_partials_finish_norm_kernel<1, 8>); break;
+            case 2: launch(ka_partials_finish_norm_kernel<2, 8>); break;
+            case 3: launch(ka_partials_finish_norm_kernel<3, 8>); break;
+            default: launch(ka_partials_finish_norm_kernel<4, 8>); break;
+        }
     }
 }

@@ -36,6 +36,12 @@ _SIGNATURES = {
         _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long,  # out, ldo, N, accumulate, M, target_waves, partial sums
         _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_long, _c_void_p],  # gamma, beta, eps, normed, its type and stride, stream
     "ka_linear_skinny_pair_in_parts": [_c_int, _c_int],
+    "ka_linear_pair_tiles_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
+    "ka_linear_pair_tiles_bf16": [
+        _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_int,                     # A1, lda1, K1, A2, lda2, K2
+        _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_void_p,               # W1, ldw1, bias1, W2, ldw2, bias2
+        _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long,     # out, ldo, N, accumulate, M, parts, partial sums
+        _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_long, _c_void_p],     # gamma, beta, eps, normed, its type and stride, stream
     "ka_linear_library_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
                                _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long, _c_void_p],
     "ka_linear_tiled_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
@@ -126,6 +132,11 @@ LIBRARY_WORKSPACE_BYTES = 128 << 20
 _ACTIVATIONS_APART = (4,)
 ACTIVATION_APART_FROM_ROWS = 256
 ACTIVATION_APART_FROM_COLUMNS = 1024
+# Tiles of 128 x 128 of the output up to which a block's two last linears go by tiles with K in parts rather than one after
+# the other to the vendor library, with the norm that follows (us, K = 2,048 + 8,192 at N = 2,048 and 2,560 + 10,240 at 2,560):
+# 65 rows 19 against 29 and 27 against 71, 256 rows 28 against 40 and 38 against 70, 512 rows 40 against 56 and 57 against 83,
+# 160 tiles (1,280 and 1,024 rows) 83 against 93 and 106 against 117; beyond, 192 tiles 99 against 94 and 200 tiles 133 both.
+PAIR_TILES_MAX = 160
 _library_space = {}
 SCRATCH_FLOATS = 8 << 20
 WIDE_FLOATS = 8 << 20              # 32 MB of partial sums for the wide skinny kernel
@@ -353,20 +364,24 @@ def linear_bf16(a, weight, bias, out, act, accumulate) -> bool:
 
 
 def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumulate: bool = True) -> bool:
-    """``out += a1 @ w1.T + b1 + a2 @ w2.T + b2`` in one launch (few rows, fp32 ``out``); with ``accumulate`` off
-    the sum replaces ``out``.
+    """``out += a1 @ w1.T + b1 + a2 @ w2.T + b2`` in one launch (few rows, fp32 ``out``), or in two by tiles with K of both
+    in parts (``pair_tile_parts``); with ``accumulate`` off the sum replaces ``out``.
     ``then_norm = (gamma, beta or None, eps, normed)``: also ``normed = LayerNorm(out)``, in the kernel
     that finishes the rows where there is one (more than 8 rows), else in a launch behind it. False:
     not covered, nothing was run (with ``then_norm``: try without)."""
     m, k1 = a1.shape
     k2 = a2.shape[1]
     n = w1.shape[0]
-    if not (0 < m <= SKINNY_MAX_ROWS) or k1 % 8 or k2 % 8 or a2.shape[0] != m or w2.shape[0] != n:
+    parts = pair_tile_parts(m, n, k1, k2)
+    if not (0 < m <= SKINNY_MAX_ROWS or parts) or k1 % 8 or k2 % 8 or a2.shape[0] != m or w2.shape[0] != n:
         return False
     if not (_operand_ok(a1, k1) and _operand_ok(w1, k1) and _operand_ok(a2, k2) and _operand_ok(w2, k2)):
         return False
     if out.dtype != torch.float32 or not _out_ok(out, m, n) or not _bias_ok(b1, n) or not _bias_ok(b2, n):
         return False
+    if parts and (out.stride(0) % 4 or any(b is not None and b.data_ptr() % 16 for b in (b1, b2))):
+        return False
+    gamma = beta = normed = None
     if then_norm is not None:
         gamma, beta, eps, normed = then_norm
         if n % 4 or n > NORM_AFTER_MAX_WIDTH or out.stride(0) % 4 or normed.dtype not in _OUT_CODE or not _out_ok(normed, m, n) \
@@ -376,6 +391,14 @@ def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumula
             return False
         if any(b is not None and b.data_ptr() % 16 for b in (b1, b2)):
             return False
+    if parts:
+        _check(lib().ka_linear_pair_tiles_bf16(
+            a1.data_ptr(), a1.stride(0), k1, a2.data_ptr(), a2.stride(0), k2, w1.data_ptr(), w1.stride(0), _ptr(b1),
+            w2.data_ptr(), w2.stride(0), _ptr(b2), out.data_ptr(), out.stride(0), n, int(bool(accumulate)), m, parts,
+            *_wide_args(a1.device, m), _ptr(gamma), _ptr(beta), float(eps) if then_norm is not None else 0.0, _ptr(normed),
+            _OUT_CODE[normed.dtype] if then_norm is not None else 0, normed.stride(0) if then_norm is not None else 0, stream_ptr()))
+        return True
+    if then_norm is not None:
         _check(lib().ka_linear_skinny_pair_norm(
             a1.data_ptr(), a1.stride(0), k1, a2.data_ptr(), a2.stride(0), k2, w1.data_ptr(), w1.stride(0), _ptr(b1),
             w2.data_ptr(), w2.stride(0), _ptr(b2), out.data_ptr(), out.stride(0), n, int(bool(accumulate)), m, chip_sizes(a1.device).skinny_target_waves,
@@ -388,6 +411,14 @@ def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumula
         w1.data_ptr(), w1.stride(0), _ptr(b1), out.data_ptr(), KA_F32, out.stride(0), n, 0, int(bool(accumulate)),
         None, 0, None, None, 0, 0, 0, 0, m, chip_sizes(a1.device).skinny_target_waves, *_wide_args(a1.device, m), stream_ptr()))
     return True
+
+
+def pair_tile_parts(m: int, n: int, k1: int, k2: int) -> int:
+    """Parts that ``linear_pair_accumulate`` cuts K of both linears into, one behind the other, where it takes them by
+    tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles)."""
+    if m <= SKINNY_MAX_ROWS or -(-m // 128) * -(-n // 128) > PAIR_TILES_MAX:
+        return 0
+    return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, WIDE_FLOATS)
 
 
 def pair_finishes_rows(m: int, n: int) -> bool:

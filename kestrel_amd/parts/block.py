@@ -14,19 +14,23 @@ from .streams import StreamReading
 def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) -> bool:
     """The parallel block for a few bf16 rows in three launches: norm + both first linears, the
     mixer's core, both last linears + residual. Needs a mixer and a feed-forward that offer their
-    stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise.
+    stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise. More rows, as long as the two last
+    linears are one product of tiles (``fast.pair_tile_parts``): the first linears are launches of their own then, and
+    a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
     ``normed``: the block's norm of ``x``, where the block before has computed it; ``then``: the norm
     the next block starts with, which the last launch computes as well where it pays (``handed``, a
     list, then gets the normalised rows)."""
     from ..ops import fast
-    from ..ops.linear import linear
+    from ..ops.linear import ACT_GATED, linear
 
     n = x.shape[0]
-    if block.dtype != torch.bfloat16 or n > fast.SKINNY_MAX_ROWS or block.feed_forward is None:
+    if block.dtype != torch.bfloat16 or block.feed_forward is None:
         return False
     m_in, f_in = block.mixer.input_projection(), block.feed_forward.input_projection()
     m_out, f_out = block.mixer.output_projection(), block.feed_forward.output_projection()
     if m_in is None or f_in is None or m_out is None or f_out is None:
+        return False
+    if n > fast.SKINNY_MAX_ROWS and (f_in[3] & ACT_GATED or not fast.pair_tile_parts(n, x.shape[1], m_out[0].shape[1], f_out[0].shape[1])):
         return False
     ws = batch.workspace
     projected = ws.get("block.mixer_in", (n, m_in[2]), block.dtype)
@@ -54,8 +58,10 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
         else:
             fused = fast.layernorm_linear(x, *ln, m_in[0], m_in[1], projected, 0, f_in[0], f_in[1], hidden, f_in[3])
     if not fused:
-        h = ws.get("block.h", tuple(x.shape), block.dtype)
-        norm.forward(x, h)
+        h = normed
+        if h is None:
+            h = ws.get("block.h", tuple(x.shape), block.dtype)
+            norm.forward(x, h)
         if not fast.linear_two_outputs(h, m_in[0], m_in[1], projected, 0, f_in[0], f_in[1], hidden, f_in[3]):
             linear(h, m_in[0], m_in[1], projected)
             linear(h, f_in[0], f_in[1], hidden, act=f_in[3])
@@ -181,7 +187,7 @@ def _two_branches_by_stages(block: "Block", h1, h2, batch, cache, delta) -> bool
         hidden = ws.get("block.ff_hidden", (n, f_in[2]), block.dtype)
         linear(h2, f_in[0], f_in[1], hidden, act=f_in[3])
     mixed = block.mixer.attend(projected, batch, cache)
-    if ff is not None and block.dtype == torch.bfloat16 and n <= fast.SKINNY_MAX_ROWS and \
+    if ff is not None and block.dtype == torch.bfloat16 and \
             fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], delta, accumulate=False):
         return True
     linear(mixed, m_out[0], m_out[1], delta)
