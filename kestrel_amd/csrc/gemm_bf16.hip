@@ -421,6 +421,56 @@ pair_tiles_kernel(PairTilesArgs p) {
 // 57 (three parts) against 83, 1,024 rows 106 against 117.
 constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5;
 
+template <int WN, int WM, int GN, int GM, int NS, int SL>
+static int launch_pair_tiles(PairTilesArgs& p, int parts, hipStream_t stream) {
+    using T = KdTile<WN, WM, GN, GM, PT_BK, NS>;
+    static bool configured = false;
+    auto kernel = pair_tiles_kernel<WN, WM, GN, GM, PT_BK, NS, SL>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM);
+        KA_CHECK(e == hipSuccess, "linear by tiles: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
+        configured = true;
+    }
+    p.tiles_m = ka_cdiv(p.M, T::BN);
+    p.tiles_n = ka_cdiv(p.N, T::BM);
+    const long launched = (((long)p.tiles_n * p.tiles_m + 7) / 8) * 8;
+    KA_CHECK(launched < (1L << 31), "linear by tiles: too many tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)launched, parts), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, p);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// Few rows (at most 64) through the same kernel, for the weight-streaming launcher: the sums of one linear, or of two added up,
+// in parts in `partial`. Returns the number of parts, 0 where the operands are not covered, -1 on an error. Bound by the weights'
+// way from HBM: what counts is that every CU has 64 KB of loads in flight, which the stages in LDS hold without registers. Tiles
+// of 64 rows by 64 weight rows, five stages in half of a CU's LDS, or by 128 and three where an output is so wide that tiles of
+// 64 alone fill half of the chip; as many parts as give every CU a workgroup (twice as many: 1 to 2 us more). At 40 rows, us,
+// the launch that adds up included, against the wide kernel of the weight-streaming file: N = 2,048, K = 2,048 + 8,192: 15.7
+// and 18.6; 2,560, 2,560 + 10,240: 22.0 and 25.7; without that launch (4 to 5 us): N = K = 4,096: 9.5 and 12; 12,288 by 4,096:
+// 22.4 and 28; 4,096 by 12,288: 19.8 and 25. Tiles of 32 rows for up to 32 gave the same.
+int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
+    if (f.M > 64 || f.K[0] % PT_BK || f.K[1] % PT_BK || f.K[0] < PT_BK || !f.partial) return 0;
+    PairTilesArgs p = {};
+    for (int s = 0; s < 2; ++s) {
+        p.A[s] = (const bf16_t*)f.A[s]; p.lda[s] = f.lda[s];
+        p.W[s] = (const bf16_t*)f.W[s]; p.ldw[s] = f.ldw[s];
+        p.steps[s] = f.K[s] / PT_BK;
+    }
+    p.M = f.M; p.N = f.N; p.partial = f.partial;
+    const int steps = p.steps[0] + p.steps[1], cus = ka_compute_units();
+    const bool wide = ka_cdiv(f.N, 64) * 2 > cus;
+    int parts = cus / ka_cdiv(f.N, wide ? 128 : 64);
+    if (parts > 8) parts = 8;                            // (what the finishing kernel asks for at once)
+    if (parts > steps / 4) parts = steps / 4;
+    if (parts < 1) parts = 1;
+    while (parts > 1 && (long)parts * f.M * f.N > f.partial_floats) --parts;
+    if ((long)parts * f.M * f.N > f.partial_floats) return 0;
+    p.per = ka_cdiv(steps, parts);
+    parts = ka_cdiv(steps, p.per);
+    if (wide ? launch_pair_tiles<1, 1, 2, 4, 3, 2>(p, parts, stream) : launch_pair_tiles<1, 1, 2, 2, 5, 2>(p, parts, stream)) return -1;
+    return parts;
+}
+
 // Parts of K for `ka_linear_pair_tiles_bf16`: as many as leave the fewest K-steps to a CU, a part more than another costing
 // the finishing kernel one more read of the output.
 static int pair_tiles_parts(int M, int N, int steps, long partial_floats) {
@@ -462,22 +512,11 @@ KA_API int ka_linear_pair_tiles_bf16(const void* A1, long lda1, int K1, const vo
     PairTilesArgs p;
     p.A[0] = (const bf16_t*)A1; p.lda[0] = lda1; p.W[0] = (const bf16_t*)W1; p.ldw[0] = ldw1; p.steps[0] = K1 / PT_BK;
     p.A[1] = (const bf16_t*)A2; p.lda[1] = lda2; p.W[1] = (const bf16_t*)W2; p.ldw[1] = ldw2; p.steps[1] = K2 / PT_BK;
-    p.M = M; p.N = N; p.tiles_n = ka_cdiv(N, PT_TILE); p.tiles_m = ka_cdiv(M, PT_TILE);
+    p.M = M; p.N = N;
     p.per = ka_cdiv(steps, parts);
     parts = ka_cdiv(steps, p.per);
     p.partial = partials;
-    const long total = (long)p.tiles_n * p.tiles_m, launched = ((total + 7) / 8) * 8;
-    KA_CHECK(launched < (1L << 31), "%s: too many tiles", who);
-    auto kernel = pair_tiles_kernel<1, 2, 4, 2, PT_BK, PT_STAGES, 2>;
-    constexpr int smem = KdTile<1, 2, 4, 2, PT_BK, PT_STAGES>::SMEM;
-    static bool configured = false;
-    if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        KA_CHECK(e == hipSuccess, "%s: cannot reserve %d bytes of LDS: %s", who, smem, hipGetErrorString(e));
-        configured = true;
-    }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)launched, parts), dim3(512), smem, stream, p);
-    KA_LAUNCH_CHECK();
+    if (launch_pair_tiles<1, 2, 4, 2, PT_STAGES, 2>(p, parts, stream)) return -1;
     if (gamma) {
         const KaThenNorm then = {gamma, beta, eps, normed, normed_dtype, ldn};
         KA_CHECK(ka_then_norm_fits(N) && normed && ldn >= N && ldn % 4 == 0, "%s: cannot normalise rows of %d", who, N);

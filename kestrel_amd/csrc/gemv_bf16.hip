@@ -549,6 +549,18 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
                                       Wb, ldwb, biasb, outb, out_dtype_b, ldob, Nb, actb, 0, nullptr, 0, nullptr,
                                       nullptr, 0, 0, 0, 0, M, target_waves, partials, partial_floats, stream);
     }
+    auto finish_parts = [&](int parts) {
+        if (then) {
+            // the finishing kernel takes whole rows and normalises them as well
+            ka_launch_finish_norm(M, Na, stream, partials, parts, biasa, A2 ? bias2 : nullptr, (float*)outa, ldoa, accumulate_a, *then);
+        } else {
+            const int quads = M * ka_cdiv(Na, 4);
+            hipLaunchKernelGGL(ka_partials_finish_kernel, dim3(ka_cdiv(quads, 256)), dim3(256), 0, stream, partials, parts,
+                               biasa, A2 ? bias2 : nullptr, outa, out_dtype_a, ldoa, M, Na, acta, accumulate_a);
+        }
+        KA_LAUNCH_CHECK();
+        return 0;
+    };
     // Up to 16 rows of two segments: where there are more strips than CUs the split kernel,
     // which gives a strip to a workgroup, takes about twice the time that it takes with one
     // strip a CU (N = 2560, K = 2560 + 10240, 16 rows: 40 us; 25 us here).
@@ -557,6 +569,14 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
     // 18.3 at 16 (N = 2048, K = 2048 + 8192).
     const bool crowded = A2 && M <= 16 && ka_linear_skinny_pair_in_parts(M, Na);      // (a single row: 19 us against 24)
     if (!Wb && partials && ((sk_wide_enabled && (M > 16 ? (A2 || !persistent_ok) : crowded)) || sk_wide_enabled >= 2)) {
+        // by tiles of 64 rows where K comes in whole K-steps (measured there), else by the wide kernel
+        KaFewRows few = {};
+        few.A[0] = args.A[0]; few.lda[0] = args.lda[0]; few.W[0] = args.a.W; few.ldw[0] = args.a.ldw; few.K[0] = K1;
+        if (A2) { few.A[1] = args.A[1]; few.lda[1] = args.lda[1]; few.W[1] = args.W2; few.ldw[1] = args.ldw2; few.K[1] = K2; }
+        few.M = M; few.N = Na; few.partial = partials; few.partial_floats = partial_floats;
+        int parts = ka_few_rows_by_tiles(few, stream);
+        if (parts < 0) return -1;
+        if (parts > 0) return finish_parts(parts);
         WideArgs wide = {};
         wide.A[0] = args.A[0]; wide.lda[0] = args.lda[0]; wide.W[0] = args.a.W; wide.ldw[0] = args.a.ldw; wide.K[0] = K1;
         if (A2) { wide.A[1] = args.A[1]; wide.lda[1] = args.lda[1]; wide.W[1] = args.W2; wide.ldw[1] = args.ldw2; wide.K[1] = K2; }
@@ -580,16 +600,7 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
                 default: hipLaunchKernelGGL(skinny_wide_kernel<4>, grid, dim3(WD_WAVES * KA_WAVE), 0, stream, wide); break;
             }
             KA_LAUNCH_CHECK();
-            if (then) {
-                // the finishing kernel takes whole rows and normalises them as well
-                ka_launch_finish_norm(M, Na, stream, partials, splits, biasa, A2 ? bias2 : nullptr, (float*)outa, ldoa, accumulate_a, *then);
-            } else {
-                const int quads = M * ka_cdiv(Na, 4);
-                hipLaunchKernelGGL(ka_partials_finish_kernel, dim3(ka_cdiv(quads, 256)), dim3(256), 0, stream, partials, splits,
-                                   biasa, A2 ? bias2 : nullptr, outa, out_dtype_a, ldoa, M, Na, acta, accumulate_a);
-            }
-            KA_LAUNCH_CHECK();
-            return 0;
+            return finish_parts(splits);
         }
     }
     // (where K was not cut into parts, a norm that follows is a launch of its own: the same kernel, no parts)

@@ -8,6 +8,19 @@
 
 typedef __attribute__((ext_vector_type(4))) float ka_floatx4;
 
+// The operands of a linear of few rows, or of two whose results are added up (K[1] = 0: one), [M, K[s]] by [N, K[s]] in bf16, rows
+// 16-byte aligned, and where the parts' sums go.
+struct KaFewRows {
+    const void* A[2];
+    const void* W[2];
+    long lda[2], ldw[2];
+    int K[2];
+    int M, N;
+    float* partial;
+    long partial_floats;
+};
+int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream);
+
 // out = act(sum of the parts + biases) (+ out): one thread per four neighbouring outputs
 static __global__ void __launch_bounds__(256)
 ka_partials_finish_kernel(const float* __restrict__ partial, int splits, const float* __restrict__ bias,

@@ -55,6 +55,23 @@ def test_pair_by_tiles(m, n, k1, k2, bias):
         assert bool(((normed.double().cpu() - want).abs() <= (2.0 ** -8 + 2.0 ** -16) * want.abs() + 2.0 ** -14 * (1 + gamma.double().abs())).all())
 
 
+# few rows: one row tile, weight tiles of 64 and of 128, parts in either linear and across the border
+@pytest.mark.parametrize("m, n, k1, k2", [(17, 64, 64, 64), (33, 516, 192, 2048), (64, 2050, 2048, 320), (40, 8260, 320, 64), (64, 16400, 64, 512)])
+def test_few_rows_of_a_pair_by_tiles(m, n, k1, k2):
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(m + n + k1)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    a1, a2, w1, w2 = rnd(m, k1).bfloat16(), rnd(m, k2 + 8).bfloat16(), rnd(n, k1 + 8).bfloat16(), rnd(n, k2).bfloat16()
+    x, bias = rnd(m, n), rnd(n)
+    d = lambda t: t.to(DEV)  # noqa: E731
+    stream = d(x)
+    assert fast.linear_pair_accumulate(d(a1), d(w1)[:, :k1], d(bias), d(a2)[:, :k2], d(w2), None, stream)
+    exact = a1.double() @ w1[:, :k1].double().T + a2[:, :k2].double() @ w2.double().T + bias.double() + x.double()
+    terms = a1.double().abs() @ w1[:, :k1].double().abs().T + a2[:, :k2].double().abs() @ w2.double().abs().T + bias.double().abs() + x.double().abs()
+    _close_to_exact(stream, (terms, k1 + k2 + 2), exact)
+
+
 @pytest.mark.parametrize("m, n, k1, k2", [(64, 256, 64, 64), (65, 256, 72, 64), (65, 256, 64, 72), (65, 258, 64, 64), (1281, 2048, 128, 128)])
 def test_what_is_not_taken_by_tiles(m, n, k1, k2):
     """Rows that the weight-streaming kernels take, K that is no multiple of a step, odd widths, more tiles than the rule allows."""
