@@ -7,7 +7,7 @@ from typing import Dict, Optional
 import torch
 
 from ..ops import core
-from ..ops.linear import ACT_GATED, activation_code, linear, linear_gated, pair_rows
+from ..ops.linear import ACT_GATED, activation_code, linear, pair_rows
 from .base import FeedForward, register_feed_forward
 from .specs import ParamSpec, RoutedExpertsSpec
 
@@ -122,6 +122,14 @@ class RoutedExperts(FeedForward):
             self.shared_pairs = first_rows("shared").contiguous()
             self.shared_down = tensors["shared.down.weight"].to(device).contiguous()
 
+    def _shared_operands(self, n: int, ws):
+        """Where the shared expert's first linear of ``n`` rows goes, and its activation: the hidden rows, or, where the pairs have a
+        launch of their own (clamps; many rows), both sums of every pair."""
+        spec = self.spec
+        if self.gated and (self.shared_clamp is not None or (self.dtype == torch.bfloat16 and n >= 256)):
+            return ws.get("experts.shared_sums", (n, 2 * spec.shared_hidden), self.dtype), 0
+        return ws.get("experts.shared_hidden", (n, spec.shared_hidden), self.dtype), self.act | (ACT_GATED if self.gated else 0)
+
     def _outputs(self, h, batch):
         """Everything but the weighted sum: the pairs' outputs, the choice, its weights, the shared expert's output and gate."""
         spec = self.spec
@@ -129,7 +137,15 @@ class RoutedExperts(FeedForward):
         ws = batch.workspace
         top = spec.top + self.joined
         logits = ws.get("experts.logits", (n, self.router.shape[0]), torch.float32)
-        linear(h, self.router, self.router_bias, logits)
+        shared = self._shared_operands(n, ws) if self.shared and not self.joined else None
+        # Few rows: the router's linear, a few workgroups that wait for memory, beside the shared expert's first in one launch
+        # (eight rows of 2,048: about 5 us a layer, 3 % of a step).
+        beside = False
+        if shared is not None and self.dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16:
+            from ..ops import fast
+            beside = fast.linear_two_outputs(h, self.router, self.router_bias, logits, 0, self.shared_pairs, None, *shared)
+        if not beside:
+            linear(h, self.router, self.router_bias, logits)
         chosen = ws.get("experts.chosen", (n, top), torch.int32)
         weights = ws.get("experts.weights", (n, top), torch.float32)
         core.route(logits, self.n_outputs, self.correction, spec.top, spec.n_groups, spec.keep_groups, spec.scale, chosen, weights,
@@ -150,18 +166,16 @@ class RoutedExperts(FeedForward):
             core.experts_linear(hidden, 1, self.down, flat, y)
         shared_out = gate = None
         if self.shared and not self.joined:
-            shared_hidden = ws.get("experts.shared_hidden", (n, spec.shared_hidden), self.dtype)
-            if not self.gated:
-                linear(h, self.shared_pairs, None, shared_hidden, act=self.act)
-            elif self.shared_clamp is not None or (self.dtype == torch.bfloat16 and n >= 256):
-                sums = ws.get("experts.shared_sums", (n, 2 * spec.shared_hidden), self.dtype)
-                linear(h, self.shared_pairs, None, sums)
+            first, act = shared
+            if not beside:
+                linear(h, self.shared_pairs, None, first, act=act)
+            shared_hidden = first
+            if self.gated and not act & ACT_GATED:           # (the pairs' sums)
+                shared_hidden = ws.get("experts.shared_hidden", (n, spec.shared_hidden), self.dtype)
                 if self.shared_clamp is not None:
-                    core.clamped_pairs(sums, shared_hidden, self.shared_clamp.limit, self.shared_clamp.slope, self.shared_clamp.shift)
+                    core.clamped_pairs(first, shared_hidden, self.shared_clamp.limit, self.shared_clamp.slope, self.shared_clamp.shift)
                 else:
-                    core.gated_pairs(sums, shared_hidden, self.act)
-            else:
-                linear_gated(h, self.shared_pairs, None, shared_hidden, self.act)
+                    core.gated_pairs(first, shared_hidden, self.act)
             shared_out = ws.get("experts.shared_out", (n, spec.dim), torch.float32)
             linear(shared_hidden, self.shared_down, None, shared_out)
             if self.gated_shared:
