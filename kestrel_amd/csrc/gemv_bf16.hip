@@ -182,7 +182,7 @@ skinny_split_kernel(SkinnyArgs p) {
 }
 
 // ----------------------------------------------------------------------------
-// The wide kernel, for 17 to 64 rows. With that many rows the activations are what the kernels
+// The wide kernel, for 17 to 64 rows of a K in no steps of 64 (else ka_few_rows_by_tiles, gemm_bf16.hip). With that many rows the activations are what the kernels
 // above read most of: every strip of 8 weight rows meets all of them, from L2. Here a workgroup
 // of eight waves takes eight neighbouring strips and a part of K, brings the activations of that
 // part into LDS once (in chunks of 256 k, two buffers in turn) and every

@@ -124,6 +124,7 @@ TILED_CONFIG = 0
 # a kernel for the case, bias, activation and the sum into the residual being its epilogues; the
 # tiled kernels of this package then take what it declines. Measured on MI355X at Moondream 2's
 # four linears: 201 against 242 us a layer at 2,048 rows, 112 against 151 at 730, 64 against 72 at 96.
+# (The two last linears of a parallel block of up to 160 tiles go by tiles all the same: PAIR_TILES_MAX.)
 LIBRARY_LINEAR = True
 LIBRARY_WORKSPACE_BYTES = 128 << 20
 # Activations that the library has no epilogue for (relu squared: ops.linear.ACT_RELU_SQUARED), and the size of an output from
