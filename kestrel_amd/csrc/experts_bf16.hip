@@ -104,6 +104,9 @@ experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, cons
 // tiles. For that the used part of the list has to be known, or the XCD with its unused end would idle: every workgroup counts
 // the tiles that have an expert, in one read of the list of tiles.
 //
+// A sum's channels meet in the order of the kernel above, so a pair's numbers are the same bits in tiles of any size and in
+// either kernel.
+//
 // Measured, us of the gated first and the fp32 second linear, before (the kernel above, which staged through registers, one wave
 // a SIMD, with sums that went through scratch memory) -> now: 62 experts of 4,096 x 896, 2,048 tokens of 6 choices 542 + 372 ->
 // 261 + 187; 512 tokens 302 + 175 -> 163 + 114; 30 experts of 2,048 x 704, 2,048 tokens of 4 choices 147 + 119 -> 81 + 60.
@@ -159,7 +162,7 @@ experts_dma_kernel(ExpertsDmaArgs g) {
         for (int b = 0; b < WM; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-    kd_product<WN, WM, GN, GM, 64, NS, SL>(eb_dma_lds, wave, lane, g.K, wsrc, xsrc, acc);
+    kd_product<WN, WM, GN, GM, 64, NS, SL, true>(eb_dma_lds, wave, lane, g.K, wsrc, xsrc, acc);
 
     // A lane ends with four neighbouring weight rows of one list row, a store instruction would touch 32 rows with 8 or 16
     // bytes each: a wave passes 32 list rows at a time through its share of LDS and stores its piece of every row whole.

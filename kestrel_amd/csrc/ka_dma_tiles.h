@@ -105,7 +105,9 @@ __device__ __forceinline__ int kd_load_channel(int row, int lane) { return ((lan
 
 // acc[a][b] += the products of this wave's tiles over K. wsrc[i], xsrc[i]: this lane's address at K-step 0 of the wave's load i
 // (rows wave * W_LOADS + i and so on, kd_load_row; valid whatever the row is). The whole workgroup takes part.
-template <int WN, int WM, int GN, int GM, int BK, int NS, int SL>
+// HALVES: which channels of a K-step meet in a product: slice j takes eight from place 8 j of either half of the step, as
+// kl_tile_product does (ka_listed_tiles.h), and the sums have its bits; without it sixteen neighbours. Both cost the same.
+template <int WN, int WM, int GN, int GM, int BK, int NS, int SL, bool HALVES = false>
 __device__ __forceinline__ void kd_product(unsigned char* lds, int wave, int lane, int K,
                                            const bf16_t* const (&wsrc)[KdTile<WN, WM, GN, GM, BK, NS>::W_LOADS],
                                            const bf16_t* const (&xsrc)[KdTile<WN, WM, GN, GM, BK, NS>::X_LOADS], floatx16 (&acc)[WN][WM]) {
@@ -126,7 +128,7 @@ __device__ __forceinline__ void kd_product(unsigned char* lds, int wave, int lan
     };
 
     // operand addresses inside a stage: tile row li of each of this wave's tiles; the k-chunk
-    // of k-step ks is ks * 2 + lg
+    // of slice ks is ks * 2 + lg, by halves lg * CPR / 2 + ks
     int wrow_off[WN], xrow_off[WM];
 #pragma unroll
     for (int a = 0; a < WN; ++a) wrow_off[a] = (wn * 32 * WN + a * 32 + li) * ROW;
@@ -160,7 +162,7 @@ __device__ __forceinline__ void kd_product(unsigned char* lds, int wave, int lan
         const unsigned char* base = lds + (stage % NS) * STAGE;
 #pragma unroll
         for (int i = 0; i < SL; ++i) {
-            const int place = (((g * SL + i) * 2 + lg) ^ swz) * 16;
+            const int slice = g * SL + i, place = ((HALVES ? lg * (CPR / 2) + slice : slice * 2 + lg) ^ swz) * 16;
 #pragma unroll
             for (int a = 0; a < WN; ++a) wa[slot][i][a] = *reinterpret_cast<const bf16x8*>(base + wrow_off[a] + place);
 #pragma unroll
