@@ -20,17 +20,70 @@ struct KaRowNorms {
     int h_bf16;
 };
 
+// However many threads a row has, its sums have the order of KA_ROW_THREADS of them, so that a row's bits do not depend on how many
+// rows a step has: "thread" t of that order owns the pieces (four channels each) t, t + KA_ROW_THREADS and so on. Where a row has
+// GROUP times as many threads, GROUP lanes of a wave share one of those: they hand each other their numbers before the wave's sum,
+// and GROUP waves make one of that order's. It costs nothing that shows: eight rows of four streams of 4,096 channels 3.9 us, as with
+// an order for each number of threads.
 template <int THREADS>
-__device__ __forceinline__ float ka_row_sum(float v, float* smem) {
-    v = ka_wave_sum(v);
+struct KaRowLanes {
+    static constexpr int GROUP = THREADS / KA_ROW_THREADS, WIDTH = KA_WAVE / GROUP, WAVES = THREADS / KA_WAVE;
+    static_assert(GROUP == 1 || GROUP == 2 || GROUP == 4, "256, 512 or 1,024 threads");
+};
+
+// First channel of this thread's piece j.
+template <int THREADS>
+__device__ __forceinline__ int ka_row_channel(int j) {
+    using L = KaRowLanes<THREADS>;
+    const int wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
+    return ((j * L::GROUP + lane / L::WIDTH) * KA_ROW_THREADS + wave * L::WIDTH + lane % L::WIDTH) * 4;
+}
+
+// Sum over the row of `q`, a number for each of this thread's pieces; the same bits in every thread. `smem` holds a float a wave.
+template <int PIECES, int THREADS>
+__device__ __forceinline__ float ka_pieces_sum(const float (&q)[PIECES], float* smem) {
+    using L = KaRowLanes<THREADS>;
+    float v = 0.f;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        if constexpr (L::GROUP == 1) {
+            v += q[j];
+        } else if constexpr (L::GROUP == 2) {
+            float a, b;
+            ka_lanes_pair<32>(q[j], a, b);
+            v += a;
+            v += b;
+        } else {
+            float a, b, c[4];
+            ka_lanes_pair<16>(q[j], a, b);
+            ka_lanes_pair<32>(a, c[0], c[2]);
+            ka_lanes_pair<32>(b, c[1], c[3]);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) v += c[p];
+        }
+    }
+    v = ka_lanes_reduce<1, L::WIDTH>(v, KaSum{});
     __syncthreads();
     if (threadIdx.x % KA_WAVE == 0) smem[threadIdx.x / KA_WAVE] = v;
     __syncthreads();
     float total = 0.f;
 #pragma unroll
-    for (int w = 0; w < THREADS / KA_WAVE; ++w) total += smem[w];
+    for (int w = 0; w < L::WAVES; w += L::GROUP) {
+        if constexpr (L::GROUP == 1) total += smem[w];
+        else if constexpr (L::GROUP == 2) total += smem[w] + smem[w + 1];
+        else total += (smem[w] + smem[w + 1]) + (smem[w + 2] + smem[w + 3]);
+    }
     return total;
 }
+
+// The same of one number a thread, KA_ROW_THREADS threads.
+__device__ __forceinline__ float ka_row_sum(float v, float* smem) {
+    const float q[1] = {v};
+    return ka_pieces_sum<1, KA_ROW_THREADS>(q, smem);
+}
+
+// Of four squares: the order is written out, so that every kernel has the same.
+__device__ __forceinline__ float ka_squares(const float4& d) { return fmaf(d.w, d.w, fmaf(d.z, d.z, fmaf(d.x, d.x, d.y * d.y))); }
 
 __device__ __forceinline__ void ka_row_store_h(const KaRowNorms& a, size_t at, float v) {
     if (a.h_bf16) reinterpret_cast<bf16_t*>(a.h)[at] = (bf16_t)v;
@@ -47,21 +100,22 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
     if constexpr (PIECES > 0) {
         typedef __attribute__((ext_vector_type(4))) __bf16 row_bf16x4;
         float4 d[PIECES], y[PIECES];
-        float s = 0.f;
+        float s[PIECES], s2[PIECES];
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * THREADS + tid) * 4;
+            const int c = ka_row_channel<THREADS>(p);
+            s[p] = 0.f;
             if (c < dim) {
                 d[p] = piece(c);
                 y[p] = *reinterpret_cast<const float4*>(x + at + c);
-                s += d[p].x * d[p].x + d[p].y * d[p].y + d[p].z * d[p].z + d[p].w * d[p].w;
+                s[p] = ka_squares(d[p]);
             }
         }
-        const float r = 1.0f / sqrtf(ka_row_sum<THREADS>(s, smem) / (float)dim + a.eps);
-        float s2 = 0.f;
+        const float r = 1.0f / sqrtf(ka_pieces_sum<PIECES, THREADS>(s, smem) / (float)dim + a.eps);
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * THREADS + tid) * 4;
+            const int c = ka_row_channel<THREADS>(p);
+            s2[p] = 0.f;
             if (c < dim) {
                 const float4 g = *reinterpret_cast<const float4*>(a.gain + c);
                 y[p].x += d[p].x * r * g.x;
@@ -69,14 +123,14 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
                 y[p].z += d[p].z * r * g.z;
                 y[p].w += d[p].w * r * g.w;
                 *reinterpret_cast<float4*>(x + at + c) = y[p];
-                s2 += y[p].x * y[p].x + y[p].y * y[p].y + y[p].z * y[p].z + y[p].w * y[p].w;
+                s2[p] = ka_squares(y[p]);
             }
         }
         if (a.h == nullptr) return;
-        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_row_sum<THREADS>(s2, smem) / (float)dim + a.eps2) : 1.f;
+        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_pieces_sum<PIECES, THREADS>(s2, smem) / (float)dim + a.eps2) : 1.f;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int c = (p * THREADS + tid) * 4;
+            const int c = ka_row_channel<THREADS>(p);
             if (c < dim) {
                 float4 v = y[p];
                 if (a.gain2) {
@@ -96,12 +150,13 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
             }
         }
     } else {
+        static_assert(THREADS == KA_ROW_THREADS, "the general form has one number of threads");
         float s = 0.f;
         for (int c = tid; c < dim; c += THREADS) {
             const float d = one(c);
             s += d * d;
         }
-        const float r = 1.0f / sqrtf(ka_row_sum<THREADS>(s, smem) / (float)dim + a.eps);
+        const float r = 1.0f / sqrtf(ka_row_sum(s, smem) / (float)dim + a.eps);
         float s2 = 0.f;
         for (int c = tid; c < dim; c += THREADS) {
             const float y = x[at + c] + one(c) * r * a.gain[c];
@@ -109,7 +164,7 @@ __device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, in
             s2 += y * y;
         }
         if (a.h == nullptr) return;
-        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_row_sum<THREADS>(s2, smem) / (float)dim + a.eps2) : 1.f;
+        const float r2 = a.gain2 ? 1.0f / sqrtf(ka_row_sum(s2, smem) / (float)dim + a.eps2) : 1.f;
         for (int c = tid; c < dim; c += THREADS) ka_row_store_h(a, at + c, x[at + c] * r2 * (a.gain2 ? a.gain2[c] : 1.f));      // (its own writes)
     }
 }

@@ -4,11 +4,12 @@
 // reads what the next sublayer sees, u = sum_t into[t] x_t, and leaves that sublayer's norm of u in h. All arithmetic is fp32.
 // What computes y is the caller's business: a load, or the weighted sum of a routed mixture's experts.
 #include "ka_common.h"
+#include "ka_rows.h"
 
 // A workgroup has a row. Of many rows each gets 256 threads and a thread several pieces of it; where there are fewer rows than two a
 // CU (a decode step) a row gets a thread per piece, up to 1,024: it then waits for memory once (48 rows of four streams of
 // 4,096: 11 -> 5.1 us between sublayers and 24 -> 8.3 behind six experts).
-constexpr int ST_THREADS = 256;
+constexpr int ST_THREADS = KA_ROW_THREADS;
 constexpr int ST_MAX_STREAMS = 16;
 
 struct StreamArgs {
@@ -27,18 +28,6 @@ struct StreamArgs {
     int S, dim;
 };
 
-template <int THREADS>
-__device__ __forceinline__ float st_block_sum(float v, float* smem) {
-    v = ka_wave_sum(v);
-    __syncthreads();
-    if (threadIdx.x % KA_WAVE == 0) smem[threadIdx.x / KA_WAVE] = v;
-    __syncthreads();
-    float total = 0.f;
-#pragma unroll
-    for (int w = 0; w < THREADS / KA_WAVE; ++w) total += smem[w];
-    return total;
-}
-
 __device__ __forceinline__ float4 st_fma4(float a, const float4& b, const float4& c) {
     return make_float4(fmaf(a, b.x, c.x), fmaf(a, b.y, c.y), fmaf(a, b.z, c.z), fmaf(a, b.w, c.w));
 }
@@ -48,7 +37,7 @@ __device__ __forceinline__ float4 st_fma4(float a, const float4& b, const float4
 template <int S, int PIECES, int THREADS, typename Piece>
 __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, float* smem) {
     typedef __attribute__((ext_vector_type(4))) __bf16 st_bf16x4;
-    const int i = blockIdx.x, tid = threadIdx.x, dim = a.dim;
+    const int i = blockIdx.x, dim = a.dim;
     float* row = a.x + (size_t)(a.rows ? a.rows[i] : i) * S * dim;
     float m[S][S], o[S], in[S];
     const bool writes = a.mix != nullptr;
@@ -63,7 +52,7 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
 #pragma unroll
     for (int s = 0; s < S; ++s) in[s] = a.into ? a.into[s] : 1.f;
     float4 u[PIECES];
-    float sum = 0.f;
+    float sum[PIECES], ss[PIECES];
     // (all that a few pieces need is asked for before anything is stored)
     constexpr int AT_ONCE = PIECES < 4 ? PIECES : 4;
 #pragma unroll
@@ -71,7 +60,7 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
         float4 v[AT_ONCE][S], y[AT_ONCE];
 #pragma unroll
         for (int p = 0; p < AT_ONCE; ++p) {
-            const int c = ((p0 + p) * THREADS + tid) * 4;
+            const int c = ka_row_channel<THREADS>(p0 + p);
             if (c >= dim) continue;
             if (a.embedded) {
                 v[p][0] = *reinterpret_cast<const float4*>(a.embedded + (size_t)i * dim + c);
@@ -83,9 +72,10 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
         }
 #pragma unroll
         for (int p = 0; p < AT_ONCE; ++p) {
-            const int c = ((p0 + p) * THREADS + tid) * 4;
+            const int c = ka_row_channel<THREADS>(p0 + p);
             float4& sums = u[p0 + p];
             sums = make_float4(0.f, 0.f, 0.f, 0.f);
+            sum[p0 + p] = 0.f;
             if (c >= dim) continue;
             if (a.embedded) {
 #pragma unroll
@@ -107,23 +97,23 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
 #pragma unroll
                 for (int s = 0; s < S; ++s) sums = st_fma4(in[s], v[p][s], sums);
             }
-            sum += (sums.x + sums.y) + (sums.z + sums.w);
+            sum[p0 + p] = (sums.x + sums.y) + (sums.z + sums.w);
         }
     }
     if (a.h == nullptr) return;
-    const float mean = a.rms ? 0.f : st_block_sum<THREADS>(sum, smem) / (float)dim;
-    float ss = 0.f;
+    const float mean = a.rms ? 0.f : ka_pieces_sum<PIECES, THREADS>(sum, smem) / (float)dim;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-        if ((p * THREADS + tid) * 4 < dim) {
+        ss[p] = 0.f;
+        if (ka_row_channel<THREADS>(p) < dim) {
             u[p] = make_float4(u[p].x - mean, u[p].y - mean, u[p].z - mean, u[p].w - mean);
-            ss += u[p].x * u[p].x + u[p].y * u[p].y + u[p].z * u[p].z + u[p].w * u[p].w;
+            ss[p] = ka_squares(u[p]);
         }
     }
-    const float r = 1.0f / sqrtf(st_block_sum<THREADS>(ss, smem) / (float)dim + a.eps);
+    const float r = 1.0f / sqrtf(ka_pieces_sum<PIECES, THREADS>(ss, smem) / (float)dim + a.eps);
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-        const int c = (p * THREADS + tid) * 4;
+        const int c = ka_row_channel<THREADS>(p);
         if (c < dim) {
             const float4 g = *reinterpret_cast<const float4*>(a.gain + c);
             float4 v = make_float4(u[p].x * r * g.x, u[p].y * r * g.y, u[p].z * r * g.z, u[p].w * r * g.w);
@@ -178,13 +168,13 @@ __device__ __forceinline__ void st_step_any(const StreamArgs& a, One one, float*
         if (a.h) sum += read(c);              // (a thread reads its own writes)
     }
     if (a.h == nullptr) return;
-    const float mean = a.rms ? 0.f : st_block_sum<ST_THREADS>(sum, smem) / (float)dim;
+    const float mean = a.rms ? 0.f : ka_row_sum(sum, smem) / (float)dim;
     float ss = 0.f;
     for (int c = tid; c < dim; c += ST_THREADS) {
         const float u = read(c) - mean;
         ss += u * u;
     }
-    const float r = 1.0f / sqrtf(st_block_sum<ST_THREADS>(ss, smem) / (float)dim + a.eps);
+    const float r = 1.0f / sqrtf(ka_row_sum(ss, smem) / (float)dim + a.eps);
     for (int c = tid; c < dim; c += ST_THREADS) {
         float v = (read(c) - mean) * r * a.gain[c];
         if (a.bias) v += a.bias[c];
