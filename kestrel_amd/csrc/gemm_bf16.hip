@@ -440,35 +440,95 @@ static int launch_pair_tiles(PairTilesArgs& p, int parts, hipStream_t stream) {
     return 0;
 }
 
-// Few rows (at most 64) through the same kernel, for the weight-streaming launcher: the sums of one linear, or of two added up,
-// in parts in `partial`. Returns the number of parts, 0 where the operands are not covered, -1 on an error. Bound by the weights'
-// way from HBM: what counts is that every CU has 64 KB of loads in flight, which the stages in LDS hold without registers. Tiles
-// of 64 rows by 64 weight rows, five stages in half of a CU's LDS, or by 128 and three where an output is so wide that tiles of
-// 64 alone fill half of the chip; as many parts as give every CU a workgroup (twice as many: 1 to 2 us more). At 40 rows, us,
-// the launch that adds up included, against the wide kernel of the weight-streaming file: N = 2,048, K = 2,048 + 8,192: 15.7
-// and 18.6; 2,560, 2,560 + 10,240: 22.0 and 25.7; without that launch (4 to 5 us): N = K = 4,096: 9.5 and 12; 12,288 by 4,096:
-// 22.4 and 28; 4,096 by 12,288: 19.8 and 25. Tiles of 32 rows for up to 32 gave the same.
-int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
-    if (f.M > 64 || f.K[0] % PT_BK || f.K[1] % PT_BK || f.K[0] < PT_BK || !f.partial) return 0;
-    PairTilesArgs p = {};
+// Few rows (at most 64), for the weight-streaming launcher: the sums of one linear, or of two added up, in parts in `partial`. Parts and
+// order of a sum are those of skinny_wide_kernel, whose bits these are: part p has the p-th range of K of either linear, and a part's sum is
+// that of the first halves of its K-steps plus that of the second.
+//
+// Bound by the weights' way from HBM: what counts is that every CU has 64 KB of loads in flight, which the stages in LDS hold without
+// registers. Tiles of 64 weight rows by all rows, five stages in half of a CU's LDS, four waves. At 40
+// rows, us, weights from HBM, the launch that adds up included, against that kernel: N = 2,048, K = 2,048 + 8,192: 15.3 and 18.6; 2,560, 2,560 +
+// 10,240: 20.1 and 24.8; N = K = 4,096: 12.8 and 16.3; 12,288 by 4,096: 30.9 and 34.2; 4,096 by 12,288: 26.4 and 31.0; at 17 and 64 rows
+// likewise.
+template <int WN, int WM, int GN, int GM, int NS>
+__global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(2, 2)))
+few_rows_kernel(KaFewRows p) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS, 16>;
+    constexpr int CPR = T::CPR;
+    extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
+    const int n0 = blockIdx.x * T::BN, part = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    int first[2], count[2];                              // this part's K-steps of either linear
+#pragma unroll
     for (int s = 0; s < 2; ++s) {
-        p.A[s] = (const bf16_t*)f.A[s]; p.lda[s] = f.lda[s];
-        p.W[s] = (const bf16_t*)f.W[s]; p.ldw[s] = f.ldw[s];
-        p.steps[s] = f.K[s] / PT_BK;
+        const int all = p.K[s] / 64, per = (all + p.parts - 1) / p.parts;
+        first[s] = min(part * per, all);
+        count[s] = min(per, all - first[s]);
     }
-    p.M = f.M; p.N = f.N; p.partial = f.partial;
-    const int steps = p.steps[0] + p.steps[1], cus = ka_compute_units();
-    const bool wide = ka_cdiv(f.N, 64) * 2 > cus;
-    int parts = cus / ka_cdiv(f.N, wide ? 128 : 64);
-    if (parts > 8) parts = 8;                            // (what the finishing kernel asks for at once)
-    if (parts > steps / 4) parts = steps / 4;
-    if (parts < 1) parts = 1;
-    while (parts > 1 && (long)parts * f.M * f.N > f.partial_floats) --parts;
-    if ((long)parts * f.M * f.N > f.partial_floats) return 0;
-    p.per = ka_cdiv(steps, parts);
-    parts = ka_cdiv(steps, p.per);
-    if (wide ? launch_pair_tiles<1, 1, 2, 4, 3, 2>(p, parts, stream) : launch_pair_tiles<1, 1, 2, 2, 5, 2>(p, parts, stream)) return -1;
-    return parts;
+    const bf16_t* w[2][T::W_LOADS];
+    const bf16_t* x[2][T::X_LOADS];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const bool has = p.K[s] > 0;
+#pragma unroll
+        for (int i = 0; i < T::W_LOADS; ++i) {
+            const int r = kd_load_row<CPR>(wave * T::W_LOADS + i, lane);
+            w[s][i] = has ? (const bf16_t*)p.W[s] + (size_t)min(n0 + r, p.N - 1) * p.ldw[s] + first[s] * 64 + kd_load_channel<CPR>(r, lane) : nullptr;
+        }
+#pragma unroll
+        for (int i = 0; i < T::X_LOADS; ++i) {
+            const int r = kd_load_row<CPR>(wave * T::X_LOADS + i, lane);
+            x[s][i] = has ? (const bf16_t*)p.A[s] + (size_t)min(r, p.M - 1) * p.lda[s] + first[s] * 64 + kd_load_channel<CPR>(r, lane) : nullptr;
+        }
+    }
+    floatx4 acc[KD_HALVES][WN][WM];
+#pragma unroll
+    for (int h = 0; h < KD_HALVES; ++h)
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b) acc[h][a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int steps = count[0] + count[1];
+    if (steps > 0)                                       // (the same for the whole workgroup)
+        kd_product_16<WN, WM, GN, GM, NS, KD_HALVES>(
+            gb_lds, wave, lane, steps, [&](int i, int st) { return st < count[0] ? w[0][i] + st * 64 : w[1][i] + (st - count[0]) * 64; },
+            [&](int i, int st) { return st < count[0] ? x[0][i] + st * 64 : x[1][i] + (st - count[0]) * 64; }, acc);
+    float* const mine = p.partial + (size_t)part * p.M * p.N;
+    const int wn = wave / GM, wm = wave % GM, col = lane % 16, quarter = lane / 16;
+#pragma unroll
+    for (int b = 0; b < WM; ++b) {
+        const int m = (wm * WM + b) * 16 + col;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int a = 0; a < WN; ++a) {
+            const int n = n0 + (wn * WN + a) * 16 + quarter * 4;
+            const floatx4 v = acc[0][a][b] + acc[1][a][b];
+            float* dst = mine + (size_t)m * p.N + n;
+            if (n + 3 < p.N && p.N % 4 == 0) *reinterpret_cast<floatx4*>(dst) = v;
+            else
+                for (int i = 0; i < 4 && n + i < p.N; ++i) dst[i] = v[i];
+        }
+    }
+}
+
+template <int WN, int WM, int GN, int GM, int NS>
+static int launch_few_rows(const KaFewRows& f, hipStream_t stream) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS, 16>;
+    static bool configured = false;
+    auto kernel = few_rows_kernel<WN, WM, GN, GM, NS>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM);
+        KA_CHECK(e == hipSuccess, "linear of few rows: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
+        configured = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3(ka_cdiv(f.N, T::BN), f.parts), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, f);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// 1: done; 0: the operands are not covered (K in steps of 64); -1: an error.
+int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
+    if (f.M < 1 || f.M > 64 || f.K[0] % 64 || f.K[1] % 64 || f.K[0] < 64 || f.parts < 1 || !f.partial) return 0;
+    return launch_few_rows<2, 2, 2, 2, 5>(f, stream) ? -1 : 1;
 }
 
 // Parts of K for `ka_linear_pair_tiles_bf16`: as many as leave the fewest K-steps to a CU, a part more than another costing

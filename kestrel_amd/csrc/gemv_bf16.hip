@@ -182,8 +182,8 @@ skinny_split_kernel(SkinnyArgs p) {
 }
 
 // ----------------------------------------------------------------------------
-// The wide kernel, for 17 to 64 rows of a K in no steps of 64 (else ka_few_rows_by_tiles, gemm_bf16.hip). With that many rows the activations are what the kernels
-// above read most of: every strip of 8 weight rows meets all of them, from L2. Here a workgroup
+// The wide kernel, for 17 to 64 rows of a K in no steps of 64 (else ka_few_rows_by_tiles, gemm_bf16.hip, which has the same
+// parts of K and the same order within one). With that many rows the activations are what the kernels above read most of: every strip of 8 weight rows meets all of them, from L2. Here a workgroup
 // of eight waves takes eight neighbouring strips and a part of K, brings the activations of that
 // part into LDS once (in chunks of 256 k, two buffers in turn) and every
 // wave multiplies its own strip with them; the parts of K meet in fp32 partial sums that a
@@ -370,7 +370,7 @@ KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enab
 // The wide kernel (17 to 64 rows, activations through LDS, parts of K in scratch memory): 1 where
 // it was measured faster, which is with two K-segments (a K too long for the persistent kernel's
 // registers: 30 against 48 us for Moondream 2's output projection + fc2 at 64 rows; one segment
-// of 2048: 21 against 15 us), 2 wherever it can run (for tests), 0 nowhere.
+// of 2048: 21 against 15 us) and K comes in no steps of 64 (those go by tiles), 2 itself wherever it can run (for tests), 0 nowhere.
 static int sk_wide_enabled = 1;
 KA_API int ka_linear_skinny_pair_in_parts(int M, int N);
 KA_API void ka_skinny_set_wide(int enabled) { sk_wide_enabled = enabled; }
@@ -569,14 +569,6 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
     // 18.3 at 16 (N = 2048, K = 2048 + 8192).
     const bool crowded = A2 && M <= 16 && ka_linear_skinny_pair_in_parts(M, Na);      // (a single row: 19 us against 24)
     if (!Wb && partials && ((sk_wide_enabled && (M > 16 ? (A2 || !persistent_ok) : crowded)) || sk_wide_enabled >= 2)) {
-        // by tiles of 64 rows where K comes in whole K-steps (measured there), else by the wide kernel
-        KaFewRows few = {};
-        few.A[0] = args.A[0]; few.lda[0] = args.lda[0]; few.W[0] = args.a.W; few.ldw[0] = args.a.ldw; few.K[0] = K1;
-        if (A2) { few.A[1] = args.A[1]; few.lda[1] = args.lda[1]; few.W[1] = args.W2; few.ldw[1] = args.ldw2; few.K[1] = K2; }
-        few.M = M; few.N = Na; few.partial = partials; few.partial_floats = partial_floats;
-        int parts = ka_few_rows_by_tiles(few, stream);
-        if (parts < 0) return -1;
-        if (parts > 0) return finish_parts(parts);
         WideArgs wide = {};
         wide.A[0] = args.A[0]; wide.lda[0] = args.lda[0]; wide.W[0] = args.a.W; wide.ldw[0] = args.a.ldw; wide.K[0] = K1;
         if (A2) { wide.A[1] = args.A[1]; wide.lda[1] = args.lda[1]; wide.W[1] = args.W2; wide.ldw[1] = args.ldw2; wide.K[1] = K2; }
@@ -591,6 +583,16 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         if (splits > ka_cdiv(kblocks, 2 * WD_CB)) splits = ka_cdiv(kblocks, 2 * WD_CB);
         while (splits > 1 && (long)splits * M * Na > partial_floats) --splits;
         if ((long)splits * M * Na <= partial_floats) {
+            // the same sums by tiles where K comes in whole steps of theirs (measured there)
+            if (sk_wide_enabled == 1) {
+                KaFewRows few = {};
+                few.M = M; few.N = Na; few.parts = splits; few.partial = partials;
+                for (int s = 0; s < (A2 ? 2 : 1); ++s) {
+                    few.A[s] = wide.A[s]; few.lda[s] = wide.lda[s]; few.W[s] = wide.W[s]; few.ldw[s] = wide.ldw[s]; few.K[s] = wide.K[s];
+                }
+                const int done = ka_few_rows_by_tiles(few, stream);
+                if (done) return done < 0 ? -1 : finish_parts(splits);
+            }
             wide.splits = splits;
             dim3 grid(groups, splits);
             switch (MB) {

@@ -71,14 +71,14 @@ __device__ __forceinline__ void at_epilogue_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The sizes that follow from a tile's shape.
-template <int WN, int WM, int GN, int GM, int BK, int NS>
+// The sizes that follow from a tile's shape; EDGE: rows and columns of an MFMA tile.
+template <int WN, int WM, int GN, int GM, int BK, int NS, int EDGE = 32>
 struct KdTile {
     static_assert(BK == 32 || BK == 64, "K-steps of 32 or 64");
     static_assert(NS >= 2 && NS <= 8, "two to eight stages");
     static_assert(GN * GM == 4 || GN * GM == 8, "four or eight waves");
     static constexpr int WAVES = GN * GM;
-    static constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM;
+    static constexpr int BN = EDGE * WN * GN, BM = EDGE * WM * GM;
     static constexpr int ROW = BK * 2;                          // bytes of a tile row
     static constexpr int CPR = BK / 8;                          // 16-byte chunks of a tile row
     static constexpr int RPL = KA_WAVE / CPR;                   // rows that one load of 1 KB brings
@@ -216,4 +216,87 @@ __device__ __forceinline__ void kd_product(unsigned char* lds, int wave, int lan
         group(std::integral_constant<int, 1>{}, t + 1);
     }
     if (t < groups) group(std::integral_constant<int, 0>{}, t);
+}
+
+// The same on MFMA tiles of 16 x 16 by 32 channels, two products a K-step of 64, for sums that have to have the order (and so the bits) of a
+// kernel that streams weights through registers, whatever the number of rows:
+//  * KD_HALVES: the first product takes channels 0 .. 31 of a step, the second 32 .. 63, each into sums of its own (skinny_wide_kernel);
+//  * KD_FOURTHS: the four lane groups hold sixteen neighbours each, the first product takes eight of each, and every fourth K-step goes
+//    into the same sums (ef_columns).
+// acc[c][a][b], c the set of sums; weight(i, step), row(i, step): this lane's address of load i at that K-step (as wsrc and xsrc above).
+enum { KD_HALVES = 2, KD_FOURTHS = 4 };
+
+template <int WN, int WM, int GN, int GM, int NS, int ORDER, typename Weight, typename Row>
+__device__ __forceinline__ void kd_product_16(unsigned char* lds, int wave, int lane, int steps, Weight weight, Row row, floatx4 (&acc)[ORDER][WN][WM]) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS, 16>;
+    constexpr int BN = T::BN, ROW = T::ROW, CPR = T::CPR, RPL = T::RPL, STAGE = T::STAGE, W_LOADS = T::W_LOADS, X_LOADS = T::X_LOADS, LPW = T::LPW;
+    const int wn = wave / GM, wm = wave % GM, col = lane % 16, quarter = lane / 16;
+    auto fetch = [&](int stage, int step) {
+        unsigned char* base = lds + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < W_LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)weight(i, step), (GD_LDS void*)(base + (wave * W_LOADS + i) * RPL * ROW), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < X_LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)row(i, step), (GD_LDS void*)(base + BN * ROW + (wave * X_LOADS + i) * RPL * ROW), 16, 0, 0);
+    };
+    int wrow_off[WN], xrow_off[WM];
+#pragma unroll
+    for (int a = 0; a < WN; ++a) wrow_off[a] = ((wn * WN + a) * 16 + col) * ROW;
+#pragma unroll
+    for (int b = 0; b < WM; ++b) xrow_off[b] = (BN + (wm * WM + b) * 16 + col) * ROW;
+    const int swz = kd_swizzle<CPR>(col);
+    // As in kd_product, a group being a whole K-step: the operands of the next step are read from LDS behind the first products of this one.
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+        if (st < steps) fetch(st, st);
+    gd_wait_younger<LPW, NS - 1>(min(NS - 1, steps - 1));
+    gd_barrier();
+    bf16x8 wa[2][2][WN], xb[2][2][WM];
+    auto operands = [&](auto slot_c, int stage) {
+        constexpr int slot = decltype(slot_c)::value;
+        const unsigned char* base = lds + (stage % NS) * STAGE;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int place = ((ORDER == KD_HALVES ? u * 4 + quarter : quarter * 2 + u) ^ swz) * 16;
+#pragma unroll
+            for (int a = 0; a < WN; ++a) wa[slot][u][a] = *reinterpret_cast<const bf16x8*>(base + wrow_off[a] + place);
+#pragma unroll
+            for (int b = 0; b < WM; ++b) xb[slot][u][b] = *reinterpret_cast<const bf16x8*>(base + xrow_off[b] + place);
+        }
+    };
+    auto step = [&](auto place_c, int st) {             // st % 4 == place
+        constexpr int place = decltype(place_c)::value, slot = place & 1;
+        if (st + 1 < steps) {
+            gd_wait_younger<LPW, NS - 2>(min(NS - 2, steps - 2 - st));
+            gd_wait_lds();
+            gd_barrier();
+            if (st + NS < steps) fetch(st % NS, st + NS);
+        }
+        operands(std::integral_constant<int, slot ^ 1>{}, st + 1);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            constexpr int fourth = place;
+            const int c = ORDER == KD_HALVES ? u : fourth;
+#pragma unroll
+            for (int a = 0; a < WN; ++a)
+#pragma unroll
+                for (int b = 0; b < WM; ++b) acc[c][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[slot][u][a], xb[slot][u][b], acc[c][a][b], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * (WN + WM), 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * WN * WM - 2, 0);
+    };
+    gd_wait_lds();
+    operands(std::integral_constant<int, 0>{}, 0);
+    int st = 0;
+    for (; st + 3 < steps; st += 4) {
+        step(std::integral_constant<int, 0>{}, st);
+        step(std::integral_constant<int, 1>{}, st + 1);
+        step(std::integral_constant<int, 2>{}, st + 2);
+        step(std::integral_constant<int, 3>{}, st + 3);
+    }
+    if (st < steps) step(std::integral_constant<int, 0>{}, st);
+    if (st + 1 < steps) step(std::integral_constant<int, 1>{}, st + 1);
+    if (st + 2 < steps) step(std::integral_constant<int, 2>{}, st + 2);
 }

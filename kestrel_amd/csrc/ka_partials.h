@@ -15,9 +15,8 @@ struct KaFewRows {
     const void* W[2];
     long lda[2], ldw[2];
     int K[2];
-    int M, N;
-    float* partial;
-    long partial_floats;
+    int M, N, parts;
+    float* partial;         // [parts, M, N]
 };
 int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream);
 

@@ -233,7 +233,8 @@ def set_skinny_wide(enabled: int) -> None:
     """Where skinny linears use the kernel that shares the activations through LDS and cuts K
     into parts: 1 (the default) where it was measured faster (two K-segments at 17 to 64 rows or
     with more strips than CUs at 5 to 16 rows; one segment too long for the persistent kernel's
-    registers at 17 to 64 rows), 2 wherever it can run (for tests), 0 nowhere."""
+    registers at 17 to 64 rows), K in steps of 64 by tiles that give the same bits; 2 that kernel
+    itself wherever it can run (for tests), 0 nowhere."""
     lib().ka_skinny_set_wide(int(enabled))
 
 

@@ -68,3 +68,31 @@ def test_rows_of_the_stream_do_not_depend_on_their_number(dim):
 
     for i, (a, b) in enumerate(zip(results(n), results(few))):
         assert torch.equal(a, b), f"result {i}"
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("n, ks", [(64, (2624,)), (1000, (4096,)), (77, (8192,)), (12288, (2688,)), (640, (64, 320)), (2056, (2048, 8192)), (4096, (192, 64))])
+def test_few_rows_have_the_bits_of_the_kernel_that_streams_weights(m, n, ks):
+    """Tiles for K in steps of 64, and the kernel with activations in LDS: the same parts of K, the same order within."""
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(m + n + sum(ks))
+    rows = [torch.randn(m, k, generator=gen).bfloat16().to(DEV) for k in ks]
+    weights = [torch.randn(n, k, generator=gen).bfloat16().to(DEV) for k in ks]
+    bias, start = torch.randn(n, generator=gen).to(DEV), torch.randn(m, n, generator=gen).to(DEV)
+    results = []
+    try:
+        for mode in (1, 2):
+            fast.set_skinny_wide(mode)
+            out = start.clone()
+            if len(ks) == 1:
+                assert fast.linear_bf16(rows[0], weights[0], bias, out, 0, True)
+            else:
+                assert fast.linear_pair_accumulate(rows[0], weights[0], bias, rows[1], weights[1], None, out)
+            results.append(out)
+    finally:
+        fast.set_skinny_wide(1)
+    if m > 16 or (len(ks) == 2 and fast.pair_finishes_rows(m, n)):         # (else rule and test name two kernels)
+        assert torch.equal(*results)
+    want = start.double() + bias.double() + sum(a.double() @ w.double().T for a, w in zip(rows, weights))
+    assert float((results[0].double() - want).norm() / want.norm()) < 2.0 ** -20
