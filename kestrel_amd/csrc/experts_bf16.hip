@@ -20,6 +20,8 @@
 
 typedef __attribute__((ext_vector_type(2))) __bf16 eb_bf16x2;
 
+constexpr int EF_MAX_PAIRS = 512;          // most pairs of a step of few
+
 template <bool TAIL>
 __global__ void __launch_bounds__(256)
 experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, const bf16_t* __restrict__ W, const int* __restrict__ sorted,
@@ -95,7 +97,7 @@ experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, cons
 // ----------------------------------------------------------------------------
 // The same linears where K is a multiple of 64: operands go from memory straight into LDS (ka_dma_tiles.h), the list's rows
 // gathered by the addresses of the loads. Eight waves and 256 weight rows a workgroup; a tile has 64, 128 or 256 list rows, as
-// many as the list was made for.
+// many as the list was made for (32: experts_dma_few_kernel).
 //
 // What bounds it: an expert sees a few hundred rows of a step, so its weights come from HBM for little more work than they cost
 // to read (62 experts of 2 x 896 x 4,096 at 198 rows each: 910 MB and 180 GFLOP, 160 us of either). The tiles that share an
@@ -125,36 +127,52 @@ struct ExpertsDmaArgs {
     int scatter;
 };
 
+// The workgroup's tile of the list and of the columns (of g.tiles_n); false: it has none.
+__device__ __forceinline__ bool experts_dma_find(const ExpertsDmaArgs& g, int& tile, int& column) {
+    int used = 0;
+    for (int t0 = 0; t0 < g.n_tiles; t0 += blockDim.x) {
+        const int t = t0 + (int)threadIdx.x;
+        used += __syncthreads_count(t < g.n_tiles && g.tile_expert[min(t, g.n_tiles - 1)] >= 0);
+    }
+    const int total = used * g.tiles_n, per_xcd = (total + 7) / 8;
+    const int at = blockIdx.x / 8, logical = blockIdx.x % 8 * per_xcd + at;
+    if (at >= per_xcd || logical >= total) return false;
+    tile = logical / g.tiles_n;
+    column = logical - tile * g.tiles_n;
+    return true;
+}
+
+// This lane's address of load i of the tile's list rows, and of its weight rows, at K-step 0 (kd_product).
+template <typename T>
+__device__ __forceinline__ const bf16_t* experts_dma_row(const ExpertsDmaArgs& g, int i0, int wave, int lane, int i) {
+    const int r = kd_load_row<T::CPR>(wave * T::X_LOADS + i, lane);
+    const long row = g.gather_div > 0 ? (long)(max(g.sorted[i0 + r], 0) / g.gather_div) : (long)i0 + r;
+    return g.a + row * g.lda + kd_load_channel<T::CPR>(r, lane);
+}
+template <typename T>
+__device__ __forceinline__ const bf16_t* experts_dma_weight(const ExpertsDmaArgs& g, int e, int n0, int wave, int lane, int i) {
+    const int r = kd_load_row<T::CPR>(wave * T::W_LOADS + i, lane);
+    return g.W + ((size_t)e * g.N + min(n0 + r, g.N - 1)) * g.K + kd_load_channel<T::CPR>(r, lane);
+}
+
 template <int WN, int WM, int GN, int GM, int NS, int SL, bool GATED, bool F32>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM)
     __attribute__((amdgpu_waves_per_eu(GN * GM / 4, (WN * WM > 8 ? 1 : 2) * (GN * GM / 4))))
 experts_dma_kernel(ExpertsDmaArgs g) {
     using T = KdTile<WN, WM, GN, GM, 64, NS>;
-    constexpr int BN = T::BN, BM = T::BM, CPR = T::CPR;
+    constexpr int BN = T::BN, BM = T::BM;
     extern __shared__ __attribute__((aligned(16))) unsigned char eb_dma_lds[];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KA_WAVE), lane = tid % KA_WAVE;
-    int used = 0;
-    for (int t0 = 0; t0 < g.n_tiles; t0 += T::WAVES * KA_WAVE)
-        used += __syncthreads_count(t0 + tid < g.n_tiles && g.tile_expert[min(t0 + tid, g.n_tiles - 1)] >= 0);
-    const int total = used * g.tiles_n, per_xcd = (total + 7) / 8;
-    const int at = blockIdx.x / 8, logical = blockIdx.x % 8 * per_xcd + at;
-    if (at >= per_xcd || logical >= total) return;
-    const int tile = logical / g.tiles_n, n0 = (logical - tile * g.tiles_n) * BN;
-    const int e = g.tile_expert[tile], i0 = tile * BM;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    int tile, column;
+    if (!experts_dma_find(g, tile, column)) return;
+    const int e = g.tile_expert[tile], i0 = tile * BM, n0 = column * BN;
     const int wn = wave / GM, wm = wave % GM, li = lane % 32, lg = lane / 32;
     const bf16_t* wsrc[T::W_LOADS];
     const bf16_t* xsrc[T::X_LOADS];
 #pragma unroll
-    for (int i = 0; i < T::X_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(wave * T::X_LOADS + i, lane);
-        const long row = g.gather_div > 0 ? (long)(max(g.sorted[i0 + r], 0) / g.gather_div) : (long)i0 + r;
-        xsrc[i] = g.a + row * g.lda + kd_load_channel<CPR>(r, lane);
-    }
+    for (int i = 0; i < T::X_LOADS; ++i) xsrc[i] = experts_dma_row<T>(g, i0, wave, lane, i);
 #pragma unroll
-    for (int i = 0; i < T::W_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(wave * T::W_LOADS + i, lane);
-        wsrc[i] = g.W + ((size_t)e * g.N + min(n0 + r, g.N - 1)) * g.K + kd_load_channel<CPR>(r, lane);
-    }
+    for (int i = 0; i < T::W_LOADS; ++i) wsrc[i] = experts_dma_weight<T>(g, e, n0, wave, lane, i);
     floatx16 acc[WN][WM];
 #pragma unroll
     for (int a = 0; a < WN; ++a)
@@ -216,7 +234,7 @@ experts_dma_kernel(ExpertsDmaArgs g) {
 }
 
 template <int WN, int WM, int GN, int GM, int NS, int SL, bool GATED, bool F32>
-static int experts_dma_launch(const ExpertsDmaArgs& g, hipStream_t stream) {
+static int experts_dma_launch(ExpertsDmaArgs g, hipStream_t stream) {
     using T = KdTile<WN, WM, GN, GM, 64, NS>;
     static bool configured = false;
     auto kernel = experts_dma_kernel<WN, WM, GN, GM, NS, SL, GATED, F32>;
@@ -225,10 +243,90 @@ static int experts_dma_launch(const ExpertsDmaArgs& g, hipStream_t stream) {
         KA_CHECK(e == hipSuccess, "ka_experts_gemm_bf16: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
         configured = true;
     }
-    static_assert(T::BN == 256, "the caller counts columns of 256");
+    g.tiles_n = ka_cdiv(g.N, T::BN);
     const long blocks = ((long)g.n_tiles * g.tiles_n + 7) / 8 * 8;
     KA_CHECK(blocks < (1L << 31), "ka_experts_gemm_bf16: too many tiles");
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * GN * GM), T::SMEM, stream, g);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// Lists of as few pairs as the kernel further down takes (ka_experts_few_bf16): its sums, on products of 16 x 16 by 32 channels, every
+// fourth K-step into the same of four sums, so that a pair's bits do not depend on which of the two a step goes to. Tiles of EF_TILE list rows
+// by 128 weight rows, four waves, two workgroups a CU: four sums of each number are 64 registers, and it is the loads in flight that count
+// (the stream of the chosen experts' weights bounds it). Both linears, us, there -> here, weights from HBM: 30 experts of 2,048 x 704, 160
+// pairs 69 -> 69, 256 75 -> 70, 512 96 -> 73; 62 of 4,096 x 896, 144 pairs 271 -> 252, 240 295 -> 256, 510 340 -> 261. Tiles of 64 list rows by
+// eight waves: 76 to 82 and 271 to 289; by 256 weight rows 106 to 110 and 390; six stages and one workgroup a CU 73 to 80 and 266 to 277.
+constexpr int EF_TILE = 32;
+
+template <int WN, int WM, int GN, int GM, int NS>
+__global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(GN * GM / 4, GN * GM / 2)))
+experts_dma_few_kernel(ExpertsDmaArgs g, int out_f32) {
+    using T = KdTile<WN, WM, GN, GM, 64, NS, 16>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char eb_dma_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    int tile, column;
+    if (!experts_dma_find(g, tile, column)) return;
+    const int e = g.tile_expert[tile], i0 = tile * T::BM, n0 = column * T::BN;
+    const bf16_t* wsrc[T::W_LOADS];
+    const bf16_t* xsrc[T::X_LOADS];
+#pragma unroll
+    for (int i = 0; i < T::X_LOADS; ++i) xsrc[i] = experts_dma_row<T>(g, i0, wave, lane, i);
+#pragma unroll
+    for (int i = 0; i < T::W_LOADS; ++i) wsrc[i] = experts_dma_weight<T>(g, e, n0, wave, lane, i);
+    floatx4 acc[KD_FOURTHS][WN][WM];
+#pragma unroll
+    for (int c = 0; c < KD_FOURTHS; ++c)
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b) acc[c][a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    kd_product_16<WN, WM, GN, GM, NS, KD_FOURTHS>(
+        eb_dma_lds, wave, lane, g.K / 64, [&](int i, int st) { return wsrc[i] + st * 64; }, [&](int i, int st) { return xsrc[i] + st * 64; }, acc);
+    const int wn = wave / GM, wm = wave % GM, col = lane % 16, quarter = lane / 16;
+    const bool gated = ka_act_gated(g.act);
+#pragma unroll
+    for (int b = 0; b < WM; ++b) {
+        const int i = i0 + (wm * WM + b) * 16 + col, p = g.sorted[i];
+        if (p < 0) continue;
+        const long at = (g.scatter ? (long)p : (long)i) * g.ldo;
+#pragma unroll
+        for (int a = 0; a < WN; ++a) {
+            floatx4 y = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < KD_FOURTHS; ++c) y += acc[c][a][b];
+            const int o = n0 + (wn * WN + a) * 16 + quarter * 4;
+            if (gated) {
+                bf16_t* op = reinterpret_cast<bf16_t*>(g.out) + at + o / 2;
+                if (o + 1 < g.N) op[0] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[0], y[1]);
+                if (o + 3 < g.N) op[1] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[2], y[3]);
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (o + r >= g.N) continue;
+                const float v = ka_activate_fast(g.act, y[r]);
+                if (out_f32) reinterpret_cast<float*>(g.out)[at + o + r] = v;
+                else reinterpret_cast<bf16_t*>(g.out)[at + o + r] = (bf16_t)v;
+            }
+        }
+    }
+}
+
+static int experts_dma_few(ExpertsDmaArgs g, int out_f32, hipStream_t stream) {
+    using T = KdTile<2, 2, 4, 1, 64, 3, 16>;
+    static_assert(T::BM == EF_TILE, "the list is made for it");
+    static bool configured = false;
+    auto kernel = experts_dma_few_kernel<2, 2, 4, 1, 3>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM);
+        KA_CHECK(e == hipSuccess, "ka_experts_gemm_bf16: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
+        configured = true;
+    }
+    g.tiles_n = ka_cdiv(g.N, T::BN);
+    const long blocks = ((long)g.n_tiles * g.tiles_n + 7) / 8 * 8;
+    KA_CHECK(blocks < (1L << 31), "ka_experts_gemm_bf16: too many tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, g, out_f32);
     KA_LAUNCH_CHECK();
     return 0;
 }
@@ -276,6 +374,12 @@ KA_API int ka_experts_gemm_tile(int n_pairs, int E, int N1, int K1, int act, int
     return cost(256) < 1.2 * cost(128) ? 256 : 128;
 }
 
+// The tile whose sums are those of ka_experts_few_bf16; 0: more pairs than that takes, or sizes that its tiles do not cover.
+KA_API int ka_experts_gemm_few_tile(int n_pairs, int N1, int K1, int act, int N2) {
+    const int ff = ka_act_outputs(act, N1);
+    return n_pairs > 0 && n_pairs <= EF_MAX_PAIRS && experts_dma_covers(N1, K1, ff, act, 0) && experts_dma_covers(N2, ff, N2, 0, 1) ? EF_TILE : 0;
+}
+
 KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const void* W, const int* sorted, const int* tile_expert,
                                 int n_tiles, int tile, int N, int K, int act, int clamped, float limit, float slope, float shift, void* out,
                                 long ldo, int scatter, int out_f32, hipStream_t stream) {
@@ -287,7 +391,8 @@ KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const v
     KA_CHECK((uintptr_t)a % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)out % 16 == 0, "%s: operands must be 16-byte aligned", who);
     if (n_tiles == 0) return 0;
     if (experts_dma_covers(N, K, ldo, act, out_f32)) {
-        const ExpertsDmaArgs g{(const bf16_t*)a, lda, gather_div, (const bf16_t*)W, sorted, tile_expert, n_tiles, ka_cdiv(N, 256), N, K, act, clamp, out, ldo, scatter};
+        const ExpertsDmaArgs g{(const bf16_t*)a, lda, gather_div, (const bf16_t*)W, sorted, tile_expert, n_tiles, 0, N, K, act, clamp, out, ldo, scatter};
+        if (tile == EF_TILE) return experts_dma_few(g, out_f32, stream);
         if (tile == 64) return experts_dma<2, 1, 4, 2, 3, 2>(g, out_f32, stream);
         if (tile == 128) return experts_dma<2, 2, 4, 2, 3, 2>(g, out_f32, stream);
         if (tile == 256) return experts_dma<2, 4, 4, 2, 2, 1>(g, out_f32, stream);
@@ -318,7 +423,6 @@ KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const v
 // the columns, 16 or 32 at a time: a lane ends with four neighbouring outputs of one pair.
 // ----------------------------------------------------------------------------
 constexpr int EF_ROWS = 16;
-constexpr int EF_MAX_PAIRS = 512;
 constexpr int EF_WAVES = 4;
 typedef __attribute__((ext_vector_type(8))) __bf16 ef_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float ef_floatx4;

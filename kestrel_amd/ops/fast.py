@@ -76,6 +76,7 @@ _SIGNATURES = {
     "ka_heads_linear_supported": [_c_long, _c_int, _c_long, _c_int, _c_int, _c_int],
     "ka_experts_gemm_supported": [_c_long, _c_int, _c_int, _c_long, _c_int, _c_int],
     "ka_experts_gemm_tile": [_c_int] * 6,
+    "ka_experts_gemm_few_tile": [_c_int] * 5,
     "ka_experts_gemm_bf16": [_c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                              _c_float, _c_float, _c_void_p, _c_long, _c_int, _c_int, _c_void_p],
     "ka_experts_few_supported": [_c_int, _c_long, _c_int, _c_int, _c_int],
@@ -1071,7 +1072,7 @@ def experts_feed_forward_bf16(h, pairs, down, chosen, hidden, y, act, workspace,
     leaves the hidden rows in list order, the second writes fp32 ``y`` ``[n top, dim]`` at the pairs' own rows. ``pairs``
     ``[E, 2 hidden, dim]`` (not gated: ``[E, hidden, dim]``), ``down`` ``[E, dim, hidden]``, ``chosen`` int32 ``[n, top]``; ``hidden`` is not used (the list's hidden rows
     live in the workspace). ``clamp`` (a ``GateClamp``): the pair's product is the clamped one. ``tile``: list rows of a tile (for tests; else
-    chosen by the sizes). False: not covered (sizes that are no multiple of 16, alignment), nothing was run."""
+    chosen by the sizes, and for as few pairs as ``experts_few_bf16`` takes the sums have the order, and the bits, of that kernel). False: not covered (sizes that are no multiple of 16, alignment), nothing was run."""
     n, top = chosen.shape
     n_experts, n_pair_rows, dim = pairs.shape
     ff = down.shape[2]
@@ -1086,7 +1087,9 @@ def experts_feed_forward_bf16(h, pairs, down, chosen, hidden, y, act, workspace,
         raise KernelError("experts: the first linear's rows do not fit the hidden size")
     if not handle.ka_experts_gemm_supported(lda, n_pair_rows, dim, ff, act, 0) or not handle.ka_experts_gemm_supported(ff, dim, ff, dim, 0, 1):
         return False
-    tile = int(tile or handle.ka_experts_gemm_tile(n * top, n_experts, n_pair_rows, dim, act, dim))
+    # (as few pairs as the kernel of few takes: its sums, whatever the list)
+    tile = int(tile or handle.ka_experts_gemm_few_tile(n * top, n_pair_rows, dim, act, dim)
+               or handle.ka_experts_gemm_tile(n * top, n_experts, n_pair_rows, dim, act, dim))
     # (sized by the step's tokens alone: the same for every replay of a captured step; the scratch tensors for the largest tile, so
     # that a step of fewer tokens never asks for more)
     capacity = -(-(n * top + n_experts * (tile - 1)) // tile) * tile

@@ -96,3 +96,28 @@ def test_few_rows_have_the_bits_of_the_kernel_that_streams_weights(m, n, ks):
         assert torch.equal(*results)
     want = start.double() + bias.double() + sum(a.double() @ w.double().T for a, w in zip(rows, weights))
     assert float((results[0].double() - want).norm() / want.norm()) < 2.0 ** -20
+
+
+@pytest.mark.parametrize("clamped", [False, True])
+@pytest.mark.parametrize("n, top, n_experts, dim, ff", [(1, 1, 1, 64, 64), (33, 4, 30, 448, 704), (128, 4, 30, 2048, 704), (85, 6, 62, 256, 896), (512, 1, 3, 192, 128),
+                                                        (40, 6, 5, 320, 64)])
+def test_lists_of_few_pairs_have_the_bits_of_the_kernel_of_few(n, top, n_experts, dim, ff, clamped):
+    """Up to 512 pairs an expert's weights are streamed past its pairs or its pairs are listed and go by tiles: the same order of every sum."""
+    from kestrel_amd.engine.batch import Workspace
+    from kestrel_amd.ops import fast
+    from kestrel_amd.ops.linear import ACT_GATED, activation_code
+    from kestrel_amd.parts.specs import GateClamp
+
+    gen = torch.Generator().manual_seed(n + dim + ff)
+    h = torch.randn(n, dim, generator=gen).bfloat16().to(DEV)
+    clamp = GateClamp(0.7, 1.702, 1.0) if clamped else None
+    chosen = torch.stack([torch.randperm(n_experts + 1, generator=gen)[:top] for _ in range(n)]).to(torch.int32).to(DEV)
+    down = (torch.randn(n_experts, dim, ff, generator=gen) * ff ** -0.5).bfloat16().to(DEV)
+    for act, rows in ((activation_code("silu") | ACT_GATED, 2 * ff), (activation_code("relu_squared"), ff)):
+        if clamped and not act & ACT_GATED:
+            continue
+        first = (torch.randn(n_experts, rows, dim, generator=gen) * dim ** -0.5).bfloat16().to(DEV)
+        few, listed = (torch.full((n * top, dim), 7.0, device=DEV) for _ in range(2))
+        assert fast.experts_few_bf16(h, first, down, chosen, torch.empty(n * top, ff, dtype=torch.bfloat16, device=DEV), few, act, clamp=clamp)
+        assert fast.experts_feed_forward_bf16(h, first, down, chosen, None, listed, act, Workspace(torch.device(DEV)), clamp=clamp)
+        assert torch.equal(few, listed)
