@@ -151,11 +151,9 @@ __global__ void __launch_bounds__(LC_THREADS) linear_chunk_local_kernel(LinearCh
 
 // SCAN: a row's chunks in order: every record gets the state its chunk starts from, the request's state is what the last
 // chunk ends with. Grid (H, rows, slices of 1,024 numbers of S), four numbers a thread. BY_CHANNEL: what a chunk's state keeps of
-// the one before comes from `factors` [chunks, H, d], key channel by key channel. KEYS_FIRST: the request's state is [H, d, dv], and
-// behind it stands the stream's row of its last token, from `x` [n, dim].
-template <bool BY_CHANNEL, bool KEYS_FIRST>
-__global__ void __launch_bounds__(LC_THREADS) linear_chunk_scan_kernel(LinearChunkArgs a, const float* __restrict__ factors, const float* __restrict__ x_rows,
-                                                                       int dim) {
+// the one before comes from `factors` [chunks, H, d], key channel by key channel.
+template <bool BY_CHANNEL>
+__global__ void __launch_bounds__(LC_THREADS) linear_chunk_scan_kernel(LinearChunkArgs a, const float* __restrict__ factors) {
     const int head = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid % KA_WAVE;
     const int t0 = a.cu_q[r], t1 = a.cu_q[r + 1];
     if (t0 >= t1) return;
@@ -166,12 +164,9 @@ __global__ void __launch_bounds__(LC_THREADS) linear_chunk_scan_kernel(LinearChu
     const int base = (int)ka_wave_sum((float)before);
     const int nc = (t1 - t0 + LC_CHUNK - 1) / LC_CHUNK;
     const int per = a.d * a.dv;
-    if (KEYS_FIRST && head == 0 && blockIdx.z == 0 && x_rows != nullptr)
-        for (int c = tid; c < dim; c += LC_THREADS) a.state[(size_t)slot * a.state_stride + (size_t)a.H * per + c] = x_rows[(size_t)(t1 - 1) * dim + c];
     const int e = (blockIdx.z * LC_THREADS + tid) * 4;
     if (e >= per) return;
-    float* st = a.state + (size_t)slot * a.state_stride + (size_t)head * per + (KEYS_FIRST ? e % a.d * a.dv + e / a.d : e);
-    const int hop = KEYS_FIRST ? a.dv : 1;
+    float* st = a.state + (size_t)slot * a.state_stride + (size_t)head * per + e;
     float* rec = a.chunks + ((size_t)base * a.H + head) * per + e;
     const size_t step = (size_t)a.H * per;
     const float l2 = BY_CHANNEL ? 0.f : a.log2_decay[head];
@@ -183,7 +178,7 @@ __global__ void __launch_bounds__(LC_THREADS) linear_chunk_scan_kernel(LinearChu
         const float f = c + 1 < nc ? whole : last;
         return make_float4(f, f, f, f);
     };
-    float4 cur = KEYS_FIRST ? make_float4(st[0], st[hop], st[2 * hop], st[3 * hop]) : *reinterpret_cast<const float4*>(st);
+    float4 cur = *reinterpret_cast<const float4*>(st);
     auto advance = [&](const float4& f, const float4& x) {
         cur.x = fmaf(f.x, cur.x, x.x);
         cur.y = fmaf(f.y, cur.y, x.y);
@@ -209,14 +204,7 @@ __global__ void __launch_bounds__(LC_THREADS) linear_chunk_scan_kernel(LinearChu
         *reinterpret_cast<float4*>(rec + c * step) = cur;
         advance(f, x);
     }
-    if constexpr (KEYS_FIRST) {
-        st[0] = cur.x;
-        st[hop] = cur.y;
-        st[2 * hop] = cur.z;
-        st[3 * hop] = cur.w;
-    } else {
-        *reinterpret_cast<float4*>(st) = cur;
-    }
+    *reinterpret_cast<float4*>(st) = cur;
 }
 
 // READ: the read-outs of one chunk and one slice of value channels. Wave w takes the tokens [32 (w % 2), + 32) and the value
@@ -366,8 +354,7 @@ KA_API int ka_linear_chunks_bf16(const void* q, const void* k, const void* v, lo
         sized = true;
     }
     hipLaunchKernelGGL(linear_chunk_local_kernel, dim3(H, n_chunks, slices), dim3(LC_THREADS), local_lds, stream, a);
-    hipLaunchKernelGGL((linear_chunk_scan_kernel<false, false>), dim3(H, n_rows, ka_cdiv((long)d * dv, 4 * LC_THREADS)), dim3(LC_THREADS), 0, stream, a,
-                       nullptr, nullptr, 0);
+    hipLaunchKernelGGL(linear_chunk_scan_kernel<false>, dim3(H, n_rows, ka_cdiv((long)d * dv, 4 * LC_THREADS)), dim3(LC_THREADS), 0, stream, a, nullptr);
     hipLaunchKernelGGL(linear_chunk_read_kernel, dim3(H, n_chunks, slices), dim3(LC_THREADS), read_lds, stream, a);
     KA_LAUNCH_CHECK();
     return 0;
@@ -383,13 +370,6 @@ KA_API int ka_linear_chunks_bf16(const void* q, const void* k, const void* v, lo
 // block's start, l_t, and up to it, B_T (b_t = B_T + l_t). Between blocks U < T a score is the product of q_t 2^(l_t) and
 // k_s 2^(B_T - b_s), both powers at most 1, on the matrix cores; within a block every power is taken by itself. So no factor,
 // however small, leaves its range. What carries a power enters its product as two bf16 numbers, as above.
-//
-// DECAYING: the same for the decaying matrix memory (recurrent_parts.hip), whose read-outs see the state before their own token's
-// update, with a bonus u for the token's own key:
-//     o_t = (S_(t-1) + v_t (u * k_t)^T) r_t,   S_t = S_(t-1) diag(w_t) + v_t k_t^T,   w_t[i] = e^(-e^(pre_t[i]))
-// A query then carries the sums up to the token before it, l_(t-1) (0 at a block's start), its own key's score is
-// sum_i r_t[i] u[i] k_t[i], and the rest stays. A decay is taken as no less than 2^-150, below which it and everything it
-// multiplies is 0 in fp32 (an infinite logarithm would make a difference of two of them nothing at all).
 // ----------------------------------------------------------------------------
 constexpr int LC_BLOCK = 16;
 constexpr int LC_BLOCKS = LC_CHUNK / LC_BLOCK;
@@ -402,24 +382,7 @@ struct GatedChunkArgs : LinearChunkArgs {
     const float* pre;           // [n, H d]
     float* factors;             // [chunks, H, d]: 2^(b_L) of every chunk
     float per_tau, q_scale;     // 1 / tau
-    const float* bonus;         // DECAYING: u [H, d]
-    // DECAYING, heads of one slice: the read-outs leave normalised and gated, out = o / rms(o) gain gate, and raw is not written
-    const float* gain;          // [H dv]
-    const bf16_t* gate;         // rows of `stride`
-    bf16_t* out;
-    long out_stride;
-    float eps;
 };
-
-template <bool DECAYING>
-__device__ __forceinline__ float lc_log2_decay(const GatedChunkArgs& a, float z) {
-    if constexpr (DECAYING) {
-        const float l = -1.4426950408889634f * __expf(z);
-        return l < -150.f ? -150.f : l;          // (NaN stays)
-    } else {
-        return ka_log2_decay<true>(z, a.per_tau);
-    }
-}
 
 __device__ __forceinline__ float lc_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -438,7 +401,6 @@ __device__ __forceinline__ void lc_stage_values(const LinearChunkArgs& a, bf16_t
 }
 
 // l of the 16 tokens of block `block` for key channel i of the head (zeros behind the last token and the last channel).
-template <bool DECAYING>
 __device__ __forceinline__ void lc_block_logs(const GatedChunkArgs& a, int head, int c0, int valid, int block, int i, float (&l)[LC_BLOCK]) {
     const float* z = a.pre + (size_t)c0 * a.H * a.d + (size_t)head * a.d + i;
     float x[LC_BLOCK];
@@ -450,14 +412,13 @@ __device__ __forceinline__ void lc_block_logs(const GatedChunkArgs& a, int head,
     float run = 0.f;
 #pragma unroll
     for (int u = 0; u < LC_BLOCK; ++u) {
-        if (i < a.d && block * LC_BLOCK + u < valid) run += lc_log2_decay<DECAYING>(a, x[u]);
+        if (i < a.d && block * LC_BLOCK + u < valid) run += ka_log2_decay<true>(x[u], a.per_tau);
         l[u] = run;
     }
 }
 
 // LOCAL: what the chunk adds to the state by its end, of one slice of value channels, and (the first slice) its factors.
 // Grid (H, chunks, slices). A wave takes a block of tokens, a lane a key channel.
-template <bool DECAYING>
 __global__ void __launch_bounds__(LC_THREADS) gated_chunk_local_kernel(GatedChunkArgs a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lc_lds[];
     int row, c0, c1;
@@ -474,7 +435,7 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_local_kernel(GatedChun
     lc_stage_values(a, VT, head, c0, valid, j0);
     for (int i = lane; i < d64; i += KA_WAVE) {
         float l[LC_BLOCK];
-        lc_block_logs<DECAYING>(a, head, c0, valid, wave, i, l);
+        lc_block_logs(a, head, c0, valid, wave, i, l);
         bf16_t k[LC_BLOCK];
 #pragma unroll
         for (int u = 0; u < LC_BLOCK; ++u) {
@@ -533,7 +494,6 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_local_kernel(GatedChun
 // READ: the read-outs of one chunk. Wave T takes the queries of block T. Grid (H, chunks, value slices at once); a workgroup
 // takes every gridDim.z-th slice of 64 value channels. In all products the queries are the column operand: a lane ends with
 // results of one query.
-template <bool DECAYING>
 __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunkArgs a) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lc_lds[];
     int row, c0, c1;
@@ -542,13 +502,9 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
     const int head = blockIdx.x, tid = threadIdx.x;
     const int valid = c1 - c0;
     const size_t out_row = (size_t)a.H * dv;
-    const bool finishes = DECAYING && a.out != nullptr;
     if (a.row_slot[row] < 0) {
         if (blockIdx.z == 0)
-            for (int e = tid; e < valid * dv; e += LC_THREADS) {
-                if (finishes) a.out[(size_t)(c0 + e / dv) * a.out_stride + (size_t)head * dv + e % dv] = (bf16_t)0.f;
-                else a.raw[(size_t)(c0 + e / dv) * out_row + (size_t)head * dv + e % dv] = 0.f;
-            }
+            for (int e = tid; e < valid * dv; e += LC_THREADS) a.raw[(size_t)(c0 + e / dv) * out_row + (size_t)head * dv + e % dv] = 0.f;
         return;
     }
     bf16_t* Qs = lc_lds;                        // [64][lq]
@@ -575,7 +531,7 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
     }
     for (int i = lane; i < d32; i += KA_WAVE) {
         float l[LC_BLOCK];
-        lc_block_logs<DECAYING>(a, head, c0, valid, wave, i, l);
+        lc_block_logs(a, head, c0, valid, wave, i, l);
 #pragma unroll
         for (int u = 0; u < LC_BLOCK; ++u) Ls[(wave * LC_BLOCK + u) * lb + i] = l[u];
     }
@@ -592,15 +548,10 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
     const int col = lane % 16, quarter = lane / 16;
     const bool active = wave * LC_BLOCK < valid;
     const int t = wave * LC_BLOCK + col;        // the lane's query (and, within the block, the lane's key)
-    // the sums that the query at `at` carries, four channels from c on: its own, or those of the token before it
-    auto query_logs = [&](int at, int c) {
-        if (DECAYING && at % LC_BLOCK == 0) return lc_floatx4{0.f, 0.f, 0.f, 0.f};
-        return *reinterpret_cast<const lc_floatx4*>(Ls + (DECAYING ? at - 1 : at) * lb + c);
-    };
     // q_t 2^(l_t) of the eight channels from c on
     auto query = [&](int c, lc_bf16x8& hi, lc_bf16x8& lo) {
         const lc_bf16x8 x = *reinterpret_cast<const lc_bf16x8*>(Qs + t * lq + c);
-        const lc_floatx4 l0 = query_logs(t, c), l1 = query_logs(t, c + 4);
+        const lc_floatx4 l0 = *reinterpret_cast<const lc_floatx4*>(Ls + t * lb + c), l1 = *reinterpret_cast<const lc_floatx4*>(Ls + t * lb + c + 4);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             bf16_t h, r;
@@ -617,21 +568,15 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
         for (int c = quarter * (d32 / 4); c < (quarter + 1) * (d32 / 4); c += 8) {
             const lc_bf16x8 k = *reinterpret_cast<const lc_bf16x8*>(Ks + t * lq + c);
             const lc_floatx4 k0 = *reinterpret_cast<const lc_floatx4*>(Ls + t * lb + c), k1 = *reinterpret_cast<const lc_floatx4*>(Ls + t * lb + c + 4);
-            float own[8];                       // DECAYING: the factors of a token's own key
-            if constexpr (DECAYING)
-#pragma unroll
-                for (int m = 0; m < 8; ++m) own[m] = c + m < d ? a.bonus[(size_t)head * d + c + m] : 0.f;
 #pragma unroll
             for (int u = 0; u < LC_BLOCK; ++u) {
                 const int at = wave * LC_BLOCK + u;
                 const lc_bf16x8 q = *reinterpret_cast<const lc_bf16x8*>(Qs + at * lq + c);
-                const lc_floatx4 l0 = query_logs(at, c), l1 = query_logs(at, c + 4);
+                const lc_floatx4 l0 = *reinterpret_cast<const lc_floatx4*>(Ls + at * lb + c), l1 = *reinterpret_cast<const lc_floatx4*>(Ls + at * lb + c + 4);
 #pragma unroll
                 for (int m = 0; m < 8; ++m) {
                     const float gap = m < 4 ? l0[m % 4] - k0[m % 4] : l1[m % 4] - k1[m % 4];
-                    float weight = lc_exp2(fminf(gap, 0.f));                 // (keys behind their query: not used)
-                    if constexpr (DECAYING) weight = u == col ? own[m] : weight;
-                    score[u] = fmaf((float)q[m] * (float)k[m], weight, score[u]);
+                    score[u] = fmaf((float)q[m] * (float)k[m], lc_exp2(fminf(gap, 0.f)), score[u]);      // (keys behind their query: not used)
                 }
             }
         }
@@ -697,7 +642,7 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
         __syncthreads();
         lc_stage_values(a, VT, head, c0, valid, j0);
         __syncthreads();
-        if (!active) continue;                  // (whole waves)
+        if (!active) continue;
         lc_floatx4 o[LC_SLICE / 16];
 #pragma unroll
         for (int j = 0; j < LC_SLICE / 16; ++j) o[j] = lc_floatx4{0.f, 0.f, 0.f, 0.f};
@@ -736,30 +681,6 @@ __global__ void __launch_bounds__(LC_THREADS) gated_chunk_read_kernel(GatedChunk
                 o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pl, o[j], 0, 0, 0);
             }
         }
-        if (finishes) {                         // (one slice: the four quarters hold a token's whole head)
-            float ss = 0.f;
-#pragma unroll
-            for (int j = 0; j < LC_SLICE / 16; ++j)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) ss = fmaf(o[j][u], o[j][u], ss);
-            ss += __shfl_xor(ss, 16);
-            ss += __shfl_xor(ss, 32);
-            const float inv = 1.0f / sqrtf(ss / (float)dv + a.eps);
-            if (t >= valid) continue;
-#pragma unroll
-            for (int j = 0; j < LC_SLICE / 16; ++j) {
-                const int c = j * 16 + quarter * 4;
-                if (c >= dv) continue;
-                const size_t at = (size_t)head * dv + c;
-                const lc_floatx4 g = *reinterpret_cast<const lc_floatx4*>(a.gain + at);
-                const lc_bf16x4 z = *reinterpret_cast<const lc_bf16x4*>(a.gate + (size_t)(c0 + t) * a.stride + at);
-                lc_bf16x4 y;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) y[u] = (bf16_t)(o[j][u] * inv * g[u] * (float)z[u]);
-                *reinterpret_cast<lc_bf16x4*>(a.out + (size_t)(c0 + t) * a.out_stride + at) = y;
-            }
-            continue;
-        }
         if (t >= valid) continue;
         float* op = a.raw + (size_t)(c0 + t) * out_row + (size_t)head * dv + j0 + quarter * 4;
 #pragma unroll
@@ -773,28 +694,6 @@ KA_API int ka_gated_chunks_supported(int d, int dv) { return d > 0 && d % 16 == 
 
 // Floats of the launches' buffer of a step of `n` tokens in `n_rows` rows: a state and its factors per chunk and head.
 KA_API long ka_gated_chunks_scratch(int n, int n_rows, int H, int d, int dv) { return (long)(n / LC_CHUNK + n_rows) * H * d * (dv + 1); }
-
-// The three launches. `x` [n, dim]: DECAYING, the rows whose last one a request keeps.
-template <bool DECAYING>
-static void gated_chunks_launch(const GatedChunkArgs& a, int n_rows, long n_chunks, const float* x, int dim, hipStream_t stream) {
-    const int d = a.d, dv = a.dv, H = a.H;
-    const int slices = ka_cdiv(dv, LC_SLICE), d32 = (d + 31) / 32 * 32, d64 = (d + 63) / 64 * 64;
-    const size_t local_lds = sizeof(bf16_t) * (size_t)(2 * d32 + LC_SLICE) * LC_ROW + sizeof(float) * LC_BLOCKS * d64;
-    const size_t read_lds = sizeof(bf16_t) * ((size_t)2 * LC_CHUNK * (d32 + LC_PAD) + (size_t)3 * LC_CHUNK * LC_ROW) +
-                            sizeof(float) * ((size_t)LC_CHUNK * (d32 + 4) + (size_t)LC_BLOCKS * d32);
-    static bool sized = false;
-    if (!sized) {
-        (void)hipFuncSetAttribute((const void*)gated_chunk_local_kernel<DECAYING>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)gated_chunk_read_kernel<DECAYING>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        sized = true;
-    }
-    // (scores are shared by the slices a workgroup takes: all of them where heads and chunks fill the GPU)
-    const int at_once = (long)H * n_chunks >= 2L * ka_compute_units() ? 1 : slices;
-    hipLaunchKernelGGL(gated_chunk_local_kernel<DECAYING>, dim3(H, n_chunks, slices), dim3(LC_THREADS), local_lds, stream, a);
-    hipLaunchKernelGGL((linear_chunk_scan_kernel<true, DECAYING>), dim3(H, n_rows, ka_cdiv((long)d * dv, 4 * LC_THREADS)), dim3(LC_THREADS), 0, stream,
-                       a, a.factors, x, dim);
-    hipLaunchKernelGGL(gated_chunk_read_kernel<DECAYING>, dim3(H, n_chunks, at_once), dim3(LC_THREADS), read_lds, stream, a);
-}
 
 KA_API int ka_gated_chunks_bf16(const void* q, const void* k, const void* v, long stride, const float* pre, float tau, float q_scale,
                                 float* state, long state_stride, const int* cu_q, const int* row_slot, float* raw, float* scratch, int n,
@@ -815,49 +714,21 @@ KA_API int ka_gated_chunks_bf16(const void* q, const void* k, const void* v, lon
     a.factors = scratch + n_chunks * H * d * dv;
     a.per_tau = 1.f / tau;
     a.q_scale = q_scale;
-    a.bonus = a.gain = nullptr;
-    a.gate = nullptr;
-    a.out = nullptr;
-    gated_chunks_launch<false>(a, n_rows, n_chunks, nullptr, 0, stream);
+    const int slices = ka_cdiv(dv, LC_SLICE), d32 = (d + 31) / 32 * 32, d64 = (d + 63) / 64 * 64;
+    const size_t local_lds = sizeof(bf16_t) * (size_t)(2 * d32 + LC_SLICE) * LC_ROW + sizeof(float) * LC_BLOCKS * d64;
+    const size_t read_lds = sizeof(bf16_t) * ((size_t)2 * LC_CHUNK * (d32 + LC_PAD) + (size_t)3 * LC_CHUNK * LC_ROW) +
+                            sizeof(float) * ((size_t)LC_CHUNK * (d32 + 4) + (size_t)LC_BLOCKS * d32);
+    static bool sized = false;
+    if (!sized) {
+        (void)hipFuncSetAttribute((const void*)gated_chunk_local_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)gated_chunk_read_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        sized = true;
+    }
+    // (scores are shared by the slices a workgroup takes: all of them where heads and chunks fill the GPU)
+    const int at_once = (long)H * n_chunks >= 2L * ka_compute_units() ? 1 : slices;
+    hipLaunchKernelGGL(gated_chunk_local_kernel, dim3(H, n_chunks, slices), dim3(LC_THREADS), local_lds, stream, a);
+    hipLaunchKernelGGL(linear_chunk_scan_kernel<true>, dim3(H, n_rows, ka_cdiv((long)d * dv, 4 * LC_THREADS)), dim3(LC_THREADS), 0, stream, a, a.factors);
+    hipLaunchKernelGGL(gated_chunk_read_kernel, dim3(H, n_chunks, at_once), dim3(LC_THREADS), read_lds, stream, a);
     KA_LAUNCH_CHECK();
     return 0;
-}
-
-// The decaying matrix memory over prompt portions (ka_decayed_memory: operands as there; `scratch` as for the gated one). Heads of up
-// to 64 channels leave normalised and gated, in `out` (returns 0, `raw` is not written); the read-outs of larger ones are left in `raw`
-// (returns 1: ka_decayed_readout finishes them).
-//
-// Token by token a head is a serial chain, 1.3 to 2.9 us per 16 tokens whatever the chip; by chunks all of a step's run at once.
-// Measured, 32 heads of 64: 2,048 tokens of one row 590 us and 16 for the norm -> 93 all together; two rows of 800 tokens
-// 251 and 11 -> 86; eight of 100 84 -> 51.
-KA_API int ka_decayed_chunks_bf16(const void* r, const void* k, const void* v, const void* gate, long stride, const float* pre, const float* u,
-                                  const float* gain, float* state, long state_stride, const float* x, int dim, const int* cu_q, const int* row_slot,
-                                  void* out, long out_stride, float* raw, float* scratch, int n, int n_rows, int H, int d, float eps,
-                                  hipStream_t stream) {
-    const char* who = "ka_decayed_chunks_bf16";
-    KA_CHECK(n >= 0 && n_rows >= 0 && H > 0 && eps >= 0.f && ka_gated_chunks_supported(d, d), "%s: heads of %d not covered", who, d);
-    KA_CHECK(pre != nullptr && u != nullptr && dim >= 0, "%s: a decay needs its pre-activations, a token its bonus", who);
-    KA_CHECK((uintptr_t)r % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 && (uintptr_t)gate % 8 == 0 && stride % 8 == 0 &&
-             (uintptr_t)raw % 16 == 0 && (uintptr_t)scratch % 16 == 0 && (uintptr_t)gain % 16 == 0 && (uintptr_t)out % 8 == 0 && out_stride % 4 == 0,
-             "%s: operands must be 16-byte aligned", who);
-    KA_CHECK(state_stride >= (long)H * d * d + (x ? dim : 0) && stride >= (long)H * d && out_stride >= (long)H * d, "%s: rows are shorter than their heads", who);
-    const long n_chunks = n / LC_CHUNK + n_rows;
-    KA_CHECK(H <= 65535 && n_rows <= 65535 && n_chunks <= 65535 && scratch != nullptr, "%s: too many heads, rows or chunks", who);
-    if (n == 0 || n_rows == 0) return 0;
-    GatedChunkArgs a;
-    static_cast<LinearChunkArgs&>(a) = LinearChunkArgs{(const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)v, stride, nullptr, state, state_stride,
-                                                       cu_q, row_slot, raw, scratch, n_rows, H, d, d, KA_ACT_NONE};
-    a.pre = pre;
-    a.factors = scratch + n_chunks * H * d * d;
-    a.per_tau = 1.f;
-    a.q_scale = 1.f;
-    a.bonus = u;
-    a.gain = gain;
-    a.gate = (const bf16_t*)gate;
-    a.out = d <= LC_SLICE ? (bf16_t*)out : nullptr;
-    a.out_stride = out_stride;
-    a.eps = eps;
-    gated_chunks_launch<true>(a, n_rows, n_chunks, x, dim, stream);
-    KA_LAUNCH_CHECK();
-    return a.out ? 0 : 1;
 }

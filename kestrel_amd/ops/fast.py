@@ -90,6 +90,7 @@ _SIGNATURES = {
     "ka_gated_chunks_scratch": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "ka_gated_chunks_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_float, _c_float, _c_void_p, _c_long, _c_void_p, _c_void_p,
                              _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_decayed_chunks_supported": [_c_int],
     "ka_decayed_chunks_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_int,
                                _c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     "ka_linear_chunks_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_void_p,
@@ -994,17 +995,17 @@ def gated_chunks_bf16(projected, offsets, pre, tau, q_scale, state, cu_q, row_sl
 
 
 def decayed_chunks_bf16(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, out, n_heads, head_dim, eps, raw, scratch) -> bool:
-    """``ops.core.decayed_memory`` for prompt portions on the matrix cores: the recurrence unrolled over chunks of 64 tokens, all chunks at
-    once in three launches (operands as there; ``scratch``: contiguous fp32 of at least ``gated_chunks_scratch`` numbers for
-    heads of ``head_dim`` by ``head_dim``). False: sizes or alignment not covered, nothing was run."""
+    """``ops.core.decayed_memory`` for prompt portions: its walk over the tokens in fp32, cut into chunks of 64 that run at once in three launches
+    (operands as there; ``scratch``: contiguous fp32 of at least ``gated_chunks_scratch`` numbers for heads of ``head_dim`` by
+    ``head_dim``). False: sizes or alignment not covered, nothing was run."""
     handle = lib()
     n, n_rows, dim = core.check_decayed_memory(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, out, n_heads, head_dim)
     if n == 0:
         return True
     width = n_heads * head_dim
     stride, out_stride = (r.stride(0), out.stride(0)) if n > 1 else (max(r.stride(0), width), max(out.stride(0), width))
-    if r.dtype != torch.bfloat16 or not handle.ka_gated_chunks_supported(int(head_dim), int(head_dim)) or stride % 8 or out_stride % 4 \
-            or any(t.data_ptr() % 16 for t in (r, k, v, gain)) or gate.data_ptr() % 8 or out.data_ptr() % 8 or n // 64 + n_rows > 65535:
+    if r.dtype != torch.bfloat16 or not handle.ka_decayed_chunks_supported(int(head_dim)) or stride % 4 or any(t.data_ptr() % 8 for t in (r, k, v)) \
+            or any(t.data_ptr() % 16 for t in (pre, u)) or n // 64 + n_rows > 65535:
         return False
     for t, numbers, what in ((scratch, gated_chunks_scratch(n, n_rows, n_heads, head_dim, head_dim), "scratch"), (raw, n * width, "read-outs")):
         if t.dtype != torch.float32 or not t.is_contiguous() or t.numel() < numbers or not t.is_cuda or t.data_ptr() % 16:
@@ -1013,7 +1014,7 @@ def decayed_chunks_bf16(r, k, v, gate, pre, u, gain, state, x, cu_q, row_slot, o
                                            gain.data_ptr(), state.data_ptr(), state.stride(0), x.data_ptr() if x is not None else None, dim,
                                            cu_q.data_ptr(), row_slot.data_ptr(), out.data_ptr(), out_stride, raw.data_ptr(), scratch.data_ptr(),
                                            n, n_rows, n_heads, head_dim, float(eps), stream_ptr())
-    if status == 1:          # (heads of more than one slice of value channels)
+    if status == 1:          # (heads of more than 64 channels)
         core.decayed_readout(raw.view(-1)[:n * width].view(n, width), gate, gain, out, n_heads, head_dim, eps)
         return True
     _check(status)

@@ -32,15 +32,15 @@ class DecayedMemory(Mixer):
     The mixer reads the fp32 stream itself (``reads_stream``): the mixes are computed in fp32 and rounded once to the
     activation type. The five projections are linears of that type; the second linear of the decay writes fp32 (with
     ``w0`` as its bias) and the exponentials are taken in the recurrence kernel, so that everything that enters the
-    recurrence besides the projections is fp32. One kernel walks over every row's tokens in order and a second normalises the read-outs
-    (``ops.core.decayed_memory``): prompts in float32, short portions, heads that the other kernels do not take. Prompts and portions in
-    bfloat16 go by chunks of 64 tokens over the matrix cores (``ops.fast.decayed_chunks_bf16``); a step of single tokens takes one launch
-    for the decay's second linear, the recurrence, norm and gate (``ops.core.decayed_step``), behind one launch for the five
+    recurrence besides the projections is fp32, and so is all of its arithmetic. One kernel walks over every row's tokens in order and a second
+    normalises the read-outs (``ops.core.decayed_memory``): prompts in float32, steps of up to 64 tokens, heads that the other kernels do not
+    take. Longer steps in bfloat16 walk over chunks of 64 tokens at once (``ops.fast.decayed_chunks_bf16``: a chunk's state is its own and
+    that of the chunk before times the product of its decays); a step of single tokens takes one launch for the decay's second linear, the recurrence, norm and gate (``ops.core.decayed_step``), behind one launch for the five
     projections in bfloat16 (``ops.fast.linears_few_bf16``). Rows without a request
     (the padding of a replayed step) write zeros and touch no state."""
 
     replays_every_step = True
-    CHUNKS_FROM_TOKENS = 65      # (64 tokens of one row: 27 us one by one, 34 by chunks; 512: 157 and 36)
+    CHUNKS_FROM_TOKENS = 65      # (65 tokens of one row: 27 us as a row, 29 in two chunks; 128: 44 and 30; eight rows of 20: 24 and 15)
     reads_stream = True
 
     def __init__(self, spec: DecayedMemorySpec) -> None:

@@ -1,4 +1,4 @@
-"""The decaying matrix memory by chunks on the matrix cores, against the recurrence in float64."""
+"""The decaying matrix memory by chunks, against the recurrence in float64."""
 
 from __future__ import annotations
 
@@ -17,8 +17,9 @@ DEV = "cuda:0"
 def test_decaying_memory_by_chunks(heads, d, decays):
     """Rows fed in pieces that begin and end anywhere in a chunk and in a block of it, a row without a request, pieces of one
     token through the other kernel in between (the state is one and the same). "sudden": decays from 1 to exactly 0 beside
-    each other. The bound: the output is rounded to bf16 (2^-9); what carries a power enters its products with sixteen bits,
-    which is far less, unless the terms cancel, as they may in a few of some thousand tokens (2^-6 for any one of them, 2^-8.5 over all)."""
+    each other. The bound: the output is rounded to bf16 (2^-9); what fp32 sums are off is far less, unless the terms cancel, as
+    they may in a few of some thousand tokens (2^-6 for any one of them, 2^-8.5 over all; the state at a finer bound in
+    test_decayed_walks_gpu.py)."""
     from kestrel_amd.ops import core, fast
 
     gen = torch.Generator().manual_seed(heads * 1000 + d)
