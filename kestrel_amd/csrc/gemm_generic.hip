@@ -1,10 +1,13 @@
 // Generic linear layer: out = act(A W^T + bias) or out += A W^T + bias.
 //
-// Plain FMA in fp32 with an LDS-tiled 64x64x16 block, any M, N, K, any mix of fp32
-// and bf16 operands. Every output element is the sum over k = 0..K-1 in that order,
-// whatever M and N are, so a row's result does not depend on what else is in the
-// batch. This is the true 32-bit path and the fallback of the bf16 path. (Many rows, and few rows, of
-// aligned fp32 operands have kernels of their own below, each with its own fixed order of the sum.)
+// Four kernels, each with an order of a sum that K alone fixes:
+//  * any M, N, K, any mix of fp32 and bf16 operands: plain FMA in fp32 with an LDS-tiled 64x64x16 block, k = 0..K-1 in that
+//    order; the fallback of the bf16 path;
+// and, of aligned fp32 operands, the true 32-bit path,
+//  * up to 16 rows of a linear without a gate: a stream of weights (gemv_f32_kernel);
+//  * else K in steps of 32: the matrix pipes (gemm_f32_mfma_kernel);
+//  * else wider FMA tiles, k in ascending order as the first (gemm_f32_kernel).
+// So a row's result does not depend on what else is in the batch, but for the step from 16 to 17 rows without a gate.
 #include "ka_common.h"
 #include "ka_dma_tiles.h"
 
@@ -495,7 +498,9 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
     int key = a_dtype * 4 + w_dtype * 2 + out_dtype;
     const bool vectors = key == 0 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 &&
                          (uintptr_t)W % 16 == 0;
-    if (vectors && M > GV_ROWS && K % F32_STEP == 0) {
+    // (a gated linear at any number of rows, since the weight-streaming kernel has no pairs: its sums then never depend on the rows
+    // beside a row. 1 to 16 rows of 2,048 inputs, 16,384 outputs: 199 to 212 us by vector tiles, 28 here; 1,408: 180 to 188 and 16.5)
+    if (vectors && (M > GV_ROWS || ka_act_gated(act)) && K % F32_STEP == 0) {
         return launch_f32_best((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream);
     }
     if (vectors && M > GV_ROWS && ka_cdiv(M, 64) <= 65535) {

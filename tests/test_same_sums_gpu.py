@@ -121,3 +121,23 @@ def test_lists_of_few_pairs_have_the_bits_of_the_kernel_of_few(n, top, n_experts
         assert fast.experts_few_bf16(h, first, down, chosen, torch.empty(n * top, ff, dtype=torch.bfloat16, device=DEV), few, act, clamp=clamp)
         assert fast.experts_feed_forward_bf16(h, first, down, chosen, None, listed, act, Workspace(torch.device(DEV)), clamp=clamp)
         assert torch.equal(few, listed)
+
+
+@pytest.mark.parametrize("n, k", [(64, 32), (130, 96), (2048, 2048), (514, 100)])
+def test_gated_linears_in_32_bits_do_not_depend_on_the_rows_beside(n, k):
+    """One to forty rows: the same bits for a row, K in steps of 32 (matrix pipes) or not (both vector kernels)."""
+    from kestrel_amd.ops import core
+    from kestrel_amd.ops.linear import ACT_GATED, activation_code
+
+    gen = torch.Generator().manual_seed(n + k)
+    a, w, bias = (torch.randn(*shape, generator=gen) for shape in ((40, k), (n, k), (n,)))
+    act = activation_code("silu") | ACT_GATED
+    results = {}
+    for m in (40, 33, 17, 16, 9, 1):
+        out = torch.full((m, n // 2), float("nan"), device=DEV)
+        core.linear_generic(a[:m].to(DEV), w.to(DEV), bias.to(DEV), out, act=act)
+        results[m] = out.cpu()
+    assert all(torch.equal(got, results[40][:m]) for m, got in results.items())
+    z = (a.double() @ w.double().T + bias.double()).view(40, n // 2, 2)
+    want = z[..., 0] * torch.sigmoid(z[..., 0]) * z[..., 1]
+    assert float((results[40].double() - want).norm() / want.norm()) < 2.0 ** -20
