@@ -312,13 +312,14 @@ KA_API int ka_experts_combine(const float* y, const void* h, long h_stride, int 
 // ----------------------------------------------------------------------------
 // The weighted sum of ka_experts_combine as the output of a sublayer whose norm stands behind it: it is normalised and
 // added into the fp32 stream x, and the norm of the new rows is computed, in the same launch (ka_rows.h). A workgroup
-// per token; the sums are those of ka_experts_combine, in its order.
+// per token; the sums are those of ka_experts_combine, in its order. In fp32 h_in may be x itself (a thread reads its channels of a row before it
+// writes them), so neither is __restrict__.
 // ----------------------------------------------------------------------------
 template <typename T, int PIECES, int THREADS>
 __global__ void __launch_bounds__(THREADS)
-experts_combine_normed_kernel(const float* __restrict__ y, const T* __restrict__ h_in, long h_stride, const int* __restrict__ chosen,
+experts_combine_normed_kernel(const float* __restrict__ y, const T* h_in, long h_stride, const int* __restrict__ chosen,
                               const float* __restrict__ weights, int top, int E, const float* __restrict__ shared,
-                              const float* __restrict__ shared_gate, long gate_stride, float* __restrict__ x, int dim, KaRowNorms a) {
+                              const float* __restrict__ shared_gate, long gate_stride, float* x, int dim, KaRowNorms a) {
     __shared__ float smem[THREADS / KA_WAVE];
     const int t = blockIdx.x;
     const float sg = shared ? (shared_gate ? 1.0f / (1.0f + expf(-shared_gate[(size_t)t * gate_stride])) : 1.f) : 0.f;

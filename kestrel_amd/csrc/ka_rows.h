@@ -92,8 +92,9 @@ __device__ __forceinline__ void ka_row_store_h(const KaRowNorms& a, size_t at, f
 
 // PIECES > 0: dim is a multiple of 4 and at most 4 PIECES THREADS, rows are 16-byte aligned; `piece(c)` gives d of the
 // channels c .. c + 3. PIECES = 0: any dim; `one(c)` gives d of channel c (asked for twice).
+// Either may read the row of x that is finished: of the thread's own channels, before these are written.
 template <int PIECES, int THREADS, typename Piece, typename One>
-__device__ __forceinline__ void ka_finish_row(float* __restrict__ x, int row, int dim, const KaRowNorms& a, Piece piece, One one,
+__device__ __forceinline__ void ka_finish_row(float* x, int row, int dim, const KaRowNorms& a, Piece piece, One one,
                                               float* smem) {
     const int tid = threadIdx.x;
     const size_t at = (size_t)row * dim;

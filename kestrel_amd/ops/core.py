@@ -1069,7 +1069,7 @@ def experts_combine_normed(y: torch.Tensor, h: torch.Tensor, chosen: torch.Tenso
                            shared: Optional[torch.Tensor], shared_gate: Optional[torch.Tensor], x: torch.Tensor, norm, then=None,
                            rows: Optional[torch.Tensor] = None) -> None:
     """The weighted sum of ``experts_combine`` as a ``delta`` of ``add_normed``: normalised and added into the fp32 stream ``x``, with
-    the norm ``then`` of the new rows (without it: the rows themselves) into ``rows`` (of ``h``'s type), in one launch."""
+    the norm ``then`` of the new rows (without it: the rows themselves) into ``rows`` (of ``h``'s type), in one launch. ``h`` may be ``x``."""
     _dev(y, h, chosen, weights, shared, shared_gate, x, rows)
     n, dim = x.shape
     top = chosen.shape[1]
