@@ -10,6 +10,8 @@
 //
 // The weights are the row operand: a lane ends with outputs of ONE list row, four neighbours at a time, so the pair of a
 // gated output meets in a lane's registers.
+//
+// First the kernel for a K in no steps of 64, tiles of KL_ROWS staged through registers (ka_listed_tiles.h).
 #include "ka_common.h"
 #include "ka_dma_tiles.h"
 #include "ka_listed_tiles.h"
@@ -22,7 +24,6 @@ typedef __attribute__((ext_vector_type(2))) __bf16 eb_bf16x2;
 
 constexpr int EF_MAX_PAIRS = 512;          // most pairs of a step of few
 
-template <bool TAIL>
 __global__ void __launch_bounds__(256)
 experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, const bf16_t* __restrict__ W, const int* __restrict__ sorted,
                     const int* __restrict__ tile_expert, int N, int K, int act, KaGateClamp clamp, void* __restrict__ out, long ldo,
@@ -43,7 +44,7 @@ experts_gemm_kernel(const bf16_t* __restrict__ a, long lda, int gather_div, cons
     auto weight_row = [&](int r) { return W + ((size_t)e * N + min((int)blockIdx.x * KL_COLS + r, N - 1)) * K; };
     kl_floatx16 acc[2][4];
     const bool swap[2] = {false, false};
-    kl_tile_product<TAIL, false>(eb_lds, K, o0 < N, swap, list_row, weight_row, acc);
+    kl_tile_product<true, false>(eb_lds, K, o0 < N, swap, list_row, weight_row, acc);
     if (o0 >= N) return;
     const bool gated = ka_act_gated(act);
 #pragma unroll
@@ -401,16 +402,11 @@ KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const v
     const dim3 grid((N + KL_COLS - 1) / KL_COLS, n_tiles);
     static bool sized = false;
     if (!sized) {
-        (void)hipFuncSetAttribute((const void*)experts_gemm_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)experts_gemm_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)experts_gemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         sized = true;
     }
-    if (K % KL_SLAB == 0)
-        hipLaunchKernelGGL(experts_gemm_kernel<false>, grid, dim3(256), KL_LDS_BYTES, stream, (const bf16_t*)a, lda, gather_div, (const bf16_t*)W,
-                           sorted, tile_expert, N, K, act, clamp, out, ldo, scatter, out_f32);
-    else
-        hipLaunchKernelGGL(experts_gemm_kernel<true>, grid, dim3(256), KL_LDS_BYTES, stream, (const bf16_t*)a, lda, gather_div, (const bf16_t*)W,
-                           sorted, tile_expert, N, K, act, clamp, out, ldo, scatter, out_f32);
+    hipLaunchKernelGGL(experts_gemm_kernel, grid, dim3(256), KL_LDS_BYTES, stream, (const bf16_t*)a, lda, gather_div, (const bf16_t*)W, sorted,
+                       tile_expert, N, K, act, clamp, out, ldo, scatter, out_f32);
     KA_LAUNCH_CHECK();
     return 0;
 }
