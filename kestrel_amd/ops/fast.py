@@ -126,7 +126,7 @@ TILED_CONFIG = 0
 # a kernel for the case, bias, activation and the sum into the residual being its epilogues; the
 # tiled kernels of this package then take what it declines. Measured on MI355X at Moondream 2's
 # four linears: 201 against 242 us a layer at 2,048 rows, 112 against 151 at 730, 64 against 72 at 96.
-# (The two last linears of a parallel block of up to 160 tiles go by tiles all the same: PAIR_TILES_MAX.)
+# (The two last linears of a block go by tiles of their own where ``pair_tiles_pay`` says so.)
 LIBRARY_LINEAR = True
 LIBRARY_WORKSPACE_BYTES = 128 << 20
 # Activations that the library has no epilogue for (relu squared: ops.linear.ACT_RELU_SQUARED), and the size of an output from
@@ -135,11 +135,20 @@ LIBRARY_WORKSPACE_BYTES = 128 << 20
 _ACTIVATIONS_APART = (4,)
 ACTIVATION_APART_FROM_ROWS = 256
 ACTIVATION_APART_FROM_COLUMNS = 1024
-# Tiles of 128 x 128 of the output up to which a block's two last linears go by tiles with K in parts rather than one after
-# the other to the vendor library, with the norm that follows (us, K = 2,048 + 8,192 at N = 2,048 and 2,560 + 10,240 at 2,560):
-# 65 rows 19 against 29 and 27 against 71, 256 rows 28 against 40 and 38 against 70, 512 rows 40 against 56 and 57 against 83,
-# 160 tiles (1,280 and 1,024 rows) 83 against 93 and 106 against 117; beyond, 192 tiles 99 against 94 and 200 tiles 133 both.
+# Tiles of 128 x 128 of the output up to which a block's two last linears can go by tiles with K in parts, and up to which they do rather than
+# one after the other to the vendor library (``pair_tiles_pay``). Both sides measured over widths of 512 to 8,192, K of 1,024 to
+# 20,480 in all and 65 to 1,536 rows, weights from HBM:
+#  * with the norm that follows, which the library has as a launch of its own, up to 128 tiles at every K (us: 1,024 in all at 2,048, 512 rows
+#    16.5 against 20.2; 4,096 at 2,048, 1,024 rows 32.9 and 36.8; 12,800 at 2,560, 512 rows 56.7 and 79.5), and to 160 where K is in
+#    parts (10,240 at 2,048 84.8 and 86.6, 12,800 at 2,560 104 and 115; in one part 5,120 at 2,560 63.1 and 59.2); beyond, 192 tiles 84 to
+#    187 against 78 to 166;
+#  * without a norm the library's two launches are only one more: up to 32 tiles at every K (1,024 at 2,048, 256 rows 14.0 and 14.3; 48 tiles
+#    15.2 and 15.0; 2,048 at 4,096, 256 rows, 64 tiles 20.0 and 18.3), to 80 where K is 6,144 or more in all (7,680 at 2,048 37.8 and
+#    48.0, 12,800 at 2,560 55.4 and 75.4; 96 tiles 55.6 and 55.1 at 10,240).
 PAIR_TILES_MAX = 160
+PAIR_TILES_NORMED = 128
+PAIR_TILES_ALONE = (32, 80)
+PAIR_TILES_LONG = 6144
 _library_space = {}
 SCRATCH_FLOATS = 8 << 20
 WIDE_FLOATS = 8 << 20              # 32 MB of partial sums for the wide skinny kernel
@@ -417,12 +426,27 @@ def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumula
     return True
 
 
+def _pair_tiles(m: int, n: int) -> int:
+    return -(-m // 128) * -(-n // 128)
+
+
 def pair_tile_parts(m: int, n: int, k1: int, k2: int) -> int:
     """Parts that ``linear_pair_accumulate`` cuts K of both linears into, one behind the other, where it takes them by
     tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles)."""
-    if m <= SKINNY_MAX_ROWS or -(-m // 128) * -(-n // 128) > PAIR_TILES_MAX:
+    if m <= SKINNY_MAX_ROWS or _pair_tiles(m, n) > PAIR_TILES_MAX:
         return 0
     return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, WIDE_FLOATS)
+
+
+def pair_tiles_pay(m: int, n: int, k1: int, k2: int, normed: bool) -> bool:
+    """Whether two last linears of more rows than the weight-streaming kernels take are faster by tiles than one after the other; ``normed``:
+    with the norm of the new rows behind them."""
+    parts, tiles = pair_tile_parts(m, n, k1, k2), _pair_tiles(m, n)
+    if not parts:
+        return False
+    if normed:
+        return tiles <= PAIR_TILES_NORMED or parts > 1
+    return tiles <= PAIR_TILES_ALONE[k1 + k2 >= PAIR_TILES_LONG]
 
 
 def pair_finishes_rows(m: int, n: int) -> bool:

@@ -15,7 +15,7 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     """The parallel block for a few bf16 rows in three launches: norm + both first linears, the
     mixer's core, both last linears + residual. Needs a mixer and a feed-forward that offer their
     stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise. More rows, as long as the two last
-    linears are one product of tiles (``fast.pair_tile_parts``): the first linears are launches of their own then, and
+    linears and the norm behind them are faster as one product of tiles (``fast.pair_tiles_pay``): the first linears are launches of their own then, and
     a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
     ``normed``: the block's norm of ``x``, where the block before has computed it; ``then``: the norm
     the next block starts with, which the last launch computes as well where it pays (``handed``, a
@@ -30,7 +30,9 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     m_out, f_out = block.mixer.output_projection(), block.feed_forward.output_projection()
     if m_in is None or f_in is None or m_out is None or f_out is None:
         return False
-    if n > fast.SKINNY_MAX_ROWS and (f_in[3] & ACT_GATED or not fast.pair_tile_parts(n, x.shape[1], m_out[0].shape[1], f_out[0].shape[1])):
+    sizes = (n, x.shape[1], m_out[0].shape[1], f_out[0].shape[1])
+    many = n > fast.SKINNY_MAX_ROWS
+    if many and (f_in[3] & ACT_GATED or not fast.pair_tiles_pay(*sizes, True)):
         return False
     ws = batch.workspace
     projected = ws.get("block.mixer_in", (n, m_in[2]), block.dtype)
@@ -80,7 +82,8 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
                                        then_norm=(*then_ln, rows)):
             handed.append(rows)
             return True
-    if not fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], x):
+    pays = not many or fast.pair_tiles_pay(*sizes, False)
+    if not (pays and fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], x)):
         linear(mixed, m_out[0], m_out[1], x, accumulate=True)
         linear(hidden, f_out[0], f_out[1], x, accumulate=True)
     return True
@@ -168,7 +171,8 @@ def settle(x, batch) -> None:
 
 def _two_branches_by_stages(block: "Block", h1, h2, batch, cache, delta) -> bool:
     """Both branches through the stages that mixer and feed-forward offer, so that the first of the last linears
-    writes ``delta`` and nobody has to clear it: for a few bf16 rows the two last linears are one launch.
+    writes ``delta`` and nobody has to clear it: for a few bf16 rows, and where it pays for more (``fast.pair_tiles_pay``), the
+    two last linears are one product.
     ``False``: a part offers no stages (its ``forward`` then adds into a cleared ``delta``)."""
     from ..ops import fast
     from ..ops.linear import linear
@@ -188,6 +192,7 @@ def _two_branches_by_stages(block: "Block", h1, h2, batch, cache, delta) -> bool
         linear(h2, f_in[0], f_in[1], hidden, act=f_in[3])
     mixed = block.mixer.attend(projected, batch, cache)
     if ff is not None and block.dtype == torch.bfloat16 and \
+            (n <= fast.SKINNY_MAX_ROWS or fast.pair_tiles_pay(n, delta.shape[1], m_out[0].shape[1], f_out[0].shape[1], False)) and \
             fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], delta, accumulate=False):
         return True
     linear(mixed, m_out[0], m_out[1], delta)
