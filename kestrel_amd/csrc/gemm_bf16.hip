@@ -445,17 +445,21 @@ static int launch_pair_tiles(PairTilesArgs& p, int parts, hipStream_t stream) {
 // that of the first halves of its K-steps plus that of the second.
 //
 // Bound by the weights' way from HBM: what counts is that every CU has 64 KB of loads in flight, which the stages in LDS hold without
-// registers. Tiles of 64 weight rows by all rows, five stages in half of a CU's LDS, four waves. At 40
-// rows, us, weights from HBM, the launch that adds up included, against that kernel: N = 2,048, K = 2,048 + 8,192: 15.3 and 18.6; 2,560, 2,560 +
-// 10,240: 20.1 and 24.8; N = K = 4,096: 12.8 and 16.3; 12,288 by 4,096: 30.9 and 34.2; 4,096 by 12,288: 26.4 and 31.0; at 17 and 64 rows
-// likewise.
+// registers. Tiles of 64 weight rows by all rows, five stages in half of a CU's LDS, four waves; an XCD's tiles are neighbours. At 40
+// rows, us, weights from HBM, the launch that adds up included, against that kernel: N = 2,048, K = 2,048 + 8,192: 15.2 and 18.6; 2,560, 2,560 +
+// 10,240: 20.1 and 24.8; N = K = 4,096: 13.0 and 16.3; 12,288 by 4,096: 31.3 and 34.2; 4,096 by 12,288: 26.4 and 31.0; at 17 and 64 rows
+// likewise. Tiles of 128 rows read LDS three times for four reads of the others and are ahead where tiles of 64 are more than three a CU, which is
+// two rounds (51,200 by 4,096 99 against 104, by 5,120 124 against 133; 40,960 by 3,072 69 against 63).
 template <int WN, int WM, int GN, int GM, int NS>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(2, 2)))
 few_rows_kernel(KaFewRows p) {
     using T = KdTile<WN, WM, GN, GM, 64, NS, 16>;
     constexpr int CPR = T::CPR;
     extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
-    const int n0 = blockIdx.x * T::BN, part = blockIdx.y;
+    const int tiles = (p.N + T::BN - 1) / T::BN, per_xcd = (tiles + 7) / 8;
+    const int tile = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;        // an XCD's tiles: neighbours
+    if (tile >= tiles) return;
+    const int n0 = tile * T::BN, part = blockIdx.y;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
     int first[2], count[2];                              // this part's K-steps of either linear
 #pragma unroll
@@ -520,7 +524,7 @@ static int launch_few_rows(const KaFewRows& f, hipStream_t stream) {
         KA_CHECK(e == hipSuccess, "linear of few rows: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
         configured = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(ka_cdiv(f.N, T::BN), f.parts), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, f);
+    hipLaunchKernelGGL(kernel, dim3(ka_cdiv(ka_cdiv(f.N, T::BN), 8) * 8, f.parts), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, f);
     KA_LAUNCH_CHECK();
     return 0;
 }
@@ -528,7 +532,8 @@ static int launch_few_rows(const KaFewRows& f, hipStream_t stream) {
 // 1: done; 0: the operands are not covered (K in steps of 64); -1: an error.
 int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
     if (f.M < 1 || f.M > 64 || f.K[0] % 64 || f.K[1] % 64 || f.K[0] < 64 || f.parts < 1 || !f.partial) return 0;
-    return launch_few_rows<2, 2, 2, 2, 5>(f, stream) ? -1 : 1;
+    const bool large = ka_cdiv(f.N, 64) > 3 * ka_compute_units();
+    return (large ? launch_few_rows<4, 2, 2, 2, 3>(f, stream) : launch_few_rows<2, 2, 2, 2, 5>(f, stream)) ? -1 : 1;
 }
 
 // Parts of K for `ka_linear_pair_tiles_bf16`: as many as leave the fewest K-steps to a CU, a part more than another costing

@@ -71,7 +71,7 @@ def test_rows_of_the_stream_do_not_depend_on_their_number(dim):
 
 
 @pytest.mark.parametrize("m", [9, 16, 17, 33, 48, 64])
-@pytest.mark.parametrize("n, ks", [(64, (2624,)), (1000, (4096,)), (77, (8192,)), (12288, (2688,)), (640, (64, 320)), (2056, (2048, 8192)), (4096, (192, 64))])
+@pytest.mark.parametrize("n, ks", [(64, (2624,)), (1000, (4096,)), (77, (8192,)), (12288, (2688,)), (640, (64, 320)), (2056, (2048, 8192)), (4096, (192, 64)), (51300, (192,)), (51300, (64, 128))])
 def test_few_rows_have_the_bits_of_the_kernel_that_streams_weights(m, n, ks):
     """Tiles for K in steps of 64, and the kernel with activations in LDS: the same parts of K, the same order within."""
     from kestrel_amd.ops import fast
