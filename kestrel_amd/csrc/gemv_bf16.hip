@@ -183,7 +183,8 @@ skinny_split_kernel(SkinnyArgs p) {
 
 // ----------------------------------------------------------------------------
 // The wide kernel, for 17 to 64 rows of a K in no steps of 64 (else ka_few_rows_by_tiles, gemm_bf16.hip, which has the same
-// parts of K and the same order within one). With that many rows the activations are what the kernels above read most of: every strip of 8 weight rows meets all of them, from L2. Here a workgroup
+// parts of K and the same order within one). With that many rows the activations are what the kernels above read most of: every
+// strip of 8 weight rows meets all of them, from L2. Here a workgroup
 // of eight waves takes eight neighbouring strips and a part of K, brings the activations of that
 // part into LDS once (in chunks of 256 k, two buffers in turn) and every
 // wave multiplies its own strip with them; the parts of K meet in fp32 partial sums that a
@@ -370,7 +371,8 @@ KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enab
 // The wide kernel (17 to 64 rows, activations through LDS, parts of K in scratch memory): 1 where
 // it was measured faster, which is with two K-segments (a K too long for the persistent kernel's
 // registers: 30 against 48 us for Moondream 2's output projection + fc2 at 64 rows; one segment
-// of 2048: 21 against 15 us) and K comes in no steps of 64 (those go by tiles), 2 itself wherever it can run (for tests), 0 nowhere.
+// of 2048: 21 against 15 us) and K comes in no steps of 64 (those go by tiles), 2 itself wherever it can run (for tests), 0
+// nowhere.
 static int sk_wide_enabled = 1;
 KA_API int ka_linear_skinny_pair_in_parts(int M, int N);
 KA_API void ka_skinny_set_wide(int enabled) { sk_wide_enabled = enabled; }
