@@ -341,31 +341,23 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
 
 // The two last linears of a block whose branches run side by side, out += A1 W1^T + A2 W2^T, for more rows than the
 // weight-streaming kernels take and fewer than fill the chip with tiles of the output: K of both, one behind the other, is cut
-// into `parts` parts of `per` K-steps (grid y), and a part's sums go out as fp32 [M, N] of its own, which the kernel that
+// into `parts` parts of `per` K-steps, and a part's sums go out as fp32 [M, N] of its own, which the kernel that
 // finishes the rows adds up (with both biases, the residual and the next block's norm).
-struct PairTilesArgs {
-    const bf16_t* A[2];     // [M, K[s]]
-    const bf16_t* W[2];     // [N, K[s]]
-    long lda[2], ldw[2];
-    int steps[2];           // K[s] / BK
-    int M, N, tiles_n, tiles_m, per;
-    float* partial;         // [parts, M, N]
-};
-
+// (KaPairTiles in ka_partials.h.)
+//
 // The rows of A are the product's first operand here: a lane then holds one column of 16 rows, and a store of the wave covers
 // two rows of 128 bytes, whole lines of the memory, without a pass through LDS.
 template <int WN, int WM, int GN, int GM, int BK, int NS, int SL>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(GN * GM / 4, GN * GM / 4)))
-pair_tiles_kernel(PairTilesArgs p) {
+pair_tiles_kernel(KaPairTiles p) {
     using T = KdTile<WN, WM, GN, GM, BK, NS>;
     constexpr int CPR = T::CPR;
     extern __shared__ __attribute__((aligned(16))) unsigned char gb_lds[];
-    const int total = p.tiles_n * p.tiles_m, per_xcd = (total + 7) / 8;
-    const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;        // an XCD's tiles: neighbours in N, whose rows of W they share
-    if (logical >= total) return;
-    const int m0 = (logical % p.tiles_m) * T::BN, n0 = (logical / p.tiles_m) * T::BM;
+    const KaPairPlace at = ka_pair_place(p, blockIdx.x);
+    if (at.part < 0) return;
+    const int m0 = at.tile_m * T::BN, n0 = at.tile_n * T::BM;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / KA_WAVE), lane = tid % KA_WAVE;
-    const int lo = blockIdx.y * p.per, hi = min(lo + p.per, p.steps[0] + p.steps[1]);
+    const int lo = at.part * p.per, hi = min(lo + p.per, p.steps[0] + p.steps[1]);
 
     floatx16 acc[WN][WM];
 #pragma unroll
@@ -399,7 +391,7 @@ pair_tiles_kernel(PairTilesArgs p) {
         kd_product<WN, WM, GN, GM, BK, NS, SL>(gb_lds, wave, lane, (last - first) * BK, asrc, wsrc, acc);
     }
 
-    float* const mine = p.partial + (size_t)blockIdx.y * p.M * p.N;
+    float* const mine = p.partial + (size_t)at.part * p.M * p.N;
     const int wn = wave / GM, wm = wave % GM, li = lane % 32, lg = lane / 32;
 #pragma unroll
     for (int b = 0; b < WM; ++b) {
@@ -419,10 +411,10 @@ pair_tiles_kernel(PairTilesArgs p) {
 // 71 us for K = 8,192 alone on 64 CUs): parts of K spread them over all CUs. Measured with the norm that follows, against the
 // vendor library's two products and the norm's launch (us; K = 2,560 + 10,240, N = 2,560): 128 rows 31 against 78, 512 rows
 // 57 (three parts) against 83, 1,024 rows 106 against 117.
-constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5;
+constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5, PT_TILE_CODE = 100;
 
 template <int WN, int WM, int GN, int GM, int NS, int SL>
-static int launch_pair_tiles(PairTilesArgs& p, int parts, hipStream_t stream) {
+static int launch_pair_tiles(KaPairTiles& p, int parts, hipStream_t stream) {
     using T = KdTile<WN, WM, GN, GM, PT_BK, NS>;
     static bool configured = false;
     auto kernel = pair_tiles_kernel<WN, WM, GN, GM, PT_BK, NS, SL>;
@@ -433,9 +425,10 @@ static int launch_pair_tiles(PairTilesArgs& p, int parts, hipStream_t stream) {
     }
     p.tiles_m = ka_cdiv(p.M, T::BN);
     p.tiles_n = ka_cdiv(p.N, T::BM);
-    const long launched = (((long)p.tiles_n * p.tiles_m + 7) / 8) * 8;
+    p.parts = parts;
+    const long launched = (((long)p.tiles_n * p.tiles_m * parts + 7) / 8) * 8;
     KA_CHECK(launched < (1L << 31), "linear by tiles: too many tiles");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)launched, parts), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)launched), dim3(KA_WAVE * T::WAVES), T::SMEM, stream, p);
     KA_LAUNCH_CHECK();
     return 0;
 }
@@ -536,27 +529,68 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
     return (large ? launch_few_rows<4, 2, 2, 2, 3>(f, stream) : launch_few_rows<2, 2, 2, 2, 5>(f, stream)) ? -1 : 1;
 }
 
-// Parts of K for `ka_linear_pair_tiles_bf16`: as many as leave the fewest K-steps to a CU, a part more than another costing
-// the finishing kernel one more read of the output. (A K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums: measured at K of
-// 10,240 and 12,800. Only their proportion matters, and whether tiles are taken at all was measured over the whole range.)
-static int pair_tiles_parts(int M, int N, int steps, long partial_floats) {
+// The tile and the parts of K for `ka_linear_pair_tiles_bf16`.
+//  * Tiles of 128 x 128: as many parts as leave the fewest K-steps to a CU, a part more than another costing the finishing kernel one more read
+//    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
+//  * The phased tiles of 256 rows where they come out 5 % ahead and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
+//    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
+//    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 %. Not where more
+//    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
+//    and 23.7 us).
+// Measured with the norm behind, the small tiles and the choice (us): N = 2,048, K = 10,240: 512 rows 43 and 38, 768 rows 55.5 and 47.0, 1,280 rows 84
+// and 66; 2,560, 12,800: 512 rows 57.6 and 49.6, 1,000 rows 104 and 76; 4,096, 20,480: 512 rows 121 and 92.
+struct PairChoice {
+    int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
+    double us;
+};
+
+static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats) {
     const int cus = ka_compute_units();
-    const long tiles = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
-    int best = 0;
-    double best_cost = 0;
+    PairChoice best = {0, 0, 0.0};
+    const long small = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
     for (int parts = 1; parts <= 8 && (long)parts * M * N <= partial_floats; ++parts) {
         const int per = ka_cdiv(steps, parts);
         if ((parts > 1 && per < 4) || ka_cdiv(steps, per) != parts) continue;
-        const double rounds = (double)((tiles * parts + cus - 1) / cus);
-        const double cost = rounds * (per + 8) * 0.55 + parts * (double)M * N * 8.0 / 4.0e6;     // us
-        if (best == 0 || cost < best_cost) { best = parts; best_cost = cost; }
+        const double rounds = (double)((small * parts + cus - 1) / cus);
+        const double us = 1.08 * (rounds * (per + 8) * 0.55 + parts * (double)M * N * 8.0 / 4.0e6);
+        if (best.parts == 0 || us < best.us) best = {0, parts, us};
+    }
+    static const struct { int tile, rows_w, rows_x; double step, full, edge, edge_full, sums; } tiles[] = {
+        {3, 128, 256, 0.83, 0.19, 8.4, -7.2, 1.93}, {1, 256, 256, 1.05, 0.51, 11.9, -8.6, 1.43}};
+    for (const auto& t : tiles) {
+        if (M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L) continue;
+        const long each = (long)ka_cdiv(N, t.rows_w) * ka_cdiv(M, t.rows_x);
+        for (int parts = 1; parts <= 8 && each * parts <= cus && (long)parts * M * N <= partial_floats; ++parts) {
+            const int per = ka_cdiv(steps, parts), last = steps - (parts - 1) * per;
+            if (per < 4 || ka_cdiv(steps, per) != parts || last < 2) continue;
+            const double load = (double)(each * parts) / cus * (each * parts) / cus;
+            const double us = 1.05 * (per * (t.step + t.full * load) + t.edge + t.edge_full * load + parts * (double)M * N * t.sums * 1e-6);
+            if (best.parts == 0 || us < best.us) best = {t.tile, parts, us};
+        }
     }
     return best;
 }
 
+static bool pair_tiles_fit(int M, int N, int K1, int K2) {
+    return M >= 1 && N >= 1 && N % 4 == 0 && K1 % PT_BK == 0 && K2 % PT_BK == 0 && K1 >= PT_BK && K2 >= PT_BK;
+}
+
+// Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered.
 KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats) {
-    if (M < 1 || N < 1 || N % 4 || K1 % PT_BK || K2 % PT_BK || K1 < PT_BK || K2 < PT_BK) return 0;
-    return pair_tiles_parts(M, N, (K1 + K2) / PT_BK, partial_floats);
+    if (!pair_tiles_fit(M, N, K1, K2)) return 0;
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats);
+    return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
+}
+
+// The same for outputs of more small tiles than a CU's worth: tiles of 256 x 256 with K in parts where they are faster than two products of the vendor
+// library and the norm behind them (its operations at 0.85 PFLOP/s, 8 us for two launches' starts and ends, 10 bytes an output at 4 TB/s). Measured,
+// us, library and tiles: N = 2,048, K = 10,240: 1,536 rows 91.5 and 74, 2,048 rows 105.5 and 88.5; 2,560, 12,800: 1,280 rows 131 and 89.5, 2,048 rows
+// 158 and 131; 2,560, 5,120: 2,048 rows 83 and 72; 4,096, 8,192: 2,048 rows 140 and 133; in one part 4,096 rows of the last 249 against 243.
+KA_API int ka_linear_pair_large_parts(int M, int N, int K1, int K2, long partial_floats) {
+    if (!pair_tiles_fit(M, N, K1, K2)) return 0;
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats);
+    const double library = 2.0 * M * N * (double)(K1 + K2) / 0.85e9 + 8.0 + (double)M * N * 10.0 / 4.0e6;
+    return c.tile == 1 && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
 KA_API int ka_linear_pair_tiles_bf16(const void* A1, long lda1, int K1, const void* A2, long lda2, int K2, const void* W1, long ldw1,
@@ -572,17 +606,18 @@ KA_API int ka_linear_pair_tiles_bf16(const void* A1, long lda1, int K1, const vo
              "%s: operands must be 16-byte aligned", who);
     KA_CHECK(((uintptr_t)bias1 | (uintptr_t)bias2) % 16 == 0 || !gamma, "%s: biases must be 16-byte aligned beside a norm", who);
     KA_CHECK(ldo >= N && ldo % 4 == 0, "%s: output stride %ld for N=%d", who, ldo, N);
-    const int steps = (K1 + K2) / PT_BK;
+    const int steps = (K1 + K2) / PT_BK, tile = parts / PT_TILE_CODE;
+    parts %= PT_TILE_CODE;
     KA_CHECK(parts >= 1 && parts <= steps && partials && (long)parts * M * N <= partial_floats, "%s: %d parts of %d steps, %ld floats", who, parts, steps,
              partial_floats);
-    PairTilesArgs p;
+    KaPairTiles p;
     p.A[0] = (const bf16_t*)A1; p.lda[0] = lda1; p.W[0] = (const bf16_t*)W1; p.ldw[0] = ldw1; p.steps[0] = K1 / PT_BK;
     p.A[1] = (const bf16_t*)A2; p.lda[1] = lda2; p.W[1] = (const bf16_t*)W2; p.ldw[1] = ldw2; p.steps[1] = K2 / PT_BK;
     p.M = M; p.N = N;
     p.per = ka_cdiv(steps, parts);
     parts = ka_cdiv(steps, p.per);
     p.partial = partials;
-    if (launch_pair_tiles<1, 2, 4, 2, PT_STAGES, 2>(p, parts, stream)) return -1;
+    if (tile ? ka_pair_phased(p, tile, parts, stream) : launch_pair_tiles<1, 2, 4, 2, PT_STAGES, 2>(p, parts, stream)) return -1;
     if (gamma) {
         const KaThenNorm then = {gamma, beta, eps, normed, normed_dtype, ldn};
         KA_CHECK(ka_then_norm_fits(N) && normed && ldn >= N && ldn % 4 == 0, "%s: cannot normalise rows of %d", who, N);

@@ -20,6 +20,30 @@ struct KaFewRows {
 };
 int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream);
 
+// The operands of two linears whose results are added up, in parts of `per` K-steps of 64.
+struct KaPairTiles {
+    const bf16_t* A[2];     // [M, K[s]]
+    const bf16_t* W[2];     // [N, K[s]]
+    long lda[2], ldw[2];
+    int steps[2];           // K[s] / 64
+    int M, N, tiles_n, tiles_m, per, parts;
+    float* partial;         // [parts, M, N]
+};
+
+// The tile and part of a workgroup; part -1: none. An XCD's workgroups are neighbours in one part of K, so that what they read of either operand
+// is the same few rows' same columns. (A part's tiles spread over all XCDs instead, every XCD reads all of K: N = 2,048, K = 10,240, 2,048 rows
+// 96.7 against 88.5 us; and 50 tiles, seven to an XCD, in five parts are a second round on seven of the XCDs: 2,560, 12,800, 1,280 rows 136 against 89.5.)
+struct KaPairPlace {
+    int part, tile_n, tile_m;
+};
+__device__ __forceinline__ KaPairPlace ka_pair_place(const KaPairTiles& p, int block) {
+    const int tiles = p.tiles_n * p.tiles_m, total = tiles * p.parts, per_xcd = (total + 7) / 8;
+    const int logical = block % 8 * per_xcd + block / 8, tile = logical % tiles;
+    if (logical >= total) return {-1, 0, 0};
+    return {logical / tiles, tile / p.tiles_m, tile % p.tiles_m};
+}
+int ka_pair_phased(const KaPairTiles& p, int tile, int parts, hipStream_t stream);
+
 // out = act(sum of the parts + biases) (+ out): one thread per four neighbouring outputs
 static __global__ void __launch_bounds__(256)
 ka_partials_finish_kernel(const float* __restrict__ partial, int splits, const float* __restrict__ bias,

@@ -37,6 +37,7 @@ _SIGNATURES = {
         _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_long, _c_void_p],  # gamma, beta, eps, normed, its type and stride, stream
     "ka_linear_skinny_pair_in_parts": [_c_int, _c_int],
     "ka_linear_pair_tiles_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
+    "ka_linear_pair_large_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
     "ka_linear_pair_tiles_bf16": [
         _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_int,                     # A1, lda1, K1, A2, lda2, K2
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_void_p,               # W1, ldw1, bias1, W2, ldw2, bias2
@@ -149,6 +150,7 @@ PAIR_TILES_MAX = 160
 PAIR_TILES_NORMED = 128
 PAIR_TILES_ALONE = (32, 80)
 PAIR_TILES_LONG = 6144
+PAIR_TILE_CODE = 100
 _library_space = {}
 SCRATCH_FLOATS = 8 << 20
 WIDE_FLOATS = 8 << 20              # 32 MB of partial sums for the wide skinny kernel
@@ -376,16 +378,16 @@ def linear_bf16(a, weight, bias, out, act, accumulate) -> bool:
     return True
 
 
-def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumulate: bool = True) -> bool:
+def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumulate: bool = True, large: bool = False) -> bool:
     """``out += a1 @ w1.T + b1 + a2 @ w2.T + b2`` in one launch (few rows, fp32 ``out``), or in two by tiles with K of both
     in parts (``pair_tile_parts``); with ``accumulate`` off the sum replaces ``out``.
     ``then_norm = (gamma, beta or None, eps, normed)``: also ``normed = LayerNorm(out)``, in the kernel
-    that finishes the rows where there is one (more than 8 rows), else in a launch behind it. False:
-    not covered, nothing was run (with ``then_norm``: try without)."""
+    that finishes the rows where there is one (more than 8 rows), else in a launch behind it. ``large``: also outputs of more
+    tiles, where ``pair_large_parts`` says so. False: not covered, nothing was run (with ``then_norm``: try without)."""
     m, k1 = a1.shape
     k2 = a2.shape[1]
     n = w1.shape[0]
-    parts = pair_tile_parts(m, n, k1, k2)
+    parts = pair_tile_parts(m, n, k1, k2) or (pair_large_parts(m, n, k1, k2) if large else 0)
     if not (0 < m <= SKINNY_MAX_ROWS or parts) or k1 % 8 or k2 % 8 or a2.shape[0] != m or w2.shape[0] != n:
         return False
     if not (_operand_ok(a1, k1) and _operand_ok(w1, k1) and _operand_ok(a2, k2) and _operand_ok(w2, k2)):
@@ -405,10 +407,11 @@ def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumula
         if any(b is not None and b.data_ptr() % 16 for b in (b1, b2)):
             return False
     if parts:
+        space = _library_workspace(a1.device)
         _check(lib().ka_linear_pair_tiles_bf16(
             a1.data_ptr(), a1.stride(0), k1, a2.data_ptr(), a2.stride(0), k2, w1.data_ptr(), w1.stride(0), _ptr(b1),
             w2.data_ptr(), w2.stride(0), _ptr(b2), out.data_ptr(), out.stride(0), n, int(bool(accumulate)), m, parts,
-            *_wide_args(a1.device, m), _ptr(gamma), _ptr(beta), float(eps) if then_norm is not None else 0.0, _ptr(normed),
+            space.data_ptr(), space.numel() // 4, _ptr(gamma), _ptr(beta), float(eps) if then_norm is not None else 0.0, _ptr(normed),
             _OUT_CODE[normed.dtype] if then_norm is not None else 0, normed.stride(0) if then_norm is not None else 0, stream_ptr()))
         return True
     if then_norm is not None:
@@ -431,11 +434,18 @@ def _pair_tiles(m: int, n: int) -> int:
 
 
 def pair_tile_parts(m: int, n: int, k1: int, k2: int) -> int:
-    """Parts that ``linear_pair_accumulate`` cuts K of both linears into, one behind the other, where it takes them by
-    tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles)."""
+    """Parts that ``linear_pair_accumulate`` cuts K of both linears into, one behind the other (and a tile's code times ``PAIR_TILE_CODE``), where
+    it takes them by tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles)."""
     if m <= SKINNY_MAX_ROWS or _pair_tiles(m, n) > PAIR_TILES_MAX:
         return 0
-    return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, WIDE_FLOATS)
+    return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4)
+
+
+def pair_large_parts(m: int, n: int, k1: int, k2: int) -> int:
+    """The same for an output of more tiles than that, in front of a norm, where large tiles in parts are faster than the vendor library; 0: they are not."""
+    if m <= SKINNY_MAX_ROWS or _pair_tiles(m, n) <= PAIR_TILES_MAX:
+        return 0
+    return lib().ka_linear_pair_large_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4)
 
 
 def pair_tiles_pay(m: int, n: int, k1: int, k2: int, normed: bool) -> bool:
@@ -445,7 +455,9 @@ def pair_tiles_pay(m: int, n: int, k1: int, k2: int, normed: bool) -> bool:
     if not parts:
         return False
     if normed:
-        return tiles <= PAIR_TILES_NORMED or parts > 1
+        # (beyond the tiles that always pay, small ones do in parts, large ones where the rule for large outputs says so)
+        return tiles <= PAIR_TILES_NORMED or 1 < parts < PAIR_TILE_CODE or \
+            lib().ka_linear_pair_large_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4) > 0
     return tiles <= PAIR_TILES_ALONE[k1 + k2 >= PAIR_TILES_LONG]
 
 

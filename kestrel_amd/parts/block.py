@@ -15,8 +15,8 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     """The parallel block for a few bf16 rows in three launches: norm + both first linears, the
     mixer's core, both last linears + residual. Needs a mixer and a feed-forward that offer their
     stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise. More rows, as long as the two last
-    linears and the norm behind them are faster as one product of tiles (``fast.pair_tiles_pay``): the first linears are launches of their own then, and
-    a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
+    linears and the norm behind them are faster as one product of tiles (``fast.pair_tiles_pay``, ``fast.pair_large_parts``): the first linears are launches
+    of their own then, and a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
     ``normed``: the block's norm of ``x``, where the block before has computed it; ``then``: the norm
     the next block starts with, which the last launch computes as well where it pays (``handed``, a
     list, then gets the normalised rows)."""
@@ -32,7 +32,9 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
         return False
     sizes = (n, x.shape[1], m_out[0].shape[1], f_out[0].shape[1])
     many = n > fast.SKINNY_MAX_ROWS
-    if many and (f_in[3] & ACT_GATED or not fast.pair_tiles_pay(*sizes, True)):
+    # (the large tiles only in front of a norm that their finishing launch takes along)
+    large = many and then is not None and then.layernorm_operands() is not None and fast.pair_large_parts(*sizes) > 0
+    if many and (f_in[3] & ACT_GATED or not (large or fast.pair_tiles_pay(*sizes, True))):
         return False
     ws = batch.workspace
     projected = ws.get("block.mixer_in", (n, m_in[2]), block.dtype)
@@ -79,7 +81,7 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     if then_ln is not None:
         rows = ws.get("block.handed", tuple(x.shape), block.dtype)
         if fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], x,
-                                       then_norm=(*then_ln, rows)):
+                                       then_norm=(*then_ln, rows), large=large):
             handed.append(rows)
             return True
     pays = not many or fast.pair_tiles_pay(*sizes, False)
