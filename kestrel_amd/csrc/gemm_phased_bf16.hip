@@ -1,7 +1,149 @@
-// Linears of prompts on the phased tiles (ka_phased_tiles.h): a block's two last linears with K of both in parts.
+// Linears of prompts on the phased tiles (ka_phased_tiles.h): the first linears of a block whose branches read the same rows, in one
+// launch, and a block's two last linears with K of both in parts.
 #include "ka_common.h"
 #include "ka_partials.h"
 #include "ka_phased_tiles.h"
+
+// out[s] = act[s](A W[s]^T + bias[s]), s = 0, 1, in bf16; the tiles of the second linear follow those of the first.
+struct KpJoint {
+    const bf16_t* A;        // [M, K]
+    long lda;
+    int M, K, tiles_m, tiles_n[2];
+    const bf16_t* W[2];     // [N[s], K]
+    const float* bias[2];   // may be null
+    bf16_t* out[2];         // [M, N[s]]
+    long ldw[2], ldo[2];
+    int N[2], act[2];
+};
+
+template <int QW0, int QW1, int QX0, int QX1, int GW, int GX>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+joint_tiles_kernel(KpJoint p) {
+    using T = KpTile<QW0, QW1, QX0, QX1, GW, GX>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char kp_lds[];
+    const int total = (p.tiles_n[0] + p.tiles_n[1]) * p.tiles_m, per_xcd = (total + 7) / 8;
+    const int logical = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;      // an XCD's tiles: neighbours in N, whose rows of W they share
+    if (logical >= total) return;
+    const int m0 = logical % p.tiles_m * T::BM, tile = logical / p.tiles_m;
+    const bool second = tile >= p.tiles_n[0];
+    const int n0 = (second ? tile - p.tiles_n[0] : tile) * T::BN;
+    const char* const W = (const char*)(second ? p.W[1] : p.W[0]);
+    const long ldw = second ? p.ldw[1] : p.ldw[0], ldo = second ? p.ldo[1] : p.ldo[0];
+    const int N = second ? p.N[1] : p.N[0], act = second ? p.act[1] : p.act[0];
+    const float* const bias = second ? p.bias[1] : p.bias[0];
+    bf16_t* const out = second ? p.out[1] : p.out[0];
+    const char* const A = (const char*)p.A;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    // (bytes from the operand's start, which the host has checked to fit in 32 bits; rows past the end are read from the last row, and never stored)
+    unsigned woff[T::LW0 + T::LW1], xoff[T::LX0 + T::LX1];
+#pragma unroll
+    for (int i = 0; i < T::LW0 + T::LW1; ++i)
+        woff[i] = (unsigned)(min(n0 + T::w_row(i, wave, lane), N - 1) * ldw + T::w_channel(i, wave, lane)) * 2u;
+#pragma unroll
+    for (int i = 0; i < T::LX0 + T::LX1; ++i)
+        xoff[i] = (unsigned)(min(m0 + T::x_row(i, wave, lane), p.M - 1) * p.lda + T::x_channel(i, wave, lane)) * 2u;
+    floatx4 acc[2][2][T::QW][T::QX];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int a = 0; a < T::QW; ++a)
+#pragma unroll
+                for (int b = 0; b < T::QX; ++b) acc[h][g][a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    asm volatile("" ::"s"(bias), "s"(out), "s"(ldo), "s"(act), "s"(p.M), "s"(N));       // (no scalar load later, on the counter of the LDS reads)
+    kp_product<QW0, QW1, QX0, QX1, GW, GX>(kp_lds, wave, lane, p.K / 64, [&](int i, int t) { return W + (size_t)t * 128 + woff[i]; },
+                                           [&](int i, int t) { return A + (size_t)t * 128 + xoff[i]; }, acc);
+    gd_barrier();                                        // the last K-step has been read by everybody
+    const int n_wave = n0 + wave / GX * T::WAVE_N, m_wave = m0 + wave % GX * T::WAVE_M, quarter = lane / 16;
+    // (N is a multiple of 8: four columns of a tile are inside it or past it together, and so are the eight of a store)
+    floatx4 add[2][T::QW];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int a = 0; a < (h ? QW1 : QW0); ++a) {
+            const int n = n_wave + (h * QW0 + a) * 16 + quarter * 4;
+            add[h][a] = bias && n < N ? *reinterpret_cast<const floatx4*>(bias + n) : floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    auto rows_out = [&](auto activate) {
+        kp_rows_out<bf16_t, QW0, QW1, QX0, QX1, GW, GX>(
+            kp_lds, wave, lane,
+            [&](auto h, auto g, auto a, auto b) {
+                floatx4 v = acc[h.value][g.value][a.value][b.value] + add[h.value][a.value];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = activate(v[i]);
+                return v;
+            },
+            [&](int r, int c, const unsigned char* from) {
+                const int m = m_wave + r, n = n_wave + c;
+                if (m < p.M && n < N) *reinterpret_cast<bf16x8*>(out + (size_t)m * ldo + n) = *reinterpret_cast<const bf16x8*>(from);
+            });
+    };
+    // (the two activations that matter have an epilogue of their own: chosen per value, an activation costs a branch a value)
+    if (act == KA_ACT_NONE) rows_out([](float x) { return x; });
+    else if (act == KA_ACT_GELU_TANH) rows_out([](float x) { return ka_gelu_tanh_fast(x); });
+    else rows_out([&](float x) { return ka_activate_fast(act, x); });
+}
+
+template <int QW0, int QW1, int QX0, int QX1, int GW, int GX>
+static int launch_joint(KpJoint p, hipStream_t stream) {
+    using T = KpTile<QW0, QW1, QX0, QX1, GW, GX>;
+    static bool configured = false;
+    auto kernel = joint_tiles_kernel<QW0, QW1, QX0, QX1, GW, GX>;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM);
+        KA_CHECK(e == hipSuccess, "joint linears: cannot reserve %d bytes of LDS: %s", T::SMEM, hipGetErrorString(e));
+        configured = true;
+    }
+    p.tiles_m = ka_cdiv(p.M, T::BM);
+    for (int s = 0; s < 2; ++s) p.tiles_n[s] = ka_cdiv(p.N[s], T::BN);
+    const long total = ((long)(p.tiles_n[0] + p.tiles_n[1]) * p.tiles_m + 7) / 8 * 8;
+    KA_CHECK(total < (1L << 31), "joint linears: too many tiles");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(512), T::SMEM, stream, p);
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// The tiles by area: of those whose workgroups are one round of the chip the smallest wins, since a K-step of it is the shortest.
+static const struct { int code, rows_w, rows_x; } KP_JOINT_TILES[] = {{6, 128, 128}, {3, 128, 256}, {5, 256, 128}, {2, 192, 256}, {4, 256, 192}, {1, 256, 256}};
+
+// The tile for two linears of the same rows in one launch, 0: not covered, or faster one after the other by the vendor library, which is so where
+// they take more than one round (14,336 outputs from 2,048, 1,200 rows: 83 against 75 us) or nearly half of the tiles is no rows (22,528 from 4,096,
+// 257 rows: 85 against 82). Measured over widths of 1,536 to 4,096 and 65 to 1,200 rows, us, library and one launch: 14,336 from 2,048: 128 rows 31.8 and
+// 25.2, 256 rows 50 and 26, 512 rows 51 and 36, 743 rows 59 and 45, 1,024 rows 69 and 54; 17,920 from 2,560, 512 rows: 70 and 55.
+KA_API int ka_linear_joint_tile(int M, int N1, int N2, int K) {
+    if (M < 1 || N1 < 8 || N2 < 8 || N1 % 8 || N2 % 8 || K % 64 || K < 128) return 0;
+    for (const auto& t : KP_JOINT_TILES)
+        if ((long)ka_cdiv(M, t.rows_x) * (ka_cdiv(N1, t.rows_w) + ka_cdiv(N2, t.rows_w)) <= ka_compute_units())
+            return t.rows_w * t.rows_x <= 128 * 256 || M * 20 >= ka_cdiv(M, t.rows_x) * t.rows_x * 11 ? t.code : 0;
+    return 0;
+}
+
+KA_API int ka_linear_joint_bf16(const void* A, long lda, int M, int K, const void* W1, long ldw1, const float* bias1, void* out1, long ldo1, int N1,
+                                int act1, const void* W2, long ldw2, const float* bias2, void* out2, long ldo2, int N2, int act2, int config,
+                                hipStream_t stream) {
+    const char* who = "ka_linear_joint_bf16";
+    KA_CHECK(M > 0 && K >= 128 && K % 64 == 0 && N1 > 0 && N1 % 8 == 0 && N2 >= 0 && N2 % 8 == 0, "%s: M=%d K=%d N=%d and %d", who, M, K, N1, N2);
+    KA_CHECK(lda >= K && ldw1 >= K && lda % 8 == 0 && ldw1 % 8 == 0 && ldo1 >= N1 && ldo1 % 8 == 0, "%s: strides", who);
+    KA_CHECK(N2 == 0 || (ldw2 >= K && ldw2 % 8 == 0 && ldo2 >= N2 && ldo2 % 8 == 0), "%s: strides of the second linear", who);
+    KA_CHECK(((uintptr_t)A | (uintptr_t)W1 | (uintptr_t)W2 | (uintptr_t)bias1 | (uintptr_t)bias2 | (uintptr_t)out1 | (uintptr_t)out2) % 16 == 0,
+             "%s: operands must be 16-byte aligned", who);
+    KA_CHECK((M - 1) * lda + K < (1L << 31) && (N1 - 1) * ldw1 + K < (1L << 31) && (N2 - 1) * ldw2 + K < (1L << 31), "%s: an operand of 4 GB", who);
+    KA_CHECK(ka_act_known(act1) && ka_act_known(act2) && !ka_act_gated(act1) && !ka_act_gated(act2), "%s: activations %d and %d", who, act1, act2);
+    KpJoint p = {};
+    p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.K = K;
+    p.W[0] = (const bf16_t*)W1; p.bias[0] = bias1; p.out[0] = (bf16_t*)out1; p.ldw[0] = ldw1; p.ldo[0] = ldo1; p.N[0] = N1; p.act[0] = act1;
+    p.W[1] = (const bf16_t*)W2; p.bias[1] = bias2; p.out[1] = (bf16_t*)out2; p.ldw[1] = ldw2; p.ldo[1] = ldo2; p.N[1] = N2; p.act[1] = act2;
+    switch (config) {
+        case 1: return launch_joint<4, 4, 2, 2, 2, 4>(p, stream);
+        case 2: return launch_joint<4, 2, 2, 2, 2, 4>(p, stream);
+        case 3: return launch_joint<2, 2, 2, 2, 2, 4>(p, stream);
+        case 4: return launch_joint<4, 4, 2, 1, 2, 4>(p, stream);
+        case 5: return launch_joint<2, 2, 2, 2, 4, 2>(p, stream);
+        case 6: return launch_joint<2, 2, 1, 1, 2, 4>(p, stream);
+    }
+    KA_CHECK(false, "%s: unknown tile %d", who, config);
+}
 
 // A block's two last linears: out += A[0] W[0]^T + A[1] W[1]^T, the K-steps of both one behind the other and cut into parts of `per`,
 // whose fp32 sums go out as [M, N] of their own for the kernel that finishes the rows.

@@ -38,11 +38,16 @@ _SIGNATURES = {
     "ka_linear_skinny_pair_in_parts": [_c_int, _c_int],
     "ka_linear_pair_tiles_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
     "ka_linear_pair_large_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
+    "ka_linear_joint_tile": [_c_int] * 4,
     "ka_linear_pair_tiles_bf16": [
         _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_int,                     # A1, lda1, K1, A2, lda2, K2
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_void_p,               # W1, ldw1, bias1, W2, ldw2, bias2
         _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long,     # out, ldo, N, accumulate, M, parts, partial sums
         _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_long, _c_void_p],     # gamma, beta, eps, normed, its type and stride, stream
+    "ka_linear_joint_bf16": [
+        _c_void_p, _c_long, _c_int, _c_int,                                                # A, lda, M, K
+        _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int,                 # W, ldw, bias, out, ldo, N, act of either linear
+        _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_void_p],   # ..., tile, stream
     "ka_linear_library_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
                                _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long, _c_void_p],
     "ka_linear_tiled_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
@@ -482,6 +487,33 @@ def linear_two_outputs(a, wa, ba, out_a, act_a, wb, bb, out_b, act_b) -> bool:
         wa.data_ptr(), wa.stride(0), _ptr(ba), out_a.data_ptr(), _OUT_CODE[out_a.dtype], out_a.stride(0), na, act_a, 0,
         wb.data_ptr(), wb.stride(0), _ptr(bb), out_b.data_ptr(), _OUT_CODE[out_b.dtype], out_b.stride(0), nb, act_b,
         m, chip_sizes(a.device).skinny_target_waves, *_wide_args(a.device, m), stream_ptr()))
+    return True
+
+
+def joint_tile(m: int, na: int, nb: int, k: int) -> int:
+    """The tile by which ``linear_joint`` runs two linears of the same rows; 0: one after the other is faster, or few rows."""
+    return lib().ka_linear_joint_tile(m, na, nb, k) if m > SKINNY_MAX_ROWS else 0
+
+
+def linear_joint(a, wa, ba, out_a, act_a, wb, bb, out_b, act_b) -> bool:
+    """``linear_two_outputs`` for more rows than the weight-streaming kernels take, into bf16, where ``joint_tile`` names a tile."""
+    m, k = a.shape
+    na, nb = wa.shape[0], wb.shape[0]
+    if (act_a | act_b) & ACT_GATED:
+        return False
+    tile = joint_tile(m, na, nb, k)
+    if not tile or not LIBRARY_LINEAR or TILED_CONFIG:
+        return False
+    if not (_operand_ok(a, k) and _operand_ok(wa, k) and _operand_ok(wb, k) and _out_ok(out_a, m, na) and _out_ok(out_b, m, nb)
+            and _bias_ok(ba, na) and _bias_ok(bb, nb)):
+        return False
+    if any(o.dtype != torch.bfloat16 or o.stride(0) % 8 for o in (out_a, out_b)) or any(b is not None and b.data_ptr() % 16 for b in (ba, bb)):
+        return False
+    if any((t.shape[0] - 1) * t.stride(0) + k >= 1 << 31 for t in (a, wa, wb)):
+        return False
+    _check(lib().ka_linear_joint_bf16(
+        a.data_ptr(), a.stride(0), m, k, wa.data_ptr(), wa.stride(0), _ptr(ba), out_a.data_ptr(), out_a.stride(0), na, act_a,
+        wb.data_ptr(), wb.stride(0), _ptr(bb), out_b.data_ptr(), out_b.stride(0), nb, act_b, tile, stream_ptr()))
     return True
 
 

@@ -14,9 +14,9 @@ from .streams import StreamReading
 def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) -> bool:
     """The parallel block for a few bf16 rows in three launches: norm + both first linears, the
     mixer's core, both last linears + residual. Needs a mixer and a feed-forward that offer their
-    stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise. More rows, as long as the two last
-    linears and the norm behind them are faster as one product of tiles (``fast.pair_tiles_pay``, ``fast.pair_large_parts``): the first linears are launches
-    of their own then, and a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
+    stages (``input_projection`` / ``output_projection``); returns ``False`` otherwise. More rows, as long as either the two first linears are
+    faster in one launch (``fast.joint_tile``) or the two last ones and the norm behind them as one product of tiles (``fast.pair_tiles_pay``,
+    ``fast.pair_large_parts``): what is not is launches of its own then, and a gated feed-forward keeps to its ``forward``, which has a better way for many rows.
     ``normed``: the block's norm of ``x``, where the block before has computed it; ``then``: the norm
     the next block starts with, which the last launch computes as well where it pays (``handed``, a
     list, then gets the normalised rows)."""
@@ -34,7 +34,8 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     many = n > fast.SKINNY_MAX_ROWS
     # (the large tiles only in front of a norm that their finishing launch takes along)
     large = many and then is not None and then.layernorm_operands() is not None and fast.pair_large_parts(*sizes) > 0
-    if many and (f_in[3] & ACT_GATED or not (large or fast.pair_tiles_pay(*sizes, True))):
+    if many and (f_in[3] & ACT_GATED or not (large or fast.pair_tiles_pay(*sizes, True) or
+                                             fast.joint_tile(n, m_in[0].shape[0], f_in[0].shape[0], x.shape[1]))):
         return False
     ws = batch.workspace
     projected = ws.get("block.mixer_in", (n, m_in[2]), block.dtype)
@@ -66,7 +67,8 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
         if h is None:
             h = ws.get("block.h", tuple(x.shape), block.dtype)
             norm.forward(x, h)
-        if not fast.linear_two_outputs(h, m_in[0], m_in[1], projected, 0, f_in[0], f_in[1], hidden, f_in[3]):
+        first = (h, m_in[0], m_in[1], projected, 0, f_in[0], f_in[1], hidden, f_in[3])
+        if not (fast.linear_joint(*first) if many else fast.linear_two_outputs(*first)):
             linear(h, m_in[0], m_in[1], projected)
             linear(h, f_in[0], f_in[1], hidden, act=f_in[3])
     mixed = block.mixer.attend(projected, batch, cache, beside) if beside is not None \
@@ -77,7 +79,7 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     # rows of 2560, which leave the prologue's kernel no registers for a third strip of weights in flight, from
     # 5 rows on: 3 to 4 %).
     handing = n > fast.SKINNY_LN_MAX_ROWS or fast.pair_finishes_rows(n, x.shape[1])
-    then_ln = then.layernorm_operands() if then is not None and handing else None
+    then_ln = then.layernorm_operands() if then is not None and handing and (not many or large or fast.pair_tiles_pay(*sizes, True)) else None
     if then_ln is not None:
         rows = ws.get("block.handed", tuple(x.shape), block.dtype)
         if fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], x,

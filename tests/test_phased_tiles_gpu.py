@@ -1,4 +1,4 @@
-"""Two last linears of prompts on the phased tiles, K of both in parts, against float64."""
+"""Linears of prompts on the phased tiles: two first linears in one launch, two last ones with K of both in parts, against float64."""
 
 from __future__ import annotations
 
@@ -15,10 +15,33 @@ def _rnd(seed):
     return lambda *shape: torch.randn(*shape, generator=gen)
 
 
-def _close(got, want, magnitudes, count):
-    """A sum of ``count`` products that are exact in 32 bits, in any order, is off by at most count 2^-24 of the sum of magnitudes."""
-    bound = count * 2.0 ** -24 * magnitudes
-    assert bool(((got.double().cpu() - want).abs() <= bound).all())
+def _close(got, want, magnitudes, count, rounded):
+    """A sum of ``count`` products that are exact in 32 bits, in any order, is off by at most count 2^-24 of the sum of magnitudes; rounding it to
+    bf16 adds half a step of 8 bits; an activation of slope at most 1.13 passes both on and adds a few steps of 24 bits of its input."""
+    bound = 1.13 * (count + 8) * 2.0 ** -24 * magnitudes + (2.0 ** -8 * want.abs() if rounded else 0.0)
+    assert bool(((got.double().cpu() - want).abs() <= bound + 2.0 ** -60).all())
+
+
+# every tile: two K-steps (none in the loop's middle), odd and even numbers of them, rows and columns at the edges of tiles and of their halves
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("m, n1, n2, k", [(65, 8, 264, 128), (257, 520, 136, 192), (128, 256, 128, 320), (383, 192, 1000, 256)])
+def test_two_first_linears_in_one_launch(tile, m, n1, n2, k):
+    from kestrel_amd.ops import fast
+
+    rnd = _rnd(m + n1 + k)
+    a, w1, w2, b1 = rnd(m, k + 8).bfloat16(), rnd(n1, k).bfloat16(), rnd(n2, k + 16).bfloat16(), rnd(n1)
+    o1, o2 = (torch.full((m, n + 8), 7.0, dtype=torch.bfloat16, device=DEV) for n in (n1, n2))
+    da, dw1, dw2, db1 = (t.to(DEV) for t in (a, w1, w2, b1))
+    for act in (1, 3):
+        fast._check(fast.lib().ka_linear_joint_bf16(
+            da.data_ptr(), k + 8, m, k, dw1.data_ptr(), k, db1.data_ptr(), o1.data_ptr(), n1 + 8, n1, 0,
+            dw2.data_ptr(), k + 16, None, o2.data_ptr(), n2 + 8, n2, act, tile, torch.cuda.current_stream().cuda_stream))
+        x, y = a[:, :k].double(), w2[:, :k].double()
+        _close(o1[:, :n1], x @ w1.double().T + b1.double(), x.abs() @ w1.double().abs().T + b1.double().abs(), k + 1, True)
+        z = x @ y.T
+        want = torch.nn.functional.gelu(z, approximate="tanh") if act == 1 else torch.nn.functional.silu(z)
+        _close(o2[:, :n2], want, x.abs() @ y.abs().T, k, True)
+        assert bool((o1[:, n1:] == 7.0).all()) and bool((o2[:, n2:] == 7.0).all())
 
 
 # every tile of it: one part and several, the border between the linears at a part's start, inside one, behind an odd number of K-steps
@@ -38,7 +61,16 @@ def test_two_last_linears_in_parts(tile, m, n, k1, k2, parts):
         torch.cuda.current_stream().cuda_stream))
     p, q, r, s = a1[:, :k1].double(), w1.double(), a2.double(), w2[:, :k2].double()
     rest = b1.double() + b2.double() + x.double()
-    _close(out, p @ q.T + r @ s.T + rest, p.abs() @ q.abs().T + r.abs() @ s.abs().T + b1.double().abs() + b2.double().abs() + x.double().abs(), k1 + k2 + 3)
+    _close(out, p @ q.T + r @ s.T + rest, p.abs() @ q.abs().T + r.abs() @ s.abs().T + b1.double().abs() + b2.double().abs() + x.double().abs(), k1 + k2 + 3, False)
+
+
+@pytest.mark.parametrize("m, n1, n2, k, tile", [(64, 6144, 8192, 2048, 0), (65, 6144, 8192, 2048, 6), (257, 6144, 8192, 2048, 3), (513, 6144, 8192, 2048, 2),
+                                                (1024, 6144, 8192, 2048, 1), (1025, 6144, 8192, 2048, 0), (257, 6144, 16384, 4096, 0), (300, 6144, 8192, 2056, 0),
+                                                (300, 6148, 8192, 2048, 0), (300, 264, 8192, 64, 0)])
+def test_where_first_linears_are_one_launch(m, n1, n2, k, tile):
+    from kestrel_amd.ops import fast
+
+    assert fast.joint_tile(m, n1, n2, k) == tile
 
 
 @pytest.mark.parametrize("m, n, k1, k2, large", [(1280, 2048, 2048, 8192, False), (1281, 2048, 2048, 8192, True), (2048, 2048, 2048, 8192, True),
@@ -52,3 +84,29 @@ def test_where_last_linears_take_large_tiles(m, n, k1, k2, large):
         bf = dict(dtype=torch.bfloat16, device=DEV)
         args = (torch.zeros(m, k1, **bf), torch.zeros(n, k1, **bf), None, torch.zeros(m, k2, **bf), torch.zeros(n, k2, **bf), None, torch.zeros(m, n, device=DEV))
         assert not fast.linear_pair_accumulate(*args) and fast.linear_pair_accumulate(*args, large=True)
+
+
+def test_a_replayed_graph_repeats_the_eager_bits():
+    from kestrel_amd.ops import fast
+
+    torch.manual_seed(5)
+    bf = dict(dtype=torch.bfloat16, device=DEV)
+    a, w1, w2, v1, v2 = (torch.randn(*s, **bf) for s in ((520, 512), (1024, 512), (2048, 512), (512, 1024), (512, 2048)))
+    fields = [(torch.empty(520, 1024, **bf), torch.empty(520, 2048, **bf), torch.empty(520, 512, device=DEV)) for _ in range(2)]
+
+    def run(o1, o2, x):
+        assert fast.linear_joint(a, w1, None, o1, 0, w2, None, o2, 1)
+        assert fast.linear_pair_accumulate(o1, v1, None, o2, v2, None, x, accumulate=False)
+
+    run(*fields[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(*fields[1])
+    for _ in range(3):
+        for t in fields[1]:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(*fields))
+        run(*fields[0])
