@@ -34,7 +34,7 @@ LIBRARIES: Dict[str, List[str]] = {
     "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_phased_bf16.hip", "gemv_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
              "gemm_library.hip"],
 }
-HEADERS = ["ka_common.h", "ka_partials.h", "ka_no_alloc.h", "ka_attention_decode.h", "ka_skinny.h", "ka_rows.h", "ka_decay.h", "ka_listed_tiles.h", "ka_dma_tiles.h", "ka_phased_tiles.h"]
+HEADERS = ["ka_common.h", "ka_partials.h", "ka_no_alloc.h", "ka_attention_decode.h", "ka_skinny.h", "ka_rows.h", "ka_decay.h", "ka_listed_tiles.h", "ka_dma_tiles.h", "ka_phased_tiles.h", "ka_conv_wide.h", "ka_gated_step.h"]
 
 # Libraries of the ROCm installation that a library of ours is linked against.
 LINK_LIBRARIES: Dict[str, List[str]] = {"fast": ["hipblaslt"]}

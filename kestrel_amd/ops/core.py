@@ -42,7 +42,7 @@ _SIGNATURES = {
                       _c_int, _c_long, _c_long, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "ka_conv_prepare": [_c_void_p, _c_int, _c_long, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                        _c_void_p, _c_int, _c_int, _c_long, _c_int, _c_float, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p],
+                        _c_void_p, _c_int, _c_int, _c_long, _c_int, _c_float, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p],
     "ka_maps_combine": [_c_void_p, _c_void_p, _c_int, _c_long, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_void_p],
     "ka_latent_prepare": [_c_void_p, _c_int, _c_long, _c_int, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int,
                           _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_int, _c_void_p],
@@ -86,6 +86,9 @@ _SIGNATURES = {
     "ka_gated_step_supported": [_c_int, _c_int, _c_int],
     "ka_gated_step": [_c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_float,
                       _c_float, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_gated_step_job": [_c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_float,
+                      _c_float, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_gated_step_job_bytes": [],
     "ka_heads_rmsnorm": [_c_void_p, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     "ka_experts_combine": [_c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
                            _c_long, _c_void_p, _c_int, _c_int, _c_void_p],
@@ -575,10 +578,11 @@ def gated_linear_attention(projected: torch.Tensor, offsets, pre: torch.Tensor, 
 
 
 def gated_step(projected: torch.Tensor, offsets, a2: torch.Tensor, a2_bias: torch.Tensor, gain: torch.Tensor, tau: float, q_scale: float, eps: float,
-               state: torch.Tensor, row_slot: torch.Tensor, out: torch.Tensor, n_heads: int, head_dim: int, value_dim: int) -> bool:
+               state: torch.Tensor, row_slot: torch.Tensor, out: torch.Tensor, n_heads: int, head_dim: int, value_dim: int, later: bool = False):
     """A step of single tokens (row ``r`` brings token ``r``) of gated linear attention in one launch: ``gated_linear_attention`` with ``pre = a2
     low + a2_bias``, then ``heads_rmsnorm``. ``offsets``: the columns of q, k, v, gate and low in ``projected`` ``[n, ..]``; ``a2`` ``[H hd, rank]`` of
-    its type. False: sizes or alignment not covered, nothing was run."""
+    its type. False: sizes or alignment not covered, nothing was run. ``later``: nothing is launched; the step is returned as ``conv_prepare`` takes it
+    (``beside``), with the tensors, which have to outlive that call, in the caller's hands."""
     _dev(projected, a2, a2_bias, gain, state, row_slot, out)
     n, rank = projected.shape[0], a2.shape[1]
     who = "gated_step"
@@ -595,10 +599,14 @@ def gated_step(projected: torch.Tensor, offsets, a2: torch.Tensor, a2_bias: torc
     oq, ok, ov, og, ol = (int(o) for o in offsets)
     _need(max(oq + n_heads * head_dim, ok + n_heads * head_dim, ov + n_heads * value_dim, og + n_heads * value_dim, ol + rank) <= projected.shape[1],
           f"{who}: the projected rows are too short")
-    _check(lib().ka_gated_step(projected.data_ptr(), projected.stride(0) if n > 1 else max(projected.stride(0), projected.shape[1]),
-                               code_of(projected.dtype), oq, ok, ov, og, ol, rank, a2.data_ptr(), a2_bias.data_ptr(), gain.data_ptr(), float(tau),
-                               float(q_scale), float(eps), state.data_ptr(), state.stride(0), row_slot.data_ptr(), out.data_ptr(),
-                               out.stride(0) if n > 1 else max(out.stride(0), n_heads * value_dim), n, n_heads, head_dim, value_dim, stream_ptr()))
+    args = (projected.data_ptr(), projected.stride(0) if n > 1 else max(projected.stride(0), projected.shape[1]), code_of(projected.dtype), oq, ok, ov, og,
+            ol, rank, a2.data_ptr(), a2_bias.data_ptr(), gain.data_ptr(), float(tau), float(q_scale), float(eps), state.data_ptr(), state.stride(0),
+            row_slot.data_ptr(), out.data_ptr(), out.stride(0) if n > 1 else max(out.stride(0), n_heads * value_dim), n, n_heads, head_dim, value_dim)
+    if later:
+        job = ctypes.create_string_buffer(lib().ka_gated_step_job_bytes())
+        _check(lib().ka_gated_step_job(*args, ctypes.addressof(job)))
+        return job
+    _check(lib().ka_gated_step(*args, stream_ptr()))
     return True
 
 
@@ -707,7 +715,7 @@ def conv_prepare(u: torch.Tensor, taps: Optional[torch.Tensor], state: Optional[
                  row_slot: torch.Tensor, token_row: torch.Tensor, positions: torch.Tensor, slots: Optional[torch.Tensor],
                  q_out: torch.Tensor, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], q_heads: int, k_heads: int,
                  head_dim: int, v_heads: int, value_dim: int, page_size: int, freqs: Optional[torch.Tensor] = None,
-                 pairing: str = "halves", unit_norm_eps: Optional[float] = None, runs=None, single_tokens: bool = False) -> None:
+                 pairing: str = "halves", unit_norm_eps: Optional[float] = None, runs=None, single_tokens: bool = False, beside=None) -> None:
     """A short causal convolution over time on every channel of the projected rows ``u`` ``[n, q | k | v]``
     (``taps`` fp32 ``[channels, K]``: ``y_t = sum_j taps[:, j] u_(t - K + 1 + j)``; ``None``: none), then the rotation of the
     first ``2 len(freqs)`` channels of every query and key head by ``place * freqs``, then queries into ``q_out`` ``[n, q]``,
@@ -715,7 +723,8 @@ def conv_prepare(u: torch.Tensor, taps: Optional[torch.Tensor], state: Optional[
     ``slots``. Inputs from before this step come from ``state`` fp32 ``[slots + 1, K - 1, channels]`` (by ``row_slot``; a slot's rows
     may lie in a wider one), which is then moved on to the last ``K - 1`` rows of ``u`` of every row. ``unit_norm_eps``: every query
     and key head is divided by its root mean square ``sqrt(mean(square) + eps)`` as well. ``runs``: (int32 first token, int32 count) of
-    the runs the tokens are cut into (``StepBatch.page_runs``); ``single_tokens``: every row brings one token."""
+    the runs the tokens are cut into (``StepBatch.page_runs``); ``single_tokens``: every row brings one token. ``beside``: a step of the same
+    single tokens (``gated_step(..., later=True)``) that neither reads nor writes what this one does, run in the same launch where that covers it."""
     _need(pairing in ROTARY_PAIRINGS, f"conv_prepare: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
     _dev(u, taps, state, cu_q, row_slot, token_row, positions, slots, q_out, k_cache, v_cache, freqs)
     n = u.shape[0]
@@ -756,7 +765,8 @@ def conv_prepare(u: torch.Tensor, taps: Optional[torch.Tensor], state: Optional[
                                  q_out.data_ptr(), q_out.stride(0) if n > 1 else q_heads * head_dim, _ptr(k_cache), _ptr(v_cache), n, n_rows,
                                  q_heads, k_heads, head_dim, v_heads, value_dim, page_size, _ptr(freqs), rot, ROTARY_PAIRINGS[pairing],
                                  state.stride(0) if K > 1 else 0, int(unit_norm_eps is not None), float(unit_norm_eps or 0.0), _ptr(first),
-                                 _ptr(count), int(first.numel()) if first is not None else 0, int(bool(single_tokens)), stream_ptr()))
+                                 _ptr(count), int(first.numel()) if first is not None else 0, int(bool(single_tokens)),
+                                 ctypes.addressof(beside) if beside is not None else None, stream_ptr()))
 
 
 def maps_combine(maps: torch.Tensor, out: torch.Tensor, n_heads: int, value_dim: int, weight: float, eps: float, out_scale: float) -> None:

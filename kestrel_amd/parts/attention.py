@@ -9,7 +9,7 @@ import torch
 from ..ops import core
 from ..ops.attention import paged_attention
 from ..ops.linear import linear
-from .base import LayerCache, Mixer, build_part, register_mixer
+from .base import LayerCache, Mixer, SideStep, build_part, register_mixer
 from .specs import AttentionSpec, CacheSpec, ParamSpec, StateSpec
 
 
@@ -271,6 +271,9 @@ class PagedAttention(Mixer):
         return fast.attention_decode_takes(job, job.a.shape[0], self.spec.n_heads, self.spec.head_dim, cache.k.shape[2],
                                            batch.max_kv)
 
+    def takes_step(self, batch) -> bool:
+        return self.prepared and bool(self.taps) and bool(batch.decode_only)
+
     def attend(self, qkv, batch, cache: LayerCache, beside=None, out=None):
         """Position encoding, cache write and attention on the projected input ``[n, q|k|v]``; ``out``: where the heads go."""
         spec = self.spec
@@ -279,9 +282,10 @@ class PagedAttention(Mixer):
         if out is None:
             out = batch.workspace.get("attn.out", (n, self.out_dim), self.dtype)
         if self.prepared:
-            if beside is not None:
+            step = beside.job if isinstance(beside, SideStep) else None
+            if beside is not None and step is None:
                 self._alone(beside)
-            return self._attend_prepared(qkv, batch, cache, group, out)
+            return self._attend_prepared(qkv, batch, cache, group, out, step)
         if self.extended:
             if beside is not None:
                 self._alone(beside)
@@ -336,9 +340,10 @@ class PagedAttention(Mixer):
                                self._slopes, self.sink)
         return out
 
-    def _attend_prepared(self, projected, batch, cache: LayerCache, group, out):
+    def _attend_prepared(self, projected, batch, cache: LayerCache, group, out, step=None):
         """Queries, keys and values made ready by one kernel (norms, rotation, factor, blend, cache write), attention with
-        the distance table where there is one, then the output gate. ``projected``: ``[n, q | k | v (| gate)]``."""
+        the distance table where there is one, then the output gate. ``projected``: ``[n, q | k | v (| gate)]``. ``step``: a job that the
+        launch of the convolutions takes along (``takes_step``)."""
         spec = self.spec
         n = projected.shape[0]
         qkv = projected[:, :self.qkv_dim] if self.gated else projected
@@ -351,7 +356,7 @@ class PagedAttention(Mixer):
         if self.shares_kv and cache.writes:
             raise RuntimeError("a layer without keys and values of its own must read another layer's cache (ScheduleEntry.reads_cache_of)")
         if self.taps:
-            qkv = self._convolve(qkv, batch, cache, group, slots)
+            qkv = self._convolve(qkv, batch, cache, group, slots, step)
         else:
             core.qkv_prepare(qkv, batch.positions, slots, cache.k, cache.v, spec.n_heads, 0 if self.shares_kv else spec.n_kv_heads,
                              spec.head_dim, self.value_dim, group.page_size, norm.scope if norm is not None else None, self._q_gain,
@@ -382,7 +387,7 @@ class PagedAttention(Mixer):
             core.gate_mul(out, gate)
         return out
 
-    def _convolve(self, qkv, batch, cache: LayerCache, group, slots):
+    def _convolve(self, qkv, batch, cache: LayerCache, group, slots, step=None):
         """The convolutions with all that follows them before attention; returns the queries."""
         spec = self.spec
         if self.taps > 1 and cache.state is None:
@@ -391,7 +396,7 @@ class PagedAttention(Mixer):
         core.conv_prepare(qkv, self._taps, cache.state, batch.cu_q, batch.row_slot, batch.token_row, batch.positions, slots, q, cache.k, cache.v,
                           spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.n_kv_heads, self.value_dim, group.page_size, self._freqs,
                           self._pairing, unit_norm_eps=float(self.qk_norm.eps) if self.qk_norm is not None else None,
-                          runs=getattr(batch, "page_runs", None), single_tokens=bool(batch.decode_only))
+                          runs=getattr(batch, "page_runs", None), single_tokens=bool(batch.decode_only), beside=step)
         return q
 
     @staticmethod

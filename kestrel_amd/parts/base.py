@@ -164,6 +164,14 @@ class SideLinear:
     act: int                              # activation code of ``ops.linear``
 
 
+class SideStep:
+    """A branch's whole work between its projections for a step of single tokens, checked and ready to run in the launch of another branch that
+    reads the same projected rows (``Mixer.takes_step``): ``job`` as ``ops.core.conv_prepare`` takes it."""
+
+    def __init__(self, job) -> None:
+        self.job = job
+
+
 class Mixer(Part):
     def cache_spec(self) -> Optional[CacheSpec]:
         """Keys and values kept per token, or ``None``."""
@@ -214,6 +222,14 @@ class Mixer(Part):
     def takes_output_weight(self, weight: float) -> bool:
         """Whether ``fold_output_weight`` can take this weight up."""
         return weight == 1.0
+
+    def takes_step(self, batch) -> bool:
+        """Whether ``attend`` takes another branch's ``SideStep`` along (``beside``) for this batch."""
+        return False
+
+    def side_step(self, projected: torch.Tensor, batch, cache: LayerCache, out: torch.Tensor) -> Optional["SideStep"]:
+        """``attend`` into ``out`` as a job for another branch's launch, or ``None`` (nothing was run)."""
+        return None
 
     def fold_output_weight(self, weight: float) -> None:
         """What ``attend`` returns is ``weight`` times what it would be from now on, at no cost and no loss (a factor that some

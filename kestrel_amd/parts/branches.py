@@ -131,9 +131,17 @@ class Branches(Mixer):
             projected = batch.workspace.get("branches.in", (n, self.in_cols[-1]), self.dtype)
             linear(h, self.in_weight, None, projected)
             heads = batch.workspace.get("branches.heads", (n, self.out_cols[-1]), self.dtype)
+            views = [(projected[:, self.in_cols[i]:self.in_cols[i + 1]], batch, self._cache_of(i, cache)) for i in range(len(self.branches))]
+            outs = [heads[:, self.out_cols[i]:self.out_cols[i + 1]] for i in range(len(self.branches))]
+            # (single tokens: what one branch does between its projections in a launch that another makes anyway)
+            host = next((i for i, branch in enumerate(self.branches) if branch.takes_step(batch)), None)
+            guest = step = None
             for i, branch in enumerate(self.branches):
-                branch.attend(projected[:, self.in_cols[i]:self.in_cols[i + 1]], batch, self._cache_of(i, cache),
-                              out=heads[:, self.out_cols[i]:self.out_cols[i + 1]])
+                if host is not None and step is None and i != host:
+                    guest, step = i, branch.side_step(*views[i], outs[i])
+            for i, branch in enumerate(self.branches):
+                if step is None or i != guest:
+                    branch.attend(*views[i], **({"beside": step} if step is not None and i == host else {}), out=outs[i])
             linear(heads, self.proj_weight, None, out, accumulate=accumulate)
             return
         if not accumulate:

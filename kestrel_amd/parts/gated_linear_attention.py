@@ -8,7 +8,7 @@ import torch
 
 from ..ops import core
 from ..ops.linear import linear
-from .base import LayerCache, Mixer, register_mixer
+from .base import LayerCache, Mixer, SideStep, register_mixer
 from .specs import GatedLinearAttentionSpec, ParamSpec, StateSpec
 
 
@@ -91,6 +91,19 @@ class GatedLinearAttention(Mixer):
     def fold_output_weight(self, weight: float) -> None:
         self.gain = self.gain * float(weight)          # (the last factor of the heads before the gate, fp32)
 
+    def _step(self, projected, batch, cache: LayerCache, out, later: bool):
+        """A step of single tokens in one launch (``core.gated_step``)."""
+        spec = self.spec
+        return core.gated_step(projected, (*self.offsets, self.gate_at, self.low_at), self.a2_weight, self.a2_bias, self.gain, float(spec.tau),
+                               float(spec.head_dim) ** -0.5, float(spec.eps), cache.state, batch.row_slot, out, spec.n_heads, spec.head_dim, spec.value_dim,
+                               later=later)
+
+    def side_step(self, projected, batch, cache: LayerCache, out) -> Optional[SideStep]:
+        if not batch.decode_only or cache.state is None or self.dtype != torch.bfloat16:
+            return None
+        job = self._step(projected, batch, cache, out, True)
+        return SideStep(job) if job else None
+
     def attend(self, projected, batch, cache: LayerCache, beside=None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The recurrence over the step's tokens, normalised and gated: the input of the output projection."""
         spec = self.spec
@@ -102,8 +115,7 @@ class GatedLinearAttention(Mixer):
             out = ws.get("gated_attention.out", (n, self.v_dim), self.dtype)
         sizes = (spec.n_heads, spec.head_dim, spec.value_dim)
         q_scale = float(spec.head_dim) ** -0.5
-        if batch.decode_only and core.gated_step(projected, (*self.offsets, self.gate_at, self.low_at), self.a2_weight, self.a2_bias, self.gain,
-                                                 float(spec.tau), q_scale, float(spec.eps), cache.state, batch.row_slot, out, *sizes):
+        if batch.decode_only and self._step(projected, batch, cache, out, False):
             return out
         pre = ws.get("gated_attention.pre", (n, self.qk_dim), torch.float32)
         linear(projected[:, self.low_at:self.low_at + self.rank], self.a2_weight, self.a2_bias, pre)
