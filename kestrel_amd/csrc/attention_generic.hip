@@ -1,5 +1,5 @@
-// Generic paged attention: one wavefront per (token, query head), any head size up
-// to 1024, any page size, fp32 or bf16 storage, all arithmetic in fp32.
+// Generic paged attention, all arithmetic in fp32: one wavefront per (token, query head), any head size up
+// to 1024, any page size, fp32 or bf16 storage; and a second kernel for fp32 storage in steps of four keys and channels, which reads whole lines.
 //
 // Every token t of the packed batch belongs to request row token_row[t] and sees
 // the cached keys at positions [kv_lo[t], kv_hi[t]) of that row (kv_lo optional,
@@ -156,6 +156,196 @@ attention_generic_kernel(const T* __restrict__ q, long q_row_stride, const T* __
     }
 }
 
+// ----------------------------------------------------------------------------
+// The same for fp32 heads of up to 256 channels (keys a multiple of four) and pages of a multiple of four keys, values in a cache of their own.
+//
+// Bound by trips to memory one behind the other. In the kernel above a lane owns a key, so a load touches 64 rows with 16 bytes each and comes
+// back to each of them for every four channels, and the values are asked for when the scores are known; one wave walks all keys. Here
+// G = 16, 32 or 64 lanes share a key (a row is one load's piece), 16 keys each; a lane's sixteen partial scores are added up across its row of 16
+// lanes so that each lane ends with one key's (fifteen lane moves for 16 keys); values come as four neighbouring keys of one channel, whole
+// pieces of a page, asked for together with the keys; and NW waves take the chunks of CK keys in turn and meet in LDS at the end.
+// 32 heads of 64, us, there and here: 3 tokens behind 31 to 160 keys 17.5 and 7.1, 8 behind 1,040 88 and 25 (5.4 TB/s), 64 behind 400 111 and 79 (5.3
+// TB/s), three prompts of 31 to 157 66 and 31, a prompt of 400 225 and 72, of 2,048 5,406 and 1,197; heads of 128: 8 behind 1,040 174 and 42, a prompt
+// of 400 453 and 108. Errors against 64 bits are no larger: a score is the sum of sixteen or more partial ones instead of one chain.
+// ----------------------------------------------------------------------------
+struct SpreadArgs {
+    const float* q;
+    long q_row_stride;
+    const float *k_cache, *v_cache;
+    const int* block_table;
+    int max_pages;
+    const int *token_row, *kv_lo, *kv_hi;
+    float* out;
+    long out_row_stride;
+    float scale;
+    int H, Hkv, hd, hdv, page_size;
+    const int* positions;
+    const float* slopes;
+    int has_sink;
+    float sink_score;
+    const float* bias_table;
+    int bias_len;
+    const float* gate;
+    long gate_row_stride;
+    const float* sinks;
+    int keep_first, maps;
+    float softcap;
+    int gate_per_head;
+};
+
+typedef __attribute__((ext_vector_type(4))) float as_floatx4;
+
+// What a wave's lanes wrote to LDS before is seen by its lanes after.
+__device__ __forceinline__ void as_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sixteen values a lane, added up over the 16 lanes of a row: lane i of the row ends with the sum of value i. A step leaves a lane the half of the
+// values that its own bit names and adds the partner's (the lane mirrored in the row, in the half row, then two and one further).
+template <int LEFT>
+__device__ __forceinline__ void as_scatter_sums(float (&v)[16], int lane) {
+    if constexpr (LEFT >= 1) {
+        constexpr int CTRL = LEFT == 8 ? 0x140 : LEFT == 4 ? 0x141 : LEFT == 2 ? 0x4E : 0xB1;
+        const bool upper = lane & LEFT;
+#pragma unroll
+        for (int i = 0; i < LEFT; ++i) {
+            const float keep = upper ? v[i + LEFT] : v[i], give = upper ? v[i] : v[i + LEFT];
+            v[i] = keep + ka_dpp_move<CTRL>(give);
+        }
+        as_scatter_sums<LEFT / 2>(v, lane);
+    }
+}
+
+template <int G, int NW>
+__global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadArgs g) {
+    constexpr int GROUPS = KA_WAVE / G, CK = 16 * GROUPS, R = G / 4;         // groups of 16 keys in a chunk of CK; channels in sixteens
+    __shared__ long k_at[NW][CK], v_at[NW][CK];
+    __shared__ __attribute__((aligned(16))) float ps[NW][CK];
+    __shared__ float sums[NW][R * 16], tops[NW], totals[NW];
+    const int t = blockIdx.x, h = blockIdx.y, wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
+    const int vh = h / g.maps / (g.H / g.Hkv), kvh = vh * g.maps + h % g.maps, Hv = g.Hkv / g.maps;
+    const int lo = g.kv_lo ? g.kv_lo[t] : 0, hi = g.kv_hi[t];
+    const int* bt = g.block_table + (size_t)g.token_row[t] * g.max_pages;
+    const int in_row = lane % G, group = lane / G;
+    const bool owns = in_row < 16;                       // (the other rows of a group hold the same keys' scores once more)
+    as_floatx4 q4 = {0.f, 0.f, 0.f, 0.f};
+    if (in_row * 4 < g.hd) {
+        const float* qp = g.q + (size_t)t * g.q_row_stride + (size_t)h * g.hd + in_row * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q4[i] = qp[i] * g.scale;
+    }
+    const float slope = g.slopes ? g.slopes[h] : 0.f;
+    const int place = (g.slopes || g.bias_table) ? g.positions[t] : 0;
+    const float* bias_row = g.bias_table ? g.bias_table + (size_t)h * g.bias_len : nullptr;
+    const float sink = g.sinks ? g.sinks[h] : g.sink_score;
+    const bool sinks_here = g.has_sink && wave == 0;
+    float m = sinks_here ? sink : -INFINITY, l = sinks_here ? 1.f : 0.f;
+    float o[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) o[r] = 0.f;
+
+    // chunks of the kept first keys, then of the window's, whose first chunk starts on a multiple of four keys
+    const int kept = min(g.keep_first, lo), kept_chunks = kept > 0 ? (kept + CK - 1) / CK : 0;
+    const int start = lo & ~3, chunks = kept_chunks + (hi > lo ? (hi - start + CK - 1) / CK : 0);
+    for (int c = wave; c < chunks; c += NW) {
+        const bool first = c < kept_chunks;
+        const int base = first ? c * CK : start + (c - kept_chunks) * CK, from = first ? 0 : lo, to = first ? kept : hi;
+        const int key = base + group * 16 + lane % 16;
+        const bool valid = key >= from && key < to;
+        {
+            const int near = min(max(key, from), to - 1), page = bt[near / g.page_size], at = near % g.page_size;
+            as_wave_sync();                              // the chunk before has been read
+            if (owns) {
+                k_at[wave][group * 16 + in_row] = (((long)page * g.Hkv + kvh) * g.page_size + at) * g.hd;
+                v_at[wave][group * 16 + in_row] = ((long)page * Hv + vh) * g.hdv * g.page_size + (at & ~3);
+            }
+            as_wave_sync();
+        }
+        as_floatx4 k4[16], v4[GROUPS][R];
+        const int channel = min(in_row * 4, g.hd - 4);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) k4[i] = *reinterpret_cast<const as_floatx4*>(g.k_cache + k_at[wave][group * 16 + i] + channel);
+#pragma unroll
+        for (int x = 0; x < GROUPS; ++x) {
+            const float* vp = g.v_cache + v_at[wave][x * 16 + lane % 4 * 4];
+#pragma unroll
+            for (int r = 0; r < R; ++r) v4[x][r] = *reinterpret_cast<const as_floatx4*>(vp + (long)min(r * 16 + lane / 4, g.hdv - 1) * g.page_size);
+        }
+        float part[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[i] = fmaf(q4[3], k4[i][3], fmaf(q4[2], k4[i][2], fmaf(q4[1], k4[i][1], q4[0] * k4[i][0])));
+        as_scatter_sums<8>(part, lane);
+        float s = ka_lanes_reduce<16, G>(part[0], KaSum{});
+        if (g.softcap > 0.f) s = g.softcap * tanhf(s / g.softcap);
+        if (g.slopes) s -= slope * (float)(place - key);
+        if (bias_row) s += bias_row[min(max(place - key, 0), g.bias_len - 1)];
+        if (!valid) s = -INFINITY;
+        const float m_new = fmaxf(m, ka_wave_max(s));
+        const float corr = m == m_new ? 1.f : expf(m - m_new);
+        const float p = valid ? expf(s - m_new) : 0.f;
+        l = l * corr + ka_wave_sum(owns ? p : 0.f);
+        m = m_new;
+        if (owns) ps[wave][group * 16 + in_row] = p;
+        as_wave_sync();
+        const bool whole = base >= from && base + CK <= to;
+#pragma unroll
+        for (int r = 0; r < R; ++r) o[r] *= corr;
+#pragma unroll
+        for (int x = 0; x < GROUPS; ++x) {
+            const int j = x * 16 + lane % 4 * 4;
+            const as_floatx4 p4 = *reinterpret_cast<const as_floatx4*>(&ps[wave][j]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                as_floatx4 v = v4[x][r];
+                if (!whole) {                            // (a place without a key may hold anything)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = base + j + i >= from && base + j + i < to ? v[i] : 0.f;
+                }
+                o[r] += fmaf(p4[3], v[3], fmaf(p4[2], v[2], fmaf(p4[1], v[1], p4[0] * v[0])));
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float y = ka_lanes_reduce<1, 4>(o[r], KaSum{});
+        if (lane % 4 == 0) sums[wave][r * 16 + lane / 4] = y;
+    }
+    if (lane == 0) {
+        tops[wave] = m;
+        totals[wave] = l;
+    }
+    __syncthreads();
+    float top = -INFINITY, total = 0.f, share[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, tops[w]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        share[w] = tops[w] == top ? 1.f : expf(tops[w] - top);           // (a wave without a key: exp(-inf), or nothing at all)
+        total += totals[w] * share[w];
+    }
+    const float inv = total > 0.f ? 1.0f / total : 0.f;
+    const float head_gate = g.gate && g.gate_per_head ? 1.0f / (1.0f + expf(-g.gate[(size_t)t * g.gate_row_stride + h])) : 1.f;
+    for (int d = threadIdx.x; d < g.hdv; d += KA_WAVE * NW) {
+        float y = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) y += sums[w][d] * share[w];
+        y *= inv * head_gate;
+        if (g.gate && !g.gate_per_head) y *= 1.0f / (1.0f + expf(-g.gate[(size_t)t * g.gate_row_stride + (size_t)h * g.hdv + d]));
+        g.out[(size_t)t * g.out_row_stride + (size_t)h * g.hdv + d] = y;
+    }
+}
+
+template <int G>
+static void launch_spread(const SpreadArgs& g, int n, hipStream_t stream) {
+    // (waves that a token's keys are cut over, by what fills the chip: a wave holds some 160 registers, three a SIMD)
+    const long heads = (long)n * g.H, cus = ka_compute_units();
+    if (heads <= 4 * cus) hipLaunchKernelGGL((attention_spread_kernel<G, 8>), dim3(n, g.H), dim3(8 * KA_WAVE), 0, stream, g);
+    else if (heads <= 16 * cus) hipLaunchKernelGGL((attention_spread_kernel<G, 4>), dim3(n, g.H), dim3(4 * KA_WAVE), 0, stream, g);
+    else hipLaunchKernelGGL((attention_spread_kernel<G, 1>), dim3(n, g.H), dim3(KA_WAVE), 0, stream, g);
+}
+
 KA_API int ka_attention_generic(const void* q, int dtype, long q_row_stride, const void* k_cache,
                                 const void* v_cache, const int* block_table, int max_pages,
                                 const int* token_row, const int* kv_lo, const int* kv_hi, void* out,
@@ -178,7 +368,16 @@ KA_API int ka_attention_generic(const void* q, int dtype, long q_row_stride, con
     KA_CHECK(page_size > 0 && max_pages > 0, "ka_attention_generic: bad paging %d %d", page_size, max_pages);
     if (n == 0) return 0;
     dim3 grid(n, H), block(KA_WAVE);
-    if (dtype == KA_F32)
+    if (dtype == KA_F32 && !values_in_keys && hd % 4 == 0 && hd <= 256 && hdv <= 256 && page_size % 4 == 0 &&
+        ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0) {
+        const SpreadArgs g{(const float*)q, q_row_stride, (const float*)k_cache, (const float*)v_cache, block_table, max_pages, token_row, kv_lo, kv_hi,
+                           (float*)out, out_row_stride, scale, H, Hkv, hd, hdv, page_size, positions, slopes, has_sink, sink_score, bias_table, bias_len,
+                           (const float*)gate, gate_row_stride, sinks, keep_first, maps, softcap, gate_per_head};
+        const int wide = hd > hdv ? hd : hdv;
+        if (wide <= 64) launch_spread<16>(g, n, stream);
+        else if (wide <= 128) launch_spread<32>(g, n, stream);
+        else launch_spread<64>(g, n, stream);
+    } else if (dtype == KA_F32)
         hipLaunchKernelGGL(attention_generic_kernel<float>, grid, block, 0, stream, (const float*)q, q_row_stride,
                            (const float*)k_cache, (const float*)v_cache, block_table, max_pages, token_row, kv_lo,
                            kv_hi, (float*)out, out_row_stride, scale, H, Hkv, hd, hdv, page_size, positions, slopes, has_sink,
