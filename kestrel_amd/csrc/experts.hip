@@ -5,151 +5,24 @@
 // A pair is p = token * top + choice. chosen[p] names the router's output that the token chose there: a number below
 // n_experts is an expert with weights, a number from n_experts on an identity expert whose output is the token's input.
 #include "ka_common.h"
+#include "ka_route.h"
 #include "ka_rows.h"
 
-constexpr int EX_MAX_OUTPUTS = 512;             // router outputs a wave can hold (8 a lane)
-constexpr int EX_MAX_GROUPS = 64;
-
-// The lowest index that holds the largest value of a wave (of at most `last`), in every lane.
-__device__ __forceinline__ int ex_wave_argmax(float v, int i, int last) {
-    const float best = ka_wave_max(v);
-    const int found = ka_lanes_reduce<1, KA_WAVE>(v == best ? i : 0x7fffffff, KaIntMin{});
-    return __builtin_amdgcn_readfirstlane(min(found, last));
-}
-
-// ----------------------------------------------------------------------------
-// The router's choice, a wave per token. logits fp32 [n, >= R] (rows `stride` apart), R router outputs.
-//     s = softmax(logits), or sigmoid(logits) one by one;  choice = s + correction (correction optional)
-//     n_groups > 0: the outputs form n_groups equal groups of neighbours, a group's score is its largest choice score, or the
-//       sum of its two largest (group_best 2), and only outputs of the `keep` best groups can be chosen;
-//     the `top` outputs with the largest choice scores are chosen (the lower index wins a tie);
-//     weights: their s divided by the sum of the chosen s (+ 1e-20), times scale.
-// mode 0: softmax scores, 2: sigmoid scores; 1 (by the logits): the choice goes by the logits themselves (no correction, no groups); the weights are the softmax over the chosen
-// logits, times scale.
-// chosen int32 [n, top], weights fp32 [n, top]; always >= 0: the rows are one longer and end in that output with weight 1 (a
-// feed-forward that every token uses, laid behind the experts).
-// ----------------------------------------------------------------------------
-template <int PER_LANE>          // outputs a lane holds
-__global__ void __launch_bounds__(KA_WAVE)
-route_kernel(const float* __restrict__ logits, long stride, const float* __restrict__ correction, int R, int top, int n_groups,
-             int keep, int group_best, float scale, int mode, int always, int* __restrict__ chosen, float* __restrict__ weights) {
-    __shared__ float choice_s[PER_LANE * KA_WAVE];
-    __shared__ float group_s[EX_MAX_GROUPS];
-    __shared__ int allowed_s[EX_MAX_GROUPS];
-    const int t = blockIdx.x, lane = threadIdx.x;
-    const bool by_logits = mode == 1, sigmoids = mode == 2;
-    const float* z = logits + (size_t)t * stride;
-    float s[PER_LANE], c[PER_LANE];
-    float top_z = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < PER_LANE; ++q) {
-        const int r = lane + q * KA_WAVE;
-        s[q] = r < R ? z[r] : -INFINITY;
-        top_z = fmaxf(top_z, s[q]);
-    }
-    top_z = ka_wave_max(top_z);
-    float total = 0.f;
-#pragma unroll
-    for (int q = 0; q < PER_LANE; ++q) {
-        c[q] = s[q];
-        if (sigmoids) s[q] = lane + q * KA_WAVE < R ? 1.0f / (1.0f + expf(-s[q])) : 0.f;
-        else s[q] = lane + q * KA_WAVE < R ? expf(s[q] - top_z) : 0.f;
-        total += s[q];
-    }
-    total = ka_wave_sum(total);
-#pragma unroll
-    for (int q = 0; q < PER_LANE; ++q) {
-        const int r = lane + q * KA_WAVE;
-        if (by_logits) continue;      // (the largest logit is among the chosen: e^(z - top) over their sum is their softmax)
-        if (!sigmoids) s[q] = s[q] / total;
-        c[q] = r < R ? s[q] + (correction ? correction[r] : 0.f) : -INFINITY;
-        if (r < R) choice_s[r] = c[q];
-    }
-    if (n_groups > 0) {
-        const int per = R / n_groups;
-        __syncthreads();
-        if (lane < n_groups) {
-            float best = -INFINITY, second = -INFINITY;
-            for (int m = 0; m < per; ++m) {
-                const float v = choice_s[lane * per + m];
-                second = fmaxf(second, fminf(v, best));
-                best = fmaxf(best, v);
-            }
-            group_s[lane] = group_best == 2 && per > 1 ? best + second : best;
-        }
-        __syncthreads();
-        if (lane < n_groups) {
-            const float own = group_s[lane];
-            int ahead = 0;              // groups that are kept before this one (the lower index wins a tie)
-            for (int g = 0; g < n_groups; ++g) ahead += group_s[g] > own || (group_s[g] == own && g < lane);
-            allowed_s[lane] = ahead < keep;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < PER_LANE; ++q) {
-            const int r = lane + q * KA_WAVE;
-            if (r < R && !allowed_s[r / per]) c[q] = -INFINITY;
-        }
-    }
-    float sum = 0.f;
-    float mine_w = 0.f;          // lane k keeps the k-th chosen score
-    int mine_i = 0;
-    unsigned taken = 0;          // bit q: this lane's entry q is chosen already
-    for (int k = 0; k < top; ++k) {
-        float v = -INFINITY;
-        int i = 0x7fffffff;
-#pragma unroll
-        for (int q = 0; q < PER_LANE; ++q) {
-            const int r = lane + q * KA_WAVE;
-            if (r < R && !(taken >> q & 1) && (c[q] > v || i == 0x7fffffff)) {
-                v = c[q];
-                i = r;
-            }
-        }
-        i = ex_wave_argmax(v, i, R - 1);
-        float sv = 0.f;
-#pragma unroll
-        for (int q = 0; q < PER_LANE; ++q)
-            if (lane + q * KA_WAVE == i) {
-                taken |= 1u << q;
-                sv = s[q];
-            }
-        sv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sv), i % KA_WAVE));       // (one lane holds it)
-        sum += sv;
-        if (lane == k % KA_WAVE) {
-            // (more than a wave of choices would need more than one register a lane: the entry point refuses it)
-            mine_w = sv;
-            mine_i = i;
-        }
-    }
-    const size_t at = (size_t)t * (always >= 0 ? top + 1 : top);
-    if (lane < top) {
-        chosen[at + lane] = mine_i;
-        weights[at + lane] = mine_w / (by_logits ? sum : sum + 1e-20f) * scale;
-    }
-    if (always >= 0 && lane == 0) {
-        chosen[at + top] = always;
-        weights[at + top] = 1.f;
-    }
+// (a launch of its own, a workgroup a token)
+template <int PER_LANE>
+__global__ void __launch_bounds__(KA_WAVE) route_kernel(RouteArgs job) {
+    __shared__ RouteRoom<PER_LANE> room;
+    ka_route_token<PER_LANE>(job, blockIdx.x, threadIdx.x, room);
 }
 
 KA_API int ka_route(const float* logits, long stride, const float* correction, int n, int R, int top, int n_groups, int keep,
                     int group_best, float scale, int mode, int always, int* chosen, float* weights, hipStream_t stream) {
-    const char* who = "ka_route";
-    KA_CHECK(mode >= 0 && mode <= 2 && (group_best == 1 || group_best == 2), "%s: unknown mode %d or group score %d", who, mode, group_best);
-    KA_CHECK(mode != 1 || (n_groups == 0 && correction == nullptr), "%s: a choice by the logits alone has no groups and no correction", who);
-    KA_CHECK(n >= 0 && R > 0 && R <= EX_MAX_OUTPUTS && stride >= R, "%s: %d router outputs (at most %d)", who, R, EX_MAX_OUTPUTS);
-    KA_CHECK(top > 0 && top <= R && top <= KA_WAVE, "%s: %d choices of %d", who, top, R);
-    KA_CHECK(n_groups >= 0 && n_groups <= EX_MAX_GROUPS && (n_groups == 0 || (R % n_groups == 0 && keep > 0 && keep <= n_groups)),
-             "%s: %d groups of which %d are kept do not divide %d outputs", who, n_groups, keep, R);
-    KA_CHECK(n_groups == 0 || keep * (R / n_groups) >= top, "%s: %d kept groups hold fewer than %d outputs", who, keep, top);
+    const RouteArgs job{logits, stride, correction, R, top, n_groups, keep, group_best, mode, always, scale, chosen, weights};
+    if (ka_route_check("ka_route", job, n)) return -1;
     if (n == 0) return 0;
-#define EX_ROUTE(PER_LANE) \
-    hipLaunchKernelGGL(route_kernel<PER_LANE>, dim3(n), dim3(KA_WAVE), 0, stream, logits, stride, correction, R, top, n_groups, keep, group_best, scale, mode, always, chosen, weights)
-    if (R <= KA_WAVE) EX_ROUTE(1);
-    else if (R <= 2 * KA_WAVE) EX_ROUTE(2);
-    else EX_ROUTE(EX_MAX_OUTPUTS / KA_WAVE);
-#undef EX_ROUTE
+    if (R <= KA_WAVE) hipLaunchKernelGGL(route_kernel<1>, dim3(n), dim3(KA_WAVE), 0, stream, job);
+    else if (R <= 2 * KA_WAVE) hipLaunchKernelGGL(route_kernel<2>, dim3(n), dim3(KA_WAVE), 0, stream, job);
+    else hipLaunchKernelGGL((route_kernel<EX_MAX_OUTPUTS / KA_WAVE>), dim3(n), dim3(KA_WAVE), 0, stream, job);
     KA_LAUNCH_CHECK();
     return 0;
 }

@@ -29,6 +29,7 @@
 //    pass): one strip per workgroup, up to 16 waves over K, rounds of blocks double-buffered.
 // Both take two targets (strips of W_a, then strips of W_b, from the same input): the fused
 // q|k|v projection and the first feed-forward linear.
+#include "ka_route.h"
 #include "ka_skinny.h"
 #include "ka_partials.h"
 
@@ -445,6 +446,59 @@ static int launch_persistent(int strips, int M, int kblocks, bool ln, size_t dyn
         case 3: return launch_persistent_per<3, false, false>(per, grid, SP_WAVES * sk_stage_elements(3) * sizeof(bf16_t), strips, stream, args);
         default: return launch_persistent_per<4, false, false>(per, grid, SP_WAVES * sk_stage_elements(4) * sizeof(bf16_t), strips, stream, args);
     }
+}
+
+// ----------------------------------------------------------------------------
+// A linear of at most eight rows by the persistent kernel and, beside it, a router's choice of at most 64 outputs for as many tokens, by one workgroup
+// more than the linear has, a wave a token. A choice alone is a launch that waits for two trips to memory: eight rows, the shared expert's second
+// linear (2,048 by 2,816) and the choice of 32 outputs 5.9 + 4.5 -> 7.0 us. (Behind the router's own linear in one workgroup that does both it is
+// slower: one CU takes 11.4 us for 30 rows of 2,048 and the choice where two launches take 8.0.)
+// ----------------------------------------------------------------------------
+template <int PER>
+__global__ void __launch_bounds__(SP_WAVES * KA_WAVE)
+skinny_choice_kernel(SkinnyArgs p, int strips, int grid, RouteArgs job, int tokens) {
+    __shared__ RouteRoom<1> room[SP_WAVES];
+    if ((int)blockIdx.x < grid) {
+        skinny_persistent_body<PER, 1, true, false, 2, false>(p, strips, blockIdx.x, grid);
+        return;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    if (wave < tokens) ka_route_token<1>(job, wave, lane, room[wave]);
+}
+
+template <int PER>
+static void launch_choice(const SkinnyArgs& args, int strips, const RouteArgs& job, int tokens, hipStream_t stream) {
+    const int slots = sk_compute_units() * (PER <= 4 ? 2 : 1), grid = ka_cdiv(strips, ka_cdiv(strips, slots));      // (as launch_persistent)
+    hipLaunchKernelGGL((skinny_choice_kernel<PER>), dim3(grid + 1), dim3(SP_WAVES * KA_WAVE), 0, stream, args, strips, grid, job, tokens);
+}
+
+// out[M, N] = A[M, K] W^T + bias in fp32 (the numbers of ka_linear_skinny_bf16) and the choice of `tokens` tokens by `logits`, which the linear does not touch.
+// 1: not covered, nothing was run.
+KA_API int ka_linear_skinny_choice(const void* A, long lda, const void* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+                                   const float* logits, long stride, const float* correction, int tokens, int R, int top, int n_groups,
+                                   int keep, int group_best, float scale, int mode, int always, int* chosen, float* weights, hipStream_t stream) {
+    const char* who = "ka_linear_skinny_choice";
+    if (M < 1 || M > 8 || tokens < 1 || tokens > SP_WAVES || R > KA_WAVE || K < 8 || K % 8 || !sk_persistent_enabled) return 1;
+    SkinnyArgs args = {};
+    args.M = M;
+    args.K[0] = K;
+    args.a = SkinnyTarget{(const bf16_t*)W, ldw, bias, out, ldo, KA_F32, N, KA_ACT_NONE, 0};
+    if (check_target(who, args.a, K)) return -1;
+    KA_CHECK(A && lda % 8 == 0 && lda >= K && (uintptr_t)A % 16 == 0, "%s: input rows must be 16-byte aligned and >= K", who);
+    args.A[0] = (const bf16_t*)A;
+    args.lda[0] = lda;
+    const int kblocks = ka_cdiv(K, SK_KBLOCK), per = ka_cdiv(kblocks, SP_WAVES), strips = args.strips_a = ka_cdiv(N, SK_STRIP);
+    if (!persistent_fits(M, kblocks, args)) return 1;
+    const RouteArgs job{logits, stride, correction, R, top, n_groups, keep, group_best, mode, always, scale, chosen, weights};
+    if (ka_route_check(who, job, tokens)) return -1;
+    if (per <= 1) launch_choice<1>(args, strips, job, tokens, stream);
+    else if (per <= 2) launch_choice<2>(args, strips, job, tokens, stream);
+    else if (per <= 4) launch_choice<4>(args, strips, job, tokens, stream);
+    else if (per <= 5) launch_choice<5>(args, strips, job, tokens, stream);
+    else if (per <= 6) launch_choice<6>(args, strips, job, tokens, stream);
+    else launch_choice<8>(args, strips, job, tokens, stream);
+    KA_LAUNCH_CHECK();
+    return 0;
 }
 
 template <int MB, bool HALF>

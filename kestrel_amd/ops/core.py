@@ -1019,6 +1019,13 @@ def route(logits: torch.Tensor, n_outputs: int, correction: Optional[torch.Tenso
     over the chosen logits, times ``scale`` (no groups, no correction). ``scores`` ``"sigmoid"``: the scores are the logits' sigmoids.
     ``group_best`` 2: a group counts by the sum of its two largest choice scores. ``always``: ``chosen`` and ``weights`` are
     ``[n, top + 1]`` and end in that number with weight 1."""
+    _check(lib().ka_route(*route_args(logits, n_outputs, correction, top, n_groups, keep_groups, scale, chosen, weights, weigh_chosen, scores, group_best, always),
+                          stream_ptr()))
+
+
+def route_args(logits, n_outputs, correction, top, n_groups, keep_groups, scale, chosen, weights, weigh_chosen=False, scores="softmax", group_best=1,
+               always=None) -> tuple:
+    """The operands of ``route``, looked over, as its entry point takes them."""
     _dev(logits, correction, chosen, weights)
     _need(scores in ROUTER_SCORES and not (weigh_chosen and scores != "softmax"), f"route: unknown scores {scores!r}")
     columns = top + (always is not None)
@@ -1029,9 +1036,9 @@ def route(logits: torch.Tensor, n_outputs: int, correction: Optional[torch.Tenso
           "route: correction fp32 [outputs]")
     _need(chosen.dtype == torch.int32 and chosen.is_contiguous() and tuple(chosen.shape) == (n, columns) and weights.dtype == torch.float32
           and weights.is_contiguous() and tuple(weights.shape) == (n, columns), "route: chosen int32 and weights fp32 [n, top]")
-    _check(lib().ka_route(logits.data_ptr(), logits.stride(0) if n > 1 else logits.shape[1], _ptr(correction), n, int(n_outputs), int(top),
-                          int(n_groups), int(keep_groups), int(group_best), float(scale), 1 if weigh_chosen else ROUTER_SCORES[scores],
-                          -1 if always is None else int(always), chosen.data_ptr(), weights.data_ptr(), stream_ptr()))
+    return (logits.data_ptr(), logits.stride(0) if n > 1 else logits.shape[1], _ptr(correction), n, int(n_outputs), int(top), int(n_groups), int(keep_groups),
+            int(group_best), float(scale), 1 if weigh_chosen else ROUTER_SCORES[scores], -1 if always is None else int(always), chosen.data_ptr(),
+            weights.data_ptr())
 
 
 def experts_linear(a: torch.Tensor, per_token: int, weights: torch.Tensor, chosen: torch.Tensor, out: torch.Tensor, act: int = 0,

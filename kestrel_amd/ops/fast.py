@@ -20,6 +20,9 @@ _c_void_p, _c_int, _c_long, _c_float = ctypes.c_void_p, ctypes.c_int, ctypes.c_l
 _SIGNATURES = {
     "ka_linear_skinny_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
                               _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long, _c_void_p],
+    "ka_linear_skinny_choice": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int,       # the linear
+                                _c_void_p, _c_long, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p,
+                                _c_void_p, _c_void_p],                                                                                  # ka_route's
     "ka_linear_skinny_fused": [
         _c_void_p, _c_long, _c_int,                                   # A1, lda1, K1
         _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_void_p,    # A2, lda2, K2, W2, ldw2, bias2
@@ -107,6 +110,8 @@ _SIGNATURES = {
 
 # Rows up to which the weight-streaming kernel is used instead of the tiled one.
 SKINNY_MAX_ROWS = 64
+# Rows up to which a linear takes a router's choice along.
+SKINNY_CHOICE_ROWS = 8
 # Rows (and their width) up to which the weight-streaming kernel can normalise its input itself.
 SKINNY_LN_MAX_ROWS = 16
 SKINNY_LN_MAX_WIDTH = 4096
@@ -487,6 +492,21 @@ def linear_two_outputs(a, wa, ba, out_a, act_a, wb, bb, out_b, act_b) -> bool:
         wa.data_ptr(), wa.stride(0), _ptr(ba), out_a.data_ptr(), _OUT_CODE[out_a.dtype], out_a.stride(0), na, act_a, 0,
         wb.data_ptr(), wb.stride(0), _ptr(bb), out_b.data_ptr(), _OUT_CODE[out_b.dtype], out_b.stride(0), nb, act_b,
         m, chip_sizes(a.device).skinny_target_waves, *_wide_args(a.device, m), stream_ptr()))
+    return True
+
+
+def linear_choice(a, weight, bias, out, *choice, **options) -> bool:
+    """``out = a @ weight.T + bias`` (fp32, few rows) and ``core.route(*choice, **options)`` beside one another in one launch
+    (the linear is not the router's). False: not covered (more than eight rows, more than 64 router outputs, long rows), nothing was run."""
+    m, k = a.shape
+    if not 0 < m <= SKINNY_CHOICE_ROWS or out.dtype != torch.float32 or k % 8 or not (_operand_ok(a, k) and _operand_ok(weight, k)
+                                                                                     and _out_ok(out, m, weight.shape[0]) and _bias_ok(bias, weight.shape[0])):
+        return False
+    status = lib().ka_linear_skinny_choice(a.data_ptr(), a.stride(0), weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), out.stride(0), m,
+                                           weight.shape[0], k, *core.route_args(*choice, **options), stream_ptr())
+    if status > 0:
+        return False
+    _check(status)
     return True
 
 

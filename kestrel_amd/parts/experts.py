@@ -131,8 +131,24 @@ class RoutedExperts(FeedForward):
             return ws.get("experts.shared_sums", (n, 2 * spec.shared_hidden), self.dtype), 0
         return ws.get("experts.shared_hidden", (n, spec.shared_hidden), self.dtype), self.act | (ACT_GATED if self.gated else 0)
 
+    def _shared_hidden(self, h, first, act, there: bool, ws):
+        """The shared expert's hidden rows (``first`` and ``act``: ``_shared_operands``; ``there``: its first linear has run)."""
+        spec = self.spec
+        if not there:
+            linear(h, self.shared_pairs, None, first, act=act)
+        if not self.gated or act & ACT_GATED:
+            return first
+        hidden = ws.get("experts.shared_hidden", (h.shape[0], spec.shared_hidden), self.dtype)       # (`first` holds the pairs' sums)
+        if self.shared_clamp is not None:
+            core.clamped_pairs(first, hidden, self.shared_clamp.limit, self.shared_clamp.slope, self.shared_clamp.shift)
+        else:
+            core.gated_pairs(first, hidden, self.act)
+        return hidden
+
     def _outputs(self, h, batch):
         """Everything but the weighted sum: the pairs' outputs, the choice, its weights, the shared expert's output and gate."""
+        from ..ops import fast
+
         spec = self.spec
         n = h.shape[0]
         ws = batch.workspace
@@ -143,20 +159,28 @@ class RoutedExperts(FeedForward):
         # (eight rows of 2,048: about 5 us a layer, 3 % of a step).
         beside = False
         if shared is not None and self.dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16:
-            from ..ops import fast
             beside = fast.linear_two_outputs(h, self.router, self.router_bias, logits, 0, self.shared_pairs, None, *shared)
-        if not beside:
-            linear(h, self.router, self.router_bias, logits)
         chosen = ws.get("experts.chosen", (n, top), torch.int32)
         weights = ws.get("experts.weights", (n, top), torch.float32)
-        core.route(logits, self.n_outputs, self.correction, spec.top, spec.n_groups, spec.keep_groups, spec.scale, chosen, weights,
-                   weigh_chosen=self.weigh_chosen, scores=self.scores, group_best=self.group_best,
-                   always=spec.n_experts if self.joined else None)
+        choice = (logits, self.n_outputs, self.correction, spec.top, spec.n_groups, spec.keep_groups, spec.scale, chosen, weights)
+        options = dict(weigh_chosen=self.weigh_chosen, scores=self.scores, group_best=self.group_best, always=spec.n_experts if self.joined else None)
+        if not beside:
+            linear(h, self.router, self.router_bias, logits)
+        # The choice, a launch that waits for memory on a wave a token, goes beside the shared expert's second linear where rows are few
+        # (eight rows of 2,048: 4 us a layer, 2 % of a step).
+        routed, shared_out = False, None
+        if shared is not None and self.dtype == torch.bfloat16 and n <= fast.SKINNY_CHOICE_ROWS:
+            shared_hidden = self._shared_hidden(h, *shared, beside, ws)
+            shared_out = ws.get("experts.shared_out", (n, spec.dim), torch.float32)
+            routed = fast.linear_choice(shared_hidden, self.shared_down, None, shared_out, *choice, **options)
+            if not routed:
+                linear(shared_hidden, self.shared_down, None, shared_out)
+        if not routed:
+            core.route(*choice, **options)
         hidden = ws.get("experts.hidden", (n * top, spec.hidden_dim), self.dtype)
         y = ws.get("experts.y", (n * top, spec.dim), torch.float32)
         done = False
         if self.dtype == torch.bfloat16 and n * top > self.PAIR_BY_PAIR_TO:
-            from ..ops import fast
             operands = (h, self.pairs, self.down, chosen, hidden, y, self.up_act)
             few_to = self.FEW_PAIRS_TO if spec.dim % 64 == 0 and spec.hidden_dim % 64 == 0 else self.FEW_PAIRS_TO_UNALIGNED
             done = n * top <= few_to and fast.experts_few_bf16(*operands, clamp=self.clamp)
@@ -165,20 +189,12 @@ class RoutedExperts(FeedForward):
             flat = chosen.view(-1)
             core.experts_linear(h, top, self.pairs, flat, hidden, self.up_act, clamp=self.clamp)
             core.experts_linear(hidden, 1, self.down, flat, y)
-        shared_out = gate = None
-        if self.shared and not self.joined:
-            first, act = shared
-            if not beside:
-                linear(h, self.shared_pairs, None, first, act=act)
-            shared_hidden = first
-            if self.gated and not act & ACT_GATED:           # (the pairs' sums)
-                shared_hidden = ws.get("experts.shared_hidden", (n, spec.shared_hidden), self.dtype)
-                if self.shared_clamp is not None:
-                    core.clamped_pairs(first, shared_hidden, self.shared_clamp.limit, self.shared_clamp.slope, self.shared_clamp.shift)
-                else:
-                    core.gated_pairs(first, shared_hidden, self.act)
-            shared_out = ws.get("experts.shared_out", (n, spec.dim), torch.float32)
-            linear(shared_hidden, self.shared_down, None, shared_out)
+        gate = None
+        if shared is not None:
+            if shared_out is None:
+                shared_hidden = self._shared_hidden(h, *shared, beside, ws)
+                shared_out = ws.get("experts.shared_out", (n, spec.dim), torch.float32)
+                linear(shared_hidden, self.shared_down, None, shared_out)
             if self.gated_shared:
                 gate = logits[:, self.n_outputs]
         return y, chosen, weights, shared_out, gate
