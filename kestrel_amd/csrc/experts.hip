@@ -66,7 +66,43 @@ __device__ __forceinline__ void ex_dots(const T* const (&w)[R], const float* __r
     for (int r = 0; r < R; ++r) y[r] = ka_wave_sum(acc[r]);
 }
 
-template <typename T>
+// The same for bf16 rows of at most AHEAD times 512: all that a wave reads of R rows is on its way at once and before the input row has been staged, one
+// trip to memory in place of up to eight. Which lane adds what in which order is as above. First and second linear, us, the loop above and this:
+// experts of 4,096 x 896, 6 pairs 24.9 + 12.2 and 21.6 + 9.6, 18 pairs 51.8 + 29.7 and 47.8 + 21.4; 2,048 x 704, 5 pairs 9.3 + 5.3 and 9.4 + 5.4,
+// 10 pairs 14.6 + 8.6 and 12.4 + 7.2, 20 pairs 24.3 + 14.7 and 21.5 + 11.8. R: four rows of up to 4,096 are 128 registers; eight rows of 2,048, as many
+// registers, are behind four of them twice (10 pairs 14.3 against 12.4).
+typedef __attribute__((ext_vector_type(8))) bf16_t ex_bf16x8;
+template <int R, int AHEAD>
+struct ExRows {
+    ex_bf16x8 x[AHEAD][R];
+    __device__ __forceinline__ void fetch(const bf16_t* const (&w)[R], int K, int lane) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[i][r] = __builtin_nontemporal_load(reinterpret_cast<const ex_bf16x8*>(w[r] + min((i * KA_WAVE + lane) * 8, K - 8)));
+    }
+    __device__ __forceinline__ void dots(const float* __restrict__ a, int K, int lane, float (&y)[R]) const {
+        float acc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = 0.f;
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int c = (i * KA_WAVE + lane) * 8;
+            if (c >= K) continue;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float h = a[c + e];
+#pragma unroll
+                for (int r = 0; r < R; ++r) acc[r] = fmaf(ka_to_float(x[i][r][e]), h, acc[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) y[r] = ka_wave_sum(acc[r]);
+    }
+};
+
+// AHEAD 0: any K, alignment and type; else bf16 rows in whole pieces of eight, at most 512 AHEAD of them.
+template <typename T, int AHEAD>
 __global__ void __launch_bounds__(256)
 experts_linear_kernel(const T* __restrict__ a, long a_stride, int a_div, const T* __restrict__ W, const int* __restrict__ chosen,
                       int E, int N, int K, int act, KaGateClamp clamp, void* __restrict__ out, long out_stride, int out_f32) {
@@ -75,8 +111,6 @@ experts_linear_kernel(const T* __restrict__ a, long a_stride, int a_div, const T
     const int e = chosen[p];
     if (e < 0 || e >= E) return;
     const T* ap = a + (size_t)(p / a_div) * a_stride;
-    for (int c = threadIdx.x; c < K; c += blockDim.x) row[c] = ka_to_float(ap[c]);
-    __syncthreads();
     const int wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
     const bool gated = ka_act_gated(act);
     const int n_out = gated ? N / 2 : N;
@@ -84,28 +118,66 @@ experts_linear_kernel(const T* __restrict__ a, long a_stride, int a_div, const T
     const bool vectors = K % (16 / sizeof(T)) == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
     constexpr int ROWS = EX_COLS / 4;           // outputs of a wave: four neighbours, or (gated) two pairs at a time
     const int j0 = blockIdx.x * EX_COLS + wave * ROWS;
-    if (j0 >= n_out) return;
     float y[ROWS];
-    if (gated) {
+    if constexpr (AHEAD > 0) {
+        // (rows past the end: not stored)
+        constexpr int R = AHEAD <= 2 ? 2 * ROWS : ROWS;
+        auto stage = [&]() {
+            for (int c = threadIdx.x * 8; c < K; c += blockDim.x * 8) {
+                const ex_bf16x8 v = *reinterpret_cast<const ex_bf16x8*>(ap + c);
 #pragma unroll
-        for (int q = 0; q < ROWS; q += 2) {
-            const T* w[4];
+                for (int i = 0; i < 8; ++i) row[c + i] = ka_to_float(v[i]);
+            }
+            __syncthreads();
+        };
+        if (gated) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[r] = We + (size_t)min(2 * (j0 + q) + r, N - 1) * K;     // (rows past the end: not stored)
-            float s[4];
-            ex_dots<T, 4>(w, row, K, lane, vectors, s);
-            y[q] = ka_gate_product<false>(act, clamp, s[0], s[1]);
-            y[q + 1] = ka_gate_product<false>(act, clamp, s[2], s[3]);
+            for (int q = 0; q < ROWS; q += R / 2) {
+                const T* w[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) w[r] = We + (size_t)min(2 * (j0 + q) + r, N - 1) * K;
+                ExRows<R, AHEAD> rows;
+                rows.fetch(w, K, lane);
+                if (q == 0) stage();
+                float s[R];
+                rows.dots(row, K, lane, s);
+#pragma unroll
+                for (int r = 0; r < R; r += 2) y[q + r / 2] = ka_gate_product<false>(act, clamp, s[r], s[r + 1]);
+            }
+        } else {
+            const T* w[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) w[r] = We + (size_t)min(j0 + r, N - 1) * K;
+            ExRows<ROWS, AHEAD> rows;
+            rows.fetch(w, K, lane);
+            stage();
+            rows.dots(row, K, lane, y);
         }
     } else {
-        const T* w[ROWS];
+        for (int c = threadIdx.x; c < K; c += blockDim.x) row[c] = ka_to_float(ap[c]);
+        __syncthreads();
+        if (j0 >= n_out) return;
+        if (gated) {
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) w[r] = We + (size_t)min(j0 + r, N - 1) * K;
-        ex_dots<T, ROWS>(w, row, K, lane, vectors, y);
+            for (int q = 0; q < ROWS; q += 2) {
+                const T* w[4];
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r)
-            if (ka_act_base(act)) y[r] = ka_activate(act, y[r]);
+                for (int r = 0; r < 4; ++r) w[r] = We + (size_t)min(2 * (j0 + q) + r, N - 1) * K;     // (rows past the end: not stored)
+                float s[4];
+                ex_dots<T, 4>(w, row, K, lane, vectors, s);
+                y[q] = ka_gate_product<false>(act, clamp, s[0], s[1]);
+                y[q + 1] = ka_gate_product<false>(act, clamp, s[2], s[3]);
+            }
+        } else {
+            const T* w[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) w[r] = We + (size_t)min(j0 + r, N - 1) * K;
+            ex_dots<T, ROWS>(w, row, K, lane, vectors, y);
+        }
     }
+    if (!gated && ka_act_base(act))
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) y[r] = ka_activate(act, y[r]);
     if (lane == 0) {
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
@@ -131,12 +203,18 @@ KA_API int ka_experts_linear(const void* a, long a_stride, int a_div, const void
     if (n_pairs == 0) return 0;
     dim3 grid((ka_act_outputs(act, N) + EX_COLS - 1) / EX_COLS, n_pairs);
     const size_t lds = (size_t)K * sizeof(float);
-    if (dtype == KA_F32)
-        hipLaunchKernelGGL(experts_linear_kernel<float>, grid, dim3(256), lds, stream, (const float*)a, a_stride, a_div, (const float*)W,
-                           chosen, E, N, K, act, clamp, out, out_stride, out_f32);
-    else
-        hipLaunchKernelGGL(experts_linear_kernel<bf16_t>, grid, dim3(256), lds, stream, (const bf16_t*)a, a_stride, a_div, (const bf16_t*)W,
-                           chosen, E, N, K, act, clamp, out, out_stride, out_f32);
+    const bool pieces = K % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)W) % 16 == 0;
+#define EX_LINEAR(T, AHEAD)                                                                                                                    \
+    hipLaunchKernelGGL((experts_linear_kernel<T, AHEAD>), grid, dim3(256), lds, stream, (const T*)a, a_stride, a_div, (const T*)W, chosen, E, N, K, act, clamp, \
+                       out, out_stride, out_f32)
+    // As few pieces ahead as the rows have (one past the end is a load for nothing). Rows of up to 512 are one trip either way, and the plain loop is
+    // ahead (8 pairs' second linear of 512 to 1,024: 2.9 and 3.7 us).
+    if (dtype == KA_F32) EX_LINEAR(float, 0);
+    else if (pieces && K > 512 && K <= 1024) EX_LINEAR(bf16_t, 2);
+    else if (pieces && K > 1024 && K <= 2048) EX_LINEAR(bf16_t, 4);
+    else if (pieces && K > 2048 && K <= 4096) EX_LINEAR(bf16_t, 8);
+    else EX_LINEAR(bf16_t, 0);
+#undef EX_LINEAR
     KA_LAUNCH_CHECK();
     return 0;
 }
