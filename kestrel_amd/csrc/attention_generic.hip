@@ -164,9 +164,9 @@ attention_generic_kernel(const T* __restrict__ q, long q_row_stride, const T* __
 // G = 16, 32 or 64 lanes share a key (a row is one load's piece), 16 keys each; a lane's sixteen partial scores are added up across its row of 16
 // lanes so that each lane ends with one key's (fifteen lane moves for 16 keys); values come as four neighbouring keys of one channel, whole
 // pieces of a page, asked for together with the keys; and NW waves take the chunks of CK keys in turn and meet in LDS at the end.
-// 32 heads of 64, us, there and here: 3 tokens behind 31 to 160 keys 17.5 and 7.1, 8 behind 1,040 88 and 25 (5.4 TB/s), 64 behind 400 111 and 79 (5.3
-// TB/s), three prompts of 31 to 157 66 and 31, a prompt of 400 225 and 72, of 2,048 5,406 and 1,197; heads of 128: 8 behind 1,040 174 and 42, a prompt
-// of 400 453 and 108. Errors against 64 bits are no larger: a score is the sum of sixteen or more partial ones instead of one chain.
+// 32 heads of 64, us, there and here: 3 tokens behind 160 keys 14.3 and 5.5, 6 behind 400 36.9 and 11.8, 64 behind 400 111 and 78 (5.4 TB/s); prompts of
+// 17 5.6 and 5.3, three of 64 36 and 13, six of 20 8.5 and 10.3, one of 200 68 and 25, of 2,048 5,406 and 1,197; heads of 128: 6 behind 400 66 and 17, a prompt
+// of 400 453 and 102. Errors against 64 bits are no larger: a score is the sum of sixteen or more partial ones instead of one chain.
 // ----------------------------------------------------------------------------
 struct SpreadArgs {
     const float* q;
@@ -339,10 +339,10 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
 
 template <int G>
 static void launch_spread(const SpreadArgs& g, int n, hipStream_t stream) {
-    // (waves that a token's keys are cut over, by what fills the chip: a wave holds some 160 registers, three a SIMD)
-    const long heads = (long)n * g.H, cus = ka_compute_units();
-    if (heads <= 4 * cus) hipLaunchKernelGGL((attention_spread_kernel<G, 8>), dim3(n, g.H), dim3(8 * KA_WAVE), 0, stream, g);
-    else if (heads <= 16 * cus) hipLaunchKernelGGL((attention_spread_kernel<G, 4>), dim3(n, g.H), dim3(4 * KA_WAVE), 0, stream, g);
+    // A token's keys over four waves where workgroups of four are two a CU at the most: 3 tokens behind 160 keys 5.5 us (one wave 8.1, eight 5.8), 16 behind
+    // 200 12.2 (15.4, 15.2), but 32 behind 64 9.7 (6.7, 17.3) and a prompt of 33 9.3 (6.1, 19.4). Only rows of a thousand keys gain by eight (6 tokens 18.1
+    // against 20.2).
+    if ((long)n * g.H <= 2L * ka_compute_units()) hipLaunchKernelGGL((attention_spread_kernel<G, 4>), dim3(n, g.H), dim3(4 * KA_WAVE), 0, stream, g);
     else hipLaunchKernelGGL((attention_spread_kernel<G, 1>), dim3(n, g.H), dim3(KA_WAVE), 0, stream, g);
 }
 
