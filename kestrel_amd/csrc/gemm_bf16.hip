@@ -526,6 +526,10 @@ static int launch_few_rows(const KaFewRows& f, hipStream_t stream) {
 int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
     if (f.M < 1 || f.M > 64 || f.K[0] % 64 || f.K[1] % 64 || f.K[0] < 64 || f.parts < 1 || !f.partial) return 0;
     const bool large = ka_cdiv(f.N, 64) > 3 * ka_compute_units();
+    // Up to 32 rows tiles of 32, which ask for half the activations, six stages in the same LDS (us, 64 rows a tile and 32, at 24 rows: 12,288 by 4,096
+    // 28.3 and 25.4, 18,944 47.0 and 44.7, 2,560 by 2,560 + 10,240 19.3 and 18.2, 2,048 by 2,048 + 8,192 14.6 and 14.1); not the tiles of 128 weight rows
+    // (51,200 by 4,096 92 and 95). Eight or twelve stages where a CU has one workgroup: 2 to 8 % slower at any number of rows.
+    if (f.M <= 32 && !large) return launch_few_rows<2, 1, 2, 2, 6>(f, stream) ? -1 : 1;
     return (large ? launch_few_rows<4, 2, 2, 2, 3>(f, stream) : launch_few_rows<2, 2, 2, 2, 5>(f, stream)) ? -1 : 1;
 }
 
