@@ -34,7 +34,6 @@ LIBRARIES: Dict[str, List[str]] = {
     "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_phased_bf16.hip", "gemv_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
              "gemm_library.hip"],
 }
-HEADERS = ["ka_common.h", "ka_partials.h", "ka_no_alloc.h", "ka_attention_decode.h", "ka_skinny.h", "ka_rows.h", "ka_decay.h", "ka_listed_tiles.h", "ka_dma_tiles.h", "ka_phased_tiles.h", "ka_conv_wide.h", "ka_gated_step.h"]
 
 # Libraries of the ROCm installation that a library of ours is linked against.
 LINK_LIBRARIES: Dict[str, List[str]] = {"fast": ["hipblaslt"]}
@@ -62,10 +61,10 @@ def _sources(name: str) -> List[Path]:
 
 
 def source_stamp(name: str) -> str:
-    """Hash of the sources, headers and flags a library is built from."""
+    """Hash of the sources, headers (all of the folder: none can be left out) and flags a library is built from."""
     digest = hashlib.sha256()
     digest.update(" ".join(HIPCC_FLAGS + LINK_LIBRARIES.get(name, [])).encode())
-    for path in [SOURCE_DIR / h for h in HEADERS] + _sources(name):
+    for path in sorted(SOURCE_DIR.glob("*.h")) + _sources(name):
         digest.update(path.name.encode())
         digest.update(path.read_bytes())
     return digest.hexdigest()[:16]

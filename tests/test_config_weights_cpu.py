@@ -272,3 +272,29 @@ def test_a_stale_library_that_cannot_be_rebuilt_is_an_error(tmp_path, monkeypatc
     monkeypatch.setattr(build, "_find_built", lambda name: (None, False))
     with pytest.raises(build.KernelBuildError, match="hipcc not found"):
         build.load("core")
+
+
+@pytest.mark.parametrize("name", ["core", "fast"])
+def test_a_library_is_stale_after_a_change_to_any_file_it_is_built_from(name, tmp_path, monkeypatch):
+    """Sources and everything they include by name, however deep, count for the stamp."""
+    import re
+    import shutil
+
+    from kestrel_amd.csrc import build
+
+    for path in build.SOURCE_DIR.iterdir():
+        if path.suffix in (".hip", ".h"):
+            shutil.copy(path, tmp_path)
+    monkeypatch.setattr(build, "SOURCE_DIR", tmp_path)
+    files, queue = set(), list(build.LIBRARIES[name])
+    while queue:
+        file = queue.pop()
+        if file not in files:
+            files.add(file)
+            queue += re.findall(r'^\s*#\s*include\s+"([^"]+)"', (tmp_path / file).read_text(), re.M)
+    assert "ka_common.h" in files
+    for file in sorted(files):
+        before, text = build.source_stamp(name), (tmp_path / file).read_text()
+        (tmp_path / file).write_text(text + "\n")
+        assert build.source_stamp(name) != before, f"{file} does not count"
+        (tmp_path / file).write_text(text)
