@@ -163,10 +163,14 @@ attention_generic_kernel(const T* __restrict__ q, long q_row_stride, const T* __
 // back to each of them for every four channels, and the values are asked for when the scores are known; one wave walks all keys. Here
 // G = 16, 32 or 64 lanes share a key (a row is one load's piece), 16 keys each; a lane's sixteen partial scores are added up across its row of 16
 // lanes so that each lane ends with one key's (fifteen lane moves for 16 keys); values come as four neighbouring keys of one channel, whole
-// pieces of a page, asked for together with the keys; and NW waves take the chunks of CK keys in turn and meet in LDS at the end.
-// 32 heads of 64, us, there and here: 3 tokens behind 160 keys 14.3 and 5.5, 6 behind 400 36.9 and 11.8, 64 behind 400 111 and 78 (5.4 TB/s); prompts of
-// 17 5.6 and 5.3, three of 64 36 and 13, six of 20 8.5 and 10.3, one of 200 68 and 25, of 2,048 5,406 and 1,197; heads of 128: 6 behind 400 66 and 17, a prompt
-// of 400 453 and 102. Errors against 64 bits are no larger: a score is the sum of sixteen or more partial ones instead of one chain.
+// pieces of a page, asked for together with the keys. A token's chunks of CK keys are dealt out to AS_PARTS parts, which meet in LDS at the end; a wave takes
+// one part or all of them one behind the other, and the sums are the same: a token's numbers do not depend on the tokens beside it.
+// 32 heads of 64, eight layers' caches in turn, us, there and here: 3 tokens behind 160 keys 17.3 and 6.6, 6 behind 400 46 and 13.7, 64 behind 400 106 and 74
+// (5.7 TB/s); prompts of 17 5.6 and 5.2, six of 20 10.6 and 9.2, three of 64 32 and 13, one of 200 67 and 24, of 2,048 5,373 and 1,078; heads of 128: 6 behind
+// 400 85 and 20, a prompt of 400 454 and 101. (All chunks in one sequence where a wave takes a token alone: 137 registers instead of 126 with heads of 64, a wave
+// less a SIMD, six of 20 12.6, three of 64 15.6; heads of 128 up to 5 % faster, a prompt of 200 35.4 against 37.3. Places behind the last key left out of the
+// loads: 172 registers, six of 20 10.2, three of 64 17.4.) Errors against 64 bits are no larger: a score is the sum of sixteen or more
+// partial ones instead of one chain.
 // ----------------------------------------------------------------------------
 struct SpreadArgs {
     const float* q;
@@ -218,13 +222,16 @@ __device__ __forceinline__ void as_scatter_sums(float (&v)[16], int lane) {
     }
 }
 
+constexpr int AS_PARTS = 4;
+
+// NW waves take the parts in turn: the sums of a token are the same whatever NW is.
 template <int G, int NW>
 __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadArgs g) {
     constexpr int GROUPS = KA_WAVE / G, CK = 16 * GROUPS, R = G / 4;         // groups of 16 keys in a chunk of CK; channels in sixteens
     __shared__ long k_at[NW][CK], v_at[NW][CK];
     __shared__ __attribute__((aligned(16))) float ps[NW][CK];
-    __shared__ float sums[NW][R * 16], tops[NW], totals[NW];
-    const int t = blockIdx.x, h = blockIdx.y, wave = threadIdx.x / KA_WAVE, lane = threadIdx.x % KA_WAVE;
+    __shared__ float sums[AS_PARTS][R * 16], tops[AS_PARTS], totals[AS_PARTS];
+    const int t = blockIdx.x, h = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
     const int vh = h / g.maps / (g.H / g.Hkv), kvh = vh * g.maps + h % g.maps, Hv = g.Hkv / g.maps;
     const int lo = g.kv_lo ? g.kv_lo[t] : 0, hi = g.kv_hi[t];
     const int* bt = g.block_table + (size_t)g.token_row[t] * g.max_pages;
@@ -240,89 +247,93 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
     const int place = (g.slopes || g.bias_table) ? g.positions[t] : 0;
     const float* bias_row = g.bias_table ? g.bias_table + (size_t)h * g.bias_len : nullptr;
     const float sink = g.sinks ? g.sinks[h] : g.sink_score;
-    const bool sinks_here = g.has_sink && wave == 0;
-    float m = sinks_here ? sink : -INFINITY, l = sinks_here ? 1.f : 0.f;
-    float o[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) o[r] = 0.f;
 
-    // chunks of the kept first keys, then of the window's, whose first chunk starts on a multiple of four keys
+    // chunks of the kept first keys, then of the window's, whose first chunk starts on a multiple of four keys; part p has every AS_PARTS-th from chunk p on
     const int kept = min(g.keep_first, lo), kept_chunks = kept > 0 ? (kept + CK - 1) / CK : 0;
     const int start = lo & ~3, chunks = kept_chunks + (hi > lo ? (hi - start + CK - 1) / CK : 0);
-    for (int c = wave; c < chunks; c += NW) {
-        const bool first = c < kept_chunks;
-        const int base = first ? c * CK : start + (c - kept_chunks) * CK, from = first ? 0 : lo, to = first ? kept : hi;
-        const int key = base + group * 16 + lane % 16;
-        const bool valid = key >= from && key < to;
-        {
-            const int near = min(max(key, from), to - 1), page = bt[near / g.page_size], at = near % g.page_size;
-            as_wave_sync();                              // the chunk before has been read
-            if (owns) {
-                k_at[wave][group * 16 + in_row] = (((long)page * g.Hkv + kvh) * g.page_size + at) * g.hd;
-                v_at[wave][group * 16 + in_row] = ((long)page * Hv + vh) * g.hdv * g.page_size + (at & ~3);
-            }
-            as_wave_sync();
-        }
-        as_floatx4 k4[16], v4[GROUPS][R];
-        const int channel = min(in_row * 4, g.hd - 4);
+    const int parts = max(1, min(AS_PARTS, chunks));     // (the first one also without a key, for the sink)
+    for (int part = wave; part < parts; part += NW) {
+        const bool sinks_here = g.has_sink && part == 0;
+        float m = sinks_here ? sink : -INFINITY, l = sinks_here ? 1.f : 0.f;
+        float o[R];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) k4[i] = *reinterpret_cast<const as_floatx4*>(g.k_cache + k_at[wave][group * 16 + i] + channel);
-#pragma unroll
-        for (int x = 0; x < GROUPS; ++x) {
-            const float* vp = g.v_cache + v_at[wave][x * 16 + lane % 4 * 4];
-#pragma unroll
-            for (int r = 0; r < R; ++r) v4[x][r] = *reinterpret_cast<const as_floatx4*>(vp + (long)min(r * 16 + lane / 4, g.hdv - 1) * g.page_size);
-        }
-        float part[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) part[i] = fmaf(q4[3], k4[i][3], fmaf(q4[2], k4[i][2], fmaf(q4[1], k4[i][1], q4[0] * k4[i][0])));
-        as_scatter_sums<8>(part, lane);
-        float s = ka_lanes_reduce<16, G>(part[0], KaSum{});
-        if (g.softcap > 0.f) s = g.softcap * tanhf(s / g.softcap);
-        if (g.slopes) s -= slope * (float)(place - key);
-        if (bias_row) s += bias_row[min(max(place - key, 0), g.bias_len - 1)];
-        if (!valid) s = -INFINITY;
-        const float m_new = fmaxf(m, ka_wave_max(s));
-        const float corr = m == m_new ? 1.f : expf(m - m_new);
-        const float p = valid ? expf(s - m_new) : 0.f;
-        l = l * corr + ka_wave_sum(owns ? p : 0.f);
-        m = m_new;
-        if (owns) ps[wave][group * 16 + in_row] = p;
-        as_wave_sync();
-        const bool whole = base >= from && base + CK <= to;
-#pragma unroll
-        for (int r = 0; r < R; ++r) o[r] *= corr;
-#pragma unroll
-        for (int x = 0; x < GROUPS; ++x) {
-            const int j = x * 16 + lane % 4 * 4;
-            const as_floatx4 p4 = *reinterpret_cast<const as_floatx4*>(&ps[wave][j]);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                as_floatx4 v = v4[x][r];
-                if (!whole) {                            // (a place without a key may hold anything)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = base + j + i >= from && base + j + i < to ? v[i] : 0.f;
+        for (int r = 0; r < R; ++r) o[r] = 0.f;
+        for (int c = part; c < chunks; c += AS_PARTS) {
+            const bool first = c < kept_chunks;
+            const int base = first ? c * CK : start + (c - kept_chunks) * CK, from = first ? 0 : lo, to = first ? kept : hi;
+            const int key = base + group * 16 + lane % 16;
+            const bool valid = key >= from && key < to;
+            {
+                const int near = min(max(key, from), to - 1), page = bt[near / g.page_size], at = near % g.page_size;
+                as_wave_sync();                          // the chunk before has been read
+                if (owns) {
+                    k_at[wave][group * 16 + in_row] = (((long)page * g.Hkv + kvh) * g.page_size + at) * g.hd;
+                    v_at[wave][group * 16 + in_row] = ((long)page * Hv + vh) * g.hdv * g.page_size + (at & ~3);
                 }
-                o[r] += fmaf(p4[3], v[3], fmaf(p4[2], v[2], fmaf(p4[1], v[1], p4[0] * v[0])));
+                as_wave_sync();
+            }
+            as_floatx4 k4[16], v4[GROUPS][R];
+            const int channel = min(in_row * 4, g.hd - 4);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) k4[i] = *reinterpret_cast<const as_floatx4*>(g.k_cache + k_at[wave][group * 16 + i] + channel);
+#pragma unroll
+            for (int x = 0; x < GROUPS; ++x) {
+                const float* vp = g.v_cache + v_at[wave][x * 16 + lane % 4 * 4];
+#pragma unroll
+                for (int r = 0; r < R; ++r) v4[x][r] = *reinterpret_cast<const as_floatx4*>(vp + (long)min(r * 16 + lane / 4, g.hdv - 1) * g.page_size);
+            }
+            float part_s[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) part_s[i] = fmaf(q4[3], k4[i][3], fmaf(q4[2], k4[i][2], fmaf(q4[1], k4[i][1], q4[0] * k4[i][0])));
+            as_scatter_sums<8>(part_s, lane);
+            float s = ka_lanes_reduce<16, G>(part_s[0], KaSum{});
+            if (g.softcap > 0.f) s = g.softcap * tanhf(s / g.softcap);
+            if (g.slopes) s -= slope * (float)(place - key);
+            if (bias_row) s += bias_row[min(max(place - key, 0), g.bias_len - 1)];
+            if (!valid) s = -INFINITY;
+            const float m_new = fmaxf(m, ka_wave_max(s));
+            const float corr = m == m_new ? 1.f : expf(m - m_new);
+            const float p = valid ? expf(s - m_new) : 0.f;
+            l = l * corr + ka_wave_sum(owns ? p : 0.f);
+            m = m_new;
+            if (owns) ps[wave][group * 16 + in_row] = p;
+            as_wave_sync();
+            const bool whole = base >= from && base + CK <= to;
+#pragma unroll
+            for (int r = 0; r < R; ++r) o[r] *= corr;
+#pragma unroll
+            for (int x = 0; x < GROUPS; ++x) {
+                const int j = x * 16 + lane % 4 * 4;
+                const as_floatx4 p4 = *reinterpret_cast<const as_floatx4*>(&ps[wave][j]);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    as_floatx4 v = v4[x][r];
+                    if (!whole) {                        // (a place without a key may hold anything)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = base + j + i >= from && base + j + i < to ? v[i] : 0.f;
+                    }
+                    o[r] += fmaf(p4[3], v[3], fmaf(p4[2], v[2], fmaf(p4[1], v[1], p4[0] * v[0])));
+                }
             }
         }
-    }
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float y = ka_lanes_reduce<1, 4>(o[r], KaSum{});
-        if (lane % 4 == 0) sums[wave][r * 16 + lane / 4] = y;
-    }
-    if (lane == 0) {
-        tops[wave] = m;
-        totals[wave] = l;
+        for (int r = 0; r < R; ++r) {
+            const float y = ka_lanes_reduce<1, 4>(o[r], KaSum{});
+            if (lane % 4 == 0) sums[part][r * 16 + lane / 4] = y;
+        }
+        if (lane == 0) {
+            tops[part] = m;
+            totals[part] = l;
+        }
     }
     __syncthreads();
-    float top = -INFINITY, total = 0.f, share[NW];
+    float top = -INFINITY, total = 0.f, share[AS_PARTS];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) top = fmaxf(top, tops[w]);
+    for (int w = 0; w < AS_PARTS; ++w) top = w < parts ? fmaxf(top, tops[w]) : top;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        share[w] = tops[w] == top ? 1.f : expf(tops[w] - top);           // (a wave without a key: exp(-inf), or nothing at all)
+    for (int w = 0; w < AS_PARTS; ++w) {
+        if (w >= parts) break;
+        share[w] = tops[w] == top ? 1.f : expf(tops[w] - top);           // (a part without a key: exp(-inf), or nothing at all)
         total += totals[w] * share[w];
     }
     const float inv = total > 0.f ? 1.0f / total : 0.f;
@@ -330,7 +341,10 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
     for (int d = threadIdx.x; d < g.hdv; d += KA_WAVE * NW) {
         float y = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) y += sums[w][d] * share[w];
+        for (int w = 0; w < AS_PARTS; ++w) {
+            if (w >= parts) break;
+            y += sums[w][d] * share[w];
+        }
         y *= inv * head_gate;
         if (g.gate && !g.gate_per_head) y *= 1.0f / (1.0f + expf(-g.gate[(size_t)t * g.gate_row_stride + (size_t)h * g.hdv + d]));
         g.out[(size_t)t * g.out_row_stride + (size_t)h * g.hdv + d] = y;
@@ -339,10 +353,10 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
 
 template <int G>
 static void launch_spread(const SpreadArgs& g, int n, hipStream_t stream) {
-    // A token's keys over four waves where workgroups of four are two a CU at the most: 3 tokens behind 160 keys 5.5 us (one wave 8.1, eight 5.8), 16 behind
-    // 200 12.2 (15.4, 15.2), but 32 behind 64 9.7 (6.7, 17.3) and a prompt of 33 9.3 (6.1, 19.4). Only rows of a thousand keys gain by eight (6 tokens 18.1
-    // against 20.2).
-    if ((long)n * g.H <= 2L * ka_compute_units()) hipLaunchKernelGGL((attention_spread_kernel<G, 4>), dim3(n, g.H), dim3(4 * KA_WAVE), 0, stream, g);
+    // A wave a part where workgroups of four waves are two a CU at the most, else one wave for all: heads of 64, us, four waves and one: 3 tokens behind 160
+    // keys 6.5 and 8.7, 16 behind 200 14.2 and 17.3, but 32 behind 64 8.9 and 8.6, a prompt of 33 9.4 and 6.4, six of 20 21 and 9.3. Long rows
+    // of many tokens do not care (64 behind 400 76 and 74).
+    if ((long)n * g.H <= 2L * ka_compute_units()) hipLaunchKernelGGL((attention_spread_kernel<G, AS_PARTS>), dim3(n, g.H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
     else hipLaunchKernelGGL((attention_spread_kernel<G, 1>), dim3(n, g.H), dim3(KA_WAVE), 0, stream, g);
 }
 

@@ -141,3 +141,35 @@ def test_gated_linears_in_32_bits_do_not_depend_on_the_rows_beside(n, k):
     z = (a.double() @ w.double().T + bias.double()).view(40, n // 2, 2)
     want = z[..., 0] * torch.sigmoid(z[..., 0]) * z[..., 1]
     assert float((results[40].double() - want).norm() / want.norm()) < 2.0 ** -20
+
+
+# (of 32 heads 16 tokens are two workgroups a CU of 256, 17 are more)
+@pytest.mark.parametrize("hd, hdv, page", [(64, 64, 16), (128, 96, 12), (256, 200, 32)])
+@pytest.mark.parametrize("window", [False, True])
+def test_attention_in_32_bits_does_not_depend_on_the_tokens_beside(hd, hdv, page, window):
+    """A token's keys by one wave or by several: the numbers of a token are the same bits alone and in a step of any size."""
+    from kestrel_amd.ops import core
+
+    gen = torch.Generator().manual_seed(hd + window)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    n, heads, kv_heads, longest = 150, 32, 8, 700
+    pages = -(-longest // page)
+    table = torch.randperm(3 * pages, generator=gen).to(torch.int32).view(3, pages).to(DEV)
+    k_cache, v_cache = rnd(3 * pages, kv_heads, page, hd).to(DEV), rnd(3 * pages, kv_heads, hdv, page).to(DEV)
+    q, sinks = rnd(n, heads * hd).to(DEV), rnd(heads).to(DEV)
+    hi = torch.randint(1, longest + 1, (n,), generator=gen).to(torch.int32)
+    hi[:4] = torch.tensor([longest, 1, 64, 65])
+    row = torch.arange(n, dtype=torch.int32) % 3
+    lo = (hi - 300).clamp(min=0).to(DEV) if window else None
+    options = dict(value_dim=hdv, keep_first=5, sinks=sinks) if window else dict(value_dim=hdv)
+    hi, row = hi.to(DEV), row.to(DEV)
+
+    def results(a, b):
+        out = torch.full((b - a, heads * hdv), float("nan"), device=DEV)
+        core.attention_generic(q[a:b], k_cache, v_cache, table, row[a:b], lo[a:b] if window else None, hi[a:b], out, hd ** -0.5, heads, kv_heads, hd, **options)
+        return out
+
+    whole = results(0, n)
+    assert bool(torch.isfinite(whole).all())
+    for size in (1, 3, 16, 17, 75):
+        assert torch.equal(torch.cat([results(a, min(n, a + size)) for a in range(0, n, size)]), whole), f"steps of {size}"
