@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
             if (!valid) s = -INFINITY;
             const float m_new = fmaxf(m, ka_wave_max(s));
             const float corr = m == m_new ? 1.f : expf(m - m_new);
-            const float p = valid ? expf(s - m_new) : 0.f;
+            const float p = s == -INFINITY ? 0.f : expf(s - m_new);      // (a table may shut out all keys of a chunk: m_new is -inf as well)
             l = l * corr + ka_wave_sum(owns ? p : 0.f);
             m = m_new;
             if (owns) ps[wave][group * 16 + in_row] = p;

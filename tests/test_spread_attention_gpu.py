@@ -103,3 +103,39 @@ def test_spread_attention(n, heads, kv_heads, maps, hd, hdv, page, options):
     # scores of fp32 operands (a few units of 2^-24 times some 8), their exponentials and averages
     assert float((got - want).abs().max()) <= 2.0 ** -18 * max(1.0, float(want.abs().max()))
     assert float((got - want).norm() / want.norm()) < 2.0 ** -20
+
+
+# (chunks of 64, 32 and 16 keys: some hold nothing but keys that the table shuts out; tokens in four waves and in one)
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("n", [3, 40])
+def test_keys_that_a_table_shuts_out(hd, n):
+    from kestrel_amd.ops import core
+
+    gen = torch.Generator().manual_seed(n + hd)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    heads, page, longest = 32, 16, 200
+    pages = -(-longest // page)
+    keys, values, q = rnd(longest, heads, hd), rnd(longest, heads, hd), rnd(n, heads * hd)
+    whole = torch.zeros(2, pages * page, heads, hd)
+    whole[0, :longest], whole[1, :longest] = keys, values
+    k_cache = whole[0].view(pages, page, heads, hd).transpose(1, 2).contiguous()
+    v_cache = whole[1].view(pages, page, heads, hd).permute(0, 2, 3, 1).contiguous()
+    hi = torch.tensor([(60, 17, 200)[t % 3] for t in range(n)], dtype=torch.int32)
+    # distances below 20 count for the first heads, those of 20 and more for the others (a row of 17 keys then sees none)
+    bias = rnd(heads, 21)
+    bias[:16, 20] = float("-inf")
+    bias[16:, :20] = float("-inf")
+    out = torch.full((n, heads * hd), float("nan"), device=DEV)
+    core.attention_generic(q.to(DEV), k_cache.to(DEV), v_cache.to(DEV), torch.arange(pages, dtype=torch.int32, device=DEV).view(1, pages),
+                           torch.zeros(n, dtype=torch.int32, device=DEV), None, hi.to(DEV), out, hd ** -0.5, heads, heads, hd,
+                           positions=(hi - 1).to(DEV), bias_table=bias.to(DEV))
+    for t in range(n):
+        for h in (0, 15, 16, 31):
+            seen = [j for j in range(int(hi[t])) if (int(hi[t]) - 1 - j < 20) == (h < 16)]
+            want = torch.zeros(hd, dtype=torch.float64)
+            if seen:
+                s = keys[seen, h].double() @ q[t, h * hd:(h + 1) * hd].double() * hd ** -0.5
+                s = s + bias[h].double()[(int(hi[t]) - 1 - torch.tensor(seen)).clamp(max=20)]
+                want = torch.softmax(s, 0) @ values[seen, h].double()
+            got = out[t, h * hd:(h + 1) * hd].cpu().double()
+            assert float((got - want).abs().max()) <= 2.0 ** -18 * max(1.0, float(want.abs().max())), (t, h)
