@@ -548,7 +548,7 @@ struct PairChoice {
     double us;
 };
 
-static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats) {
+static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased) {
     const int cus = ka_compute_units();
     PairChoice best = {0, 0, 0.0};
     const long small = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
@@ -562,7 +562,7 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
     static const struct { int tile, rows_w, rows_x; double step, full, edge, edge_full, sums; } tiles[] = {
         {3, 128, 256, 0.83, 0.19, 8.4, -7.2, 1.93}, {1, 256, 256, 1.05, 0.51, 11.9, -8.6, 1.43}};
     for (const auto& t : tiles) {
-        if (M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L) continue;
+        if (!phased || M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L) continue;
         const long each = (long)ka_cdiv(N, t.rows_w) * ka_cdiv(M, t.rows_x);
         for (int parts = 1; parts <= 8 && each * parts <= cus && (long)parts * M * N <= partial_floats; ++parts) {
             const int per = ka_cdiv(steps, parts), last = steps - (parts - 1) * per;
@@ -579,10 +579,10 @@ static bool pair_tiles_fit(int M, int N, int K1, int K2) {
     return M >= 1 && N >= 1 && N % 4 == 0 && K1 % PT_BK == 0 && K2 % PT_BK == 0 && K1 >= PT_BK && K2 >= PT_BK;
 }
 
-// Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered.
-KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats) {
+// Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles, whose offsets have to fit in 32 bits.
+KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats, int phased) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased);
     return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
@@ -592,7 +592,7 @@ KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial
 // 158 and 131; 2,560, 5,120: 2,048 rows 83 and 72; 4,096, 8,192: 2,048 rows 140 and 133; in one part 4,096 rows of the last 249 against 243.
 KA_API int ka_linear_pair_large_parts(int M, int N, int K1, int K2, long partial_floats) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true);
     const double library = 2.0 * M * N * (double)(K1 + K2) / 0.85e9 + 8.0 + (double)M * N * 10.0 / 4.0e6;
     return c.tile == 1 && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
 }

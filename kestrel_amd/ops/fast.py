@@ -39,7 +39,7 @@ _SIGNATURES = {
         _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long,  # out, ldo, N, accumulate, M, target_waves, partial sums
         _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_long, _c_void_p],  # gamma, beta, eps, normed, its type and stride, stream
     "ka_linear_skinny_pair_in_parts": [_c_int, _c_int],
-    "ka_linear_pair_tiles_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
+    "ka_linear_pair_tiles_parts": [_c_int, _c_int, _c_int, _c_int, _c_long, _c_int],
     "ka_linear_pair_large_parts": [_c_int, _c_int, _c_int, _c_int, _c_long],
     "ka_linear_joint_tile": [_c_int] * 4,
     "ka_linear_pair_tiles_bf16": [
@@ -397,7 +397,9 @@ def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumula
     m, k1 = a1.shape
     k2 = a2.shape[1]
     n = w1.shape[0]
-    parts = pair_tile_parts(m, n, k1, k2) or (pair_large_parts(m, n, k1, k2) if large else 0)
+    # (operands whose offsets pass 32 bits: not by the phased tiles)
+    far = m > SKINNY_MAX_ROWS and any((t.shape[0] - 1) * t.stride(0) + t.shape[1] >= 1 << 31 for t in (a1, w1, a2, w2))
+    parts = pair_tile_parts(m, n, k1, k2, not far) or (pair_large_parts(m, n, k1, k2) if large and not far else 0)
     if not (0 < m <= SKINNY_MAX_ROWS or parts) or k1 % 8 or k2 % 8 or a2.shape[0] != m or w2.shape[0] != n:
         return False
     if not (_operand_ok(a1, k1) and _operand_ok(w1, k1) and _operand_ok(a2, k2) and _operand_ok(w2, k2)):
@@ -443,12 +445,13 @@ def _pair_tiles(m: int, n: int) -> int:
     return -(-m // 128) * -(-n // 128)
 
 
-def pair_tile_parts(m: int, n: int, k1: int, k2: int) -> int:
+def pair_tile_parts(m: int, n: int, k1: int, k2: int, phased: bool = True) -> int:
     """Parts that ``linear_pair_accumulate`` cuts K of both linears into, one behind the other (and a tile's code times ``PAIR_TILE_CODE``), where
-    it takes them by tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles)."""
+    it takes them by tiles; 0: it does not (few rows, a K that is no multiple of the tile's step, or an output of too many tiles). ``phased`` off:
+    by the small tiles alone (operands whose offsets do not fit in 32 bits)."""
     if m <= SKINNY_MAX_ROWS or _pair_tiles(m, n) > PAIR_TILES_MAX:
         return 0
-    return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4)
+    return lib().ka_linear_pair_tiles_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4, int(phased))
 
 
 def pair_large_parts(m: int, n: int, k1: int, k2: int) -> int:

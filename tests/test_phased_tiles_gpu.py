@@ -86,6 +86,30 @@ def test_where_last_linears_take_large_tiles(m, n, k1, k2, large):
         assert not fast.linear_pair_accumulate(*args) and fast.linear_pair_accumulate(*args, large=True)
 
 
+@pytest.mark.parametrize("m, large", [(768, False), (1536, True)])
+def test_rows_over_more_than_4_gb(m, large):
+    """A view whose offsets pass 32 bits of bytes goes where it went without phased tiles: by the small ones, or to the caller's other way."""
+    from kestrel_amd.ops import fast
+
+    n, k1, k2 = 2048, 2048, 8192
+    rnd = _rnd(m)
+    rows = [rnd(m, k).bfloat16().to(DEV) for k in (k1, k2)]
+    weights = [(rnd(n, k) * k ** -0.5).bfloat16().to(DEV) for k in (k1, k2)]
+    stride = (1 << 31) // (m - 1) // 8 * 8 + 8
+    wide = torch.empty(m * stride, dtype=torch.bfloat16, device=DEV).as_strided((m, k2), (stride, 1))
+    wide.copy_(rows[1])
+    assert (m - 1) * stride + k2 >= 1 << 31
+    assert (fast.pair_large_parts(m, n, k1, k2) if large else fast.pair_tile_parts(m, n, k1, k2)) >= fast.PAIR_TILE_CODE
+    out = torch.zeros(m, n, device=DEV)
+    done = fast.linear_pair_accumulate(rows[0], weights[0], None, wide, weights[1], None, out, large=large)
+    assert done == (not large)
+    if done:
+        x = [t.double().cpu() for t in (*rows, *weights)]
+        _close(out, x[0] @ x[2].T + x[1] @ x[3].T, x[0].abs() @ x[2].abs().T + x[1].abs() @ x[3].abs().T, k1 + k2, False)
+    else:
+        assert bool((out == 0.0).all())
+
+
 def test_a_replayed_graph_repeats_the_eager_bits():
     from kestrel_amd.ops import fast
 
