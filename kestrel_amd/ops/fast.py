@@ -150,9 +150,10 @@ ACTIVATION_APART_FROM_COLUMNS = 1024
 # one after the other to the vendor library (``pair_tiles_pay``). Both sides measured over widths of 512 to 8,192, K of 1,024 to
 # 20,480 in all and 65 to 1,536 rows, weights from HBM:
 #  * with the norm that follows, which the library has as a launch of its own, up to 128 tiles at every K (us: 1,024 in all at 2,048, 512 rows
-#    16.5 against 20.2; 4,096 at 2,048, 1,024 rows 32.9 and 36.8; 12,800 at 2,560, 512 rows 56.7 and 79.5), and to 160 where K is in
-#    parts (10,240 at 2,048 84.8 and 86.6, 12,800 at 2,560 104 and 115; in one part 5,120 at 2,560 63.1 and 59.2); beyond, 192 tiles 84 to
-#    187 against 78 to 166;
+#    16.5 against 20.2; 4,096 at 2,048, 1,024 rows 32.9 and 36.8; 12,800 at 2,560, 512 rows 56.5 and 79.5), and to 160 where the small tiles
+#    would have K in parts, by whichever tile is then the one (tiles and library: 10,240 at 2,048 61.5 and 92 for 1,025 rows, 66 and 94 for
+#    1,280; 6,144 46.3 and 58.5, 50.1 and 58.5; 12,800 at 2,560 72 and 113 for 769 rows, 77 and 117 for 1,024; 5,120 at 1,024, 2,049 rows
+#    42.5 and 49.6); beyond: ``pair_large_parts``;
 #  * without a norm the library's two launches are only one more: up to 32 tiles at every K (1,024 at 2,048, 256 rows 14.0 and 14.3; 48 tiles
 #    15.2 and 15.0; 2,048 at 4,096, 256 rows, 64 tiles 20.0 and 18.3), to 80 where K is 6,144 or more in all (7,680 at 2,048 37.8 and
 #    48.0, 12,800 at 2,560 55.4 and 75.4; 96 tiles 55.6 and 55.1 at 10,240).
@@ -468,9 +469,8 @@ def pair_tiles_pay(m: int, n: int, k1: int, k2: int, normed: bool) -> bool:
     if not parts:
         return False
     if normed:
-        # (beyond the tiles that always pay, small ones do in parts, large ones where the rule for large outputs says so)
-        return tiles <= PAIR_TILES_NORMED or 1 < parts < PAIR_TILE_CODE or \
-            lib().ka_linear_pair_large_parts(m, n, k1, k2, LIBRARY_WORKSPACE_BYTES // 4) > 0
+        # (beyond the tiles that always pay: where the small ones would come in parts, whichever tile is then taken)
+        return tiles <= PAIR_TILES_NORMED or pair_tile_parts(m, n, k1, k2, False) > 1
     return tiles <= PAIR_TILES_ALONE[k1 + k2 >= PAIR_TILES_LONG]
 
 

@@ -33,3 +33,17 @@ def test_where_pairs_go_by_tiles(m, n, k1, k2, normed, alone, monkeypatch):
     rows = SimpleNamespace(shape=(m, n))
     assert block._two_branches_by_stages(two, rows, rows, batch, None, rows)
     assert seen == ["one", "one"] + (["pair"] if alone or m <= fast.SKINNY_MAX_ROWS else ["one", "one"])
+
+
+# (129 to 160 tiles: with K in parts they pay whatever tile is chosen, its borders are no borders of the rule)
+@pytest.mark.parametrize("n, k1, k2, pays", [(2048, 2048, 8192, True), (2048, 1024, 5888, True), (2048, 2048, 4096, True), (2560, 2560, 10240, True),
+                                             (1536, 1536, 6144, True), (4096, 4096, 8192, True), (1024, 1024, 4992, True), (2048, 2048, 2048, False),
+                                             (2560, 512, 2560, False)])
+def test_pairs_in_parts_pay_up_to_160_tiles_of_any_kind(n, k1, k2, pays):
+    from kestrel_amd.ops import fast
+
+    across = -(-n // 128)
+    rows = range(128 // across * 128 + 1, 160 // across * 128 + 1, 13)
+    tiles = {fast.pair_tile_parts(m, n, k1, k2) // fast.PAIR_TILE_CODE for m in rows}
+    assert [fast.pair_tiles_pay(m, n, k1, k2, True) for m in rows] == [pays] * len(rows)
+    assert not pays or tiles & {1, 3}
