@@ -123,9 +123,9 @@ KA_API int ka_linear_joint_bf16(const void* A, long lda, int M, int K, const voi
                                 int act1, const void* W2, long ldw2, const float* bias2, void* out2, long ldo2, int N2, int act2, int config,
                                 hipStream_t stream) {
     const char* who = "ka_linear_joint_bf16";
-    KA_CHECK(M > 0 && K >= 128 && K % 64 == 0 && N1 > 0 && N1 % 8 == 0 && N2 >= 0 && N2 % 8 == 0, "%s: M=%d K=%d N=%d and %d", who, M, K, N1, N2);
+    KA_CHECK(M > 0 && K >= 128 && K % 64 == 0 && N1 > 0 && N1 % 8 == 0 && N2 > 0 && N2 % 8 == 0, "%s: M=%d K=%d N=%d and %d", who, M, K, N1, N2);
     KA_CHECK(lda >= K && ldw1 >= K && lda % 8 == 0 && ldw1 % 8 == 0 && ldo1 >= N1 && ldo1 % 8 == 0, "%s: strides", who);
-    KA_CHECK(N2 == 0 || (ldw2 >= K && ldw2 % 8 == 0 && ldo2 >= N2 && ldo2 % 8 == 0), "%s: strides of the second linear", who);
+    KA_CHECK(ldw2 >= K && ldw2 % 8 == 0 && ldo2 >= N2 && ldo2 % 8 == 0, "%s: strides of the second linear", who);
     KA_CHECK(((uintptr_t)A | (uintptr_t)W1 | (uintptr_t)W2 | (uintptr_t)bias1 | (uintptr_t)bias2 | (uintptr_t)out1 | (uintptr_t)out2) % 16 == 0,
              "%s: operands must be 16-byte aligned", who);
     KA_CHECK((M - 1) * lda + K < (1L << 31) && (N1 - 1) * ldw1 + K < (1L << 31) && (N2 - 1) * ldw2 + K < (1L << 31), "%s: an operand of 4 GB", who);
@@ -216,7 +216,7 @@ static int launch_pair(KaPairTiles p, int parts, hipStream_t stream) {
     return 0;
 }
 
-// tile: 256 x 256 (W x A rows) 1, 128 x 256 3, 256 x 128 5. Every part needs two K-steps.
+// tile: 256 x 256 (W x A rows) 1, 128 x 256 3. Every part needs two K-steps.
 int ka_pair_phased(const KaPairTiles& p, int tile, int parts, hipStream_t stream) {
     const int steps = p.steps[0] + p.steps[1];
     KA_CHECK(parts >= 1 && p.per >= 2 && (parts - 1) * p.per < steps && parts * p.per >= steps && steps - (parts - 1) * p.per >= 2,
@@ -226,7 +226,6 @@ int ka_pair_phased(const KaPairTiles& p, int tile, int parts, hipStream_t stream
     switch (tile) {
         case 1: return launch_pair<4, 4, 2, 2, 2, 4>(p, parts, stream);
         case 3: return launch_pair<2, 2, 2, 2, 2, 4>(p, parts, stream);
-        case 5: return launch_pair<2, 2, 2, 2, 4, 2>(p, parts, stream);
     }
     KA_CHECK(false, "pair of linears: unknown tile %d", tile);
 }
