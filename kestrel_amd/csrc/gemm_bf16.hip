@@ -410,7 +410,7 @@ pair_tiles_kernel(KaPairTiles p) {
 // Bound by the K-steps that follow one another on a CU, 0.5 to 0.6 us each whatever the stages in flight (three to five: 73 to
 // 71 us for K = 8,192 alone on 64 CUs): parts of K spread them over all CUs. Measured with the norm that follows, against the
 // vendor library's two products and the norm's launch (us; K = 2,560 + 10,240, N = 2,560): 128 rows 31 against 78, 512 rows
-// 57 (three parts) against 83, 1,024 rows 106 against 117.
+// 56.5 (three parts) against 83, 1,024 rows 108 against 117.
 constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5, PT_TILE_CODE = 100;
 
 template <int WN, int WM, int GN, int GM, int NS, int SL>
@@ -538,11 +538,13 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
 //    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
 //  * The phased tiles of 256 rows where they come out 5 % ahead and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
 //    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
-//    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 %. Not where more
+//    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 % on the average. Not where more
 //    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
 //    and 23.7 us).
-// Measured with the norm behind, the small tiles and the choice (us): N = 2,048, K = 10,240: 512 rows 43 and 38, 768 rows 55.5 and 47.0, 1,280 rows 84
-// and 66; 2,560, 12,800: 512 rows 57.6 and 49.6, 1,000 rows 104 and 76; 4,096, 20,480: 512 rows 121 and 92.
+// Measured with the norm behind, small tiles in the parts they would come in and the phased ones chosen (us): N = 2,048, K = 10,240: 768 rows 54.0 and 47.7,
+// 1,280 rows 84.4 and 66.0; 2,560, 12,800: 385 rows 49.6 and 47.9, 448 rows 52.5 and 49.1, 1,024 rows 108 and 77; 4,096, 12,288, 640 rows 97 and 80.
+// Where the two estimates meet the choice can be the slower one: 2,560, 12,800, 512 rows, small tiles 56.5 (estimated 53.0), phased ones in
+// six parts 50.5 (53.7); at 2,048, 10,240, 512 rows it is right (37.0 and 39.9).
 struct PairChoice {
     int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
     double us;

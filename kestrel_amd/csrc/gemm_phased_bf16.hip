@@ -107,10 +107,13 @@ static int launch_joint(KpJoint p, hipStream_t stream) {
 // The tiles by area: of those whose workgroups are one round of the chip the smallest wins, since a K-step of it is the shortest.
 static const struct { int code, rows_w, rows_x; } KP_JOINT_TILES[] = {{6, 128, 128}, {3, 128, 256}, {5, 256, 128}, {2, 192, 256}, {4, 256, 192}, {1, 256, 256}};
 
-// The tile for two linears of the same rows in one launch, 0: not covered, or faster one after the other by the vendor library, which is so where
-// they take more than one round (14,336 outputs from 2,048, 1,200 rows: 83 against 75 us) or nearly half of the tiles is no rows (22,528 from 4,096,
-// 257 rows: 85 against 82). Measured over widths of 1,536 to 4,096 and 65 to 1,200 rows, us, library and one launch: 14,336 from 2,048: 128 rows 31.8 and
-// 25.2, 256 rows 50 and 26, 512 rows 51 and 36, 743 rows 59 and 45, 1,024 rows 69 and 54; 17,920 from 2,560, 512 rows: 70 and 55.
+// The tile for two linears of the same rows in one launch, 0: not covered, or left to the vendor library one after the other. That is so where nearly half of
+// the tiles is no rows (22,528 from 4,096, 257 rows: 85 us in one launch, 82 by the library), and where they take more than one round, in which neither
+// side is ahead everywhere (us, library and the best of the tiles 256 x 256, 192 x 256 and 128 x 256; 14,336 from 2,048: 1,100 rows 74 and 84, 1,300 rows 90
+// and 86, 1,536 rows 88 and 89, 2,048 rows 104 and 106; 17,920 from 2,560: 1,024 rows 105 and 106, 1,200 rows 128 and 109, 1,536 rows 125 and 127, 1,792 rows
+// 162 and 131): a rule for those rows would go by the fill of the last round, and has not been measured at other widths. Within one round, widths of 1,536 to
+// 4,096, 65 to 1,024 rows, library and one launch: 14,336 from 2,048: 128 rows 31.8 and 25.2, 256 rows 50 and 26, 512 rows 51 and 36, 743 rows 59
+// and 45, 1,024 rows 69 and 55; 17,920 from 2,560, 512 rows: 70 and 55.
 KA_API int ka_linear_joint_tile(int M, int N1, int N2, int K) {
     if (M < 1 || N1 < 8 || N2 < 8 || N1 % 8 || N2 % 8 || K % 64 || K < 128) return 0;
     for (const auto& t : KP_JOINT_TILES)

@@ -1,5 +1,5 @@
 // The short causal convolution with rotation and cache write (sequence_parts.hip) for bf16 rows as a function of a workgroup's place, so that
-// more than one kernel can hold it: the plain launch and the launch that runs it beside the step of a recurrence (linear_attention.hip).
+// more than one kernel can hold it: the plain launch and the launch that runs it beside the step of a recurrence (both in sequence_parts.hip).
 #pragma once
 #include "ka_common.h"
 

@@ -32,7 +32,8 @@ struct KaPairTiles {
 
 // The tile and part of a workgroup; part -1: none. An XCD's workgroups are neighbours in one part of K, so that what they read of either operand
 // is the same few rows' same columns. (A part's tiles spread over all XCDs instead, every XCD reads all of K: N = 2,048, K = 10,240, 2,048 rows
-// 96.7 against 88.5 us; and 50 tiles, seven to an XCD, in five parts are a second round on seven of the XCDs: 2,560, 12,800, 1,280 rows 136 against 89.5.)
+// 96.7 against 88.5 us; and 50 tiles, seven to an XCD, in five parts are a second round on seven of the XCDs: 2,560, 12,800, 1,280 rows 136 against 89.5.
+// Tiles of 128 x 128 gain less: 2,048, 10,240, 512 rows 38.6 and 37.0, 2,560, 12,800, 512 rows 57.5 and 56.5.)
 struct KaPairPlace {
     int part, tile_n, tile_m;
 };

@@ -161,6 +161,7 @@ PAIR_TILES_MAX = 160
 PAIR_TILES_NORMED = 128
 PAIR_TILES_ALONE = (32, 80)
 PAIR_TILES_LONG = 6144
+# A code of parts and tile: parts + PAIR_TILE_CODE * tile (0: 128 x 128; 1 and 3: the phased tiles).
 PAIR_TILE_CODE = 100
 _library_space = {}
 SCRATCH_FLOATS = 8 << 20
@@ -298,9 +299,9 @@ def _wide_scratch_buffer(device: torch.device) -> torch.Tensor:
 
 
 def _library_workspace(device: torch.device) -> torch.Tensor:
-    """Scratch memory the vendor library's kernels may use (parts of K that meet in it), one buffer
-    per device, made at the first call (a step's first run is never inside a graph capture).
-    Calls on one device must not overlap."""
+    """Scratch memory the vendor library's kernels may use (parts of K that meet in it), and the fp32 sums of the parts of
+    ``linear_pair_accumulate`` by tiles; one buffer per device, made at the first call (a step's first run is never
+    inside a graph capture). Calls of either on one device must not overlap."""
     key = _device_index(device)
     if key not in _library_space:
         _library_space[key] = torch.empty(LIBRARY_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
@@ -310,7 +311,8 @@ def _library_workspace(device: torch.device) -> torch.Tensor:
 def prepare(device: torch.device) -> int:
     """Everything these kernels keep per device, made now instead of at the first call that needs it
     (which may be the first step of a live request): the partial results of decode attention, the
-    partial sums of the wide skinny kernel and the vendor library's workspace. Returns their bytes."""
+    partial sums of the wide skinny kernel and the workspace of the vendor library and of pairs of
+    linears by tiles. Returns their bytes."""
     buffers = (scratch(device), _library_workspace(device), _wide_scratch_buffer(device))
     return sum(b.numel() * b.element_size() for b in buffers)
 
