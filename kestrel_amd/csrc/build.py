@@ -31,7 +31,7 @@ ARCH = "gfx950"
 LIBRARIES: Dict[str, List[str]] = {
     "core": ["ka_error.hip", "elementwise.hip", "gemm_generic.hip", "attention_generic.hip", "mixer_parts.hip", "sequence_parts.hip", "recurrent_parts.hip", "linear_attention.hip", "stream_parts.hip", "experts.hip",
              "sampling.hip", "peaks.hip"],
-    "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_phased_bf16.hip", "gemv_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
+    "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_phased_bf16.hip", "gemv_bf16.hip", "gemv_share_bf16.hip", "gemv_share_long_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
              "gemm_library.hip"],
 }
 
@@ -137,7 +137,9 @@ def build(name: str, verbose: bool = True) -> Path:
     for src in sources:
         obj = objdir / (src.stem + ".o")
         cmd = [hipcc, *HIPCC_FLAGS, "-I", str(SOURCE_DIR), "-c", str(src), "-o", str(obj)]
-        procs.append((src, obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env=env)))
+        # (into a file: the compiler warns once a kernel and pass, and a pipe that nobody reads until it ends stops it when full)
+        with open(obj.with_suffix(".log"), "wb") as log:
+            procs.append((src, obj, subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT, env=env)))
     objects = []
     pending = list(procs)
     last_note = time.time()
@@ -147,8 +149,8 @@ def build(name: str, verbose: bool = True) -> Path:
             if proc.poll() is None:
                 continue
             pending.remove(item)
-            output = proc.stdout.read().decode(errors="replace")
             if proc.returncode != 0:
+                output = obj.with_suffix(".log").read_text(errors="replace")
                 for _, _, other in pending:
                     other.kill()
                 raise KernelBuildError(f"hipcc failed on {src.name}:\n{output}")
