@@ -367,6 +367,8 @@ static int sk_compute_units() { return ka_compute_units(); }
 
 // The persistent kernel is used wherever it fits; switching it off is for measurements and for
 // tests of the split kernel on sizes that it otherwise never sees.
+int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, hipStream_t stream);      // gemv_share_bf16.hip
+
 static int sk_persistent_enabled = 1;
 KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enabled; }
 // The wide kernel (17 to 64 rows, activations through LDS, parts of K in scratch memory): 1 where
@@ -588,6 +590,8 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         const size_t dyn = (size_t)M * (K1 + SK_PAD) * sizeof(bf16_t);
         KA_CHECK(dyn <= 96 * 1024, "%s: %d rows of %d do not fit in LDS", who, M, K1);
         KA_CHECK(persistent_fits(M, kblocks, args), "%s: K=%d or the biases do not suit the LayerNorm prologue", who, K1);
+        const int shared = sk_persistent_enabled ? ka_skinny_share(args, strips, kblocks, true, stream) : 1;
+        if (shared <= 0) return shared;
         if (launch_persistent(strips, M, kblocks, true, dyn, stream, args)) return -1;
         KA_LAUNCH_CHECK();
         return 0;
@@ -666,6 +670,15 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         if (then)
             ka_launch_finish_norm(M, Na, stream, nullptr, 0, nullptr, nullptr, (float*)outa, ldoa, 0, *then);
     };
+    if (sk_persistent_enabled) {
+        const int shared = ka_skinny_share(args, strips, kblocks, false, stream);
+        if (shared < 0) return -1;
+        if (shared == 0) {
+            norm_after();
+            KA_LAUNCH_CHECK();
+            return 0;
+        }
+    }
     if (persistent_ok) {
         if (launch_persistent(strips, M, kblocks, false, 0, stream, args)) return -1;
         KA_LAUNCH_CHECK();

@@ -20,6 +20,14 @@ constexpr int SK_PAD = 8;          // bf16 of padding per LDS row (keeps 16-byte
 constexpr int SP_WAVES = 8;        // waves of a persistent workgroup
 constexpr int SP_MAX_PER = 8;      // most k-blocks per wave it keeps activations for
 
+// A barrier for what went through LDS: loads from memory stay on their way.
+__device__ __forceinline__ void sk_lds_barrier() {
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0), the other counters at their maximum
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Orders the LDS traffic of one wave: what its lanes wrote before is seen by its lanes after.
 __device__ __forceinline__ void sk_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -173,13 +181,16 @@ template <int XV, bool EARLY>
 __device__ __forceinline__ void sk_fetch_row(const SkinnyArgs& p, int m, int lane, RowOperands<XV, EARLY>& row) {
     const int K = p.K[0];
     const float* src = p.ln_x + (size_t)m * K;
+    // (no shift: the scale once more, which sk_normalise_row leaves out. A load under a branch, or a value chosen as soon as it is
+    // loaded, would make the wave wait for everything in flight)
+    const float* shift = p.ln_beta ? p.ln_beta : p.ln_gamma;
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int k = min((j * KA_WAVE + lane) * 4, K - 4);
         row.x[j] = *reinterpret_cast<const floatx4*>(src + k);
         if constexpr (EARLY) {
             row.gamma[j] = *reinterpret_cast<const floatx4*>(p.ln_gamma + k);
-            row.beta[j] = p.ln_beta ? *reinterpret_cast<const floatx4*>(p.ln_beta + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+            row.beta[j] = *reinterpret_cast<const floatx4*>(shift + k);
         }
     }
 }
@@ -210,7 +221,7 @@ __device__ __forceinline__ void sk_normalise_row(const SkinnyArgs& p, bf16_t* xs
             floatx4 gm, bt;
             if constexpr (EARLY) {
                 gm = row.gamma[j];
-                bt = row.beta[j];
+                bt = p.ln_beta ? row.beta[j] : floatx4{0.f, 0.f, 0.f, 0.f};
             } else {
                 gm = *reinterpret_cast<const floatx4*>(p.ln_gamma + k);
                 bt = p.ln_beta ? *reinterpret_cast<const floatx4*>(p.ln_beta + k) : floatx4{0.f, 0.f, 0.f, 0.f};
