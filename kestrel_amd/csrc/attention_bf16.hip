@@ -448,7 +448,7 @@ constexpr int ad_waves_per_simd(int HD, int WAVES, int TP) {
 constexpr int AD_SMALL_TILE_PAGES = 2;
 constexpr int AD_SMALL_TILE_MAX_PAGES = 128;   // rows of up to this many pages get the small tiles
 
-template <int HD, int WAVES, int TP>
+template <int HD, int WAVES, int TP, bool SHORT>
 __global__ void __launch_bounds__(KA_WAVE * WAVES)
     __attribute__((amdgpu_waves_per_eu(ad_waves_per_simd(HD, WAVES, TP), ad_waves_per_simd(HD, WAVES, TP))))
 attn_decode_kernel(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* __restrict__ k_cache,
@@ -456,7 +456,7 @@ attn_decode_kernel(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t
                    const int* __restrict__ token_row, const int* __restrict__ kv_lo,
                    const int* __restrict__ kv_hi, bf16_t* __restrict__ out, long out_row_stride, float scale,
                    int H, int Hkv, float* __restrict__ partial, DecodeFuse fz) {
-    attn_decode_body<HD, WAVES, false, TP>(q, q_row_stride, k_cache, v_cache, block_table, max_pages, token_row, kv_lo, kv_hi,
+    attn_decode_body<HD, WAVES, SHORT, false, TP>(q, q_row_stride, k_cache, v_cache, block_table, max_pages, token_row, kv_lo, kv_hi,
                                            out, out_row_stride, scale, H, Hkv, partial, fz, blockIdx.x, blockIdx.y, blockIdx.z,
                                            gridDim.z);
 }
@@ -749,8 +749,9 @@ static int decode_launch(const char* who, const void* q, long q_row_stride, cons
     // (Rows of up to 2,048 keys, going by the width of the block table: behind 4,096 keys a row the larger tile
     // came out 2 to 3 % ahead at 24 and 32 rows, level at 48 and 64.)
     const bool small_tiles = waves == 4 && hd <= 64 && max_pages <= AD_SMALL_TILE_MAX_PAGES && groups * 2 >= 3L * cus && groups <= 8L * cus;
+    const bool short_rows = max_pages <= AT_LDS_PAGES;
 #define KA_AD(HDV, WV, TPV)                                                                                         \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, WV, TPV>), grid, block, 0, stream, (const bf16_t*)q, q_row_stride, \
+    hipLaunchKernelGGL((short_rows ? attn_decode_kernel<HDV, WV, TPV, true> : attn_decode_kernel<HDV, WV, TPV, false>), grid, block, 0, stream, (const bf16_t*)q, q_row_stride, \
                        (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, token_row, kv_lo,   \
                        kv_hi, (bf16_t*)out, out_row_stride, scale, H, Hkv, partial, fz)
 #define KA_AD_SMALL(HDV)                                                                                            \

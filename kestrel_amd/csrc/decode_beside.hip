@@ -41,7 +41,7 @@ struct BesideAttention {
     DecodeFuse fz;
 };
 
-template <int HD, int PER>
+template <int HD, int PER, bool SHORT>
 __global__ void __launch_bounds__(BS_WAVES * KA_WAVE) __attribute__((amdgpu_waves_per_eu(4, 4)))
 attn_decode_beside_kernel(BesideAttention a, SkinnyArgs p, int strips, int attention_groups, int linear_groups) {
     const int b = blockIdx.x;
@@ -53,7 +53,7 @@ attn_decode_beside_kernel(BesideAttention a, SkinnyArgs p, int strips, int atten
         return;
     }
     const int t = index % a.n, h = index / a.n % a.H, split = index / (a.n * a.H);
-    attn_decode_body<HD, BS_WAVES, true>(a.q, a.q_row_stride, a.k_cache, a.v_cache, a.block_table, a.max_pages, a.token_row,
+    attn_decode_body<HD, BS_WAVES, SHORT, true>(a.q, a.q_row_stride, a.k_cache, a.v_cache, a.block_table, a.max_pages, a.token_row,
                                    a.kv_lo, a.kv_hi, a.out, a.out_row_stride, a.scale, a.H, a.Hkv, a.partial, a.fz, t, h,
                                    split, a.splits);
 }
@@ -118,21 +118,22 @@ KA_API int ka_attention_decode_beside_bf16(const void* q, long q_row_stride, con
     KA_CHECK(attention_groups + linear_groups < (1L << 31), "%s: too many workgroups", who);
     const int per = ka_cdiv(ka_cdiv(K, SK_KBLOCK), SP_WAVES);
     dim3 grid((unsigned)(attention_groups + linear_groups)), block(BS_WAVES * KA_WAVE);
-#define KA_BS_LAUNCH(HDV, PERV)                                                                                     \
+#define KA_BS_LAUNCH(HDV, PERV, SHORTV)                                                                             \
     {                                                                                                               \
         static size_t reserved = 0;                                                                                 \
         if (dyn > reserved) {                                                                                       \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_decode_beside_kernel<HDV, PERV>), \
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_decode_beside_kernel<HDV, PERV, SHORTV>),\
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);               \
             KA_CHECK(e == hipSuccess, "%s: cannot reserve %zu bytes of LDS", who, dyn);                             \
             reserved = dyn;                                                                                         \
         }                                                                                                           \
-        hipLaunchKernelGGL((attn_decode_beside_kernel<HDV, PERV>), grid, block, dyn, stream, a, p, strips,          \
+        hipLaunchKernelGGL((attn_decode_beside_kernel<HDV, PERV, SHORTV>), grid, block, dyn, stream, a, p, strips,  \
                            (int)attention_groups, linear_groups);                                                   \
     }
 #define KA_BS(HDV)                                                                                                  \
     case HDV:                                                                                                       \
-        if (per <= 1) KA_BS_LAUNCH(HDV, 1) else if (per <= 2) KA_BS_LAUNCH(HDV, 2) else KA_BS_LAUNCH(HDV, 4)        \
+        if (max_pages > AT_LDS_PAGES) KA_BS_LAUNCH(HDV, 4, false)                                                   \
+        else if (per <= 1) KA_BS_LAUNCH(HDV, 1, true) else if (per <= 2) KA_BS_LAUNCH(HDV, 2, true) else KA_BS_LAUNCH(HDV, 4, true) \
         break;
     switch (hd) {
         KA_BS(16) KA_BS(32) KA_BS(48) KA_BS(64)
