@@ -75,7 +75,7 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 
 // Many rows in fp32 where K is a multiple of 32: true fp32 products and sums on the matrix pipes (v_mfma_f32_32x32x2_f32, twice
 // the rate of the vector unit without packed FMAs), operands straight from memory into swizzled LDS as in ka_dma_tiles.h (a
-// K-step of 32 numbers is the same 128 bytes a row), two stages.
+// K-step of 32 numbers is the same 128 bytes a row, of 16 the same 64), NS stages of STEP numbers.
 //
 // The order of a sum is fixed by K alone. Every sixteen k are summed from zero (of every eight in the order 0 4 1 5 2 6 3 7: a lane
 // holds four neighbours), these sums are added in order within a part, K being cut into F32_PARTS parts, and the parts' sums
@@ -91,14 +91,15 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 constexpr int F32_PARTS = 4;
 constexpr int F32_STEP = 32;
 
-template <int WN, int WM, int GN, int GM, int KG>
+template <int WN, int WM, int GN, int GM, int KG, int STEP, int NS>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM * KG)
 gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
                      float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
     static_assert(KG == 1 || KG == F32_PARTS, "the parts one after the other, or one a group of waves");
     constexpr int WAVES = GN * GM, BN = 32 * WN * GN, BM = 32 * WM * GM;
-    constexpr int ROW = F32_STEP * 4, CPR = 8, RPL = KA_WAVE / CPR, STAGE = (BN + BM) * ROW;
+    constexpr int ROW = STEP * 4, CPR = ROW / 16, RPL = KA_WAVE / CPR, STAGE = (BN + BM) * ROW;
     constexpr int W_LOADS = BN / RPL / WAVES, X_LOADS = BM / RPL / WAVES;
+    static_assert(W_LOADS * RPL * WAVES == BN && X_LOADS * RPL * WAVES == BM, "the tile does not divide over the waves' loads");
     extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
     const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8;
     const int logical = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
@@ -119,7 +120,7 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
         const int r = kd_load_row<CPR>(part_wave * X_LOADS + i, lane);
         xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2;
     }
-    unsigned char* mine = gf_lds + group * 2 * STAGE;
+    unsigned char* mine = gf_lds + group * NS * STAGE;
     auto fetch = [&](int stage, int k) {
         unsigned char* base = mine + stage * STAGE;
 #pragma unroll
@@ -140,22 +141,26 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
                 for (int v = 0; v < 16; ++v) x[a][b][v] = 0.f;
     };
     clear(acc);
-    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP, k_steps = K / F32_STEP;
+    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP * (F32_STEP / STEP), k_steps = K / STEP;
     // this wave's steps: all of K, or its group's part
     const int first = KG == 1 ? 0 : group * part_steps;
     const int steps = max(0, min(KG == 1 ? k_steps : part_steps, k_steps - first));
     const int rounds = KG == 1 ? k_steps : min(part_steps, k_steps);           // (the same for every wave: barriers)
-    if (steps > 0) fetch(0, first * F32_STEP);
-    int done = 0;                                                              // KG == 1: parts added into `sum`
-    for (int s = 0; s < rounds; ++s) {
-        gd_wait_loads<0>();                                                    // own loads of this step have landed
-        gd_wait_lds();                                                         // own reads of the step before are in registers
-        gd_barrier();
-        if (s + 1 < steps) fetch((s + 1) & 1, (first + s + 1) * F32_STEP);
-        if (s < steps) {
-            const unsigned char* base = mine + (s & 1) * STAGE;
 #pragma unroll
-            for (int g = 0; g < F32_STEP / 16; ++g) {
+    for (int s = 0; s < NS - 1; ++s)
+        if (s < steps) fetch(s, (first + s) * STEP);
+    int done = 0;                                                              // KG == 1: parts added into `sum`
+    int stage = 0;                                                             // of step s
+    for (int s = 0; s < rounds; ++s) {
+        gd_wait_younger<W_LOADS + X_LOADS, NS - 2>(steps - 1 - s);             // own loads of this step have landed
+        gd_wait_lds();                                                         // own reads of the step before are in registers
+        if constexpr (WAVES > 1) gd_barrier();                                 // (a wave that has its part of K to itself reads what it asked for)
+        if (s + NS - 1 < steps) fetch(stage == 0 ? NS - 1 : stage - 1, (first + s + NS - 1) * STEP);
+        if (s < steps) {
+            const unsigned char* base = mine + stage * STAGE;
+            stage = stage + 1 == NS ? 0 : stage + 1;
+#pragma unroll
+            for (int g = 0; g < STEP / 16; ++g) {
                 floatx4 w[2][WN], x[2][WM];
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -243,12 +248,13 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
     }
 }
 
-template <int WN, int WM, int GN, int GM, int KG>
+template <int WN, int WM, int GN, int GM, int KG, int STEP, int NS>
 static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
-    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * 2 * (BN + BM) * F32_STEP * 4;
+    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * NS * (BN + BM) * STEP * 4;
+    static_assert(KG == 1 || smem >= KG * GN * GM * WN * WM * 4 * KA_WAVE * 16, "the parts' sums fit");
     static bool configured = false;
-    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG>;
+    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG, STEP, NS>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         KA_CHECK(e == hipSuccess, "ka_linear_generic: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
@@ -265,19 +271,25 @@ static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, c
 
 // The tile: the one that takes the fewest blocks of 32 x 32 x K one after the other on the fullest CU, weighed by the rate the
 // tile reaches where CUs are full (TFLOP/s: smaller tiles read L2 and LDS more often per product). All give the same bits.
-// (us with 64 x 128, 64 x 64, 64 x 32 and 32 x 32 before the sums were cut into sixteens: 303 rows of 2,048 x 6,144 150, 82, 94,
-// 96; 157 rows 93, 82, 50, 54; 17 rows of 2,048 x 2,048 88, 40, 24, 19; 2,048 rows of 8,192 x 2,048 604, 630, 683, 766.)
+// K-steps: of 32 where a workgroup has a CU to itself and where every wave waits for nobody (tiles of 32 x 32, a part of K a wave: no barrier; with one
+// a step 2,048 of 8,192 took 144 us at 304 rows, 133 without); of 16, half the LDS and so two or three workgroups a CU, where there are more tiles
+// of 64 x 32 or 64 x 64 than CUs (304 rows, steps of 32 and 16: 8,192 of 2,048 124 and 116, 6,144 of 2,048 87.2 and 86.9, at 320 rows 87.6 and 83.0, at
+// 450 129 and 121; one a CU, 64 rows of 2,048 x 2,048 by 64 x 32: 25.9 and 32.5). Three and four stages of 16 were slower at every size.
 static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
     const int cus = ka_compute_units();
-    auto cost = [&](int bn, int bm, float rate) { return ka_cdiv((long)ka_cdiv(N, bn) * ka_cdiv(M, bm), cus) * (float)(bn * bm) / rate; };
-    const float t128 = cost(64, 128, 112.f), t64 = cost(64, 64, 104.f), t32 = cost(64, 32, 90.f), t1 = cost(32, 32, 85.f);
+    auto tiles = [&](int bn, int bm) { return (long)ka_cdiv(N, bn) * ka_cdiv(M, bm); };
+    auto cost = [&](int bn, int bm, float rate) { return ka_cdiv(tiles(bn, bm), cus) * (float)(bn * bm) / rate; };
+    const float t128 = cost(64, 128, 112.f), t64 = cost(64, 64, 112.f), t32 = cost(64, 32, 95.f), t1 = cost(32, 32, 92.f);
     const float best = fminf(fminf(t128, t64), fminf(t32, t1));
 #define KA_F32(...) return launch_f32_mfma<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
-    if (t128 <= best) KA_F32(1, 2, 2, 2, 1);
-    if (t64 <= best) KA_F32(1, 2, 2, 1, F32_PARTS);
-    if (t32 <= best) KA_F32(1, 1, 2, 1, F32_PARTS);
-    KA_F32(1, 1, 1, 1, F32_PARTS);
+    if (t128 <= best) KA_F32(1, 2, 2, 2, 1, 32, 2);
+    if (t64 <= best) KA_F32(1, 2, 2, 1, F32_PARTS, 16, 2);
+    if (t32 <= best) {
+        if (tiles(64, 32) > cus) KA_F32(1, 1, 2, 1, F32_PARTS, 16, 2);
+        KA_F32(1, 1, 2, 1, F32_PARTS, 32, 2);
+    }
+    KA_F32(1, 1, 1, 1, F32_PARTS, 32, 2);
 #undef KA_F32
 }
 
@@ -378,7 +390,8 @@ gemm_f32_kernel(const float* __restrict__ A, long lda, const float* __restrict__
 // loop over the rows that are there are not hoisted over each other), and a step's activations, which come from the CU's cache,
 // serve all C columns. Measured, us, before -> now, three rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x 8,192, 8,192 x 2,048 and the
 // head of 2,048 x 51,200: 14.3, 11.0, 23.5, 35.8 and 124 -> 12.7, 6.7, 16.5, 19.6 and 79; one row 11.1, 8.9, 15.7, 22.4 and 78 -> 10.1,
-// 4.6, 12.6, 12.5 (5.4 TB/s) and 64.
+// 4.6, 12.6, 12.5 (5.4 TB/s) and 64. Forms for exactly three and for six rows (instead of four and eight, one or two of them read for nothing): three rows
+// of 8,192 x 2,048 19.3 -> 16.7, 2,048 x 8,192 16.3 -> 15.8; six 22.6 -> 21.8, 19.3 -> 18.2.
 constexpr int GV_ROWS = 16;      // most rows
 constexpr int GV_WAVES = 4;      // waves per workgroup
 
@@ -463,14 +476,14 @@ static void launch_gemv_form(const float* A, long lda, const float* W, long ldw,
 
 // Columns a wave: more of them ask the cache for fewer activations, fewer of them leave more waves to wait for memory. Two are
 // best over most of the range; one where there are less than 16 waves a CU and at most four rows (2,048 columns of 8,192 at three
-// rows: 19.6 us, 22.5 with two, 22.8 with four), four from eight rows and 32 waves a CU on (51,200 x 2,048 at sixteen rows:
+// rows: 19.6 us, 22.5 with two, 22.8 with four), four from five rows and 32 waves a CU on (51,200 x 2,048 at sixteen rows:
 // 210, 228 with two, 306 with one).
 template <int MB>
 static void launch_gemv(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K, int act,
                         int accumulate, hipStream_t stream) {
     const int cus = ka_compute_units();
     if (MB <= 4 && N < 16 * cus) launch_gemv_form<MB, 1>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
-    else if (MB >= 8 && N >= 32 * cus) launch_gemv_form<MB, 4>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
+    else if (MB >= 6 && N >= 32 * cus) launch_gemv_form<MB, 4>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
     else launch_gemv_form<MB, 2>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream);
 }
 
@@ -517,7 +530,9 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
 #define KA_GEMV(MB) launch_gemv<MB>((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream)
         if (M <= 1) KA_GEMV(1);
         else if (M <= 2) KA_GEMV(2);
+        else if (M <= 3) KA_GEMV(3);
         else if (M <= 4) KA_GEMV(4);
+        else if (M <= 6) KA_GEMV(6);
         else if (M <= 8) KA_GEMV(8);
         else KA_GEMV(16);
 #undef KA_GEMV
