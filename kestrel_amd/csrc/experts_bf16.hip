@@ -436,6 +436,41 @@ struct ExpertsFewArgs {
     int out_f32;
 };
 
+// Four neighbouring outputs, o to o + 3, of a pair.
+__device__ __forceinline__ void ef_store(const ExpertsFewArgs& g, const ef_floatx4 y, int pair, int o) {
+    const size_t row = (size_t)pair * g.ldo;
+    if (ka_act_gated(g.act)) {
+        bf16_t* op = reinterpret_cast<bf16_t*>(g.out) + row + o / 2;
+        if (o + 1 < g.N) op[0] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[0], y[1]);
+        if (o + 3 < g.N) op[1] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[2], y[3]);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (o + r >= g.N) continue;
+        const float v = ka_activate_fast(g.act, y[r]);
+        if (g.out_f32) reinterpret_cast<float*>(g.out)[row + o + r] = v;
+        else reinterpret_cast<bf16_t*>(g.out)[row + o + r] = (bf16_t)v;
+    }
+}
+
+// The waves' sums through LDS and the outputs of MB * 16 columns; pair: the pair of this lane's column of a block.
+template <int MB>
+__device__ __forceinline__ void ef_finish(const ExpertsFewArgs& g, const ef_floatx4 (&acc)[MB], const int (&pair)[MB], int count, int first, int row0,
+                                          float* sums) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    const int col = lane % 16, quarter = lane / 16;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) *reinterpret_cast<ef_floatx4*>(sums + ((wave * MB + m) * KA_WAVE + lane) * 4) = acc[m];
+    __syncthreads();
+    if (wave >= MB) return;
+    ef_floatx4 y = ef_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < EF_WAVES; ++v) y += *reinterpret_cast<const ef_floatx4*>(sums + ((v * MB + wave) * KA_WAVE + lane) * 4);
+    if (first + wave * 16 + col >= count) return;
+    ef_store(g, y, pair[MB == 1 ? 0 : wave], row0 + quarter * 4);
+}
+
 template <int MB, int U>
 __device__ __forceinline__ void ef_columns(const ExpertsFewArgs& g, const bf16_t* W, const int* list, int count, int first, int row0,
                                            float* sums) {
@@ -475,34 +510,77 @@ __device__ __forceinline__ void ef_columns(const ExpertsFewArgs& g, const bf16_t
 #pragma unroll
             for (int m = 0; m < MB; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u][m], acc[m], 0, 0, 0);
     }
-#pragma unroll
-    for (int m = 0; m < MB; ++m) *reinterpret_cast<ef_floatx4*>(sums + ((wave * MB + m) * KA_WAVE + lane) * 4) = acc[m];
-    __syncthreads();
-    if (wave >= MB) return;
-    ef_floatx4 y = ef_floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int v = 0; v < EF_WAVES; ++v) y += *reinterpret_cast<const ef_floatx4*>(sums + ((v * MB + wave) * KA_WAVE + lane) * 4);
-    if (first + wave * 16 + col >= count) return;
-    const size_t row = (size_t)pair[MB == 1 ? 0 : wave] * g.ldo;
-    const int o = row0 + quarter * 4;
-    if (ka_act_gated(g.act)) {
-        bf16_t* op = reinterpret_cast<bf16_t*>(g.out) + row + o / 2;
-        if (o + 1 < g.N) op[0] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[0], y[1]);
-        if (o + 3 < g.N) op[1] = (bf16_t)ka_gate_product<true>(g.act, g.clamp, y[2], y[3]);
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if (o + r >= g.N) continue;
-        const float v = ka_activate_fast(g.act, y[r]);
-        if (g.out_f32) reinterpret_cast<float*>(g.out)[row + o + r] = v;
-        else reinterpret_cast<bf16_t*>(g.out)[row + o + r] = (bf16_t)v;
-    }
+    ef_finish<MB>(g, acc, pair, count, first, row0, sums);
 }
 
+// Up to eight columns of a K in steps of 64: the same products in the same order, operands straight into LDS. A wave's share of a step is whole lines of
+// 16 weight rows and of the pairs' rows, in a ring of NS steps of its own (no barrier): in registers they cost a workgroup a place on the CU for every few
+// loads in flight, and an instruction touches a half of each of 16 lines. Both linears, us, registers -> three stages (two, four): 30 experts of 2,048 x 704,
+// top 4, 1 row 20.5 -> 15.8 (15.8, 17.2), 8 rows 49.0 -> 43.5 (43.7, 47.6), 32 rows 67 -> 60; 62 of 4,096 x 896, top 6, 8 rows 176 -> 155 (157, 161), 32
+// rows 281 -> 238 (5.5 TB/s). What is left at few bytes is a workgroup's way: the choices, its one or two rounds of steps, the waves' sums. A workgroup of
+// one wave that keeps the four sums apart (no such end) took 50.0 and 202 at 8 rows: its stream is one chain of steps.
+constexpr int ES_PAIRS = 8;
+constexpr int ES_STAGES = 3;
+constexpr int ES_STAGE = (EF_ROWS + ES_PAIRS) * 128;
+
+template <int NS>
+__device__ __forceinline__ void ef_stream(const ExpertsFewArgs& g, const bf16_t* W, const int* list, int count, int first, int row0,
+                                          unsigned char* lds) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    const int col = lane % 16, quarter = lane / 16;
+    unsigned char* const mine = lds + wave * NS * ES_STAGE;
+    const int steps = (g.K / 64 - wave + EF_WAVES - 1) / EF_WAVES;                 // this wave's: wave, wave + 4, ...
+    // what this lane asks for: a piece of the weight rows lane / 8 and lane / 8 + 8, and of the pair lane / 8 (rows and pairs past the end: not stored)
+    const bf16_t* wsrc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = kd_load_row<8>(i, lane);
+        wsrc[i] = W + (size_t)min(row0 + r, g.N - 1) * g.K + kd_load_channel<8>(r, lane);
+    }
+    const int asked = list[min(first + kd_load_row<8>(0, lane), count - 1)];
+    const bf16_t* const xsrc = g.a + (size_t)(asked / g.gather_div) * g.lda + kd_load_channel<8>(kd_load_row<8>(0, lane), lane);
+    auto fetch = [&](int stage, int s) {
+        unsigned char* const base = mine + stage * ES_STAGE;
+        const int k = (wave + s * EF_WAVES) * 64;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + k), (GD_LDS void*)(base + i * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc + k), (GD_LDS void*)(base + EF_ROWS * 128), 16, 0, 0);
+    };
+    for (int s = 0; s < NS && s < steps; ++s) fetch(s, s);
+    ef_floatx4 acc[1] = {{0.f, 0.f, 0.f, 0.f}};
+    const int wplace = col * 128, xplace = EF_ROWS * 128 + col % ES_PAIRS * 128;
+    int stage = 0;                                                                 // of step s
+    for (int s = 0; s < steps; ++s) {
+        gd_wait_younger<3, NS - 1>(steps - 1 - s);                                 // this step has landed
+        asm volatile("" ::: "memory");
+        const unsigned char* const base = mine + stage * ES_STAGE;
+        ef_bf16x8 w[2], x[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            w[h] = *reinterpret_cast<const ef_bf16x8*>(base + wplace + (((quarter * 2 + h) ^ kd_swizzle<8>(col)) * 16));
+            x[h] = *reinterpret_cast<const ef_bf16x8*>(base + xplace + (((quarter * 2 + h) ^ kd_swizzle<8>(col % ES_PAIRS)) * 16));
+        }
+        gd_wait_lds();                                                             // and is in registers: its place is free
+        asm volatile("" ::: "memory");
+        if (s + NS < steps) fetch(stage, s + NS);
+        stage = stage + 1 == NS ? 0 : stage + 1;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h], x[h], acc[0], 0, 0, 0);
+    }
+    __syncthreads();                                                               // (the sums take the place of the stages)
+    const int pair[1] = {list[min(first + col, count - 1)]};
+    ef_finish<1>(g, acc, pair, count, first, row0, reinterpret_cast<float*>(lds));
+}
+
+constexpr int es_room(int NS) { return NS * EF_WAVES * ES_STAGE > EF_WAVES * 2 * KA_WAVE * 16 ? NS * EF_WAVES * ES_STAGE : EF_WAVES * 2 * KA_WAVE * 16; }
+
+// NS: stages of ef_stream (K in steps of 64: the host's check); 0: any K.
+template <int NS>
 __global__ void __launch_bounds__(EF_WAVES * KA_WAVE) experts_few_kernel(ExpertsFewArgs g) {
     __shared__ int list[EF_MAX_PAIRS];
-    __shared__ __attribute__((aligned(16))) float sums[EF_WAVES * 2 * KA_WAVE * 4];
+    __shared__ __attribute__((aligned(16))) unsigned char room[es_room(NS)];
+    float* const sums = reinterpret_cast<float*>(room);
     const int e = blockIdx.y, lane = threadIdx.x % KA_WAVE;
     // (every wave makes the list by itself: all write the same numbers)
     int mine[EF_MAX_PAIRS / KA_WAVE];
@@ -520,7 +598,10 @@ __global__ void __launch_bounds__(EF_WAVES * KA_WAVE) experts_few_kernel(Experts
     const bf16_t* W = g.W + (size_t)e * g.N * g.K;
     const int row0 = blockIdx.x * EF_ROWS;
     for (int first = 0; first < count;) {
-        if (count - first <= 16) {
+        if (NS > 0 && count - first <= ES_PAIRS) {
+            if constexpr (NS > 0) ef_stream<NS>(g, W, list, count, first, row0, room);
+            first += ES_PAIRS;
+        } else if (count - first <= 16) {
             ef_columns<1, 8>(g, W, list, count, first, row0, sums);
             first += 16;
         } else {
@@ -546,7 +627,8 @@ KA_API int ka_experts_few_bf16(const void* a, long lda, int gather_div, const vo
     KA_CHECK(!ka_act_gated(act) || !out_f32, "%s: a gated linear writes bf16", who);
     KA_CHECK((uintptr_t)a % 16 == 0 && (uintptr_t)W % 16 == 0, "%s: operands must be 16-byte aligned", who);
     const ExpertsFewArgs g{(const bf16_t*)a, lda, gather_div, (const bf16_t*)W, chosen, n_pairs, N, K, act, {clamped, limit, slope, shift}, out, ldo, out_f32};
-    hipLaunchKernelGGL(experts_few_kernel, dim3(ka_cdiv(N, EF_ROWS), E), dim3(EF_WAVES * KA_WAVE), 0, stream, g);
+    auto kernel = K % 64 == 0 ? experts_few_kernel<ES_STAGES> : experts_few_kernel<0>;
+    hipLaunchKernelGGL(kernel, dim3(ka_cdiv(N, EF_ROWS), E), dim3(EF_WAVES * KA_WAVE), 0, stream, g);
     KA_LAUNCH_CHECK();
     return 0;
 }
