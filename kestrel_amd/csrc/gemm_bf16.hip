@@ -536,21 +536,23 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
 // The tile and the parts of K for `ka_linear_pair_tiles_bf16`.
 //  * Tiles of 128 x 128: as many parts as leave the fewest K-steps to a CU, a part more than another costing the finishing kernel one more read
 //    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
-//  * The phased tiles of 256 rows where they come out 5 % ahead and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
+//  * The phased tiles of 256 rows where their estimate is no more than 1 % behind and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
 //    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
 //    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 % on the average. Not where more
 //    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
 //    and 23.7 us).
 // Measured with the norm behind, small tiles in the parts they would come in and the phased ones chosen (us): N = 2,048, K = 10,240: 768 rows 54.0 and 47.7,
 // 1,280 rows 84.4 and 66.0; 2,560, 12,800: 385 rows 49.6 and 47.9, 448 rows 52.5 and 49.1, 1,024 rows 108 and 77; 4,096, 12,288, 640 rows 97 and 80.
-// Where the two estimates meet the choice can be the slower one: 2,560, 12,800, 512 rows, small tiles 56.5 (estimated 53.0), phased ones in
-// six parts 50.5 (53.7); at 2,048, 10,240, 512 rows it is right (37.0 and 39.9).
+// Where the two estimates meet (estimates' ratio, small tiles and phased ones as measured): 2,560, 12,800, 512 rows 0.964, 57.1 and 48.5; 480 rows 0.956, 55.4
+// and 48.2; 2,560, 5,120, 640 rows 0.974, 39.1 and 34.8; 2,048, 10,240, 400 to 512 rows 0.962 to 1.006, 33.9 to 36.5 and 33.6 to 35.0; 576 rows
+// 1.020, 41.3 and 42.2; 1,024, 5,120, 900 rows 1.042, 23.1 and 26.0.
 struct PairChoice {
     int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
     double us;
 };
 
-static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased) {
+// lead: how far ahead the phased tiles' estimate has to be (0.99: 1 % behind).
+static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased, double lead) {
     const int cus = ka_compute_units();
     PairChoice best = {0, 0, 0.0};
     const long small = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
@@ -563,6 +565,7 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
     }
     static const struct { int tile, rows_w, rows_x; double step, full, edge, edge_full, sums; } tiles[] = {
         {3, 128, 256, 0.83, 0.19, 8.4, -7.2, 1.93}, {1, 256, 256, 1.05, 0.51, 11.9, -8.6, 1.43}};
+    PairChoice large = {0, 0, 0.0};
     for (const auto& t : tiles) {
         if (!phased || M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L) continue;
         const long each = (long)ka_cdiv(N, t.rows_w) * ka_cdiv(M, t.rows_x);
@@ -570,9 +573,13 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
             const int per = ka_cdiv(steps, parts), last = steps - (parts - 1) * per;
             if (per < 4 || ka_cdiv(steps, per) != parts || last < 2) continue;
             const double load = (double)(each * parts) / cus * (each * parts) / cus;
-            const double us = 1.05 * (per * (t.step + t.full * load) + t.edge + t.edge_full * load + parts * (double)M * N * t.sums * 1e-6);
-            if (best.parts == 0 || us < best.us) best = {t.tile, parts, us};
+            const double us = per * (t.step + t.full * load) + t.edge + t.edge_full * load + parts * (double)M * N * t.sums * 1e-6;
+            if (large.parts == 0 || us < large.us) large = {t.tile, parts, us};
         }
+    }
+    if (large.parts && (best.parts == 0 || lead * large.us < best.us)) {
+        best = large;
+        best.us *= 1.05;               // (what the vendor library is compared with)
     }
     return best;
 }
@@ -584,7 +591,7 @@ static bool pair_tiles_fit(int M, int N, int K1, int K2) {
 // Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles, whose offsets have to fit in 32 bits.
 KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats, int phased) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, 0.99);
     return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
@@ -594,7 +601,7 @@ KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial
 // 158 and 131; 2,560, 5,120: 2,048 rows 83 and 72; 4,096, 8,192: 2,048 rows 140 and 133; in one part 4,096 rows of the last 249 against 243.
 KA_API int ka_linear_pair_large_parts(int M, int N, int K1, int K2, long partial_floats) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true, 1.05);
     const double library = 2.0 * M * N * (double)(K1 + K2) / 0.85e9 + 8.0 + (double)M * N * 10.0 / 4.0e6;
     return c.tile == 1 && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
