@@ -30,15 +30,15 @@ class RoutedExperts(FeedForward):
     (``ops.core.experts_linear``; fp32 always does); up to ``FEW_PAIRS_TO`` every chosen expert's weights are streamed once past its pairs
     (``ops.fast.experts_few_bf16``); beyond, the pairs are listed by expert first and each expert's go through the matrix cores in
     tiles (``ops.fast.experts_feed_forward_bf16``); where width or hidden size is no multiple of 64 the tiles are the slower ones
-    and their turn comes at ``FEW_PAIRS_TO_UNALIGNED``. Measured, both linears, 31 experts of 2,048 x 704, choices of 5: 4 tokens 38 us pair
-    by pair, 38 streamed once, 8 tokens 62 and 56 (lists 61); 30 of them, choices of 4, streamed once and by lists: 16 tokens 59 and 65, 40
-    tokens 69 and 69, 64 tokens 75 and 69, 128 tokens 96 and 73; 62 experts of 4,096 x 896, choices of 6: 16 tokens 235 and 223, 24 tokens 267
-    and 245, 40 tokens 289 and 252. Up to 512 pairs both give the same bits, beyond that all lists do; either way a pair's result
+    and their turn comes at ``FEW_PAIRS_TO_UNALIGNED``. Measured, both linears, 31 experts of 2,048 x 704, choices of 5: 4 tokens 28 us pair
+    by pair, 31 streamed once, 8 tokens 46 and 44; streamed once and by lists: 24 tokens 60 and 69, 40 tokens 66 and 71, 48 tokens (240 pairs) 71.5
+    and 71.0, 64 tokens 80 and 72; 30 of them, choices of 4: 32 tokens 60 and 66, 48 tokens 63 and 66, 64 tokens 68 and 67; 62 experts of 4,096 x
+    896, choices of 6: 16 tokens 206 and 216, 40 tokens 248 and 257, 64 tokens 264 and 259. Up to 512 pairs both give the same bits, beyond that all lists do; either way a pair's result
     depends on its own row alone."""
 
     replays_every_step = True
     PAIR_BY_PAIR_TO = 20
-    FEW_PAIRS_TO = 128
+    FEW_PAIRS_TO = 240
     FEW_PAIRS_TO_UNALIGNED = 512
 
     def __init__(self, spec: RoutedExpertsSpec) -> None:
