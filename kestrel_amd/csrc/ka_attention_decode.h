@@ -197,7 +197,7 @@ attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* 
 
     typedef __attribute__((address_space(1))) const int* at_global_ints;
     const at_global_ints bt = (at_global_ints)(block_table + (size_t)row * max_pages);
-    const int n_pages = (max(hi, 0) + AT_PAGE - 1) / AT_PAGE;
+    const int n_pages = min((max(hi, 0) + AT_PAGE - 1) / AT_PAGE, max_pages);
     const bool table_in_lds = SHORT || n_pages <= AT_LDS_PAGES;
     if (table_in_lds) {   // the row's block table goes to LDS once (see the prompt kernel)
         for (int i = threadIdx.x; i < n_pages; i += KA_WAVE * WAVES) pages[i] = bt[i];
