@@ -413,10 +413,11 @@ KA_API int ka_experts_gemm_bf16(const void* a, long lda, int gather_div, const v
 
 // ----------------------------------------------------------------------------
 // The same linears for a step of few pairs (a decode step), where all that matters is to read every chosen expert's
-// weights once: no lists are made beforehand, and weights go from memory to the matrix cores without LDS. A workgroup owns
+// weights once: no lists are made beforehand. A workgroup owns
 // 16 weight rows of one expert; it looks through the choices for its expert's pairs (an expert that nobody chose ends there), its
 // four waves take every fourth step of 64 inputs each and their sums meet in LDS. Weights are the row operand and pairs
-// the columns, 16 or 32 at a time: a lane ends with four neighbouring outputs of one pair.
+// the columns: a lane ends with four neighbouring outputs of one pair. Up to eight pairs of an expert go with the weights straight into LDS
+// where K is in steps of 64 (ef_stream); 16 or 32 at a time, and any other K, from memory to the matrix cores without LDS.
 // ----------------------------------------------------------------------------
 constexpr int EF_ROWS = 16;
 constexpr int EF_WAVES = 4;

@@ -19,7 +19,8 @@
 // load under a branch makes the compiler wait for ALL loads in flight before the next MFMA,
 // and the loop then pays a trip to memory per round instead of streaming.
 //
-// Two kernels:
+// Up to eight rows, a workgroup whose share is a few strips asks for all of it at once (ka_share.h, with the rule and what both
+// sides measure in gemv_share_bf16.hip and gemv_share_long_bf16.hip). Otherwise two kernels:
 //  * persistent (one K-segment, K up to 64 * 8 * 8): a workgroup loads its share of the
 //    activations into registers ONCE (normalising fp32 rows itself if asked to: the LayerNorm
 //    prologue) and then walks over strips blockIdx.x, + gridDim.x, ...: only weights are

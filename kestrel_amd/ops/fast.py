@@ -150,7 +150,7 @@ ACTIVATION_APART_FROM_COLUMNS = 1024
 # one after the other to the vendor library (``pair_tiles_pay``). Both sides measured over widths of 512 to 8,192, K of 1,024 to
 # 20,480 in all and 65 to 1,536 rows, weights from HBM:
 #  * with the norm that follows, which the library has as a launch of its own, up to 128 tiles at every K (us: 1,024 in all at 2,048, 512 rows
-#    16.5 against 20.2; 4,096 at 2,048, 1,024 rows 32.9 and 36.8; 12,800 at 2,560, 512 rows 56.5 and 79.5), and to 160 where the small tiles
+#    16.5 against 20.2; 4,096 at 2,048, 1,024 rows 32.9 and 36.8; 12,800 at 2,560, 512 rows 48.5 and 79.5), and to 160 where the small tiles
 #    would have K in parts, by whichever tile is then the one (tiles and library: 10,240 at 2,048 61.5 and 92 for 1,025 rows, 66 and 94 for
 #    1,280; 6,144 46.3 and 58.5, 50.1 and 58.5; 12,800 at 2,560 72 and 113 for 769 rows, 77 and 117 for 1,024; 5,120 at 1,024, 2,049 rows
 #    42.5 and 49.6); beyond: ``pair_large_parts``;
