@@ -102,3 +102,22 @@ def test_a_norm_in_front(form, m, na, nb, k):
     for w, out in ((wa, out_a),) + (((wb, out_b),) if nb else ()):
         slack = h_slack @ w.double().abs().T + (k + 4) * 2.0 ** -24 * (h.abs() @ w.double().abs().T)
         assert bool(((out.cpu().double() - h @ w.double().T).abs() <= slack).all())
+
+
+# outputs of two segments: strips of which a CU holds one or two
+@pytest.mark.parametrize("n, k1, k2", [(2048, 2048, 8192), (2560, 2560, 10240), (4096, 4096, 6144), (4096, 2048, 704)])
+def test_two_segments_do_not_depend_on_the_rows_beside(n, k1, k2):
+    """One row alone, among three and among as many as go this way: the same bits."""
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(n + k1 + k2)
+    a = [_rows(gen, 8, k).to(DEV) for k in (k1, k2)]
+    w = [_rows(gen, n, k, k ** -0.5).to(DEV) for k in (k1, k2)]
+    start = torch.randn(8, n, generator=gen).to(DEV)
+    most = 4 if fast.pair_finishes_rows(8, n) else 8           # (five to eight rows of more strips than CUs: K in parts)
+    results = {}
+    for m in (most, 3, 1):
+        out = start[:m].clone()
+        assert fast.linear_pair_accumulate(a[0][:m], w[0], None, a[1][:m], w[1], None, out)
+        results[m] = out
+    assert torch.equal(results[most][:3], results[3]) and torch.equal(results[most][:1], results[1])
