@@ -12,12 +12,15 @@
 
 constexpr int SH_ROWS = 8;                        // most rows
 __host__ __device__ constexpr int sh_threads(bool ln) { return (SP_WAVES + (ln ? 4 : 0)) * KA_WAVE; }
-// LDS: the strips' sums [NS][SP_WAVES][KA_WAVE]; with a norm, two counts of waves (16 bytes), each wave's part of every row's sums, and
-// the rows, [M][K + SK_PAD] in bf16.
+// LDS: the strips' sums [NS][SP_WAVES][KA_WAVE]; with a norm, in their place before there are any, the rows in fp32, [M][K], and behind them
+// three counts of waves (16 bytes), each row's mean and reciprocal deviation, and the normalised rows, [M][K + SK_PAD] in bf16.
 constexpr int SH_NORM = 4;                        // waves that normalise, beside the eight that multiply
-__host__ __device__ constexpr int sh_red_bytes(int NS) { return NS * SP_WAVES * KA_WAVE * 16; }
-constexpr int SH_STATS_BYTES = 16 + SH_NORM * SH_ROWS * 8;
 __host__ __device__ constexpr int sh_min(int a, int b) { return a < b ? a : b; }
+__host__ __device__ constexpr int sh_first_bytes(int NS, bool ln, int M, int K) {
+    const int sums = NS * SP_WAVES * KA_WAVE * 16, rows = ln ? M * K * 4 : 0;
+    return sums > rows ? sums : rows;
+}
+constexpr int SH_STATS_BYTES = 16 + SH_ROWS * 8;
 
 // Workgroup `block` of `grid`: strips block, block + grid, ... (NS of them; past the last strip it reads the last one again and stores nothing).
 // U: k-blocks of a wave. AHEAD: blocks asked for before the first is multiplied (all NS * U, or as many as registers hold).
@@ -26,8 +29,11 @@ __host__ __device__ constexpr int sh_min(int a, int b) { return a < b ? a : b; }
 // LN: the rows are fp32 and normalised here, by waves of their own: a wave is held where it asks for more than the memory takes, so one that first asked
 // for its weights would begin with the norm when most of them have come (stamps, 14,336 outputs of 2,048, 8 rows: rows normalised 10.6 us into
 // 12.7), and one that asks for them behind it leaves the memory idle. These waves share the channels, not the rows: scale and shift are then read once a
-// workgroup (with a row a wave, once a row: 16 K bytes of every 16 K + 8 M K at eight rows). A wave that multiplies waits for the
-// rows and not for the other waves: at a barrier it would wait for the last one's requests.
+// workgroup (with a row a wave, once a row: 16 K bytes of every 16 K + 8 M K at eight rows). The sums of a row have the order of sk_row_statistics, as in every
+// kernel with a norm in front, so a row's numbers do not depend on the rows beside it: the channels that the waves have brought meet in LDS, and a wave
+// takes the sums of whole rows from there (sums by the waves' own channels: 0.1 to 0.3 us less up to 2,048 wide, up to 1.2 less at 2,560 and eight rows of
+// few outputs, nothing from 8,192 outputs on). A wave that multiplies waits for the rows and not for the other waves: at a barrier it would wait for the
+// last one's requests.
 template <int U, int NS, int AHEAD, bool LN, bool PAIR, bool X_BESIDE>
 __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int total_strips, const int block, const int grid, unsigned char* lds) {
     static_assert(AHEAD <= NS * U && AHEAD > 0, "blocks ahead");
@@ -36,10 +42,13 @@ __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int
     constexpr bool ACCUMULATES = NS == 1 && !LN;
     constexpr int WAVES = sh_threads(LN) / KA_WAVE, ADDENDS = (NS + WAVES - 1) / WAVES;
     floatx4* const red = reinterpret_cast<floatx4*>(lds);
-    int* const rows_done = reinterpret_cast<int*>(lds + sh_red_bytes(NS));             // waves whose part of the rows is in LDS
-    int* const sums_done = rows_done + 1;                                              // waves whose part of the rows' sums is
-    float2* const stats = reinterpret_cast<float2*>(rows_done + 4);                    // [SH_NORM][SH_ROWS]
-    bf16_t* const xs = reinterpret_cast<bf16_t*>(lds + sh_red_bytes(NS) + SH_STATS_BYTES);
+    float* const raw = reinterpret_cast<float*>(lds);                                  // [M][K]
+    unsigned char* const behind = lds + sh_first_bytes(NS, LN, p.M, p.K[0]);
+    int* const raw_done = reinterpret_cast<int*>(behind);                              // waves whose part of the fp32 rows is in LDS
+    int* const stats_done = raw_done + 1;                                              // waves whose rows' statistics are
+    int* const rows_done = raw_done + 2;                                               // waves whose part of the normalised rows is
+    float2* const stats = reinterpret_cast<float2*>(raw_done + 4);                     // [SH_ROWS]
+    bf16_t* const xs = reinterpret_cast<bf16_t*>(behind + SH_STATS_BYTES);
     auto await = [](const int* count) {
         while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < SH_NORM) __builtin_amdgcn_s_sleep(1);
         asm volatile("" ::: "memory");
@@ -113,14 +122,9 @@ __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int
     if (LN && wave >= SP_WAVES) {
         if constexpr (LN) {
             constexpr int XJ = (2 * U + SH_NORM - 1) / SH_NORM;       // pieces of four channels a lane and row
+            constexpr bool KEPT = XJ <= 2;                             // (else read once more: 24 pieces beside a whole row spill)
             const int part = wave - SP_WAVES;
             auto channel = [&](int j) { return ((j * SH_NORM + part) * KA_WAVE + lane) * 4; };
-            auto count = [&](int v) {                                  // channels of a row that wave v has
-                int n = 0;
-#pragma unroll
-                for (int j = 0; j < XJ; ++j) n += max(0, min(KA_WAVE * 4, K0 - (j * SH_NORM + v) * KA_WAVE * 4));
-                return (float)n;
-            };
             const float* const shift = p.ln_beta ? p.ln_beta : p.ln_gamma;        // (no shift: the scale once more, left out below)
             floatx4 xf[SH_ROWS][XJ], gamma[XJ], beta[XJ];
 #pragma unroll
@@ -134,51 +138,32 @@ __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int
                 gamma[j] = *(const SK_GLOBAL floatx4*)(p.ln_gamma + min(channel(j), K0 - 4));
                 beta[j] = *(const SK_GLOBAL floatx4*)(shift + min(channel(j), K0 - 4));
             }
-            if (part == 0 && lane == 0) *rows_done = *sums_done = 0;
+            if (part == 0 && lane == 0) *rows_done = *raw_done = *stats_done = 0;
             sk_lds_barrier();
-            const float mine = count(part);
-            float s_mine = 0.f, q_mine = 0.f;                          // lane `of`: this wave's sum of row `of`, and its squares about their own mean
+            auto report = [&](int* count) {
+                __builtin_amdgcn_s_waitcnt(0xc07f);                    // (what this wave wrote is in LDS)
+                asm volatile("" ::: "memory");
+                if (lane == 0) __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            };
 #pragma unroll
             for (int of = 0; of < SH_ROWS; ++of)
                 if (of < M) {
-                    float s = 0.f, q = 0.f;
-#pragma unroll
-                    for (int j = 0; j < XJ; ++j) {
-                        if (channel(j) >= K0) xf[of][j] = zero4;
-                        s += (xf[of][j][0] + xf[of][j][1]) + (xf[of][j][2] + xf[of][j][3]);
-                    }
-                    s = ka_wave_sum(s);
-                    const float centre = p.ln_uncentred || mine == 0.f ? 0.f : s / mine;
 #pragma unroll
                     for (int j = 0; j < XJ; ++j)
-                        if (channel(j) < K0) {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) q += (xf[of][j][i] - centre) * (xf[of][j][i] - centre);
-                        }
-                    q = ka_wave_sum(q);
-                    s_mine = lane == of ? s : s_mine;
-                    q_mine = lane == of ? q : q_mine;
+                        if (channel(j) < K0) *reinterpret_cast<floatx4*>(raw + of * K0 + channel(j)) = xf[of][j];
                 }
-            if (lane < SH_ROWS) stats[part * SH_ROWS + lane] = make_float2(s_mine, q_mine);
-            __builtin_amdgcn_s_waitcnt(0xc07f);
-            asm volatile("" ::: "memory");
-            if (lane == 0) __hip_atomic_fetch_add(sums_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            await(sums_done);
-            // row lane % 8: the squares about its mean are those about each part's own, and the parts' means about the row's
-            float total = 0.f, squares = 0.f;
-            float2 parts[SH_NORM];
+            report(raw_done);
+            await(raw_done);
+#pragma unroll 1
+            for (int of = part; of < M; of += SH_NORM) {
+                floatx4 row[2 * U];
 #pragma unroll
-            for (int v = 0; v < SH_NORM; ++v) {
-                parts[v] = stats[v * SH_ROWS + lane % SH_ROWS];
-                total += parts[v].x;
+                for (int j = 0; j < 2 * U; ++j) row[j] = *reinterpret_cast<const floatx4*>(raw + of * K0 + min((j * KA_WAVE + lane) * 4, K0 - 4));
+                const float2 mean_rstd = sk_row_statistics(p, K0, lane, row);
+                if (lane == 0) stats[of] = mean_rstd;
             }
-            const float row_mean = p.ln_uncentred ? 0.f : total / (float)K0;
-#pragma unroll
-            for (int v = 0; v < SH_NORM; ++v) {
-                const float n = count(v), d = p.ln_uncentred || n == 0.f ? 0.f : parts[v].x / n - row_mean;
-                squares += parts[v].y + n * d * d;
-            }
-            const float row_rstd = 1.0f / sqrtf(squares / (float)K0 + p.ln_eps);
+            report(stats_done);
+            await(stats_done);
             const bool shifted = p.ln_beta != nullptr, stored = p.ln_store != nullptr && block == 0;
 #pragma unroll
             for (int j = 0; j < XJ; ++j)
@@ -186,9 +171,10 @@ __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int
 #pragma unroll
             for (int of = 0; of < SH_ROWS; ++of)
                 if (of < M) {
-                    const float mean = ka_lane_value(row_mean, of), rstd = ka_lane_value(row_rstd, of);
+                    const float mean = stats[of].x, rstd = stats[of].y;
 #pragma unroll
                     for (int j = 0; j < XJ; ++j) {
+                        if constexpr (!KEPT) xf[of][j] = *reinterpret_cast<const floatx4*>(raw + of * K0 + min(channel(j), K0 - 4));
                         bf16x4 y;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) y[i] = (bf16_t)((xf[of][j][i] - mean) * rstd * gamma[j][i] + beta[j][i]);
@@ -199,9 +185,7 @@ __device__ __forceinline__ void skinny_share_body(const SkinnyArgs& p, const int
                         }
                     }
                 }
-            __builtin_amdgcn_s_waitcnt(0xc07f);
-            asm volatile("" ::: "memory");
-            if (lane == 0) __hip_atomic_fetch_add(rows_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            report(rows_done);
         }
     } else {
         if constexpr (!LN && !X_BESIDE) sk_static_for<U>([&](auto u) { x[u.value] = load_x(u.value); });
@@ -263,7 +247,7 @@ skinny_share_kernel(SkinnyArgs p, int strips) {
 template <int U, int NS, int AHEAD, bool LN, bool PAIR, bool X_BESIDE>
 static int launch_share(const SkinnyArgs& args, int strips, hipStream_t stream) {
     auto kernel = skinny_share_kernel<U, NS, AHEAD, LN, PAIR, X_BESIDE>;
-    const int lds = sh_red_bytes(NS) + (LN ? SH_STATS_BYTES + args.M * (args.K[0] + SK_PAD) * (int)sizeof(bf16_t) : 0);
+    const int lds = sh_first_bytes(NS, LN, args.M, args.K[0]) + (LN ? SH_STATS_BYTES + args.M * (args.K[0] + SK_PAD) * (int)sizeof(bf16_t) : 0);
     static int reserved = 64 * 1024;
     if (lds > reserved) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);

@@ -195,25 +195,33 @@ __device__ __forceinline__ void sk_fetch_row(const SkinnyArgs& p, int m, int lan
     }
 }
 
-template <int XV, bool EARLY>
-__device__ __forceinline__ void sk_normalise_row(const SkinnyArgs& p, bf16_t* xs, int m, int lane, RowOperands<XV, EARLY>& row) {
-    const int K = p.K[0], ld = K + SK_PAD;
+// Mean and reciprocal deviation of a row of K that one wave holds, four channels at (j * KA_WAVE + lane) * 4 a lane and j: the one order of these sums,
+// whatever kernel normalises the row. x past K becomes zero.
+template <int XV>
+__device__ __forceinline__ float2 sk_row_statistics(const SkinnyArgs& p, const int K, const int lane, floatx4 (&x)[XV]) {
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
-        if ((j * KA_WAVE + lane) * 4 >= K) row.x[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        s += (row.x[j][0] + row.x[j][1]) + (row.x[j][2] + row.x[j][3]);
+        if ((j * KA_WAVE + lane) * 4 >= K) x[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        s += (x[j][0] + x[j][1]) + (x[j][2] + x[j][3]);
     }
-    float mean = p.ln_uncentred ? 0.f : ka_wave_sum(s) / (float)K;
+    const float mean = p.ln_uncentred ? 0.f : ka_wave_sum(s) / (float)K;
     float q = 0.f;
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         if ((j * KA_WAVE + lane) * 4 < K) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) q += (row.x[j][i] - mean) * (row.x[j][i] - mean);
+            for (int i = 0; i < 4; ++i) q += (x[j][i] - mean) * (x[j][i] - mean);
         }
     }
-    float rstd = 1.0f / sqrtf(ka_wave_sum(q) / (float)K + p.ln_eps);
+    return make_float2(mean, 1.0f / sqrtf(ka_wave_sum(q) / (float)K + p.ln_eps));
+}
+
+template <int XV, bool EARLY>
+__device__ __forceinline__ void sk_normalise_row(const SkinnyArgs& p, bf16_t* xs, int m, int lane, RowOperands<XV, EARLY>& row) {
+    const int K = p.K[0], ld = K + SK_PAD;
+    const float2 of = sk_row_statistics(p, K, lane, row.x);
+    const float mean = of.x, rstd = of.y;
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int k = (j * KA_WAVE + lane) * 4;

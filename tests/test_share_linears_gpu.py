@@ -121,3 +121,28 @@ def test_two_segments_do_not_depend_on_the_rows_beside(n, k1, k2):
         assert fast.linear_pair_accumulate(a[0][:m], w[0], None, a[1][:m], w[1], None, out)
         results[m] = out
     assert torch.equal(results[most][:3], results[3]) and torch.equal(results[most][:1], results[1])
+
+
+# K: two to five blocks a wave, in steps of 64 and not; outputs: one to seven strips a CU
+@pytest.mark.parametrize("n, k", [(2048, 1096), (6144, 1536), (4100, 2008), (14336, 2048), (40, 2048), (6144, 2560), (2052, 2104)])
+@pytest.mark.parametrize("form", ["shift", "no shift", "uncentred"])
+def test_a_norm_in_front_does_not_depend_on_the_rows_beside(form, n, k):
+    """One to sixteen rows, on either side of eight: the same bits of a row, and of what is left of the norm. Rows of one sign, whose sums have to round."""
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(n + k)
+    x = (torch.randn(16, k, generator=gen).abs() * torch.linspace(0.5, 40.0, 16)[:, None]).to(DEV)
+    gamma, beta = torch.randn(k, generator=gen).to(DEV), torch.randn(k, generator=gen).to(DEV)
+    w = _rows(gen, n, k, k ** -0.5).to(DEV)
+    results = {}
+    for m in (16, 9, 8, 7, 4, 1):
+        out, left = torch.full((m, n), float("nan"), device=DEV), torch.full((m, k), float("nan"), dtype=torch.bfloat16, device=DEV)
+        if form == "uncentred":
+            assert fast.layernorm_linear(x[:m], gamma, None, 1e-5, w, None, out, 0, centred=False)
+            left = None
+        else:
+            assert fast.layernorm_linear(x[:m], gamma, beta if form == "shift" else None, 1e-5, w, None, out, 0, store=left)
+        results[m] = (out, left)
+    for m, (out, left) in results.items():
+        assert torch.equal(out, results[16][0][:m]), m
+        assert left is None or torch.equal(left, results[16][1][:m]), m
