@@ -368,7 +368,7 @@ static int sk_compute_units() { return ka_compute_units(); }
 
 // The persistent kernel is used wherever it fits; switching it off is for measurements and for
 // tests of the split kernel on sizes that it otherwise never sees.
-int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, hipStream_t stream);      // gemv_share_bf16.hip
+int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, int split_waves, hipStream_t stream);      // gemv_share_bf16.hip
 
 static int sk_persistent_enabled = 1;
 KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enabled; }
@@ -504,16 +504,23 @@ KA_API int ka_linear_skinny_choice(const void* A, long lda, const void* W, long 
     return 0;
 }
 
+// Waves over K of the split kernel, 4, 8 or 16 (the nearest): enough workgroups x waves to fill the chip, no more than there are rounds for.
+// 16 waves leave 128 registers a lane, enough only for the half-column form.
+static int sk_split_waves(int M, int strips, int kblocks, int target_waves) {
+    const int MB = ka_cdiv(M, 16), un = MB == 1 ? 4 : MB == 2 ? 2 : 1;
+    const int wanted = ka_cdiv(target_waves, strips), rounds = ka_cdiv(kblocks, un), waves = wanted < rounds ? wanted : rounds;
+    return waves >= 12 && M <= 8 ? 16 : waves >= 6 ? 8 : 4;
+}
+
 template <int MB, bool HALF>
 static int launch_split(int waves, int strips, hipStream_t stream, const SkinnyArgs& args) {
-    // (rounded to the nearest of 4, 8 and 16)
-    if (waves >= 12) {
-        if constexpr (HALF) {      // 16 waves leave 128 registers a lane: enough only for the half-column form
+    if constexpr (HALF) {
+        if (waves == 16) {
             hipLaunchKernelGGL((skinny_split_kernel<MB, 16, HALF>), dim3(strips), dim3(16 * KA_WAVE), 0, stream, args);
             return 0;
         }
     }
-    if (waves >= 6) hipLaunchKernelGGL((skinny_split_kernel<MB, 8, HALF>), dim3(strips), dim3(8 * KA_WAVE), 0, stream, args);
+    if (waves == 8) hipLaunchKernelGGL((skinny_split_kernel<MB, 8, HALF>), dim3(strips), dim3(8 * KA_WAVE), 0, stream, args);
     else hipLaunchKernelGGL((skinny_split_kernel<MB, 4, HALF>), dim3(strips), dim3(4 * KA_WAVE), 0, stream, args);
     return 0;
 }
@@ -591,7 +598,7 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         const size_t dyn = (size_t)M * (K1 + SK_PAD) * sizeof(bf16_t);
         KA_CHECK(dyn <= 96 * 1024, "%s: %d rows of %d do not fit in LDS", who, M, K1);
         KA_CHECK(persistent_fits(M, kblocks, args), "%s: K=%d or the biases do not suit the LayerNorm prologue", who, K1);
-        const int shared = sk_persistent_enabled ? ka_skinny_share(args, strips, kblocks, true, stream) : 1;
+        const int shared = sk_persistent_enabled ? ka_skinny_share(args, strips, kblocks, true, 0, stream) : 1;
         if (shared <= 0) return shared;
         if (launch_persistent(strips, M, kblocks, true, dyn, stream, args)) return -1;
         KA_LAUNCH_CHECK();
@@ -671,8 +678,9 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         if (then)
             ka_launch_finish_norm(M, Na, stream, nullptr, 0, nullptr, nullptr, (float*)outa, ldoa, 0, *then);
     };
+    const int waves = sk_split_waves(M, strips, kblocks, target_waves);
     if (sk_persistent_enabled) {
-        const int shared = ka_skinny_share(args, strips, kblocks, false, stream);
+        const int shared = ka_skinny_share(args, strips, kblocks, false, persistent_ok ? 0 : waves, stream);
         if (shared < 0) return -1;
         if (shared == 0) {
             norm_after();
@@ -687,10 +695,6 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         KA_LAUNCH_CHECK();
         return 0;
     }
-    // waves over K: enough workgroups x waves to fill the chip, no more than there are rounds for
-    int waves = ka_cdiv(target_waves, strips);
-    const int un = MB == 1 ? 4 : MB == 2 ? 2 : 1;
-    if (waves > ka_cdiv(kblocks, un)) waves = ka_cdiv(kblocks, un);
     int rc;
     if (M <= 8) rc = launch_split<1, true>(waves, strips, stream, args);
     else switch (MB) {

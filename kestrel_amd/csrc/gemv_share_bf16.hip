@@ -28,9 +28,13 @@ int ka_skinny_share_long(const SkinnyArgs& args, int strips, int per, bool crowd
 // rows 22.0 -> 19.2; 9,280 of 2,048, one row 10.5 -> 9.3, eight 11.2 -> 9.0; 5,632 of 2,048 gated, eight 8.7 -> 7.0; 4,096 of 4,096, eight 9.7 -> 8.7;
 // 2,048 of 2,048 4.2 -> 4.1; 2,048 of 2,048 + 8,192, one row 9.8 -> 9.3, eight 12.5 -> 12.1; 2,560 of 2,560 + 10,240, four rows 24.0 -> 21.7.
 // What bounds them now: requests, which the memory takes at 5 to 5.5 TB/s once all CUs ask, and 2 us of a launch's start and end.
+// split_waves: the waves over K that the split kernel would take, where that one has the call otherwise (else 0). With four of them there the call stays there:
+// nine to sixteen rows have four as well, and eight here would be another order of a row's sums. (Where it would take sixteen, nine to sixteen rows have the eight of here; error
+// of the fp32 sums against 64 bits, 256 to 1,488 outputs of 3,072 to 10,752: 1.147e-7 of their norm with eight waves, 1.131e-7 with sixteen.)
 // 1: not covered, nothing was run.
-int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, hipStream_t stream) {
+int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, int split_waves, hipStream_t stream) {
     const bool pair = args.A[1] != nullptr;
+    if (split_waves == 4) return 1;
     const int cus = ka_compute_units(), per = ka_cdiv(kblocks, SP_WAVES), NS = ka_cdiv(strips, cus);
     if (args.M > SH_ROWS || !persistent_bias_ok(args.a) || !persistent_bias_ok(args.b)) return 1;
     for (long ld : {args.a.ldw, args.b.ldw, args.ldw2, args.lda[0], args.lda[1]})

@@ -146,3 +146,20 @@ def test_a_norm_in_front_does_not_depend_on_the_rows_beside(form, n, k):
     for m, (out, left) in results.items():
         assert torch.equal(out, results[16][0][:m]), m
         assert left is None or torch.equal(left, results[16][1][:m]), m
+
+
+# Where the split kernel has nine to sixteen rows: with four waves over K (many strips, or accumulation over a short K), with eight, with eight where it had
+# sixteen up to eight rows (few strips)
+@pytest.mark.parametrize("n, k, accumulate", [(3288, 4608, False), (4096, 8448, True), (512, 1024, True), (2048, 1280, True), (2048, 1288, True), (2048, 4608, False),
+                                              (3272, 8448, True), (256, 8448, False), (1000, 4096, True)])
+def test_a_long_or_accumulated_linear_does_not_depend_on_the_rows_beside(n, k, accumulate):
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(n + k)
+    a, w, start = _rows(gen, 16, k).to(DEV), _rows(gen, n, k, k ** -0.5).to(DEV), torch.randn(16, n, generator=gen).to(DEV)
+    results = {}
+    for m in (16, 9, 8, 5, 1):
+        results[m] = start[:m].clone()
+        assert fast.linear_bf16(a[:m], w, None, results[m], 0, accumulate)
+    for m, out in results.items():
+        assert torch.equal(out, results[16][:m]), m
