@@ -40,6 +40,7 @@ int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, in
     for (long ld : {args.a.ldw, args.b.ldw, args.ldw2, args.lda[0], args.lda[1]})
         if (ld >= 1L << 26) return 1;          // (offsets of eight rows in 32 bits)
     if (args.bias2 && (args.a.N % 4 || (uintptr_t)args.bias2 % 16)) return 1;
+    if (args.a.accumulate && args.b.W) return 1;        // (the body adds a's old values, whichever target a strip has)
     if (args.a.accumulate && (args.a.N % 4 || args.a.ldo % 4 || (uintptr_t)args.a.out % 16)) return 1;
     if (ln) {
         // (rows of up to 1,024: the persistent kernel. In the form for two blocks the compiler keeps the rows in memory, 7.5 against 5.2 us)

@@ -163,3 +163,25 @@ def test_a_long_or_accumulated_linear_does_not_depend_on_the_rows_beside(n, k, a
         assert fast.linear_bf16(a[:m], w, None, results[m], 0, accumulate)
     for m, out in results.items():
         assert torch.equal(out, results[16][:m]), m
+
+
+@pytest.mark.parametrize("m", [1, 5, 8, 12])
+@pytest.mark.parametrize("na, nb, k", [(64, 136, 512), (136, 64, 1024), (1000, 1048, 4096)])
+def test_accumulation_into_the_first_of_two_targets(m, na, nb, k):
+    """The entry point's accumulation is the first target's alone: the second one's outputs are new, also where it is the wider one, and
+    its rows lie beside numbers that stay."""
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(m + na + k)
+    a, wa, wb = _rows(gen, m, k), _rows(gen, na, k, k ** -0.5), _rows(gen, nb, k, k ** -0.5)
+    start = torch.randn(m, na, generator=gen)
+    ad, wad, wbd, out_a = a.to(DEV), wa.to(DEV), wb.to(DEV), start.to(DEV)
+    room = torch.full((m, nb + 8), 7.0, device=DEV)
+    out_b = room[:, :nb]
+    fast._check(fast.lib().ka_linear_skinny_fused(
+        ad.data_ptr(), k, k, None, 0, 0, None, 0, None, None, None, None, 0.0, wad.data_ptr(), k, None, out_a.data_ptr(), 0, na, na, 0, 1,
+        wbd.data_ptr(), k, None, out_b.data_ptr(), 0, nb + 8, nb, 0, m, fast.chip_sizes(ad.device).skinny_target_waves, None, 0, fast.stream_ptr()))
+    want_a = a.double() @ wa.double().T + start.double()
+    assert bool(((out_a.cpu().double() - want_a).abs() <= _sum_slack(a, wa, k) + 2.0 ** -23 * (start.abs() + want_a.abs())).all())
+    assert bool(((out_b.cpu().double() - a.double() @ wb.double().T).abs() <= _sum_slack(a, wb, k) + 1e-30).all())
+    assert bool((room[:, nb:] == 7.0).all())
