@@ -145,7 +145,8 @@ attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* 
     const int lo = kv_lo ? kv_lo[t] : 0;
     const bool fused = fz.slots != nullptr && kv_hi[t] > 0;
     const int pos = kv_hi[t] - 1;                 // fused: the token's own position, whose key is not cached yet
-    const int hi = fused ? pos : kv_hi[t];        // cached keys this token reads: [lo, hi)
+    // cached keys this token reads: [lo, hi), no more than its row of the table has pages for
+    const int hi = (int)min((long)(fused ? pos : kv_hi[t]), (long)max_pages * AT_PAGE);
     // this unit's rounds: round r holds the keys [tile0, tile_hi) of round_keys(r) (a row without keys,
     // hi <= lo, has no pages and no rounds: nothing of the cache is touched)
     constexpr bool EVEN = WAVES == 4;
@@ -197,7 +198,7 @@ attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* 
 
     typedef __attribute__((address_space(1))) const int* at_global_ints;
     const at_global_ints bt = (at_global_ints)(block_table + (size_t)row * max_pages);
-    const int n_pages = min((max(hi, 0) + AT_PAGE - 1) / AT_PAGE, max_pages);
+    const int n_pages = (max(hi, 0) + AT_PAGE - 1) / AT_PAGE;
     const bool table_in_lds = SHORT || n_pages <= AT_LDS_PAGES;
     if (table_in_lds) {   // the row's block table goes to LDS once (see the prompt kernel)
         for (int i = threadIdx.x; i < n_pages; i += KA_WAVE * WAVES) pages[i] = bt[i];
