@@ -749,9 +749,15 @@ static int decode_launch(const char* who, const void* q, long q_row_stride, cons
     // (Rows of up to 2,048 keys, going by the width of the block table: behind 4,096 keys a row the larger tile
     // came out 2 to 3 % ahead at 24 and 32 rows, level at 48 and 64.)
     const bool small_tiles = waves == 4 && hd <= 64 && max_pages <= AD_SMALL_TILE_MAX_PAGES && groups * 2 >= 3L * cus && groups <= 8L * cus;
-    const bool short_rows = max_pages <= AT_LDS_PAGES;
+    // Tables that fit in LDS read as LDS (SHORT): what it saves is waits of a chain of trips to memory. Up to 64 channels it is ahead or level everywhere (us, either
+    // pointer and LDS: one row of 700 keys 7.50 and 7.28, eight of 1,050 15.15 and 15.04, 24 of 1,050 33.5 and 33.6). Above, where registers leave few waves, it
+    // is ahead where few workgroups wait for their chains (80: one row of 4,000 40.0 and 38.9, four of 1,050 14.75 and 14.51; 128: 41.2 and 40.6, 15.0 and
+    // 14.5; 160: 73.5 and 68.9; 256: four of 1,050 29.0 and 26.7) and behind where memory is the bound, from about a workgroup on every other CU
+    // on (80: eight rows of 4,000 56.2 and 57.1; 128: 47.2 and 48.0; 192: 94.2 and 97.6; 256: 115 and 126).
+    const bool table_fits = max_pages <= AT_LDS_PAGES;
+    const bool short_rows = table_fits && (hd <= 64 || (waves == 8 && groups * (hd <= 96 ? 2 : 4) <= cus));
 #define KA_AD(HDV, WV, TPV)                                                                                         \
-    hipLaunchKernelGGL((short_rows ? attn_decode_kernel<HDV, WV, TPV, true> : attn_decode_kernel<HDV, WV, TPV, false>), grid, block, 0, stream, (const bf16_t*)q, q_row_stride, \
+    hipLaunchKernelGGL((short_rows ? attn_decode_kernel<HDV, WV, TPV, HDV <= 64 || WV == 8> : attn_decode_kernel<HDV, WV, TPV, false>), grid, block, 0, stream, (const bf16_t*)q, q_row_stride, \
                        (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, token_row, kv_lo,   \
                        kv_hi, (bf16_t*)out, out_row_stride, scale, H, Hkv, partial, fz)
 #define KA_AD_SMALL(HDV)                                                                                            \

@@ -130,15 +130,17 @@ KA_API int ka_attention_decode_beside_bf16(const void* q, long q_row_stride, con
         hipLaunchKernelGGL((attn_decode_beside_kernel<HDV, PERV, SHORTV>), grid, block, dyn, stream, a, p, strips,  \
                            (int)attention_groups, linear_groups);                                                   \
     }
+#define KA_BS_TABLE(HDV, PERV)                                                                                      \
+    { if (max_pages <= AT_LDS_PAGES) KA_BS_LAUNCH(HDV, PERV, true) else KA_BS_LAUNCH(HDV, PERV, false) }
 #define KA_BS(HDV)                                                                                                  \
     case HDV:                                                                                                       \
-        if (max_pages > AT_LDS_PAGES) KA_BS_LAUNCH(HDV, 4, false)                                                   \
-        else if (per <= 1) KA_BS_LAUNCH(HDV, 1, true) else if (per <= 2) KA_BS_LAUNCH(HDV, 2, true) else KA_BS_LAUNCH(HDV, 4, true) \
+        if (per <= 1) KA_BS_TABLE(HDV, 1) else if (per <= 2) KA_BS_TABLE(HDV, 2) else KA_BS_TABLE(HDV, 4)           \
         break;
     switch (hd) {
         KA_BS(16) KA_BS(32) KA_BS(48) KA_BS(64)
     }
 #undef KA_BS
+#undef KA_BS_TABLE
 #undef KA_BS_LAUNCH
     KA_LAUNCH_CHECK();
     if (splits > 1) {

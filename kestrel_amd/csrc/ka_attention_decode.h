@@ -116,7 +116,7 @@ __device__ __forceinline__ void at_rotated(const RotaryOperands& r, const Rotary
 // than one tile and the kernel is a chain of trips (few rows), no gain where it streams (many rows).
 // (A tile's values asked for together with its keys instead: slower, 11.8 against 11.2 us for the
 // attention of one row with eight waves.)
-// SHORT: no row has more than AT_LDS_PAGES pages (the host goes by the width of the block table).
+// SHORT: no row has more than AT_LDS_PAGES pages (the host goes by the width of the block table, and by what it measured).
 template <int HD, int WAVES, bool SHORT, bool AHEAD = false, int TP = AD_TILE_PAGES>
 __device__ __forceinline__ void
 attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* __restrict__ k_cache,
@@ -196,13 +196,14 @@ attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* 
         for (int u = 0; u < VU; ++u) vnew[u] = vrow[min(u * 32 + lane / 2, HD - 1)];
     }
 
-    typedef __attribute__((address_space(1))) const int* at_global_ints;
-    const at_global_ints bt = (at_global_ints)(block_table + (size_t)row * max_pages);
-    const int n_pages = (max(hi, 0) + AT_PAGE - 1) / AT_PAGE;
-    const bool table_in_lds = SHORT || n_pages <= AT_LDS_PAGES;
-    if (table_in_lds) {   // the row's block table goes to LDS once (see the prompt kernel)
-        for (int i = threadIdx.x; i < n_pages; i += KA_WAVE * WAVES) pages[i] = bt[i];
-        __syncthreads();
+    const int* bt = block_table + (size_t)row * max_pages;
+    {   // the row's block table goes to LDS once (see the prompt kernel)
+        const int n_pages = (max(hi, 0) + AT_PAGE - 1) / AT_PAGE;
+        if (SHORT || n_pages <= AT_LDS_PAGES) {
+            for (int i = threadIdx.x; i < n_pages; i += KA_WAVE * WAVES) pages[i] = bt[i];
+            __syncthreads();
+            if constexpr (!SHORT) bt = pages;
+        }
     }
     // q, and the token's own key and value, have had the time of the block table's trip
     float qf[8];
@@ -256,120 +257,115 @@ attn_decode_body(const bf16_t* __restrict__ q, long q_row_stride, const bf16_t* 
     // has room for TP pages and may hold fewer: what it does not hold is masked like any other place
     // outside (jumping over its arithmetic, the same for all lanes, cuts the tile's straight run of
     // instructions into pieces: 1,215 against 1,247 tok/s at one row).
-    // The table is read as what it is, LDS or memory, in a loop of its own each: through one pointer to either, every entry is a load that counts as both,
-    // and each use of one waits for all keys and values in flight. (A kernel with both loops has registers for neither at head size 80: 20.8 against 17.8 us,
-    // eight rows; hence SHORT. One row's 750 keys beside a linear 11.7 -> 11.4 us, eight rows of 800 to 1,050 16.1 -> 15.7.)
-    auto walk = [&](auto page_of) {
-        auto load_keys = [&](int tile0, int tile_hi, bf16x8 (&dst)[KL]) {
+    // SHORT reads the table as what it is, LDS: through one pointer to LDS or memory every entry is a load that counts as both, and each use of one waits for
+    // all keys and values in flight. (A kernel with a loop for each has registers for neither at head size 80, four waves: 67.2 against 57.3 us, 64 rows of 500.)
+    auto page_of = [&](int i) {
+        if constexpr (SHORT) return pages[i];
+        else return bt[i];
+    };
+    auto load_keys = [&](int tile0, int tile_hi, bf16x8 (&dst)[KL]) {
 #pragma unroll
-            for (int i = 0; i < KL; ++i) {
-                int key = tile0 + i * KPI + ks;
-                int kc = max(min(key, tile_hi - 1), lo);   // a place that holds data (pages below lo may be gone)
-                int page = page_of(kc / AT_PAGE);
-                dst[i] = at_load8(k_cache + (((size_t)page * Hkv + kvh) * AT_PAGE + kc % AT_PAGE) * HD + dg * 8);
-            }
-        };
-        // round r of this unit: keys [tile0, tile_hi)
-        auto round_keys = [&](int r, int& tile0, int& tile_hi) {
-            const int page0 = mine0 + r * (EVEN ? per : units * TP);
-            tile0 = page0 * AT_PAGE;
-            tile_hi = min(mine_hi, (page0 + per) * AT_PAGE);
-        };
-        bf16x8 kreg[KL], knext[AHEAD ? KL : 1];
-        if constexpr (AHEAD) {
-            if (rounds > 0) {
-                int t0, t1;
-                round_keys(0, t0, t1);
-                load_keys(t0, t1, kreg);
-            }
-        }
-        for (int r = 0; r < rounds; ++r) {
-            int tile0, tile_hi;
-            round_keys(r, tile0, tile_hi);
-            if constexpr (AHEAD) {
-                // (past the last round: the last round's keys once more, which nobody uses)
-                int n0, n1;
-                round_keys(min(r + 1, rounds - 1), n0, n1);
-                load_keys(n0, n1, knext);
-            } else {
-                load_keys(tile0, tile_hi, kreg);
-            }
-            __builtin_amdgcn_sched_barrier(0);     // all of them, before the first is used
-            float sc[KL];
-            float mx = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < KL; ++i) {
-                int key = tile0 + i * KPI + ks;
-                bool ok = key >= lo && key < tile_hi;
-                float dot = 0.f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) dot = fmaf(qf[j], (float)kreg[i][j], dot);
-                dot = ka_lanes_reduce<1, LPK>(dot, KaSum{});           // the LPK lanes of a key
-                sc[i] = ok ? dot : -INFINITY;
-                mx = fmaxf(mx, sc[i]);
-            }
-            mx = ka_lanes_reduce<LPK, KA_WAVE>(mx, KaMax{});            // (the lanes of a key hold one value)
-            float m_new = fmaxf(m_i, mx);                               // finite: the tile holds a key of [lo, hi)
-            // the values: asked for as soon as the keys' registers are free, all at once; the softmax
-            // below runs while they are on their way
-            bf16x8 vreg[TP][VU];
-#pragma unroll
-            for (int pg = 0; pg < TP; ++pg) {
-                int kc = max(min(tile0 + pg * AT_PAGE, tile_hi - 1), lo);
-                int page = page_of(kc / AT_PAGE);
-#pragma unroll
-                for (int u = 0; u < VU; ++u) {
-                    int d = min(u * 32 + lane / 2, HD - 1);
-                    vreg[pg][u] = at_load8(v_cache + (((size_t)page * Hkv + kvh) * HD + d) * AT_PAGE + (lane & 1) * 8);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            float alpha = exp2f(m_i - m_new);
-            float rowsum = 0.f;
-            at_wave_sync();                        // the previous tile's probabilities have been read
-#pragma unroll
-            for (int i = 0; i < KL; ++i) {
-                float p = exp2f(sc[i] - m_new);
-                rowsum += p;
-                if (dg_lane == 0) ps[wave][i * KPI + ks] = p;
-            }
-            rowsum = ka_lanes_reduce<LPK, KA_WAVE>(rowsum, KaSum{});
-            l_i = l_i * alpha + rowsum;
-            m_i = m_new;
-#pragma unroll
-            for (int u = 0; u < VU; ++u) acc[u] *= alpha;
-            at_wave_sync();
-            // values: a page is HD rows of 16 keys; a lane holds 8 keys (half a row) per load
-#pragma unroll
-            for (int pg = 0; pg < TP; ++pg) {
-                const int half = lane & 1;
-                const int first = tile0 + pg * AT_PAGE + half * 8;
-                float pv[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) pv[j] = ps[wave][pg * AT_PAGE + half * 8 + j];
-#pragma unroll
-                for (int u = 0; u < VU; ++u) {
-                    float sum = 0.f;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        int key = first + j;                      // slots outside the data may hold anything
-                        float x = key >= lo && key < tile_hi ? (float)vreg[pg][u][j] : 0.f;
-                        sum = fmaf(pv[j], x, sum);
-                    }
-                    acc[u] += sum;
-                }
-            }
-            if constexpr (AHEAD) {
-#pragma unroll
-                for (int i = 0; i < KL; ++i) kreg[i] = knext[i];
-            }
+        for (int i = 0; i < KL; ++i) {
+            int key = tile0 + i * KPI + ks;
+            int kc = max(min(key, tile_hi - 1), lo);   // a place that holds data (pages below lo may be gone)
+            int page = page_of(kc / AT_PAGE);
+            dst[i] = at_load8(k_cache + (((size_t)page * Hkv + kvh) * AT_PAGE + kc % AT_PAGE) * HD + dg * 8);
         }
     };
-    if constexpr (SHORT) {
-        walk([&](int i) { return pages[i]; });
-    } else {
-        if (table_in_lds) walk([&](int i) { return pages[i]; });
-        else walk([&](int i) { return bt[i]; });
+    // round r of this unit: keys [tile0, tile_hi)
+    auto round_keys = [&](int r, int& tile0, int& tile_hi) {
+        const int page0 = mine0 + r * (EVEN ? per : units * TP);
+        tile0 = page0 * AT_PAGE;
+        tile_hi = min(mine_hi, (page0 + per) * AT_PAGE);
+    };
+    bf16x8 kreg[KL], knext[AHEAD ? KL : 1];
+    if constexpr (AHEAD) {
+        if (rounds > 0) {
+            int t0, t1;
+            round_keys(0, t0, t1);
+            load_keys(t0, t1, kreg);
+        }
+    }
+    for (int r = 0; r < rounds; ++r) {
+        int tile0, tile_hi;
+        round_keys(r, tile0, tile_hi);
+        if constexpr (AHEAD) {
+            // (past the last round: the last round's keys once more, which nobody uses)
+            int n0, n1;
+            round_keys(min(r + 1, rounds - 1), n0, n1);
+            load_keys(n0, n1, knext);
+        } else {
+            load_keys(tile0, tile_hi, kreg);
+        }
+        __builtin_amdgcn_sched_barrier(0);     // all of them, before the first is used
+        float sc[KL];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            int key = tile0 + i * KPI + ks;
+            bool ok = key >= lo && key < tile_hi;
+            float dot = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) dot = fmaf(qf[j], (float)kreg[i][j], dot);
+            dot = ka_lanes_reduce<1, LPK>(dot, KaSum{});           // the LPK lanes of a key
+            sc[i] = ok ? dot : -INFINITY;
+            mx = fmaxf(mx, sc[i]);
+        }
+        mx = ka_lanes_reduce<LPK, KA_WAVE>(mx, KaMax{});            // (the lanes of a key hold one value)
+        float m_new = fmaxf(m_i, mx);                               // finite: the tile holds a key of [lo, hi)
+        // the values: asked for as soon as the keys' registers are free, all at once; the softmax
+        // below runs while they are on their way
+        bf16x8 vreg[TP][VU];
+#pragma unroll
+        for (int pg = 0; pg < TP; ++pg) {
+            int kc = max(min(tile0 + pg * AT_PAGE, tile_hi - 1), lo);
+            int page = page_of(kc / AT_PAGE);
+#pragma unroll
+            for (int u = 0; u < VU; ++u) {
+                int d = min(u * 32 + lane / 2, HD - 1);
+                vreg[pg][u] = at_load8(v_cache + (((size_t)page * Hkv + kvh) * HD + d) * AT_PAGE + (lane & 1) * 8);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float alpha = exp2f(m_i - m_new);
+        float rowsum = 0.f;
+        at_wave_sync();                        // the previous tile's probabilities have been read
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            float p = exp2f(sc[i] - m_new);
+            rowsum += p;
+            if (dg_lane == 0) ps[wave][i * KPI + ks] = p;
+        }
+        rowsum = ka_lanes_reduce<LPK, KA_WAVE>(rowsum, KaSum{});
+        l_i = l_i * alpha + rowsum;
+        m_i = m_new;
+#pragma unroll
+        for (int u = 0; u < VU; ++u) acc[u] *= alpha;
+        at_wave_sync();
+        // values: a page is HD rows of 16 keys; a lane holds 8 keys (half a row) per load
+#pragma unroll
+        for (int pg = 0; pg < TP; ++pg) {
+            const int half = lane & 1;
+            const int first = tile0 + pg * AT_PAGE + half * 8;
+            float pv[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) pv[j] = ps[wave][pg * AT_PAGE + half * 8 + j];
+#pragma unroll
+            for (int u = 0; u < VU; ++u) {
+                float sum = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    int key = first + j;                      // slots outside the data may hold anything
+                    float x = key >= lo && key < tile_hi ? (float)vreg[pg][u][j] : 0.f;
+                    sum = fmaf(pv[j], x, sum);
+                }
+                acc[u] += sum;
+            }
+        }
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int i = 0; i < KL; ++i) kreg[i] = knext[i];
+        }
     }
     // the two halves of a channel row
 #pragma unroll

@@ -66,3 +66,32 @@ def test_a_row_longer_than_its_table_reads_what_the_table_holds(hd, waves, width
             values = torch.cat([case.v[t][:end, head // 2].double(), v_new[t, head // 2][None]])
             want[t, head] = torch.softmax(keys @ q[t, head] * hd ** -0.5, dim=0) @ values
     _close(out, want.view(4, -1), torch.bfloat16)
+
+
+# K of the linear beside it: one, two and four blocks of 64 a wave
+@pytest.mark.parametrize("h, hkv, hd, k", [(4, 4, 64, 512), (6, 2, 48, 520), (2, 1, 16, 1024), (32, 32, 64, 2048)])
+def test_a_wider_table_changes_nothing_beside_a_linear(h, hkv, hd, k):
+    """The launch with a linear layer on the side, rows behind tables of their own width, of 2,048 and of 2,049 entries: the same bits of both."""
+    from kestrel_amd.ops import fast
+    from kestrel_amd.parts import SideLinear
+
+    gen = torch.Generator().manual_seed(hd + k)
+    lens = [1000, 33, 64][:max(1, 128 // h)]
+    case = PagedCase(lens, [1] * len(lens), h, hkv, hd, 16, torch.bfloat16, seed=hd)
+    n = len(lens)
+    a, w = (torch.randn(rows, k, generator=gen).bfloat16().to(DEV) for rows in (n, 520))
+    q, rows = case.q.to(DEV), case.table
+    results = []
+    for width in (rows.shape[1], 2048, 2049):
+        table = torch.zeros(rows.shape[0], width, dtype=torch.int32, device=DEV)
+        table[:, :rows.shape[1]] = rows
+        out, linear = torch.full((n, h * hd), float("nan"), dtype=torch.bfloat16, device=DEV), torch.full((n, 520), float("nan"), device=DEV)
+        job = SideLinear(a, w, None, linear, 0)
+        assert fast.attention_decode_takes(job, n, h, hd, 16, case.batch.max_kv)
+        assert fast.attention_decode_bf16(q, case.k_cache, case.v_cache, table, case.token_row, None, case.kv_hi, out, hd ** -0.5, h, hkv, hd, case.batch, beside=job)
+        results.append((out, linear))
+    _close(results[0][0], case.reference(hd ** -0.5), torch.bfloat16)
+    want = a.double() @ w.double().T
+    assert bool(((results[0][1].double() - want).abs() <= (k + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+    for out, linear in results[1:]:
+        assert torch.equal(out, results[0][0]) and torch.equal(linear, results[0][1])
