@@ -27,18 +27,26 @@ class RoutedExperts(FeedForward):
     (``[E, 2 hidden, dim]``, plain ones ``[E, hidden, dim]``; ``[E, dim, hidden]``). A step runs: the router's linear (fp32), the choice
     (``ops.core.route``), the experts' two linears, and the weighted sum. In bf16, by the number of pairs (token, choice): a
     step of up to ``PAIR_BY_PAIR_TO`` computes every pair by itself, its expert's weights streamed for it
-    (``ops.core.experts_linear``; fp32 always does); up to ``FEW_PAIRS_TO`` every chosen expert's weights are streamed once past its pairs
-    (``ops.fast.experts_few_bf16``); beyond, the pairs are listed by expert first and each expert's go through the matrix cores in
-    tiles (``ops.fast.experts_feed_forward_bf16``); where width or hidden size is no multiple of 64 the tiles are the slower ones
-    and their turn comes at ``FEW_PAIRS_TO_UNALIGNED``. Measured, both linears, 31 experts of 2,048 x 704, choices of 5: 4 tokens 28 us pair
-    by pair, 31 streamed once, 8 tokens 46 and 44; streamed once and by lists: 24 tokens 60 and 69, 40 tokens 66 and 71, 48 tokens (240 pairs) 71.5
-    and 71.0, 64 tokens 80 and 72; 30 of them, choices of 4: 32 tokens 60 and 66, 48 tokens 63 and 66, 64 tokens 68 and 67; 62 experts of 4,096 x
-    896, choices of 6: 16 tokens 206 and 216, 40 tokens 248 and 257, 64 tokens 264 and 259. Up to 512 pairs both give the same bits, beyond that all lists do; either way a pair's result
+    (``ops.core.experts_linear``; fp32 always does); up to ``few_pairs_to()`` every chosen expert's weights are streamed past its pairs
+    (``ops.fast.experts_few_bf16``: once up to 32 pairs of an expert, once more for every further 32); beyond, the pairs are listed by expert first and each
+    expert's go through the matrix cores in tiles (``ops.fast.experts_feed_forward_bf16``). Where width or hidden size is no multiple of 64 the tiles are the
+    slower ones and their turn comes at ``FEW_PAIRS_TO_UNALIGNED``; else at ``FEW_PAIRS_TO``, and with many experts at
+    ``FEW_PAIRS_AN_EXPERT`` an expert on the average, up to ``FEW_PAIRS_SPREAD_TO``: the stream's own form takes eight pairs of an expert, and fewer on
+    the average leave room for choices that crowd. A shared expert among the experts, which has a pair of every token, keeps the lower line. Measured, both linears, streamed and by lists, us; choices spread evenly, crowded (an
+    expert's frequency as its rank to the power of -1.5), and over half of the experts: 62 experts of 4,096 x 896, choices of 6, 126 pairs 227 and 238, 152
+    and 160, 138 and 139; 198 pairs 235 and 250, 180 and 189, 142 and 140; 240 pairs 246 and 252, 204 and 192, 156 and 142. 30 experts of
+    2,048 x 704, choices of 4, 128 pairs 61 and 69, 50 and 59, 42 and 42; 160 pairs 63 and 67, 53 and 58, 44 and 41; 240 pairs 70 and 68, 68
+    and 69, 54 and 43. 30 of them beside a shared one, choices of 5, 130 pairs 68 and 72, 59 and 60, 52 and 45; 200 pairs 80 and 71, 75
+    and 64, 66 and 48. 16 experts of 2,048 x 1,408, choices of 4, 128 pairs 72 and 68, 69 and 70, 52 and 47; 160 pairs 77 and 69, 75 and
+    71, 56 and 47; 8 of them, choices of 2, 160 pairs 58 and 51, 63 and 48, 58 and 39. Pair by pair and streamed, 31 experts, choices of 5: 4 tokens 28
+    and 31, 8 tokens 46 and 44. Up to 512 pairs both give the same bits, beyond that all lists do; either way a pair's result
     depends on its own row alone."""
 
     replays_every_step = True
     PAIR_BY_PAIR_TO = 20
-    FEW_PAIRS_TO = 240
+    FEW_PAIRS_TO = 128
+    FEW_PAIRS_SPREAD_TO = 240
+    FEW_PAIRS_AN_EXPERT = 4
     FEW_PAIRS_TO_UNALIGNED = 512
 
     def __init__(self, spec: RoutedExpertsSpec) -> None:
@@ -145,6 +153,14 @@ class RoutedExperts(FeedForward):
             core.gated_pairs(first, hidden, self.act)
         return hidden
 
+    def few_pairs_to(self) -> int:
+        """Most pairs of a step that go past streamed weights instead of by lists."""
+        spec = self.spec
+        if spec.dim % 64 or spec.hidden_dim % 64:
+            return self.FEW_PAIRS_TO_UNALIGNED
+        spread = 0 if self.joined else min(self.FEW_PAIRS_AN_EXPERT * spec.n_experts, self.FEW_PAIRS_SPREAD_TO)
+        return max(self.FEW_PAIRS_TO, spread)
+
     def _outputs(self, h, batch):
         """Everything but the weighted sum: the pairs' outputs, the choice, its weights, the shared expert's output and gate."""
         from ..ops import fast
@@ -182,8 +198,7 @@ class RoutedExperts(FeedForward):
         done = False
         if self.dtype == torch.bfloat16 and n * top > self.PAIR_BY_PAIR_TO:
             operands = (h, self.pairs, self.down, chosen, hidden, y, self.up_act)
-            few_to = self.FEW_PAIRS_TO if spec.dim % 64 == 0 and spec.hidden_dim % 64 == 0 else self.FEW_PAIRS_TO_UNALIGNED
-            done = n * top <= few_to and fast.experts_few_bf16(*operands, clamp=self.clamp)
+            done = n * top <= self.few_pairs_to() and fast.experts_few_bf16(*operands, clamp=self.clamp)
             done = done or fast.experts_feed_forward_bf16(*operands, ws, clamp=self.clamp)
         if not done:
             flat = chosen.view(-1)
