@@ -269,22 +269,34 @@ static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, c
     return 0;
 }
 
-// The tile: the one that takes the fewest blocks of 32 x 32 x K one after the other on the fullest CU, weighed by the rate the
-// tile reaches where CUs are full (TFLOP/s: smaller tiles read L2 and LDS more often per product). All give the same bits.
+// The tile: the one that is done first by what was measured (us per 2,048 of K: a first part, and as much again for every round of one tile a CU). All give the
+// same bits. Fitted to every tile's times at 17 to 2,048 rows of 1,024 x 1,024, 2,048 x 2,048, 2,560 x 2,560, 6,144 x 2,048, 8,192 x 2,048, 2,048 x 8,192 and 10,240 x 2,560
+// (outputs x inputs), tiles a CU rounded up, us per 2,048 of K, average of all sizes:
+//              1     2     3     4     5     6     7     8    10    12
+//   64 x 128   98   157   231   309
+//   64 x 64    45    83   122   159   198   235   269
+//   64 x 32    28    49    70    92   112   132   153   174   216   258
+//   32 x 32    17    29    41    51    61    73    82    95   116   138
+// What it chooses is 0.2 % behind the fastest tile on the average and 3.5 % at most (1,024 x 1,024, 350 rows). By a rate for each tile alone, without the
+// first part, it was up to 20 % behind: tiles of 64 x 128 one a CU do not overlap a start with anything (2,048 x 2,048, 1,024 rows 105 us, now 90).
 // K-steps: of 32 where a workgroup has a CU to itself and where every wave waits for nobody (tiles of 32 x 32, a part of K a wave: no barrier; with one
 // a step 2,048 of 8,192 took 144 us at 304 rows, 133 without); of 16, half the LDS and so two or three workgroups a CU, where there are more tiles
-// of 64 x 32 or 64 x 64 than CUs (304 rows, steps of 32 and 16: 8,192 of 2,048 124 and 116, 6,144 of 2,048 87.2 and 86.9, at 320 rows 87.6 and 83.0, at
-// 450 129 and 121; one a CU, 64 rows of 2,048 x 2,048 by 64 x 32: 25.9 and 32.5). Three and four stages of 16 were slower at every size.
+// of 64 x 32 or 64 x 64 than CUs (steps of 32 and 16, 64 x 64: 6,144 of 2,048, 304 rows 88.0 and 84.7, 450 rows 128.7 and 123.5; 64 x 32: 8,192 of 2,048,
+// 304 rows 122.7 and 112.9; one a CU: 64 x 64 of 2,048 x 8,192, 450 rows 161.5 and 163.3, 64 x 32 of 2,048 x 2,048, 64 rows 26.9 and 33.1).
+// Three and four stages of 16 were slower at every size.
 static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
     const int cus = ka_compute_units();
     auto tiles = [&](int bn, int bm) { return (long)ka_cdiv(N, bn) * ka_cdiv(M, bm); };
-    auto cost = [&](int bn, int bm, float rate) { return ka_cdiv(tiles(bn, bm), cus) * (float)(bn * bm) / rate; };
-    const float t128 = cost(64, 128, 112.f), t64 = cost(64, 64, 112.f), t32 = cost(64, 32, 95.f), t1 = cost(32, 32, 92.f);
+    auto us = [&](int bn, int bm, float first, float round) { return first + ka_cdiv(tiles(bn, bm), cus) * round; };
+    const float t128 = us(64, 128, 40.f, 62.f), t64 = us(64, 64, 3.5f, 39.5f), t32 = us(64, 32, 8.f, 21.f), t1 = us(32, 32, 6.f, 11.f);
     const float best = fminf(fminf(t128, t64), fminf(t32, t1));
 #define KA_F32(...) return launch_f32_mfma<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
     if (t128 <= best) KA_F32(1, 2, 2, 2, 1, 32, 2);
-    if (t64 <= best) KA_F32(1, 2, 2, 1, F32_PARTS, 16, 2);
+    if (t64 <= best) {
+        if (tiles(64, 64) > cus) KA_F32(1, 2, 2, 1, F32_PARTS, 16, 2);
+        KA_F32(1, 2, 2, 1, F32_PARTS, 32, 2);
+    }
     if (t32 <= best) {
         if (tiles(64, 32) > cus) KA_F32(1, 1, 2, 1, F32_PARTS, 16, 2);
         KA_F32(1, 1, 2, 1, F32_PARTS, 32, 2);
