@@ -75,7 +75,7 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 
 // Many rows in fp32 where K is a multiple of 32: true fp32 products and sums on the matrix pipes (v_mfma_f32_32x32x2_f32, twice
 // the rate of the vector unit without packed FMAs), operands straight from memory into swizzled LDS as in ka_dma_tiles.h (a
-// K-step of 32 numbers is the same 128 bytes a row, of 16 the same 64), NS stages of STEP numbers.
+// K-step of 32 numbers is the same 128 bytes a row, of 16 the same 64), two stages of STEP numbers.
 //
 // The order of a sum is fixed by K alone. Every sixteen k are summed from zero (of every eight in the order 0 4 1 5 2 6 3 7: a lane
 // holds four neighbours), these sums are added in order within a part, K being cut into F32_PARTS parts, and the parts' sums
@@ -91,7 +91,7 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 constexpr int F32_PARTS = 4;
 constexpr int F32_STEP = 32;
 
-template <int WN, int WM, int GN, int GM, int KG, int STEP, int NS>
+template <int WN, int WM, int GN, int GM, int KG, int STEP>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM * KG)
 gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
                      float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
@@ -120,7 +120,7 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
         const int r = kd_load_row<CPR>(part_wave * X_LOADS + i, lane);
         xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2;
     }
-    unsigned char* mine = gf_lds + group * NS * STAGE;
+    unsigned char* mine = gf_lds + group * 2 * STAGE;
     auto fetch = [&](int stage, int k) {
         unsigned char* base = mine + stage * STAGE;
 #pragma unroll
@@ -146,19 +146,15 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
     const int first = KG == 1 ? 0 : group * part_steps;
     const int steps = max(0, min(KG == 1 ? k_steps : part_steps, k_steps - first));
     const int rounds = KG == 1 ? k_steps : min(part_steps, k_steps);           // (the same for every wave: barriers)
-#pragma unroll
-    for (int s = 0; s < NS - 1; ++s)
-        if (s < steps) fetch(s, (first + s) * STEP);
+    if (steps > 0) fetch(0, first * STEP);
     int done = 0;                                                              // KG == 1: parts added into `sum`
-    int stage = 0;                                                             // of step s
     for (int s = 0; s < rounds; ++s) {
-        gd_wait_younger<W_LOADS + X_LOADS, NS - 2>(steps - 1 - s);             // own loads of this step have landed
+        gd_wait_loads<0>();                                                    // own loads of this step have landed
         gd_wait_lds();                                                         // own reads of the step before are in registers
         if constexpr (WAVES > 1) gd_barrier();                                 // (a wave that has its part of K to itself reads what it asked for)
-        if (s + NS - 1 < steps) fetch(stage == 0 ? NS - 1 : stage - 1, (first + s + NS - 1) * STEP);
+        if (s + 1 < steps) fetch((s + 1) & 1, (first + s + 1) * STEP);
         if (s < steps) {
-            const unsigned char* base = mine + stage * STAGE;
-            stage = stage + 1 == NS ? 0 : stage + 1;
+            const unsigned char* base = mine + (s & 1) * STAGE;
 #pragma unroll
             for (int g = 0; g < STEP / 16; ++g) {
                 floatx4 w[2][WN], x[2][WM];
@@ -248,13 +244,13 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
     }
 }
 
-template <int WN, int WM, int GN, int GM, int KG, int STEP, int NS>
+template <int WN, int WM, int GN, int GM, int KG, int STEP>
 static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
-    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * NS * (BN + BM) * STEP * 4;
+    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * 2 * (BN + BM) * STEP * 4;
     static_assert(KG == 1 || smem >= KG * GN * GM * WN * WM * 4 * KA_WAVE * 16, "the parts' sums fit");
     static bool configured = false;
-    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG, STEP, NS>;
+    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG, STEP>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         KA_CHECK(e == hipSuccess, "ka_linear_generic: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
@@ -292,16 +288,16 @@ static int launch_f32_best(const float* A, long lda, const float* W, long ldw, c
     const float t128 = us(64, 128, 40.f, 62.f), t64 = us(64, 64, 3.5f, 39.5f), t32 = us(64, 32, 8.f, 21.f), t1 = us(32, 32, 6.f, 11.f);
     const float best = fminf(fminf(t128, t64), fminf(t32, t1));
 #define KA_F32(...) return launch_f32_mfma<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
-    if (t128 <= best) KA_F32(1, 2, 2, 2, 1, 32, 2);
+    if (t128 <= best) KA_F32(1, 2, 2, 2, 1, 32);
     if (t64 <= best) {
-        if (tiles(64, 64) > cus) KA_F32(1, 2, 2, 1, F32_PARTS, 16, 2);
-        KA_F32(1, 2, 2, 1, F32_PARTS, 32, 2);
+        if (tiles(64, 64) > cus) KA_F32(1, 2, 2, 1, F32_PARTS, 16);
+        KA_F32(1, 2, 2, 1, F32_PARTS, 32);
     }
     if (t32 <= best) {
-        if (tiles(64, 32) > cus) KA_F32(1, 1, 2, 1, F32_PARTS, 16, 2);
-        KA_F32(1, 1, 2, 1, F32_PARTS, 32, 2);
+        if (tiles(64, 32) > cus) KA_F32(1, 1, 2, 1, F32_PARTS, 16);
+        KA_F32(1, 1, 2, 1, F32_PARTS, 32);
     }
-    KA_F32(1, 1, 1, 1, F32_PARTS, 32, 2);
+    KA_F32(1, 1, 1, 1, F32_PARTS, 32);
 #undef KA_F32
 }
 
