@@ -410,7 +410,7 @@ pair_tiles_kernel(KaPairTiles p) {
 // Bound by the K-steps that follow one another on a CU, 0.5 to 0.6 us each whatever the stages in flight (three to five: 73 to
 // 71 us for K = 8,192 alone on 64 CUs): parts of K spread them over all CUs. Measured with the norm that follows, against the
 // vendor library's two products and the norm's launch (us; K = 2,560 + 10,240, N = 2,560): 128 rows 31 against 78, 512 rows
-// 56.5 (three parts) against 83, 1,024 rows 108 against 117.
+// 56.5 (three parts) against 83, 1,024 rows 108 against 117 (where the phased tiles of 256 rows take over: pair_tiles_choice).
 constexpr int PT_TILE = 128, PT_BK = 64, PT_STAGES = 5, PT_TILE_CODE = 100;
 
 template <int WN, int WM, int GN, int GM, int NS, int SL>

@@ -366,10 +366,10 @@ skinny_wide_kernel(WideArgs p) {
 // ----------------------------------------------------------------------------
 static int sk_compute_units() { return ka_compute_units(); }
 
-// The persistent kernel is used wherever it fits; switching it off is for measurements and for
-// tests of the split kernel on sizes that it otherwise never sees.
 int ka_skinny_share(const SkinnyArgs& args, int strips, int kblocks, bool ln, int split_waves, hipStream_t stream);      // gemv_share_bf16.hip
 
+// Whole shares at once and the persistent kernel: switching both off is for measurements and for tests of the split kernel on sizes
+// that it otherwise never sees (the LayerNorm prologue then still runs in the persistent kernel, the only other one that has it).
 static int sk_persistent_enabled = 1;
 KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enabled; }
 // The wide kernel (17 to 64 rows, activations through LDS, parts of K in scratch memory): 1 where
@@ -383,9 +383,8 @@ KA_API void ka_skinny_set_wide(int enabled) { sk_wide_enabled = enabled; }
 
 template <int PER, int MB, bool HALF, bool LN>
 static int launch_persistent_one(int grid, size_t dyn, int strips, hipStream_t stream, const SkinnyArgs& args) {
-    // two strips ahead where one workgroup has a CU (and its registers) to itself (three, which the
-    // registers would still hold, were measured slower: 6.56k against 6.72k tok/s at batch 8; for five
-    // k-blocks a wave, K = 2560, likewise: 523 against 537 tok/s at one row)
+    // two strips ahead where one workgroup has a CU (and its registers) to itself (measured when every layer's linears of at most
+    // eight rows ran here; three, which the registers would still hold, were 1 to 3 % of a decode step slower)
     constexpr int DEPTH = LN && PER <= 4 ? 3 : 2;
     if (dyn > 0) {
         static size_t reserved = 0;

@@ -1,7 +1,8 @@
 // Linears of at most eight rows whose workgroups hold their whole share of the weights: all of it is asked for at once.
 //
-// The products are those of ka_skinny.h, in the same order (the same bits): strips of 8 weight rows, eight waves that take the k-blocks of a
-// strip in turn, the waves' sums added in their order. What differs is that nothing of a workgroup's way depends on a number known at
+// The products are those of ka_skinny.h: strips of 8 weight rows, eight waves that take the k-blocks of a strip in turn, the waves' sums added in their
+// order, rows with a norm in front summed by sk_row_statistics. So a row has the bits that the persistent kernel gives it, and those of the split kernel where
+// that one has eight waves over K. What differs is that nothing of a workgroup's way depends on a number known at
 // run time only: strips and blocks are unrolled, so that every load can be issued where it stands and waited for by count. A loop over
 // strips cannot have that here: what a round has asked for moves to other registers for the next one, and the compiler waits for all of it
 // to do so; a value chosen as soon as it is loaded (no bias: zero) waits for it there too. With few strips a workgroup, which is what a

@@ -12,7 +12,8 @@ DEV = "cuda:0"
 
 # K: one step for one of the four waves, less than a step each, as many steps as stages and more, the loop for any K; N: less than 16 rows, a rest
 @pytest.mark.parametrize("n, k", [(8, 64), (24, 128), (36, 192), (40, 704), (1408, 2048), (20, 832), (40, 200)])
-# pairs per expert: one, eight, nine (eight and one), seventeen to thirty-three (32 at a time by the loop, then the rest)
+# pairs per expert: one and eight (the stream), nine to sixteen (16 columns by the loop), seventeen (32 by the loop), thirty-three and forty (32 by the loop, the
+# rest of up to eight by the stream)
 @pytest.mark.parametrize("counts", [(1, 0, 3), (8, 9, 1), (16, 17, 2), (33, 0, 40)])
 @pytest.mark.parametrize("per", [1, 3])
 def test_one_linear_of_listed_pairs(per, counts, n, k):
@@ -40,7 +41,7 @@ def test_one_linear_of_listed_pairs(per, counts, n, k):
 
 @pytest.mark.parametrize("k", [192, 2048])
 def test_a_pair_has_the_same_bits_alone_and_among_others(k):
-    """Alone, among eight, nine and thirty-three pairs of its expert: by the stream, by the loops, by either for the rest."""
+    """Alone and among eight pairs of its expert (the stream), nine and sixteen (the loop of 16), thirty-three (the loop of 32, the last one by the stream)."""
     from kestrel_amd.ops import fast
 
     gen = torch.Generator().manual_seed(k)

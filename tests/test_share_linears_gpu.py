@@ -185,3 +185,33 @@ def test_accumulation_into_the_first_of_two_targets(m, na, nb, k):
     assert bool(((out_a.cpu().double() - want_a).abs() <= _sum_slack(a, wa, k) + 2.0 ** -23 * (start.abs() + want_a.abs())).all())
     assert bool(((out_b.cpu().double() - a.double() @ wb.double().T).abs() <= _sum_slack(a, wb, k) + 1e-30).all())
     assert bool((room[:, nb:] == 7.0).all())
+
+
+# more than nine strips a CU, which the kernel that loops over strips has
+@pytest.mark.parametrize("m", [1, 5, 8])
+@pytest.mark.parametrize("n, k", [(20484, 520), (20484, 2048), (51200, 1024), (51200, 2048), (18436, 2560), (18436, 4096)])
+def test_more_strips_than_a_share(m, n, k):
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(m + n + k)
+    a, w, bias = _rows(gen, m, k).to(DEV), _rows(gen, n, k, k ** -0.5).to(DEV), torch.randn(n, generator=gen).to(DEV)
+    out = torch.full((m, n), float("nan"), device=DEV)
+    assert fast.linear_bf16(a, w, bias, out, 0, False)
+    want = a.double() @ w.double().T + bias.double()
+    slack = (k + 4) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 2.0 ** -23 * want.abs()
+    assert bool(((out.double() - want).abs() <= slack).all())
+
+
+@pytest.mark.parametrize("n, k", [(520, 512), (2048, 2048), (4100, 1544), (6148, 2560), (18436, 1024)])
+def test_one_linear_does_not_depend_on_the_rows_beside(n, k):
+    """Up to 64 rows where the kernel that loops over strips keeps their activations (K up to 2,560): the same bits of a row."""
+    from kestrel_amd.ops import fast
+
+    gen = torch.Generator().manual_seed(n + k)
+    a, w = _rows(gen, 64, k).to(DEV), _rows(gen, n, k, k ** -0.5).to(DEV)
+    results = {}
+    for m in (64, 17, 16, 9, 8, 5, 1):
+        results[m] = torch.full((m, n), float("nan"), device=DEV)
+        assert fast.linear_bf16(a[:m], w, None, results[m], 0, False)
+    for m, out in results.items():
+        assert torch.equal(out, results[64][:m]), m
