@@ -536,22 +536,25 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
 // The tile and the parts of K for `ka_linear_pair_tiles_bf16`.
 //  * Tiles of 128 x 128: as many parts as leave the fewest K-steps to a CU, a part more than another costing the finishing kernel one more read
 //    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
-//  * The phased tiles of 256 rows where their estimate is no more than 1 % behind and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
+//  * The phased tiles of 256 rows where their estimate is ahead, by 1 % if they take 32 us or more, else by 5 %, and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
 //    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
 //    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 % on the average. Not where more
 //    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
 //    and 23.7 us).
 // Measured with the norm behind, small tiles in the parts they would come in and the phased ones chosen (us): N = 2,048, K = 10,240: 768 rows 54.0 and 47.7,
 // 1,280 rows 84.4 and 66.0; 2,560, 12,800: 385 rows 49.6 and 47.9, 448 rows 52.5 and 49.1, 1,024 rows 108 and 77; 4,096, 12,288, 640 rows 97 and 80.
-// Where the two estimates meet (estimates' ratio, small tiles and phased ones as measured): 2,560, 12,800, 512 rows 0.964, 57.1 and 48.5; 480 rows 0.956, 55.4
-// and 48.2; 2,560, 5,120, 640 rows 0.974, 39.1 and 34.8; 2,048, 10,240, 400 to 512 rows 0.962 to 1.006, 33.9 to 36.5 and 33.6 to 35.0; 576 rows
-// 1.020, 41.3 and 42.2; 1,024, 5,120, 900 rows 1.042, 23.1 and 26.0.
+// Where the two estimates meet, both sides measured at 336 sizes (512 to 4,096 wide, K of 2,560 to 20,480, estimates' ratio of 0.93 to 1.03): the phased tiles of
+// 32 us or more that this takes are 5 % ahead on the average, up to 16 % (2,560, 12,800: 480 rows 55.4 and 48.2 us, 512 rows 57.3 and 50.0; 2,048, 12,800, 512 rows 47.6 and 41.0), and 3 % behind at
+// most (768, 10,240, 1,049 rows 32.2 and 33.2; 3,072, 20,480, 309 rows 72.5 and 74.3); shorter ones are up to 20 % behind, their start and end being more
+// than the estimate has (1,024, 5,120, 769 rows 22.4 and 26.1; 2,048, 4,096, 771 rows 28.6 and 30.3; 1,024, 8,192, 769 rows 28.7 and 31.1).
 struct PairChoice {
     int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
     double us;
 };
 
-// lead: how far ahead the phased tiles' estimate has to be (0.99: 1 % behind).
+constexpr double PT_LONG_US = 32.0, PT_LEAD_SHORT = 1.05;
+
+// lead: how far ahead the estimate of phased tiles of PT_LONG_US or more has to be.
 static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased, double lead) {
     const int cus = ka_compute_units();
     PairChoice best = {0, 0, 0.0};
@@ -577,7 +580,7 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
             if (large.parts == 0 || us < large.us) large = {t.tile, parts, us};
         }
     }
-    if (large.parts && (best.parts == 0 || lead * large.us < best.us)) {
+    if (large.parts && (best.parts == 0 || (large.us < PT_LONG_US ? PT_LEAD_SHORT : lead) * large.us < best.us)) {
         best = large;
         best.us *= 1.05;               // (what the vendor library is compared with)
     }
@@ -591,7 +594,7 @@ static bool pair_tiles_fit(int M, int N, int K1, int K2) {
 // Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles, whose offsets have to fit in 32 bits.
 KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats, int phased) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, 0.99);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, 1.01);
     return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
