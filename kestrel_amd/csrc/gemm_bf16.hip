@@ -536,26 +536,32 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
 // The tile and the parts of K for `ka_linear_pair_tiles_bf16`.
 //  * Tiles of 128 x 128: as many parts as leave the fewest K-steps to a CU, a part more than another costing the finishing kernel one more read
 //    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
-//  * The phased tiles of 256 rows where their estimate is ahead, by 1 % if they take 32 us or more, else by 5 %, and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
+//  * The phased tiles of 256 rows where their estimate says so (pair_lead) and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
 //    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
 //    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 % on the average. Not where more
 //    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
 //    and 23.7 us).
 // Measured with the norm behind, small tiles in the parts they would come in and the phased ones chosen (us): N = 2,048, K = 10,240: 768 rows 54.0 and 47.7,
 // 1,280 rows 84.4 and 66.0; 2,560, 12,800: 385 rows 49.6 and 47.9, 448 rows 52.5 and 49.1, 1,024 rows 108 and 77; 4,096, 12,288, 640 rows 97 and 80.
-// Where the two estimates meet, both sides measured at 336 sizes (512 to 4,096 wide, K of 2,560 to 20,480, estimates' ratio of 0.93 to 1.03): the phased tiles of
-// 32 us or more that this takes are 5 % ahead on the average, up to 16 % (2,560, 12,800: 480 rows 55.4 and 48.2 us, 512 rows 57.3 and 50.0; 2,048, 12,800, 512 rows 47.6 and 41.0), and 3 % behind at
-// most (768, 10,240, 1,049 rows 32.2 and 33.2; 3,072, 20,480, 309 rows 72.5 and 74.3); shorter ones are up to 20 % behind, their start and end being more
-// than the estimate has (1,024, 5,120, 769 rows 22.4 and 26.1; 2,048, 4,096, 771 rows 28.6 and 30.3; 1,024, 8,192, 769 rows 28.7 and 31.1).
 struct PairChoice {
     int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
     double us;
 };
 
-constexpr double PT_LONG_US = 32.0, PT_LEAD_SHORT = 1.05;
+// How far ahead of the small tiles' the estimate of phased tiles that take `us` has to be (0.99: 1 % behind will do). Both sides measured at 336 sizes where the estimates meet
+// (512 to 4,096 wide, K of 2,560 to 20,480, their ratio 0.93 to 1.03):
+//  * Short ones are up to 20 % slower, their start and end being more than the estimate has (1,024, 5,120, 769 rows 22.4 and 26.1 us; 2,048, 4,096, 771 rows 28.6 and
+//    30.3; 1,024, 8,192, 769 rows 28.7 and 31.1).
+//  * Longer ones that this takes are 5 % faster on the average, up to 16 % (2,560, 12,800: 480 rows 55.4 and 48.2, 512 rows 57.3 and 50.0; 2,048, 12,800, 512
+//    rows 47.6 and 41.0), and 3 % slower at most (768, 10,240, 1,049 rows 32.2 and 33.2; 3,072, 20,480, 309 rows 72.5 and 74.3).
+//  * Rows that fill the last tile count for the phased ones (2,048, 10,240, 490 rows 36.4 and 35.1 at a ratio of 0.998; 1,536, 12,800, 513 rows 43.1 and 46.9 at 1.005).
+static double pair_lead(int M, double us) {
+    if (us < 33.0) return 1.05;
+    return M * 10L >= ka_cdiv(M, 256) * 256 * 8L ? 0.99 : 1.01;
+}
 
-// lead: how far ahead the estimate of phased tiles of PT_LONG_US or more has to be.
-static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased, double lead) {
+// large_only: the small tiles are not among what the caller can take; the phased ones then have to be well ahead of them.
+static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats, bool phased, bool large_only) {
     const int cus = ka_compute_units();
     PairChoice best = {0, 0, 0.0};
     const long small = (long)ka_cdiv(N, PT_TILE) * ka_cdiv(M, PT_TILE);
@@ -580,7 +586,7 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
             if (large.parts == 0 || us < large.us) large = {t.tile, parts, us};
         }
     }
-    if (large.parts && (best.parts == 0 || (large.us < PT_LONG_US ? PT_LEAD_SHORT : lead) * large.us < best.us)) {
+    if (large.parts && (best.parts == 0 || (large_only ? 1.05 : pair_lead(M, large.us)) * large.us < best.us)) {
         best = large;
         best.us *= 1.05;               // (what the vendor library is compared with)
     }
@@ -594,7 +600,7 @@ static bool pair_tiles_fit(int M, int N, int K1, int K2) {
 // Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles, whose offsets have to fit in 32 bits.
 KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats, int phased) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, 1.01);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, false);
     return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
@@ -604,7 +610,7 @@ KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial
 // 158 and 131; 2,560, 5,120: 2,048 rows 83 and 72; 4,096, 8,192: 2,048 rows 140 and 133; in one part 4,096 rows of the last 249 against 243.
 KA_API int ka_linear_pair_large_parts(int M, int N, int K1, int K2, long partial_floats) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
-    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true, 1.05);
+    const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true, true);
     const double library = 2.0 * M * N * (double)(K1 + K2) / 0.85e9 + 8.0 + (double)M * N * 10.0 / 4.0e6;
     return c.tile == 1 && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
