@@ -440,9 +440,8 @@ static int launch_pair_tiles(KaPairTiles& p, int parts, hipStream_t stream) {
 // Bound by the weights' way from HBM: what counts is that every CU has 64 KB of loads in flight, which the stages in LDS hold without
 // registers. Tiles of 64 weight rows by all rows, five stages in half of a CU's LDS, four waves; an XCD's tiles are neighbours. At 40
 // rows, us, weights from HBM, the launch that adds up included, against that kernel: N = 2,048, K = 2,048 + 8,192: 15.2 and 18.6; 2,560, 2,560 +
-// 10,240: 20.1 and 24.8; N = K = 4,096: 13.0 and 16.3; 12,288 by 4,096: 31.3 and 34.2; 4,096 by 12,288: 26.4 and 31.0; at 17 and 64 rows
-// likewise. Tiles of 128 rows read LDS three times for four reads of the others and are ahead where tiles of 64 are more than three a CU, which is
-// two rounds (51,200 by 4,096 99 against 104, by 5,120 124 against 133; 40,960 by 3,072 69 against 63).
+// 10,240: 20.1 and 24.8; N = K = 4,096: 13.0 and 16.3; 4,096 by 12,288: 26.4 and 31.0; at 17 and 64 rows likewise. (One linear whose K would be in one part goes by
+// gemm_few_bf16.hip, but for outputs in no fours.)
 template <int WN, int WM, int GN, int GM, int NS>
 __global__ void __launch_bounds__(KA_WAVE * GN * GM) __attribute__((amdgpu_waves_per_eu(2, 2)))
 few_rows_kernel(KaFewRows p) {
@@ -525,12 +524,9 @@ static int launch_few_rows(const KaFewRows& f, hipStream_t stream) {
 // 1: done; 0: the operands are not covered (K in steps of 64); -1: an error.
 int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
     if (f.M < 1 || f.M > 64 || f.K[0] % 64 || f.K[1] % 64 || f.K[0] < 64 || f.parts < 1 || !f.partial) return 0;
-    const bool large = ka_cdiv(f.N, 64) > 3 * ka_compute_units();
-    // Up to 32 rows tiles of 32, which ask for half the activations, six stages in the same LDS (us, 64 rows a tile and 32, at 24 rows: 12,288 by 4,096
-    // 28.3 and 25.4, 18,944 47.0 and 44.7, 2,560 by 2,560 + 10,240 19.3 and 18.2, 2,048 by 2,048 + 8,192 14.6 and 14.1); not the tiles of 128 weight rows
-    // (51,200 by 4,096 92 and 95). Eight or twelve stages where a CU has one workgroup: 2 to 8 % slower at any number of rows.
-    if (f.M <= 32 && !large) return launch_few_rows<2, 1, 2, 2, 6>(f, stream) ? -1 : 1;
-    return (large ? launch_few_rows<4, 2, 2, 2, 3>(f, stream) : launch_few_rows<2, 2, 2, 2, 5>(f, stream)) ? -1 : 1;
+    // Up to 32 rows tiles of 32, which ask for half the activations, six stages in the same LDS (us, 64 rows a tile and 32, at 24 rows: 2,560 by 2,560 + 10,240
+    // 19.3 and 18.2, 2,048 by 2,048 + 8,192 14.6 and 14.1). Eight or twelve stages where a CU has one workgroup: 2 to 8 % slower at any number of rows.
+    return (f.M <= 32 ? launch_few_rows<2, 1, 2, 2, 6>(f, stream) : launch_few_rows<2, 2, 2, 2, 5>(f, stream)) ? -1 : 1;
 }
 
 // The tile and the parts of K for `ka_linear_pair_tiles_bf16`.

@@ -377,6 +377,7 @@ KA_API void ka_skinny_set_persistent(int enabled) { sk_persistent_enabled = enab
 // registers: 30 against 48 us for Moondream 2's output projection + fc2 at 64 rows; one segment
 // of 2048: 21 against 15 us) and K comes in no steps of 64 (those go by tiles), 2 itself wherever it can run (for tests), 0
 // nowhere.
+int ka_few_rows_whole(const SkinnyArgs& args, bool halves, hipStream_t stream);      // gemm_few_bf16.hip
 static int sk_wide_enabled = 1;
 KA_API int ka_linear_skinny_pair_in_parts(int M, int N);
 KA_API void ka_skinny_set_wide(int enabled) { sk_wide_enabled = enabled; }
@@ -607,6 +608,18 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
     // would read all activations from L2 once per strip (78 us for 48 rows, K = 2560, N = 17920;
     // the wide kernel shares them through LDS). Two targets go one after the other.
     const bool persistent_ok = !A2 && !accumulate_a && sk_persistent_enabled && persistent_fits(M, kblocks, args);
+    // All of K by one tile where that is ahead (measured there): what the persistent kernel would take, and where the wide kernel's K would be in one part.
+    auto one_part = [&](int N) { return 2 * ka_cdiv(N, WD_WAVES * SK_STRIP) > sk_compute_units(); };
+    const int groups = ka_cdiv(Na, WD_WAVES * SK_STRIP);
+    if (M > 16 && !A2 && sk_wide_enabled == 1 && (persistent_ok || (partials && one_part(Na) && (!Wb || one_part(Nb))))) {
+        const int done = ka_few_rows_whole(args, !persistent_ok, stream);
+        if (done < 0) return -1;
+        if (done == 0) {
+            if (then) ka_launch_finish_norm(M, Na, stream, nullptr, 0, nullptr, nullptr, (float*)outa, ldoa, 0, *then);
+            KA_LAUNCH_CHECK();
+            return 0;
+        }
+    }
     if (M > 16 && Wb && partials && sk_wide_enabled && !persistent_ok) {
         int rc = skinny_fused(SkinnyExtras{}, A1, lda1, K1, nullptr, 0, 0, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0.f,
                                         Wa, ldwa, biasa, outa, out_dtype_a, ldoa, Na, acta, accumulate_a, nullptr, 0,
@@ -644,7 +657,6 @@ static int skinny_fused(const SkinnyExtras& extras, const void* A1, long lda1, i
         // K = 2048 + 8192, 32 groups of strips: 8 parts 18.1 us at 32 rows and 19.6 at 64, finishing
         // kernel included; 6 parts 21.4 and 22.3, 10 parts 22.6 and 27.4, 16 parts 21.1 and 25.1),
         // every part at least two chunks
-        const int groups = ka_cdiv(Na, WD_WAVES * SK_STRIP);
         int splits = sk_compute_units() / groups;
         if (splits < 1) splits = 1;
         if (splits > ka_cdiv(kblocks, 2 * WD_CB)) splits = ka_cdiv(kblocks, 2 * WD_CB);
