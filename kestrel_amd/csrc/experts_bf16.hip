@@ -181,6 +181,11 @@ experts_dma_kernel(ExpertsDmaArgs g) {
         for (int b = 0; b < WM; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+    // (the pairs of this wave's list rows, a row a lane: asked for where the rows are stored, each was a trip to memory that the store waited for. F32, us: 30 experts of
+    // 2,048 x 704, 2,048 tokens of 4 choices 62.9 -> 57.6)
+    int pairs[WM];
+#pragma unroll
+    for (int b = 0; b < WM; ++b) pairs[b] = g.sorted[i0 + (wm * WM + b) * 32 + li];
     kd_product<WN, WM, GN, GM, 64, NS, SL, true>(eb_dma_lds, wave, lane, g.K, wsrc, xsrc, acc);
 
     // A lane ends with four neighbouring weight rows of one list row, a store instruction would touch 32 rows with 8 or 16
@@ -219,12 +224,14 @@ experts_dma_kernel(ExpertsDmaArgs g) {
 #pragma unroll
         for (int r0 = 0; r0 < 32; r0 += RPI) {
             const int rl = r0 + lane / CH, c = lane % CH, i = i0 + wm * 32 * WM + b * 32 + rl, o = o_wave + c * PER;
-            const int p = g.sorted[i];
+            const int p = __shfl(pairs[b], rl);
             if (p >= 0 && o < n_out) {
                 const unsigned char* from = mine + rl * RS + c * 16;
                 E* op = reinterpret_cast<E*>(g.out) + (g.scatter ? (long)p : (long)i) * g.ldo + o;
                 if (o + PER <= n_out) {
-                    *reinterpret_cast<floatx4*>(op) = *reinterpret_cast<const floatx4*>(from);
+                    // (the fp32 rows are more than the caches of an XCD hold, and pass by them: 62 experts of 4,096 x 896, 1,204 tokens of 6 choices 149 -> 132 us)
+                    if constexpr (F32) __builtin_nontemporal_store(*reinterpret_cast<const floatx4*>(from), reinterpret_cast<floatx4*>(op));
+                    else *reinterpret_cast<floatx4*>(op) = *reinterpret_cast<const floatx4*>(from);
                 } else {
                     for (int x = 0; x < PER && o + x < n_out; ++x) op[x] = reinterpret_cast<const E*>(from)[x];
                 }
