@@ -4,6 +4,7 @@
 // reads what the next sublayer sees, u = sum_t into[t] x_t, and leaves that sublayer's norm of u in h. All arithmetic is fp32.
 // What computes y is the caller's business: a load, or the weighted sum of a routed mixture's experts.
 #include "ka_common.h"
+#include "ka_route.h"
 #include "ka_rows.h"
 
 // A workgroup has a row. Of many rows each gets 256 threads and a thread several pieces of it; where there are fewer rows than two a
@@ -33,24 +34,37 @@ __device__ __forceinline__ float4 st_fma4(float a, const float4& b, const float4
 }
 
 // S streams in registers, PIECES pieces of four channels a thread (dim a multiple of 4 and at most 4 PIECES THREADS, rows
-// 16-byte aligned). `piece(c)` gives y of the channels c .. c + 3.
-template <int S, int PIECES, int THREADS, typename Piece>
-__device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, float* smem) {
-    typedef __attribute__((ext_vector_type(4))) __bf16 st_bf16x4;
+// 16-byte aligned). `piece(c)` gives y of the channels c .. c + 3. `early()` runs behind the first requests, `keep(c, b)` sees the bf16 rows of h.
+typedef __attribute__((ext_vector_type(4))) __bf16 st_bf16x4;
+
+template <int S, int PIECES, int THREADS, typename Piece, typename Early, typename Keep>
+__device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, float* smem, Early early, Keep keep) {
     const int i = blockIdx.x, dim = a.dim;
     float* row = a.x + (size_t)(a.rows ? a.rows[i] : i) * S * dim;
     float m[S][S], o[S], in[S];
     const bool writes = a.mix != nullptr;
-    if (writes) {
+    // The numbers of the streams and (of short rows) the norm's are asked for behind the row and arrive with it; where they are used they would come behind what `early`
+    // asks for. (A step without that: 2.8 us at one row of four streams of 2,048 either way.)
+    auto numbers = [&] {
+        if (writes) {
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
+            for (int s = 0; s < S; ++s) {
 #pragma unroll
-            for (int t = 0; t < S; ++t) m[s][t] = a.mix[s * S + t];
-            o[s] = a.out[s];
+                for (int t = 0; t < S; ++t) m[s][t] = a.mix[s * S + t];
+                o[s] = a.out[s];
+            }
         }
-    }
 #pragma unroll
-    for (int s = 0; s < S; ++s) in[s] = a.into ? a.into[s] : 1.f;
+        for (int s = 0; s < S; ++s) in[s] = a.into ? a.into[s] : 1.f;
+    };
+    constexpr bool NORM_EARLY = PIECES <= 2;
+    float4 gain[PIECES], bias[PIECES];
+    auto norm_of = [&](int p) {
+        const int c = min(ka_row_channel<THREADS>(p), dim - 4);
+        const float* const g = a.h ? a.gain : row;                  // (without a norm any address; not used)
+        gain[p] = *reinterpret_cast<const float4*>(g + c);
+        bias[p] = *reinterpret_cast<const float4*>((a.h && a.bias ? a.bias : g) + c);
+    };
     float4 u[PIECES];
     float sum[PIECES], ss[PIECES];
     // (all that a few pieces need is asked for before anything is stored)
@@ -69,6 +83,14 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
                 for (int s = 0; s < S; ++s) v[p][s] = *reinterpret_cast<const float4*>(row + (size_t)s * dim + c);
             }
             if (writes) y[p] = piece(c);
+        }
+        if (p0 == 0) {
+            if constexpr (NORM_EARLY) {
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) norm_of(p);
+            }
+            numbers();
+            early();
         }
 #pragma unroll
         for (int p = 0; p < AT_ONCE; ++p) {
@@ -115,12 +137,10 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
     for (int p = 0; p < PIECES; ++p) {
         const int c = ka_row_channel<THREADS>(p);
         if (c < dim) {
-            const float4 g = *reinterpret_cast<const float4*>(a.gain + c);
+            if constexpr (!NORM_EARLY) norm_of(p);
+            const float4 g = gain[p];
             float4 v = make_float4(u[p].x * r * g.x, u[p].y * r * g.y, u[p].z * r * g.z, u[p].w * r * g.w);
-            if (a.bias) {
-                const float4 b = *reinterpret_cast<const float4*>(a.bias + c);
-                v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
-            }
+            if (a.bias) v = make_float4(v.x + bias[p].x, v.y + bias[p].y, v.z + bias[p].z, v.w + bias[p].w);
             if (a.h_bf16) {
                 st_bf16x4 b;
                 b[0] = (bf16_t)v.x;
@@ -128,11 +148,17 @@ __device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, f
                 b[2] = (bf16_t)v.z;
                 b[3] = (bf16_t)v.w;
                 *reinterpret_cast<st_bf16x4*>(reinterpret_cast<bf16_t*>(a.h) + (size_t)i * dim + c) = b;
+                keep(c, b);
             } else {
                 *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.h) + (size_t)i * dim + c) = v;
             }
         }
     }
+}
+
+template <int S, int PIECES, int THREADS, typename Piece>
+__device__ __forceinline__ void st_step_regs(const StreamArgs& a, Piece piece, float* smem) {
+    st_step_regs<S, PIECES, THREADS>(a, piece, smem, [] {}, [](int, const st_bf16x4&) {});
 }
 
 // Any number of streams up to ST_MAX_STREAMS, any dim. `one(c)` gives y of channel c.
@@ -191,6 +217,76 @@ __global__ void __launch_bounds__(THREADS) streams_step_kernel(StreamArgs a, con
         st_step_regs<S, PIECES, THREADS>(a, [&](int c) { return *reinterpret_cast<const float4*>(yr + c); }, smem);
     else
         st_step_any(a, [&](int c) { return yr[c]; }, smem);
+}
+
+// The step in front of a routed mixture, of few rows: the same row's router logits and its choice in the launch that leaves h. The router's linear of few rows is a
+// handful of workgroups that wait for memory, and the choice behind it a wave a row that waits again; here the router's weights (120 to 500 KB, from L2 for all rows
+// but the first) are asked for beside the streams, in registers, and h meets them out of LDS: a wave takes every (THREADS / 64)-th output.
+// A row's numbers depend on that row alone. One CU brings the weights at 30 to 40 GB/s beyond the first trip, so long rows gain only where the linear alone is slow
+// (us, 30 outputs of 2,048, one row: step, linear and choice 9.4, this 7.5; 62 of 4,096: 11.9 and 15.7, 40 rows 21.4 and 16.5). 1,024 threads leave 128 registers: two
+// outputs ahead spilled, 25.8 us.
+struct StreamRoute {
+    const bf16_t* router;       // [outputs, dim], rows ld apart
+    long ld;
+    int outputs;                // rows of the router's linear: those of the choice, and what else rides along
+    const float* bias;          // [outputs] or null
+    float* logits;              // [n, >= outputs], rows logits_ld apart
+    long logits_ld;
+};
+constexpr int ST_ROUTE_OUTPUTS = 128;
+
+template <int S, int THREADS>
+__global__ void __launch_bounds__(THREADS) streams_route_kernel(StreamArgs a, const float* __restrict__ y, StreamRoute q, RouteArgs choice) {
+    typedef __attribute__((ext_vector_type(8))) __bf16 st_bf16x8;
+    constexpr int WAVES = THREADS / KA_WAVE, LOADS = THREADS * 4 / (8 * KA_WAVE), AHEAD = THREADS == 512 ? 4 : 1;     // loads of 16 bytes a lane and output; outputs asked for ahead
+    __shared__ float smem[WAVES], logits[ST_ROUTE_OUTPUTS];
+    __shared__ __attribute__((aligned(16))) bf16_t row[THREADS * 4];
+    __shared__ RouteRoom<1> room;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE, dim = a.dim;
+    const float* yr = y + (size_t)blockIdx.x * dim;
+    st_bf16x8 w[AHEAD][LOADS];
+    auto ask = [&](st_bf16x8 (&to)[LOADS], int r) {
+        const bf16_t* from = q.router + (size_t)min(r, q.outputs - 1) * q.ld;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) to[i] = *reinterpret_cast<const st_bf16x8*>(from + min((i * KA_WAVE + lane) * 8, dim - 8));
+    };
+    st_step_regs<S, 1, THREADS>(
+        a, [&](int c) { return *reinterpret_cast<const float4*>(yr + c); }, smem,
+        [&] {
+#pragma unroll
+            for (int g = 0; g < AHEAD; ++g) ask(w[g], wave + g * WAVES);
+        },
+        [&](int c, const st_bf16x4& b) { *reinterpret_cast<st_bf16x4*>(row + c) = b; });
+    __syncthreads();
+    st_bf16x8 h[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) h[i] = *reinterpret_cast<const st_bf16x8*>(row + (i * KA_WAVE + lane) * 8);
+    for (int r0 = wave; r0 < q.outputs; r0 += AHEAD * WAVES) {
+#pragma unroll
+        for (int g = 0; g < AHEAD; ++g) {
+            const int r = r0 + g * WAVES;
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                float part = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) part = fmaf((float)w[g][i][e], (float)h[i][e], part);
+                sum += (i * KA_WAVE + lane) * 8 < dim ? part : 0.f;
+            }
+            ask(w[g], r + AHEAD * WAVES);
+            sum = ka_wave_sum(sum);
+            if (r < q.outputs && lane == 0) {
+                if (q.bias) sum += q.bias[r];
+                logits[r] = sum;
+                q.logits[(size_t)blockIdx.x * q.logits_ld + r] = sum;
+            }
+        }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    choice.logits = logits;
+    choice.stride = 0;
+    ka_route_token<1>(choice, blockIdx.x, lane, room);
 }
 
 // y = sum_k weights[t, k] * (chosen[t, k] < E ? pairs[t top + k] : h_in[t]) + sigmoid(shared_gate[t]) * shared[t], as
@@ -304,6 +400,38 @@ KA_API int ka_streams_step(float* x, const float* embedded, const float* y, cons
 #define ST_LAUNCH(S_, P_, T_) hipLaunchKernelGGL((streams_step_kernel<S_, P_, T_>), dim3(n), dim3(T_), 0, stream, a, y)
     ST_DISPATCH(ST_LAUNCH)
 #undef ST_LAUNCH
+    KA_LAUNCH_CHECK();
+    return 0;
+}
+
+// ka_streams_step of rows that are written and read, and ka_route of the logits h router^T (+ router_bias) in the same launch. 1: not covered, nothing was run.
+KA_API int ka_streams_step_route(float* x, const float* y, const float* mix, const float* out, const float* into, const float* gain, const float* bias, float eps,
+                                 int rms, void* h, int n, int S, int dim, const void* router, long ldr, int outputs, const float* router_bias,
+                                 float* logits, long stride, const float* correction, int tokens, int R, int top, int n_groups, int keep, int group_best, float scale,
+                                 int mode, int always, int* chosen, float* weights, hipStream_t stream) {
+    const char* who = "ka_streams_step_route";
+    const StreamArgs a{x, nullptr, mix, out, into, nullptr, gain, bias, eps, rms, h, 1, S, dim};
+    if (const int status = st_check(who, a, n, KA_BF16)) return status;
+    KA_CHECK(mix != nullptr && y != nullptr && h != nullptr, "%s: a step that writes and reads", who);
+    const RouteArgs choice{logits, stride, correction, R, top, n_groups, keep, group_best, mode, always, scale, chosen, weights};
+    if (ka_route_check(who, choice, tokens)) return -1;
+    KA_CHECK(tokens == n && outputs >= R && stride >= outputs && ldr >= dim, "%s: %d outputs of which %d are chosen among, %d of %d rows", who, outputs, R, tokens, n);
+    const int pieces = st_pieces(a, n, y, nullptr);
+    if ((pieces != 11 && pieces != 12) || R > KA_WAVE || outputs > ST_ROUTE_OUTPUTS || dim % 8 || ldr % 8 || (uintptr_t)router % 16) return 1;
+    if (n == 0) return 0;
+    const StreamRoute q{(const bf16_t*)router, ldr, outputs, router_bias, logits, stride};
+#define ST_ROUTE(S_)                                                                                                                  \
+    case S_:                                                                                                                          \
+        if (pieces == 11) hipLaunchKernelGGL((streams_route_kernel<S_, 512>), dim3(n), dim3(512), 0, stream, a, y, q, choice);        \
+        else hipLaunchKernelGGL((streams_route_kernel<S_, 1024>), dim3(n), dim3(1024), 0, stream, a, y, q, choice);                   \
+        break;
+    switch (S) {
+        ST_ROUTE(1)
+        ST_ROUTE(2)
+        ST_ROUTE(3)
+        ST_ROUTE(4)
+    }
+#undef ST_ROUTE
     KA_LAUNCH_CHECK();
     return 0;
 }

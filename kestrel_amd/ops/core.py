@@ -78,6 +78,9 @@ _SIGNATURES = {
                           _c_float, _c_float, _c_void_p, _c_long, _c_int, _c_void_p],
     "ka_streams_step": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_int,
                         _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_streams_step_route": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_int, _c_void_p, _c_int, _c_int, _c_int,
+                              _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_long, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
+                              _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p],
     "ka_streams_experts": [_c_void_p, _c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_long,
                            _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                            _c_void_p],
@@ -664,6 +667,30 @@ def streams_step(x: torch.Tensor, y: Optional[torch.Tensor] = None, mix: Optiona
     _check(lib().ka_streams_step(x.data_ptr(), _ptr(embedded), _ptr(y), _ptr(mix), _ptr(out), _ptr(into), _ptr(rows), _ptr(gain), _ptr(bias), eps,
                                  rms, _ptr(h), code_of(h.dtype) if h is not None else KA_F32, n if rows is None else rows.numel(), S, dim,
                                  stream_ptr()))
+
+
+def streams_step_route(x: torch.Tensor, y: torch.Tensor, mix: torch.Tensor, out: torch.Tensor, reading, h: torch.Tensor, router: torch.Tensor,
+                       router_bias: Optional[torch.Tensor], logits: torch.Tensor, *choice, **options) -> bool:
+    """``streams_step`` that writes ``y`` and leaves bf16 ``h``, and in the same launch ``logits = h @ router.T (+ router_bias)`` and
+    ``route(logits, *choice, **options)``. False: not covered (an fp32 router, rows of at most 1,024 or more than 4,096, more than four streams or 64 outputs to
+    choose among, many rows), nothing was run."""
+    n, S, dim = x.shape
+    who = "streams_step_route"
+    into, gain, bias, eps, rms = _stream_args(who, x, mix, out, reading, h)
+    _dev(y, router, router_bias, logits)
+    _need(y.dtype == torch.float32 and y.is_contiguous() and tuple(y.shape) == (n, dim), f"{who}: fp32 rows [n, dim]")
+    _need(reading is not None, f"{who}: the router's input is what is read")
+    if h.dtype != torch.bfloat16 or router.dtype != torch.bfloat16 or router.stride(1) != 1 or router.data_ptr() % 16:
+        return False
+    outputs = router.shape[0]
+    _need(router.shape[1] == dim and logits.shape[1] >= outputs and logits.stride(1) == 1, f"{who}: a router [outputs, dim] and its logits [n, outputs]")
+    _need(router_bias is None or (router_bias.dtype == torch.float32 and router_bias.is_contiguous() and router_bias.numel() == outputs), f"{who}: router_bias fp32 [outputs]")
+    status = lib().ka_streams_step_route(x.data_ptr(), y.data_ptr(), _ptr(mix), _ptr(out), _ptr(into), _ptr(gain), _ptr(bias), eps, rms, h.data_ptr(), n, S, dim,
+                                         router.data_ptr(), router.stride(0), outputs, _ptr(router_bias), *route_args(logits, *choice, **options), stream_ptr())
+    if status > 0:
+        return False
+    _check(status)
+    return True
 
 
 def streams_experts(x: torch.Tensor, pairs: torch.Tensor, h_in: torch.Tensor, chosen: torch.Tensor, weights: torch.Tensor, n_experts: int,

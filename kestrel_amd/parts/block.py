@@ -397,7 +397,7 @@ def _streams(block: "Block", x, batch, cache, normed=None, then=None):
 
     One launch stands between two sublayers: it writes the one's output into the streams and leaves the norm of what the
     next one reads (``then``, a ``StreamReading``, behind the last: its rows are handed over). A feed-forward that offers
-    ``mix_streams`` takes that launch's work into its own last one."""
+    ``mix_streams`` takes that launch's work into its own last one, and one with ``choose_streams`` its choice into the one in front of it."""
     from ..ops import core
 
     ws = batch.workspace
@@ -423,9 +423,12 @@ def _streams(block: "Block", x, batch, cache, normed=None, then=None):
         core.streams_step(x, delta, block.streams.matrix, block.streams.out, last, handed)
         return handed
     h2 = ws.get("block.h2", (n, dim), block.dtype)
-    core.streams_step(x, delta, block.streams.matrix, block.streams.out, block.reader2.operands(), h2)
+    reading = block.reader2.operands()
+    chosen = callable(getattr(ff, "choose_streams", None)) and ff.choose_streams(x, delta, block.streams, reading, h2, batch)
+    if not chosen:
+        core.streams_step(x, delta, block.streams.matrix, block.streams.out, reading, h2)
     if callable(getattr(ff, "mix_streams", None)):
-        ff.mix_streams(h2, batch, x, block.streams2, last, handed)
+        ff.mix_streams(h2, batch, x, block.streams2, last, handed, **({"chosen": True} if chosen else {}))
         return handed
     into_delta(ff, h2, batch)
     core.streams_step(x, delta, block.streams2.matrix, block.streams2.out, last, handed)

@@ -48,6 +48,7 @@ class RoutedExperts(FeedForward):
     FEW_PAIRS_SPREAD_TO = 240
     FEW_PAIRS_AN_EXPERT = 4
     FEW_PAIRS_TO_UNALIGNED = 512
+    CHOICE_BEHIND_TO, CHOICE_BEHIND_ROWS, CHOICE_BEHIND_FROM = 2048, 16, 2560
 
     def __init__(self, spec: RoutedExpertsSpec) -> None:
         super().__init__(spec)
@@ -161,7 +162,34 @@ class RoutedExperts(FeedForward):
         spread = 0 if self.joined else min(self.FEW_PAIRS_AN_EXPERT * spec.n_experts, self.FEW_PAIRS_SPREAD_TO)
         return max(self.FEW_PAIRS_TO, spread)
 
-    def _outputs(self, h, batch):
+    def _choice(self, n: int, ws):
+        """Where the router's logits of ``n`` rows go, and the operands of ``ops.core.route`` behind them."""
+        spec = self.spec
+        top = spec.top + self.joined
+        logits = ws.get("experts.logits", (n, self.router.shape[0]), torch.float32)
+        chosen = ws.get("experts.chosen", (n, top), torch.int32)
+        weights = ws.get("experts.weights", (n, top), torch.float32)
+        choice = (self.n_outputs, self.correction, spec.top, spec.n_groups, spec.keep_groups, spec.scale, chosen, weights)
+        options = dict(weigh_chosen=self.weigh_chosen, scores=self.scores, group_best=self.group_best, always=spec.n_experts if self.joined else None)
+        return logits, choice, options
+
+    def choose_streams(self, x, y, streams, reading, h, batch) -> bool:
+        """``ops.core.streams_step`` in front of this feed-forward (``mix_streams`` is then told that it has ``chosen``), with the router's linear and the choice in the
+        same launch where they would be launches of their own. False: nothing was run."""
+        from ..ops import fast
+
+        n, dim = h.shape
+        if self.dtype != torch.bfloat16 or not 0 < n <= fast.SKINNY_MAX_ROWS:
+            return False
+        # Rows of up to 2,048, where no shared expert's launches take the router's linear and the choice along (three launches and one, us, 30 outputs of 2,048: one row 9.4
+        # and 7.5, 40 rows 12.7 and 8.0; 62: 9.9 and 8.9, 13.0 and 9.4); longer ones where the linear would come in parts (62 of 4,096: one row 11.9 and
+        # 15.7, 20 rows 19.6 and 16.4, 40 rows 21.4 and 16.5; 64 of 3,072: 14.7 and 15.9, 16.0 and 16.0), which no launch takes along.
+        if not (dim <= self.CHOICE_BEHIND_TO and (self.joined or not self.shared) or n > self.CHOICE_BEHIND_ROWS and dim > self.CHOICE_BEHIND_FROM):
+            return False
+        logits, choice, options = self._choice(n, batch.workspace)
+        return core.streams_step_route(x, y, streams.matrix, streams.out, reading, h, self.router, self.router_bias, logits, *choice, **options)
+
+    def _outputs(self, h, batch, chosen_already: bool = False):
         """Everything but the weighted sum: the pairs' outputs, the choice, its weights, the shared expert's output and gate."""
         from ..ops import fast
 
@@ -169,23 +197,21 @@ class RoutedExperts(FeedForward):
         n = h.shape[0]
         ws = batch.workspace
         top = spec.top + self.joined
-        logits = ws.get("experts.logits", (n, self.router.shape[0]), torch.float32)
+        logits, choice, options = self._choice(n, ws)
+        choice = (logits, *choice)
+        chosen, weights = choice[-2:]
         shared = self._shared_operands(n, ws) if self.shared and not self.joined else None
         # Few rows: the router's linear, a few workgroups that wait for memory, beside the shared expert's first in one launch
         # (eight rows of 2,048: about 5 us a layer, 3 % of a step).
         beside = False
-        if shared is not None and self.dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16:
+        if shared is not None and not chosen_already and self.dtype == torch.bfloat16 and self.router.dtype == torch.bfloat16:
             beside = fast.linear_two_outputs(h, self.router, self.router_bias, logits, 0, self.shared_pairs, None, *shared)
-        chosen = ws.get("experts.chosen", (n, top), torch.int32)
-        weights = ws.get("experts.weights", (n, top), torch.float32)
-        choice = (logits, self.n_outputs, self.correction, spec.top, spec.n_groups, spec.keep_groups, spec.scale, chosen, weights)
-        options = dict(weigh_chosen=self.weigh_chosen, scores=self.scores, group_best=self.group_best, always=spec.n_experts if self.joined else None)
-        if not beside:
+        if not beside and not chosen_already:
             linear(h, self.router, self.router_bias, logits)
         # The choice, a launch that waits for memory on a wave a token, goes beside the shared expert's second linear where rows are few
         # (eight rows of 2,048: 4 us a layer, 2 % of a step).
-        routed, shared_out = False, None
-        if shared is not None and self.dtype == torch.bfloat16 and n <= fast.SKINNY_CHOICE_ROWS:
+        routed, shared_out = chosen_already, None
+        if shared is not None and not routed and self.dtype == torch.bfloat16 and n <= fast.SKINNY_CHOICE_ROWS:
             shared_hidden = self._shared_hidden(h, *shared, beside, ws)
             shared_out = ws.get("experts.shared_out", (n, spec.dim), torch.float32)
             routed = fast.linear_choice(shared_hidden, self.shared_down, None, shared_out, *choice, **options)
@@ -226,10 +252,11 @@ class RoutedExperts(FeedForward):
         y, chosen, weights, shared_out, gate = self._outputs(h, batch)
         core.experts_combine_normed(y, h, chosen, weights, self.pairs.shape[0], shared_out, gate, x, norm, then, rows)
 
-    def mix_streams(self, h, batch, x, streams, reading, rows) -> None:
+    def mix_streams(self, h, batch, x, streams, reading, rows, chosen: bool = False) -> None:
         """The feed-forward of ``h`` written into the streams ``x`` by the numbers of ``streams`` (a ``StreamMix``), by the launch that
-        takes the weighted sum; what ``reading`` sees of the new streams goes into ``rows`` (``ops.core.streams_step``)."""
-        y, chosen, weights, shared_out, gate = self._outputs(h, batch)
+        takes the weighted sum; what ``reading`` sees of the new streams goes into ``rows`` (``ops.core.streams_step``). ``chosen``:
+        ``choose_streams`` has made the choice."""
+        y, chosen, weights, shared_out, gate = self._outputs(h, batch, chosen)
         core.streams_experts(x, y, h, chosen, weights, self.pairs.shape[0], shared_out, gate, streams.matrix, streams.out, reading, rows)
 
     def forward(self, h, batch, residual) -> None:
