@@ -3,6 +3,7 @@
 #include "ka_common.h"
 #include "ka_partials.h"
 #include "ka_phased_tiles.h"
+#include "ka_quad_tiles.h"
 
 // out[s] = act[s](A W[s]^T + bias[s]), s = 0, 1, in bf16; the tiles of the second linear follow those of the first.
 struct KpJoint {
@@ -104,22 +105,60 @@ static int launch_joint(KpJoint p, hipStream_t stream) {
     return 0;
 }
 
-// The tiles by area: of those whose workgroups are one round of the chip the smallest wins, since a K-step of it is the shortest.
-static const struct { int code, rows_w, rows_x; } KP_JOINT_TILES[] = {{6, 128, 128}, {3, 128, 256}, {5, 256, 128}, {2, 192, 256}, {4, 256, 192}, {1, 256, 256}};
-
-// The tile for two linears of the same rows in one launch, 0: not covered, or left to the vendor library one after the other. That is so where nearly half of
-// the tiles is no rows (22,528 from 4,096, 257 rows: 85 us in one launch, 82 by the library), and where they take more than one round, in which neither
-// side is ahead everywhere (us, library and the best of the tiles 256 x 256, 192 x 256 and 128 x 256; 14,336 from 2,048: 1,100 rows 74 and 84, 1,300 rows 90
+// The tile for two linears of the same rows in one launch, 0: not covered, or left to the vendor library one after the other. Of the tiles whose workgroups are one round of the chip
+// the smallest wins, since a K-step of it is the shortest: four waves a tile up to 160 x 256 (ka_quad_tiles.h), above that the phased ones.
+// Measured, us, the library's two launches, the phased tiles (128 x 128, 128 x 256, 192 x 256) that ran here before, and these; 14,336 from 2,048: 96 rows 31.7, 23.1, 18.6; 256 rows 50,
+// 26, 25.8; 384 rows 49, 31.5, 30.0; 512 rows 51, 34, 33.6; 17,920 from 2,560: 96 rows 43, 32.5, 30.4; 256 rows 70, 45, 37.8; 512 rows 71, 54, 47.3. Over widths of 768 to 4,096 and 65 to
+// 1,024 rows the tile chosen is the fastest but in three cases of 98 (4 % behind), and one launch 1.2 to 2.6 times as fast as the library's two. That is not so where nearly half of a
+// large tile is no rows (22,528 from 4,096, 257 rows: 85 us in one launch, 82 by the library), and where the tiles take more than one round, in which neither
+// side is ahead everywhere (library and the best of the tiles 256 x 256, 192 x 256 and 128 x 256; 14,336 from 2,048: 1,100 rows 74 and 84, 1,300 rows 90
 // and 86, 1,536 rows 88 and 89, 2,048 rows 104 and 106; 17,920 from 2,560: 1,024 rows 105 and 106, 1,200 rows 128 and 109, 1,536 rows 125 and 127, 1,792 rows
-// 162 and 131): a rule for those rows would go by the fill of the last round, and has not been measured at other widths. Within one round, widths of 1,536 to
-// 4,096, 65 to 1,024 rows, library and one launch: 14,336 from 2,048: 128 rows 31.8 and 25.2, 256 rows 50 and 26, 512 rows 51 and 36, 743 rows 59
-// and 45, 1,024 rows 69 and 55; 17,920 from 2,560, 512 rows: 70 and 55.
+// 162 and 131): a rule for those rows would go by the fill of the last round, and has not been measured at other widths.
+static const struct { int code, rows_w, rows_x; } KP_JOINT_TILES[] = {{6, 64, 128}, {7, 96, 128}, {8, 128, 128}, {5, 160, 128}, {3, 128, 192}, {9, 96, 256}, {10, 160, 192},
+                                                                      {11, 128, 256}, {12, 160, 256}, {2, 192, 256}, {4, 256, 192}, {1, 256, 256}};
+static bool kp_phased(int code) { return code == 1 || code == 2 || code == 4; }
+
 KA_API int ka_linear_joint_tile(int M, int N1, int N2, int K) {
     if (M < 1 || N1 < 8 || N2 < 8 || N1 % 8 || N2 % 8 || K % 64 || K < 128) return 0;
     for (const auto& t : KP_JOINT_TILES)
         if ((long)ka_cdiv(M, t.rows_x) * (ka_cdiv(N1, t.rows_w) + ka_cdiv(N2, t.rows_w)) <= ka_compute_units())
-            return t.rows_w * t.rows_x <= 128 * 256 || M * 20 >= ka_cdiv(M, t.rows_x) * t.rows_x * 11 ? t.code : 0;
+            return !kp_phased(t.code) || M * 20 >= ka_cdiv(M, t.rows_x) * t.rows_x * 11 ? t.code : 0;
     return 0;
+}
+
+// The tile for one linear of more rows than the weight-streaming kernels take, 0: left to the vendor library. The smallest whose workgroups are one round, as above, if they are enough:
+// with K up to 1,024 a sixth of the CUs (and 1,024 outputs); up to 2,304 five eighths, below which the library cuts K (us, library and tile: 2,048 of 2,048, 448 rows, 112
+// workgroups 12.1 and 12.1; 1,024 of 2,048, 768 rows, 96 workgroups 11.3 and 11.9); up to 4,608 seven eighths, or two thirds of the smallest tile, whose stages run furthest ahead (4,096 of
+// 4,096, 768 rows, 192 of 128 x 128 33.9 and 38.5; 2,048 of 4,096, 768 rows, 192 of 64 x 128 23.4 and 21.3). Over 976 sizes (512 to 12,416 outputs, K of 512 to 8,192, 80 to 2,048
+// rows, bf16 and fp32 out, weights from HBM) what this takes is 19 % faster on the average, up to 1.7 times (5,632 of 704, 256 rows 13.1 and 7.6), and 4 % behind at most (6,144 of 704, 1,024
+// rows into fp32, 14.4 and 15.0): 2,048 of 2,048, 2,048 rows 21.4 and 18.8; 4,096 of 2,048 31.5 and 29.7; 5,632 of 2,048, 512 rows 24.3 and 17.6. Longer K and more than a round: the library.
+KA_API int ka_linear_quad_tile(int M, int N, int K) {
+    if (M < 1 || N < 8 || N % 8 || K < 64 || K % 64) return 0;
+    const long cus = ka_compute_units();
+    for (const auto& t : KP_JOINT_TILES) {
+        if (kp_phased(t.code)) break;
+        const long tiles = (long)ka_cdiv(M, t.rows_x) * ka_cdiv(N, t.rows_w);
+        if (tiles > cus) continue;
+        if (K <= 1024) return tiles * 6 >= cus && N >= 1024 ? t.code : 0;
+        if (K <= 2304) return tiles * 8 >= cus * 5 ? t.code : 0;
+        return K <= 4608 && (tiles * 8 >= cus * 7 || (t.code == 6 && tiles * 3 >= cus * 2)) ? t.code : 0;
+    }
+    return 0;
+}
+
+// One linear by the tiles of four waves into bf16 or fp32.
+KA_API int ka_linear_quad_bf16(const void* A, long lda, const void* W, long ldw, const float* bias, void* out, int out_dtype, long ldo, int M, int N, int K, int act,
+                               int accumulate, int code, hipStream_t stream) {
+    const char* who = "ka_linear_quad_bf16";
+    KA_CHECK(M > 0 && K >= 64 && K % 64 == 0 && N > 0 && N % 8 == 0, "%s: M=%d K=%d N=%d", who, M, K, N);
+    KA_CHECK(lda >= K && ldw >= K && lda % 8 == 0 && ldw % 8 == 0 && ldo >= N && ldo % 8 == 0, "%s: strides", who);
+    KA_CHECK(((uintptr_t)A | (uintptr_t)W | (uintptr_t)bias | (uintptr_t)out) % 16 == 0, "%s: operands must be 16-byte aligned", who);
+    KA_CHECK((M - 1) * lda + K < (1L << 31) && (N - 1) * ldw + K < (1L << 31), "%s: an operand of 4 GB", who);
+    KA_CHECK(ka_act_known(act) && !ka_act_gated(act) && (out_dtype == KA_F32 || out_dtype == KA_BF16) && !(accumulate && out_dtype != KA_F32), "%s: activation %d, output %d", who, act, out_dtype);
+    KqLinears q = {};
+    q.A = (const bf16_t*)A; q.lda = lda; q.M = M; q.K = K; q.accumulate = accumulate;
+    q.W[0] = (const bf16_t*)W; q.ldw[0] = ldw; q.bias[0] = bias; q.out[0] = out; q.ldo[0] = ldo; q.N[0] = N; q.act[0] = act;
+    return out_dtype == KA_F32 ? ka_quad_f32(q, code, stream) : ka_quad_bf16(q, code, stream);
 }
 
 KA_API int ka_linear_joint_bf16(const void* A, long lda, int M, int K, const void* W1, long ldw1, const float* bias1, void* out1, long ldo1, int N1,
@@ -140,12 +179,14 @@ KA_API int ka_linear_joint_bf16(const void* A, long lda, int M, int K, const voi
     switch (config) {
         case 1: return launch_joint<4, 4, 2, 2, 2, 4>(p, stream);
         case 2: return launch_joint<4, 2, 2, 2, 2, 4>(p, stream);
-        case 3: return launch_joint<2, 2, 2, 2, 2, 4>(p, stream);
         case 4: return launch_joint<4, 4, 2, 1, 2, 4>(p, stream);
-        case 5: return launch_joint<2, 2, 2, 2, 4, 2>(p, stream);
-        case 6: return launch_joint<2, 2, 1, 1, 2, 4>(p, stream);
     }
-    KA_CHECK(false, "%s: unknown tile %d", who, config);
+    KqLinears q = {};
+    q.A = p.A; q.lda = p.lda; q.M = p.M; q.K = p.K;
+    for (int i = 0; i < 2; ++i) {
+        q.W[i] = p.W[i]; q.ldw[i] = p.ldw[i]; q.bias[i] = p.bias[i]; q.out[i] = p.out[i]; q.ldo[i] = p.ldo[i]; q.N[i] = p.N[i]; q.act[i] = p.act[i];
+    }
+    return ka_quad_bf16(q, config, stream);
 }
 
 // A block's two last linears: out += A[0] W[0]^T + A[1] W[1]^T, the K-steps of both one behind the other and cut into parts of `per`,

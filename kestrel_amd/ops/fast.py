@@ -51,6 +51,8 @@ _SIGNATURES = {
         _c_void_p, _c_long, _c_int, _c_int,                                                # A, lda, M, K
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int,                 # W, ldw, bias, out, ldo, N, act of either linear
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_void_p],   # ..., tile, stream
+    "ka_linear_quad_tile": [_c_int, _c_int, _c_int],
+    "ka_linear_quad_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "ka_linear_library_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
                                _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_long, _c_void_p],
     "ka_linear_tiled_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,
@@ -137,7 +139,7 @@ TILED_CONFIG = 0
 # a kernel for the case, bias, activation and the sum into the residual being its epilogues; the
 # tiled kernels of this package then take what it declines. Measured on MI355X at Moondream 2's
 # four linears: 201 against 242 us a layer at 2,048 rows, 112 against 151 at 730, 64 against 72 at 96.
-# (The two last linears of a block go by tiles of their own where ``pair_tiles_pay`` says so.)
+# (The two last linears of a block go by tiles of their own where ``pair_tiles_pay`` says so, and a linear whose tiles are one round of the chip where ``quad_tile`` names one.)
 LIBRARY_LINEAR = True
 LIBRARY_WORKSPACE_BYTES = 128 << 20
 # Activations that the library has no epilogue for (relu squared: ops.linear.ACT_RELU_SQUARED), and the size of an output from
@@ -372,6 +374,11 @@ def linear_bf16(a, weight, bias, out, act, accumulate) -> bool:
                                             int(accumulate), chip_sizes(a.device).skinny_target_waves, *_wide_args(a.device, m), stream_ptr()))
     else:
         if LIBRARY_LINEAR and TILED_CONFIG == 0:
+            tile = quad_tile(a, weight, bias, out, act)
+            if tile:
+                _check(handle.ka_linear_quad_bf16(a.data_ptr(), a.stride(0), weight.data_ptr(), weight.stride(0), _ptr(bias), out.data_ptr(), _OUT_CODE[out.dtype],
+                                                  out.stride(0), m, n, k, act, int(accumulate), tile, stream_ptr()))
+                return True
             space = _library_workspace(a.device)
             # (an activation the library has no epilogue for: a pass of its own over the products)
             apart = act in _ACTIVATIONS_APART and m >= ACTIVATION_APART_FROM_ROWS and n >= ACTIVATION_APART_FROM_COLUMNS \
@@ -389,6 +396,16 @@ def linear_bf16(a, weight, bias, out, act, accumulate) -> bool:
                                            out.data_ptr(), _OUT_CODE[out.dtype], out.stride(0), m, n, k, act,
                                            int(accumulate), TILED_CONFIG, *_wide_args(a.device, m), stream_ptr()))
     return True
+
+
+def quad_tile(a, weight, bias, out, act: int) -> int:
+    """The tile by which this package's own kernel runs a linear of more than ``SKINNY_MAX_ROWS`` rows; 0: the vendor library is faster, or it is not covered."""
+    (m, k), n = a.shape, weight.shape[0]
+    tile = lib().ka_linear_quad_tile(m, n, k)
+    if not tile or act & ACT_GATED or out.stride(0) < n or out.stride(0) % 8 or (bias is not None and bias.data_ptr() % 16) \
+            or any(t.stride(0) < k or (t.shape[0] - 1) * t.stride(0) + k >= 1 << 31 for t in (a, weight)):
+        return 0
+    return tile
 
 
 def linear_pair_accumulate(a1, w1, b1, a2, w2, b2, out, then_norm=None, accumulate: bool = True, large: bool = False) -> bool:
