@@ -195,6 +195,10 @@ struct SpreadArgs {
     int keep_first, maps;
     float softcap;
     int gate_per_head;
+    // a step of single tokens whose keys and values are not cached yet: they lie behind the queries of `q`
+    const int* slots;           // where they go (< 0: nowhere)
+    const float* table;         // [places, rot]: cosines, then sines
+    int rot, interleaved;
 };
 
 typedef __attribute__((ext_vector_type(4))) float as_floatx4;
@@ -224,8 +228,25 @@ __device__ __forceinline__ void as_scatter_sums(float (&v)[16], int lane) {
 
 constexpr int AS_PARTS = 4;
 
-// NW waves take the parts in turn: the sums of a token are the same whatever NW is.
-template <int G, int NW>
+// Four channels of a head from `d` on, the first `rot` of them rotated (as rope_cache_kernel does).
+__device__ __forceinline__ as_floatx4 as_rotated(const float* head, const float* cs, int rot, int interleaved, int d) {
+    as_floatx4 y = *reinterpret_cast<const as_floatx4*>(head + d);
+    const int half = rot / 2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int c = d + e;
+        if (c >= rot) continue;
+        const int i = interleaved ? c / 2 : (c < half ? c : c - half), ia = interleaved ? 2 * i : i, ib = interleaved ? 2 * i + 1 : i + half;
+        const float a = head[ia], b = head[ib], co = cs[i], si = cs[half + i];
+        y[e] = c == ia ? a * co - b * si : b * co + a * si;
+    }
+    return y;
+}
+
+// NW waves take the parts in turn: the sums of a token are the same whatever NW is. STEP: the token's own key and value come from the projected row, rotated here, and the first
+// head that reads them puts them into the cache; in a chunk of keys they take the place of what the cache holds there. (As a launch in front and this
+// one, us, 32 heads of 64: three tokens behind 160 keys 9.6 and 8.0, six behind 400 17.1 and 14.8, six behind 2,000 48.8 and 42.9; heads of 80, three behind 160 10.6 and 10.4.)
+template <int G, int NW, bool STEP>
 __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadArgs g) {
     constexpr int GROUPS = KA_WAVE / G, CK = 16 * GROUPS, R = G / 4;         // groups of 16 keys in a chunk of CK; channels in sixteens
     __shared__ long k_at[NW][CK], v_at[NW][CK];
@@ -238,7 +259,31 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
     const int in_row = lane % G, group = lane / G;
     const bool owns = in_row < 16;                       // (the other rows of a group hold the same keys' scores once more)
     as_floatx4 q4 = {0.f, 0.f, 0.f, 0.f};
-    if (in_row * 4 < g.hd) {
+    as_floatx4 own_k = {0.f, 0.f, 0.f, 0.f};
+    float own_v[R];
+    const int slot = STEP ? g.slots[t] : -1;
+    if constexpr (STEP) {
+        const float *row = g.q + (size_t)t * g.q_row_stride, *krow = row + (size_t)g.H * g.hd + (size_t)kvh * g.hd, *vrow = row + (size_t)(g.H + g.Hkv) * g.hd + (size_t)kvh * g.hd;
+        const float* cs = g.rot ? g.table + (size_t)g.positions[t] * g.rot : nullptr;
+#pragma unroll
+        for (int r = 0; r < R; ++r) own_v[r] = vrow[min(r * 16 + lane / 4, g.hdv - 1)];
+        if (in_row * 4 < g.hd) {
+            q4 = as_rotated(row + (size_t)h * g.hd, cs, g.rot, g.interleaved, in_row * 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q4[i] *= g.scale;
+            own_k = as_rotated(krow, cs, g.rot, g.interleaved, in_row * 4);
+        }
+        if (slot >= 0 && wave == 0 && h % (g.H / g.Hkv) == 0) {
+            const long page = slot / g.page_size;
+            const int off = slot % g.page_size;
+            if (group == 0 && in_row * 4 < g.hd)
+                *reinterpret_cast<as_floatx4*>(const_cast<float*>(g.k_cache) + ((page * g.Hkv + kvh) * g.page_size + off) * g.hd + in_row * 4) = own_k;
+            if (lane % 4 == 0)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (r * 16 + lane / 4 < g.hdv) const_cast<float*>(g.v_cache)[((page * g.Hkv + kvh) * g.hdv + r * 16 + lane / 4) * g.page_size + off] = own_v[r];
+        }
+    } else if (in_row * 4 < g.hd) {
         const float* qp = g.q + (size_t)t * g.q_row_stride + (size_t)h * g.hd + in_row * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) q4[i] = qp[i] * g.scale;
@@ -263,8 +308,13 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
             const int base = first ? c * CK : start + (c - kept_chunks) * CK, from = first ? 0 : lo, to = first ? kept : hi;
             const int key = base + group * 16 + lane % 16;
             const bool valid = key >= from && key < to;
+            int own = -1;                                // STEP: the place in the chunk of the token's own key
             {
                 const int near = min(max(key, from), to - 1), page = bt[near / g.page_size], at = near % g.page_size;
+                if constexpr (STEP) {
+                    const unsigned long long hit = __ballot(owns && valid && page * g.page_size + at == slot);
+                    if (hit) own = (int)__builtin_ctzll(hit) / G * 16 + (int)__builtin_ctzll(hit) % G;
+                }
                 as_wave_sync();                          // the chunk before has been read
                 if (owns) {
                     k_at[wave][group * 16 + in_row] = (((long)page * g.Hkv + kvh) * g.page_size + at) * g.hd;
@@ -281,6 +331,16 @@ __global__ void __launch_bounds__(KA_WAVE * NW) attention_spread_kernel(SpreadAr
                 const float* vp = g.v_cache + v_at[wave][x * 16 + lane % 4 * 4];
 #pragma unroll
                 for (int r = 0; r < R; ++r) v4[x][r] = *reinterpret_cast<const as_floatx4*>(vp + (long)min(r * 16 + lane / 4, g.hdv - 1) * g.page_size);
+            }
+            if (STEP && own >= 0) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) k4[i] = group * 16 + i == own ? own_k : k4[i];
+#pragma unroll
+                for (int x = 0; x < GROUPS; ++x)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v4[x][r][i] = x * 16 + lane % 4 * 4 + i == own ? own_v[r] : v4[x][r][i];
             }
             float part_s[16];
 #pragma unroll
@@ -356,8 +416,8 @@ static void launch_spread(const SpreadArgs& g, int n, hipStream_t stream) {
     // A wave a part where workgroups of four waves are two a CU at the most, else one wave for all: heads of 64, us, four waves and one: 3 tokens behind 160
     // keys 6.5 and 8.7, 16 behind 200 14.2 and 17.3, but 32 behind 64 8.9 and 8.6, a prompt of 33 9.4 and 6.4, six of 20 21 and 9.3. Long rows
     // of many tokens do not care (64 behind 400 76 and 74).
-    if ((long)n * g.H <= 2L * ka_compute_units()) hipLaunchKernelGGL((attention_spread_kernel<G, AS_PARTS>), dim3(n, g.H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
-    else hipLaunchKernelGGL((attention_spread_kernel<G, 1>), dim3(n, g.H), dim3(KA_WAVE), 0, stream, g);
+    if ((long)n * g.H <= 2L * ka_compute_units()) hipLaunchKernelGGL((attention_spread_kernel<G, AS_PARTS, false>), dim3(n, g.H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
+    else hipLaunchKernelGGL((attention_spread_kernel<G, 1, false>), dim3(n, g.H), dim3(KA_WAVE), 0, stream, g);
 }
 
 KA_API int ka_attention_generic(const void* q, int dtype, long q_row_stride, const void* k_cache,
@@ -386,7 +446,7 @@ KA_API int ka_attention_generic(const void* q, int dtype, long q_row_stride, con
         ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0) {
         const SpreadArgs g{(const float*)q, q_row_stride, (const float*)k_cache, (const float*)v_cache, block_table, max_pages, token_row, kv_lo, kv_hi,
                            (float*)out, out_row_stride, scale, H, Hkv, hd, hdv, page_size, positions, slopes, has_sink, sink_score, bias_table, bias_len,
-                           (const float*)gate, gate_row_stride, sinks, keep_first, maps, softcap, gate_per_head};
+                           (const float*)gate, gate_row_stride, sinks, keep_first, maps, softcap, gate_per_head, nullptr, nullptr, 0, 0};
         const int wide = hd > hdv ? hd : hdv;
         if (wide <= 64) launch_spread<16>(g, n, stream);
         else if (wide <= 128) launch_spread<32>(g, n, stream);
@@ -405,4 +465,25 @@ KA_API int ka_attention_generic(const void* q, int dtype, long q_row_stride, con
         KA_CHECK(false, "ka_attention_generic: unsupported dtype %d", dtype);
     KA_LAUNCH_CHECK();
     return 0;
+}
+
+// A step of single tokens in 32 bits: rotation, cache write and attention in one launch. qkv rows: [H hd q | Hkv hd k | Hkv hd v], not changed. 1: done; 0: not covered,
+// nothing was run; -1: an error.
+KA_API int ka_attention_step_f32(const float* qkv, long row_stride, float* k_cache, float* v_cache, const int* block_table, int max_pages, const int* token_row, const int* kv_lo,
+                                 const int* kv_hi, float* out, long out_row_stride, float scale, int n, int H, int Hkv, int hd, int page_size, const int* positions,
+                                 const int* slots, const float* table, int table_rows, int rot, int interleaved, hipStream_t stream) {
+    const char* who = "ka_attention_step_f32";
+    KA_CHECK(n > 0 && H > 0 && Hkv > 0 && hd > 0 && H % Hkv == 0 && H <= 65535, "%s: n=%d heads %d, %d of %d", who, n, H, Hkv, hd);
+    KA_CHECK(page_size > 0 && max_pages > 0 && slots && row_stride >= (long)(H + 2 * Hkv) * hd && out_row_stride >= (long)H * hd, "%s: pages of %d, %d a row, strides %ld and %ld", who,
+             page_size, max_pages, row_stride, out_row_stride);
+    KA_CHECK(rot >= 0 && rot <= hd && rot % 2 == 0 && (rot == 0 || (table && table_rows > 0 && positions)), "%s: rotation of %d channels", who, rot);
+    // (one workgroup a CU at the most: with 214 to 240 registers instead of 126 to 160 two of them share a CU worse; 16 tokens of 32 heads behind 200 keys 19.5 us, the two launches 18.3)
+    if ((long)n * H > ka_compute_units() || hd % 4 || hd > 256 || page_size % 4 || row_stride % 4 || ((uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)qkv) % 16) return 0;
+    const SpreadArgs g{qkv, row_stride, k_cache, v_cache, block_table, max_pages, token_row, kv_lo, kv_hi, out, out_row_stride, scale, H, Hkv, hd, hd, page_size, positions,
+                       nullptr, 0, 0.f, nullptr, 0, nullptr, 0, nullptr, 0, 1, 0.f, 0, slots, table, rot, interleaved};
+    if (hd <= 64) hipLaunchKernelGGL((attention_spread_kernel<16, AS_PARTS, true>), dim3(n, H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
+    else if (hd <= 128) hipLaunchKernelGGL((attention_spread_kernel<32, AS_PARTS, true>), dim3(n, H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
+    else hipLaunchKernelGGL((attention_spread_kernel<64, AS_PARTS, true>), dim3(n, H), dim3(AS_PARTS * KA_WAVE), 0, stream, g);
+    KA_LAUNCH_CHECK();
+    return 1;
 }

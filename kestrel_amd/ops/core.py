@@ -29,6 +29,13 @@ _SIGNATURES = {
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "ka_linear_generic": [_c_void_p, _c_int, _c_long, _c_void_p, _c_int, _c_long, _c_void_p, _c_void_p, _c_int,
                           _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_linears_first_f32": [_c_void_p, _c_long, _c_void_p, _c_void_p, _c_float,                            # x, ldx, norm
+                             _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int,            # W, ldw, bias, out, ldo, N, act of either linear
+                             _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+    "ka_linears_last_f32": [_c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_void_p, _c_long, _c_void_p,
+                            _c_void_p, _c_long, _c_int, _c_int, _c_void_p],
+    "ka_attention_step_f32": [_c_void_p, _c_long, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_long, _c_float,
+                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "ka_attention_generic": [_c_void_p, _c_int, _c_long, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p,
                              _c_void_p, _c_void_p, _c_void_p, _c_long, _c_float, _c_int, _c_int, _c_int, _c_int,
                              _c_int, _c_int, _c_void_p, _c_void_p, _c_int, _c_float, _c_void_p, _c_int, _c_void_p, _c_long,
@@ -1188,6 +1195,72 @@ def linear_generic(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     _check(lib().ka_linear_generic(a.data_ptr(), code_of(a.dtype), a.stride(0), weight.data_ptr(),
                                    code_of(weight.dtype), weight.stride(0), _ptr(bias), out.data_ptr(),
                                    code_of(out.dtype), out.stride(0), m, n, k, act, int(accumulate), stream_ptr()))
+
+
+# Most rows of the launches of two fp32 linears (GP_ROWS in csrc/gemv_pairs_f32.hip).
+FEW_F32_ROWS = 8
+
+
+def _f32_rows(t: torch.Tensor, rows: int, columns: int) -> bool:
+    return t.dtype == torch.float32 and t.dim() == 2 and tuple(t.shape) == (rows, columns) and t.stride(1) == 1 and t.stride(0) >= columns
+
+
+def _f32_vector(t: Optional[torch.Tensor], n: int) -> bool:
+    return t is None or (t.dtype == torch.float32 and t.numel() == n and t.is_contiguous())
+
+
+def linears_first_f32(x: torch.Tensor, norm, wa: torch.Tensor, ba: Optional[torch.Tensor], out_a: torch.Tensor, act_a: int,
+                      wb: torch.Tensor, bb: Optional[torch.Tensor], out_b: torch.Tensor, act_b: int) -> bool:
+    """``out_a = act_a(h @ wa.T + ba)`` and ``out_b = act_b(h @ wb.T + bb)`` of a few fp32 rows in one launch, ``h = LayerNorm(x)`` with ``norm =
+    (gamma, beta or None, eps)``, or ``x`` itself (``None``); the same bits as in a launch each. False: not covered, nothing was run."""
+    m, k = x.shape
+    na, nb = wa.shape[0], wb.shape[0]
+    gamma, beta, eps = norm if norm is not None else (None, None, 0.0)
+    if not (m and _f32_rows(x, m, k) and _f32_rows(wa, na, k) and _f32_rows(wb, nb, k) and _f32_rows(out_a, m, na) and _f32_rows(out_b, m, nb)
+            and _f32_vector(ba, na) and _f32_vector(bb, nb) and _f32_vector(gamma, k) and _f32_vector(beta, k)):
+        return False
+    _dev(x, gamma, beta, wa, ba, out_a, wb, bb, out_b)
+    status = lib().ka_linears_first_f32(x.data_ptr(), x.stride(0), _ptr(gamma), _ptr(beta), float(eps), wa.data_ptr(), wa.stride(0), _ptr(ba), out_a.data_ptr(),
+                                        out_a.stride(0), na, act_a, wb.data_ptr(), wb.stride(0), _ptr(bb), out_b.data_ptr(), out_b.stride(0), nb, act_b, m, k, stream_ptr())
+    _check(min(status, 0))
+    return status == 1
+
+
+def linears_last_f32(a1: torch.Tensor, w1: torch.Tensor, b1: Optional[torch.Tensor], a2: torch.Tensor, w2: torch.Tensor, b2: Optional[torch.Tensor],
+                     out: torch.Tensor) -> bool:
+    """``out += a1 @ w1.T + b1``, then ``out += a2 @ w2.T + b2``, of a few fp32 rows in one launch; the same bits as in a launch each. False: not covered,
+    nothing was run."""
+    (m, k1), (n, k2) = a1.shape, w2.shape
+    if not (m and _f32_rows(a1, m, k1) and _f32_rows(w1, n, k1) and _f32_rows(a2, m, k2) and _f32_rows(w2, n, k2) and _f32_rows(out, m, n)
+            and _f32_vector(b1, n) and _f32_vector(b2, n)):
+        return False
+    _dev(a1, w1, b1, a2, w2, b2, out)
+    status = lib().ka_linears_last_f32(a1.data_ptr(), a1.stride(0), k1, w1.data_ptr(), w1.stride(0), _ptr(b1), a2.data_ptr(), a2.stride(0), k2, w2.data_ptr(),
+                                       w2.stride(0), _ptr(b2), out.data_ptr(), out.stride(0), m, n, stream_ptr())
+    _check(min(status, 0))
+    return status == 1
+
+
+def attention_step_f32(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, table: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: torch.Tensor,
+                       block_table: torch.Tensor, token_row: torch.Tensor, kv_lo: Optional[torch.Tensor], kv_hi: torch.Tensor, out: torch.Tensor, scale: float,
+                       n_heads: int, n_kv_heads: int, head_dim: int, pairing: str = "halves") -> bool:
+    """``rope_cache`` and ``attention_generic`` of single fp32 tokens, each of a row of its own, in one launch; the queries in ``qkv`` stay as they are. False: not
+    covered, nothing was run."""
+    n, page_size = qkv.shape[0], k_cache.shape[2]
+    ints = [positions, slots, token_row, kv_hi] + ([kv_lo] if kv_lo is not None else [])
+    if not (n and qkv.dtype == torch.float32 and qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == (n_heads + 2 * n_kv_heads) * head_dim
+            and _f32_rows(out, n, n_heads * head_dim) and all(t.dtype == torch.int32 and t.numel() == n and t.is_contiguous() for t in ints)
+            and block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.is_contiguous()
+            and (table is None or (table.dtype == torch.float32 and table.dim() == 2 and table.is_contiguous())) and pairing in ROTARY_PAIRINGS):
+        return False
+    _check_caches("attention_step", k_cache, v_cache, qkv.dtype, n_kv_heads, page_size, head_dim)
+    _dev(qkv, *ints, block_table, table, k_cache, v_cache, out)
+    rows, rot = table.shape if table is not None else (0, 0)
+    status = lib().ka_attention_step_f32(qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1],
+                                         token_row.data_ptr(), _ptr(kv_lo), kv_hi.data_ptr(), out.data_ptr(), out.stride(0), float(scale), n, n_heads, n_kv_heads, head_dim,
+                                         page_size, positions.data_ptr(), slots.data_ptr(), _ptr(table), rows, rot, ROTARY_PAIRINGS[pairing], stream_ptr())
+    _check(min(status, 0))
+    return status == 1
 
 
 def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,

@@ -308,6 +308,10 @@ class PagedAttention(Mixer):
         if beside is not None:
             self._alone(beside)
         slots = group.slots if cache.writes else None
+        if batch.decode_only and slots is not None and qkv.dtype == torch.float32 and \
+                core.attention_step_f32(qkv, batch.positions, slots, self._table, cache.k, cache.v, group.block_table, batch.token_row, group.kv_lo, batch.kv_hi,
+                                        out, self.scale, spec.n_heads, spec.n_kv_heads, spec.head_dim, self._pairing):
+            return out
         done = False
         if qkv.dtype == torch.bfloat16 and halves:
             from ..ops import fast

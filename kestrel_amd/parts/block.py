@@ -93,6 +93,39 @@ def _parallel_few_rows(block: "Block", x, batch, cache, normed, then, handed) ->
     return True
 
 
+def _parallel_few_rows_f32(block: "Block", x, batch, cache, normed) -> bool:
+    """The parallel block for a few fp32 rows in three launches, as ``_parallel_few_rows`` has them: norm and both first linears, the mixer's core, both last
+    linears; what ``ops.core`` does not cover is a launch each. Returns ``False`` (nothing was run) where the parts do not offer their stages."""
+    from ..ops import core
+    from ..ops.linear import ACT_GATED, linear
+
+    n = x.shape[0]
+    if block.dtype != torch.float32 or n > core.FEW_F32_ROWS or block.feed_forward is None:
+        return False
+    m_in, f_in = block.mixer.input_projection(), block.feed_forward.input_projection()
+    m_out, f_out = block.mixer.output_projection(), block.feed_forward.output_projection()
+    if m_in is None or f_in is None or m_out is None or f_out is None or f_in[3] & ACT_GATED:
+        return False
+    ws = batch.workspace
+    projected = ws.get("block.mixer_in", (n, m_in[2]), block.dtype)
+    hidden = ws.get("block.ff_hidden", (n, f_in[2]), block.dtype)
+    first = (m_in[0], m_in[1], projected, 0, f_in[0], f_in[1], hidden, f_in[3])
+    ln = block.norm.layernorm_operands() if normed is None else None
+    if ln is None or not core.linears_first_f32(x, ln, *first):
+        h = normed
+        if h is None:
+            h = ws.get("block.h", tuple(x.shape), block.dtype)
+            block.norm.forward(x, h)
+        if not core.linears_first_f32(h, None, *first):
+            linear(h, m_in[0], m_in[1], projected)
+            linear(h, f_in[0], f_in[1], hidden, act=f_in[3])
+    mixed = block.mixer.attend(projected, batch, cache)
+    if not core.linears_last_f32(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], x):
+        linear(mixed, m_out[0], m_out[1], x, accumulate=True)
+        linear(hidden, f_out[0], f_out[1], x, accumulate=True)
+    return True
+
+
 def _parallel(block: "Block", x, batch, cache, normed=None, then=None):
     """``x + mixer(norm(x)) + ff(norm(x))``: both branches read the same normalised input (a block without a
     feed-forward has the first branch only).
@@ -102,6 +135,8 @@ def _parallel(block: "Block", x, batch, cache, normed=None, then=None):
     handed = []
     if _parallel_few_rows(block, x, batch, cache, normed, then, handed):
         return handed[0] if handed else None
+    if _parallel_few_rows_f32(block, x, batch, cache, normed):
+        return None
     h = normed
     if h is None:
         h = batch.workspace.get("block.h", tuple(x.shape), block.dtype)
