@@ -2,7 +2,7 @@
 
 from __future__ import annotations
 
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 from typing import Dict, Optional, Tuple
 
 import torch
@@ -90,4 +90,61 @@ class StepBatch:
     decode_only: bool = False
     causal_only: bool = True            # no token sees past its own position
     wants_every_token: bool = False     # ``logit_rows`` is 0, 1, ..., n_tokens - 1: every token's logits, in order
+    whole_last: bool = False            # every token through the last layer, whichever are wanted (a warm-up: scratch of any step)
     host: dict = field(default_factory=dict)
+
+    def wanted_alone(self) -> Optional["WantedTokens"]:
+        """The tokens whose logits are wanted as a step of their own, where that pays (``WantedTokens``)."""
+        return WantedTokens(self) if not self.whole_last and WantedTokens.pays(self) else None
+
+
+class WantedTokens:
+    """The tokens of a step whose logits are wanted, as a step of its own: what is left to do behind the last kernel that reads a
+    token's row for another token's sake (the last layer's keys, values and states).
+
+    ``batch`` lists them as single tokens, in the order of the logits, that read their requests' caches and write nothing. Its columns, and whatever a
+    part hands over on the way, are picked out of the step by ``gather``, the columns by its first call."""
+
+    # Most wanted tokens, and tokens of the step to each of them: attention over single tokens reads a request's keys once for each of them.
+    MOST, SHARE = 64, 2
+
+    @classmethod
+    def pays(cls, batch: "StepBatch") -> bool:
+        wanted = int(batch.logit_rows.numel())
+        return not batch.decode_only and wanted <= cls.MOST and wanted * cls.SHARE <= batch.n_tokens
+
+    def __init__(self, batch: "StepBatch") -> None:
+        self.rows = batch.logit_rows
+        self.count = int(self.rows.numel())
+        self._workspace = batch.workspace
+        self._columns = []
+
+        def column(name: str, source: torch.Tensor) -> torch.Tensor:
+            own = self.buffer(name, source)
+            self._columns.append((source, own))
+            return own
+
+        groups = {key: replace(g, slots=g.slots[:0], kv_lo=None if g.kv_lo is None else column(f"kv_lo{key}", g.kv_lo))
+                  for key, g in batch.groups.items()}
+        self.batch = replace(
+            batch, n_tokens=self.count, n_rows=self.count, token_ids=batch.token_ids[:0], positions=column("positions", batch.positions),
+            token_row=column("token_row", batch.token_row), kv_hi=column("kv_hi", batch.kv_hi), row_slot=batch.row_slot[:0], cu_q=batch.cu_q[:0],
+            kv_len=batch.kv_len[:0], groups=groups, query_blocks={}, page_runs=None, position_axes=None, given_embeds=None, given_rows=None, max_q=1,
+            decode_only=True, wants_every_token=True, host={})
+
+    def buffer(self, name: str, like: torch.Tensor) -> torch.Tensor:
+        """Scratch for the wanted rows of ``like``."""
+        return self._workspace.get("wanted." + name, (self.count, *like.shape[1:]), like.dtype)
+
+    def gather(self, *pairs) -> None:
+        """``dst[i] = src[rows[i]]`` for every ``(src, dst)``."""
+        from ..ops import core
+
+        core.gather_rows(self.rows, [*self._columns, *pairs])
+        self._columns = []
+
+    def take(self, name: str, source: torch.Tensor, *pairs) -> torch.Tensor:
+        """The wanted rows of ``source`` in scratch memory, and ``pairs`` besides."""
+        own = self.buffer(name, source)
+        self.gather((source, own), *pairs)
+        return own

@@ -805,7 +805,13 @@ class ModelRunner:
                 continue
             slot = self.admit(tokens, tokens)
             try:
-                self.step([StepEntry(slot, np.zeros(tokens, dtype=np.int64), want=list(range(min(tokens, wanted_rows, rows))))])
+                entries = [StepEntry(slot, np.zeros(tokens, dtype=np.int64), want=list(range(min(tokens, wanted_rows, rows))))]
+                if tokens == sizes[0]:
+                    # (the last layer's scratch for as many tokens, too: a step may want most of its tokens)
+                    batch = self.build_batch(entries)
+                    batch.whole_last = True
+                    self.model.forward(batch, self.layer_caches)
+                self.step(entries)
             finally:
                 self.release(slot)
         torch.cuda.synchronize(self.device)

@@ -172,6 +172,7 @@ class DecoderModel:
             first = self.blocks[plan.schedule[0].layer].reader if plan.schedule else None
             handed = ws.get("block.h", (batch.n_tokens, plan.dim), self.dtype) if first is not None else None
             core.streams_step(x, embedded=embedded, reading=first.operands() if first is not None else None, h=handed)
+        rows = batch.logit_rows
         for index, entry in enumerate(plan.schedule):
             after = plan.schedule[index + 1] if index + 1 < len(plan.schedule) else None
             # (a junction between two runs changes the stream: no norm is handed across it)
@@ -183,7 +184,14 @@ class DecoderModel:
                 settle(x, batch)
                 self.junctions[before].forward(x, batch, passage=int(getattr(entry, "passage", 0)))
                 handed = None
-            handed = self.blocks[entry.layer].forward(x, batch, caches[index], normed=handed, then=then)
+            block = self.blocks[entry.layer]
+            few = batch.wanted_alone() if after is None and block.narrows else None
+            if few is not None:
+                # nobody reads the last layer's rows but for the wanted ones: from here on the step is those tokens
+                x, handed = block.forward_wanted(x, batch, caches[index], few, normed=handed, then=final if few.count else None)
+                batch, rows = few.batch, None
+                break
+            handed = block.forward(x, batch, caches[index], normed=handed, then=then)
         settle(x, batch)       # (what the last block has left to be added into the stream)
         wanted = int(batch.logit_rows.numel())
         logits = ws.get("model.logits", (wanted, plan.vocab_size), torch.float32)
@@ -191,12 +199,12 @@ class DecoderModel:
             normed = handed if batch.decode_only and getattr(batch, "wants_every_token", False) else None
             if normed is None:
                 normed = ws.get("model.head_in", (wanted, plan.dim), self.dtype)
-                core.streams_step(x, reading=final.operands(), h=normed, rows=batch.logit_rows)
+                core.streams_step(x, reading=final.operands(), h=normed, rows=rows)
             linear(normed, self.head_weight, self.head_bias, logits)
         elif wanted:
             if not self._head_with_norm(x, batch, logits):
                 normed = ws.get("model.head_in", (wanted, plan.dim), self.dtype)
-                self.final_norm.forward(x, normed, rows=batch.logit_rows)
+                self.final_norm.forward(x, normed, rows=rows)
                 linear(normed, self.head_weight, self.head_bias, logits)
         if wanted:
             if plan.logit_scale != 1.0 or plan.logit_softcap is not None:

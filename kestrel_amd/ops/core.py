@@ -22,6 +22,7 @@ _c_void_p, _c_int, _c_long, _c_float = ctypes.c_void_p, ctypes.c_int, ctypes.c_l
 _SIGNATURES = {
     "ka_embed": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int, _c_int, _c_float, _c_void_p],
     "ka_adjust_logits": [_c_void_p, _c_long, _c_float, _c_float, _c_void_p],
+    "ka_gather_rows": [_c_void_p, _c_int, _c_int] + [_c_void_p] * 6,
     "ka_scatter_rows": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p],
     "ka_layernorm": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_int, _c_int,
                      _c_void_p],
@@ -274,6 +275,34 @@ def scatter_rows(src: torch.Tensor, rows: torch.Tensor, out: torch.Tensor) -> No
     _need(rows.dtype == torch.int32 and rows.numel() == m and rows.is_contiguous(), "scatter_rows: rows int32 [m]")
     _check(lib().ka_scatter_rows(src.data_ptr(), code_of(src.dtype), rows.data_ptr(), out.data_ptr(), m, dim,
                                  stream_ptr()))
+
+
+GATHER_PAIRS = 12          # most pairs of one launch (GR_PAIRS)
+
+
+def gather_rows(rows: torch.Tensor, pairs) -> None:
+    """``dst[i] = src[rows[i]]`` for every ``(src, dst)`` of ``pairs`` (same type and shape behind the first axis; rows may lie in wider ones)."""
+    m = rows.numel()
+    _need(rows.dtype == torch.int32 and rows.is_contiguous(), "gather_rows: rows int32 [m]")
+    _dev(rows)
+    table = []
+    for src, dst in pairs:
+        _dev(src, dst)
+        _need(src.dtype == dst.dtype and dst.shape[0] == m and tuple(src.shape[1:]) == tuple(dst.shape[1:]), "gather_rows: pairs of one type and row")
+        size, row = src.element_size(), 1
+        for t in (src, dst):
+            row = 1
+            for extent, stride in zip(reversed(t.shape[1:]), reversed(t.stride()[1:])):
+                _need(extent == 1 or stride == row, "gather_rows: a row's numbers must lie side by side")
+                row *= extent
+        table.append((src.data_ptr(), src.stride(0) * size, dst.data_ptr(), dst.stride(0) * size, row * size))
+    if m == 0:
+        return
+    for at in range(0, len(table), GATHER_PAIRS):
+        part = table[at:at + GATHER_PAIRS]
+        columns = [(kind * len(part))(*(row[i] for row in part)) for i, kind in
+                   enumerate((ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p, ctypes.c_long, ctypes.c_long))]
+        _check(lib().ka_gather_rows(rows.data_ptr(), m, len(part), *columns, stream_ptr()))
 
 
 def layernorm(x: torch.Tensor, gamma: torch.Tensor, beta: Optional[torch.Tensor], eps: float, out: torch.Tensor,

@@ -285,12 +285,11 @@ class PagedAttention(Mixer):
             step = beside.job if isinstance(beside, SideStep) else None
             if beside is not None and step is None:
                 self._alone(beside)
-            return self._attend_prepared(qkv, batch, cache, group, out, step)
+            return self._read_prepared(*self._prepare(qkv, batch, cache, group, step), batch, cache, group, out)
         if self.extended:
             if beside is not None:
                 self._alone(beside)
-            return self._attend_extended(qkv, batch, cache, group, out)
-        halves = self._pairing == "halves"
+            return self._read_extended(self._unit_norm(qkv, batch, cache, group), batch, cache, group, out)
         if qkv.dtype == torch.bfloat16 and self._decodes_fused(batch, cache):
             from ..ops import fast
             k_new = qkv[:, self.q_dim:self.q_dim + self.kv_dim]
@@ -312,8 +311,14 @@ class PagedAttention(Mixer):
                 core.attention_step_f32(qkv, batch.positions, slots, self._table, cache.k, cache.v, group.block_table, batch.token_row, group.kv_lo, batch.kv_hi,
                                         out, self.scale, spec.n_heads, spec.n_kv_heads, spec.head_dim, self._pairing):
             return out
+        return self._read(self._rotate(qkv, batch, cache, group), batch, cache, group, out)
+
+    def _rotate(self, qkv, batch, cache: LayerCache, group):
+        """Position encoding and cache write, in place."""
+        spec = self.spec
+        slots = group.slots if cache.writes else None
         done = False
-        if qkv.dtype == torch.bfloat16 and halves:
+        if qkv.dtype == torch.bfloat16 and self._pairing == "halves":
             from ..ops import fast
             done = fast.rope_cache_bf16(qkv, batch.positions, slots, self._table, cache.k, cache.v, spec.n_heads,
                                         spec.n_kv_heads, spec.head_dim, group.page_size,
@@ -321,18 +326,57 @@ class PagedAttention(Mixer):
         if not done:
             core.rope_cache(qkv, batch.positions, slots, self._table, cache.k, cache.v, spec.n_heads, spec.n_kv_heads,
                             spec.head_dim, group.page_size, self._pairing)
+        return qkv
+
+    def _read(self, qkv, batch, cache: LayerCache, group, out):
+        """Attention of rotated queries."""
+        spec = self.spec
         paged_attention(qkv, cache.k, cache.v, group.block_table, batch.token_row, group.kv_lo, batch.kv_hi, out,
                         self.scale, spec.n_heads, spec.n_kv_heads, spec.head_dim, batch)
         return out
 
-    def _attend_extended(self, qkv, batch, cache: LayerCache, group, out):
-        """Queries and keys to unit norm, the cache write, then attention with the terms the specification names."""
+    def attend_wanted(self, qkv, batch, cache: LayerCache, wanted, *also, out=None):
+        """``attend`` where only the tokens of ``wanted`` are read: keys and values of all tokens go into the cache, those tokens' queries are
+        picked out (and the pairs of ``also`` with them) and read it as single tokens. Returns their heads."""
+        group = batch.groups[cache.group]
+        gate = None
+        if self.prepared:
+            q, gate = self._prepare(qkv, batch, cache, group)
+        elif self.extended:
+            q = self._unit_norm(qkv, batch, cache, group)
+        else:
+            q = self._rotate(qkv, batch, cache, group)
+        q = q[:, :self.q_dim]
+        q_few = wanted.buffer("q", q)
+        pairs = [(q, q_few), *also]
+        if gate is not None:
+            pairs.append((gate, wanted.buffer("gate", gate)))
+            gate = pairs[-1][1]
+        wanted.gather(*pairs)
+        if out is None:
+            out = wanted.batch.workspace.get("attn.out", (wanted.count, self.out_dim), self.dtype)
+        few = wanted.batch
+        if wanted.count == 0:
+            return out
+        if self.prepared:
+            return self._read_prepared(q_few, gate, few, cache, few.groups[cache.group], out)
+        if self.extended:
+            return self._read_extended(q_few, few, cache, few.groups[cache.group], out)
+        return self._read(q_few, few, cache, few.groups[cache.group], out)
+
+    def _unit_norm(self, qkv, batch, cache: LayerCache, group):
+        """Queries and keys to unit norm and the cache write, in place."""
         spec = self.spec
         slots = group.slots if cache.writes else None
         # (a decode step's tokens are each a run of their own: nothing to gain from the lists there)
         core.unit_norm_cache(qkv, slots, cache.k, cache.v, spec.n_heads, spec.n_kv_heads, spec.head_dim, self.value_dim,
                              group.page_size, self.unit_norm_eps,
                              runs=None if batch.decode_only else getattr(batch, "page_runs", None))
+        return qkv
+
+    def _read_extended(self, qkv, batch, cache: LayerCache, group, out):
+        """Attention of what ``_unit_norm`` left, with the terms the specification names."""
+        spec = self.spec
         if qkv.dtype == torch.bfloat16:
             from ..ops import fast
             if fast.attention_biased_bf16(qkv, cache.k, cache.v, group.block_table, batch.token_row, group.kv_lo, batch.kv_hi,
@@ -344,10 +388,9 @@ class PagedAttention(Mixer):
                                self._slopes, self.sink)
         return out
 
-    def _attend_prepared(self, projected, batch, cache: LayerCache, group, out, step=None):
-        """Queries, keys and values made ready by one kernel (norms, rotation, factor, blend, cache write), attention with
-        the distance table where there is one, then the output gate. ``projected``: ``[n, q | k | v (| gate)]``. ``step``: a job that the
-        launch of the convolutions takes along (``takes_step``)."""
+    def _prepare(self, projected, batch, cache: LayerCache, group, step=None):
+        """Queries, keys and values made ready by one kernel (norms, rotation, factor, blend, cache write). ``projected``: ``[n, q | k | v (| gate)]``.
+        ``step``: a job that the launch of the convolutions takes along (``takes_step``). Returns the queries and the gate (or ``None``)."""
         spec = self.spec
         n = projected.shape[0]
         qkv = projected[:, :self.qkv_dim] if self.gated else projected
@@ -368,7 +411,11 @@ class PagedAttention(Mixer):
                              (self.growth.coef, self.growth.every) if self.growth is not None else None,
                              self.blend.role if self.blend is not None else None, other, self._blend_weight,
                              values_from_keys=self.values_from_keys)
-        gate = projected[:, self.qkv_dim:] if self.gated else None
+        return qkv, projected[:, self.qkv_dim:] if self.gated else None
+
+    def _read_prepared(self, qkv, gate, batch, cache: LayerCache, group, out):
+        """Attention of what ``_prepare`` left, with the distance table where there is one, then the output gate."""
+        spec = self.spec
         more = dict(sinks=self._sinks, softcap=self.softcap, gate_per_head=self.gate_per_head)
         done = gated = False          # (gated: the attention kernel has applied the output gate in its epilogue)
         if qkv.dtype == torch.bfloat16:
@@ -410,10 +457,25 @@ class PagedAttention(Mixer):
 
     def mix(self, h, batch, cache: LayerCache, out, accumulate: bool) -> None:
         """The mixer's output written into (or added to) fp32 ``out``."""
+        mixed = self.attend(self.project(h, batch), batch, cache)
+        linear(mixed, self.proj_weight, self.proj_bias, out, accumulate=accumulate)
+
+    def project(self, h, batch):
+        """The mixer's first linear."""
         qkv = batch.workspace.get("attn.qkv", (h.shape[0], self.in_dim), self.dtype)
         linear(h, self.qkv_weight, self.qkv_bias, qkv)
-        mixed = self.attend(qkv, batch, cache)
-        linear(mixed, self.proj_weight, self.proj_bias, out, accumulate=accumulate)
+        return qkv
+
+    @property
+    def only_reads(self) -> bool:
+        """Whether nothing of a token's row is kept for another token."""
+        return self.shares_kv and not self.taps
+
+    def mix_wanted(self, h, batch, cache: LayerCache, out, wanted, *also) -> None:
+        """``mix`` for the tokens of ``wanted``, in their order (``attend_wanted``)."""
+        mixed = self.attend_wanted(self.project(h, batch), batch, cache, wanted, *also)
+        if wanted.count:
+            linear(mixed, self.proj_weight, self.proj_bias, out)
 
     def forward(self, h, batch, cache: LayerCache, residual) -> None:
         self.mix(h, batch, cache, residual, True)

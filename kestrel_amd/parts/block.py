@@ -126,12 +126,52 @@ def _parallel_few_rows_f32(block: "Block", x, batch, cache, normed) -> bool:
     return True
 
 
-def _parallel(block: "Block", x, batch, cache, normed=None, then=None):
+def _parallel_wanted(block: "Block", x, batch, cache, normed, wanted):
+    """The parallel block that leaves the wanted tokens alone: the mixer's first linear and what it keeps of all tokens, everything else for those."""
+    from ..ops import fast
+    from ..ops.linear import linear
+
+    ff, ws = block.feed_forward, batch.workspace
+    h = normed
+    if h is None:
+        h = ws.get("block.h", tuple(x.shape), block.dtype)
+        block.norm.forward(x, h)
+    few, h_few = wanted.buffer("x", x), wanted.buffer("h", h)
+    m_out = block.mixer.output_projection() if callable(getattr(block.mixer, "attend_wanted", None)) else None
+    f_in, f_out = (ff.input_projection(), ff.output_projection()) if ff is not None else (None, None)
+    if m_out is None:
+        # (a mixer that only adds: into the stream of all tokens)
+        wanted.gather((h, h_few))
+        block.mixer.forward(h, batch, cache, x)
+        wanted.gather((x, few))
+        mixed = None
+    else:
+        mixed = block.mixer.attend_wanted(block.mixer.project(h, batch), batch, cache, wanted, (x, few), (h, h_few))
+    if wanted.count == 0:
+        return few, None
+    if mixed is not None and f_in is not None and f_out is not None:
+        hidden = ws.get("block.ff_hidden", (wanted.count, f_in[2]), block.dtype)
+        linear(h_few, f_in[0], f_in[1], hidden, act=f_in[3])
+        if block.dtype == torch.bfloat16 and fast.linear_pair_accumulate(mixed, m_out[0], m_out[1], hidden, f_out[0], f_out[1], few):
+            return few, None
+        linear(mixed, m_out[0], m_out[1], few, accumulate=True)
+        linear(hidden, f_out[0], f_out[1], few, accumulate=True)
+        return few, None
+    if mixed is not None:
+        linear(mixed, m_out[0], m_out[1], few, accumulate=True)
+    if ff is not None:
+        ff.forward(h_few, wanted.batch, few)
+    return few, None
+
+
+def _parallel(block: "Block", x, batch, cache, normed=None, then=None, wanted=None):
     """``x + mixer(norm(x)) + ff(norm(x))``: both branches read the same normalised input (a block without a
     feed-forward has the first branch only).
 
     Reference: ``kestrel/models/moondream/text.py:222-275``.
     """
+    if wanted is not None:
+        return _parallel_wanted(block, x, batch, cache, normed, wanted)
     handed = []
     if _parallel_few_rows(block, x, batch, cache, normed, then, handed):
         return handed[0] if handed else None
@@ -147,7 +187,7 @@ def _parallel(block: "Block", x, batch, cache, normed=None, then=None):
     return None
 
 
-_parallel.hands_over = True
+_parallel.hands_over = _parallel.narrows = True
 
 
 def _sequential_few_rows(block: "Block", x, batch, cache) -> bool:
@@ -301,7 +341,28 @@ class StreamRounding:
         return None
 
 
-def _output_norms(block: "Block", x, batch, cache, normed=None, then=None):
+def _into_delta(part, delta, *operands) -> None:
+    """A part's output written into fp32 ``delta``."""
+    if callable(getattr(part, "mix", None)):
+        part.mix(*operands, delta, False)
+    else:
+        delta.zero_()
+        part.forward(*operands, delta)
+
+
+def _mix_wanted(block: "Block", h, x, batch, cache, delta, wanted):
+    """``(x, delta)`` of the wanted tokens: their rows of the stream and the mixer's output for them. The mixer leaves what later steps read of
+    all tokens; one that offers ``mix_wanted`` does only that for the others."""
+    few, out = wanted.buffer("x", x), wanted.buffer("delta", delta)
+    if callable(getattr(block.mixer, "mix_wanted", None)):
+        block.mixer.mix_wanted(h, batch, cache, out, wanted, (x, few))
+    else:
+        _into_delta(block.mixer, delta, h, batch, cache)
+        wanted.gather((x, few), (delta, out))
+    return few, out
+
+
+def _output_norms(block: "Block", x, batch, cache, normed=None, then=None, wanted=None):
     """``x += norm(mixer(x)); x += norm2(ff(x))``: the parts read the stream itself (rounded to the activation type, or,
     for a mixer that says ``reads_stream``, as it is) and the norms stand behind them. Each part writes its output into
     an fp32 buffer (``mix``; a part without it adds into a cleared buffer through ``forward``); one launch normalises it, adds it
@@ -309,14 +370,33 @@ def _output_norms(block: "Block", x, batch, cache, normed=None, then=None):
     that offers ``mix_normed`` takes that launch's work into its own last one."""
     from ..ops import core
 
-    ws = batch.workspace
+    mixer, ws = block.mixer, batch.workspace
+    if wanted is not None and getattr(mixer, "only_reads", False):
+        # (nobody else reads anything of a token's row here: the whole block for the wanted tokens alone)
+        few = wanted.buffer("x", x)
+        rows = (normed, wanted.buffer("h", normed)) if normed is not None else None
+        wanted.gather((x, few), *([rows] if rows else []))
+        return few, _output_norms(block, few, wanted.batch, cache, rows[1] if rows else None, then) if wanted.count else None
     delta = ws.get("block.delta", tuple(x.shape), torch.float32)
-    rounds = block.dtype != torch.float32
+    source = x
+    if block.dtype != torch.float32 and not getattr(mixer, "reads_stream", False):
+        source = normed
+        if source is None:
+            source = ws.get("block.h", tuple(x.shape), block.dtype)
+            core.cast_columns(x, source)
+    if wanted is not None:
+        x, delta = _mix_wanted(block, source, x, batch, cache, delta, wanted)
+        return x, _output_norms_behind(block, x, wanted.batch, delta, then) if wanted.count else None
+    _into_delta(mixer, delta, source, batch, cache)
+    return _output_norms_behind(block, x, batch, delta, then)
 
-    def rounded(name: str):
-        h = ws.get(name, tuple(x.shape), block.dtype)
-        core.cast_columns(x, h)
-        return h
+
+def _output_norms_behind(block: "Block", x, batch, delta, then):
+    """What ``_output_norms`` does behind the mixer, whose output is ``delta``."""
+    from ..ops import core
+
+    ws = batch.workspace
+    rounds = block.dtype != torch.float32
 
     def add(norm, rows) -> bool:
         """``x += norm(delta)``, the stream's rounding into ``rows`` (``None``: not wanted); returns whether ``rows`` was written."""
@@ -332,15 +412,6 @@ def _output_norms(block: "Block", x, batch, cache, normed=None, then=None):
             core.add_scaled(x, summed, 1.0)
         return False
 
-    mixer = block.mixer
-    source = x
-    if rounds and not getattr(mixer, "reads_stream", False):
-        source = normed if normed is not None else rounded("block.h")
-    if callable(getattr(mixer, "mix", None)):
-        mixer.mix(source, batch, cache, delta, False)
-    else:
-        delta.zero_()
-        mixer.forward(source, batch, cache, delta)
     handed = ws.get("block.handed", tuple(x.shape), block.dtype) if rounds and isinstance(then, StreamRounding) and then.wanted else None
     ff = block.feed_forward
     if ff is None:
@@ -354,15 +425,11 @@ def _output_norms(block: "Block", x, batch, cache, normed=None, then=None):
     if callable(getattr(ff, "mix_normed", None)) and second is not None:
         ff.mix_normed(h, batch, x, second, None, handed)
         return handed
-    if callable(getattr(ff, "mix", None)):
-        ff.mix(h, batch, delta, False)
-    else:
-        delta.zero_()
-        ff.forward(h, batch, delta)
+    _into_delta(ff, delta, h, batch)
     return handed if add(block.norm2, handed) else None
 
 
-_output_norms.hands_over = True
+_output_norms.hands_over = _output_norms.narrows = True
 
 
 def _add_normed(norm, delta, x, then, rows, ws) -> bool:
@@ -384,29 +451,29 @@ def _add_normed(norm, delta, x, then, rows, ws) -> bool:
     return second is not None
 
 
-def _norms_around(block: "Block", x, batch, cache, normed=None, then=None):
+def _norms_around(block: "Block", x, batch, cache, normed=None, then=None, wanted=None):
     """``x += norm_after(mixer(norm(x))); x += norm2_after(ff(norm2(x)))``: a norm before and behind each sublayer.
 
     A sublayer writes its output into an fp32 buffer (``mix``); one launch then normalises it, adds it into the stream
     and computes the norm that the next reader of the stream begins with: ``norm2`` behind the mixer, and behind the
     feed-forward the first norm of the block that follows (``then``), whose rows are handed over. A feed-forward that
     offers ``mix_normed`` takes that launch's work into its own last one."""
-    ws = batch.workspace
-    ff = block.feed_forward
-    delta = ws.get("block.delta", tuple(x.shape), torch.float32)
+    delta = batch.workspace.get("block.delta", tuple(x.shape), torch.float32)
     h = normed
     if h is None:
-        h = ws.get("block.h", tuple(x.shape), block.dtype)
+        h = batch.workspace.get("block.h", tuple(x.shape), block.dtype)
         block.norm.forward(x, h)
+    if wanted is not None:
+        x, delta = _mix_wanted(block, h, x, batch, cache, delta, wanted)
+        return x, _norms_around_behind(block, x, wanted.batch, delta, then) if wanted.count else None
+    _into_delta(block.mixer, delta, h, batch, cache)
+    return _norms_around_behind(block, x, batch, delta, then)
 
-    def into_delta(part, *operands):
-        if callable(getattr(part, "mix", None)):
-            part.mix(*operands, delta, False)
-        else:
-            delta.zero_()
-            part.forward(*operands, delta)
 
-    into_delta(block.mixer, h, batch, cache)
+def _norms_around_behind(block: "Block", x, batch, delta, then):
+    """What ``_norms_around`` does behind the mixer, whose output is ``delta``."""
+    ws = batch.workspace
+    ff = block.feed_forward
     handed = ws.get("block.handed", tuple(x.shape), block.dtype)
     if ff is None:
         return handed if _add_normed(block.norm_after, delta, x, then, handed, ws) else None
@@ -419,14 +486,14 @@ def _norms_around(block: "Block", x, batch, cache, normed=None, then=None):
         if first is not None:
             ff.mix_normed(h, batch, x, first, second, handed if second is not None else None)
             return handed if second is not None else None
-    into_delta(ff, h, batch)
+    _into_delta(ff, delta, h, batch)
     return handed if _add_normed(block.norm2_after, delta, x, then, handed, ws) else None
 
 
-_norms_around.hands_over = True
+_norms_around.hands_over = _norms_around.narrows = True
 
 
-def _streams(block: "Block", x, batch, cache, normed=None, then=None):
+def _streams(block: "Block", x, batch, cache, normed=None, then=None, wanted=None):
     """The stream as several copies ``x`` ``[n, S, dim]`` (hyper-connections): ``u = sum_s in[s] x_s``, ``y = mixer(norm(u))``,
     ``x_t <- sum_s mix[s, t] x_s + out[t] y``, then the same with the feed-forward and its own numbers and norm.
 
@@ -435,23 +502,26 @@ def _streams(block: "Block", x, batch, cache, normed=None, then=None):
     ``mix_streams`` takes that launch's work into its own last one, and one with ``choose_streams`` its choice into the one in front of it."""
     from ..ops import core
 
+    n, _count, dim = x.shape
+    delta = batch.workspace.get("block.delta", (n, dim), torch.float32)
+    h = normed
+    if h is None:
+        h = batch.workspace.get("block.h", (n, dim), block.dtype)
+        core.streams_step(x, reading=block.reader.operands(), h=h)
+    if wanted is not None:
+        x, delta = _mix_wanted(block, h, x, batch, cache, delta, wanted)
+        return x, _streams_behind(block, x, wanted.batch, delta, then) if wanted.count else None
+    _into_delta(block.mixer, delta, h, batch, cache)
+    return _streams_behind(block, x, batch, delta, then)
+
+
+def _streams_behind(block: "Block", x, batch, delta, then):
+    """What ``_streams`` does behind the mixer, whose output is ``delta``."""
+    from ..ops import core
+
     ws = batch.workspace
     n, _count, dim = x.shape
     ff = block.feed_forward
-    delta = ws.get("block.delta", (n, dim), torch.float32)
-    h = normed
-    if h is None:
-        h = ws.get("block.h", (n, dim), block.dtype)
-        core.streams_step(x, reading=block.reader.operands(), h=h)
-
-    def into_delta(part, *operands):
-        if callable(getattr(part, "mix", None)):
-            part.mix(*operands, delta, False)
-        else:
-            delta.zero_()
-            part.forward(*operands, delta)
-
-    into_delta(block.mixer, h, batch, cache)
     last = then.operands() if then is not None else None
     handed = ws.get("block.handed", (n, dim), block.dtype) if then is not None else None
     if ff is None:
@@ -465,12 +535,12 @@ def _streams(block: "Block", x, batch, cache, normed=None, then=None):
     if callable(getattr(ff, "mix_streams", None)):
         ff.mix_streams(h2, batch, x, block.streams2, last, handed, **({"chosen": True} if chosen else {}))
         return handed
-    into_delta(ff, h2, batch)
+    _into_delta(ff, delta, h2, batch)
     core.streams_step(x, delta, block.streams2.matrix, block.streams2.out, last, handed)
     return handed
 
 
-_streams.hands_over = True
+_streams.hands_over = _streams.narrows = True
 
 
 ARRANGEMENTS: Dict[str, Callable] = {"parallel": _parallel, "sequential": _sequential,
@@ -483,7 +553,8 @@ def register_arrangement(name: str, fn: Callable) -> None:
     attribute ``hands_over = True`` is called as ``fn(block, x, batch, cache, normed=, then=)``:
     ``normed`` is ``block.norm`` of ``x`` if the block before has computed it (else ``None``), ``then``
     the first norm of the block that follows (or ``None``); it may return that norm of its result, or
-    ``None``."""
+    ``None``. One with ``narrows = True`` besides is given ``wanted=`` (a ``WantedTokens``) where only those tokens' rows are read
+    behind it, and returns ``(their rows of the stream, that norm of them or None)`` then."""
     ARRANGEMENTS[name] = fn
 
 
@@ -570,3 +641,15 @@ class Block:
             return self._run(self, x, batch, cache, normed=normed, then=then)
         self._run(self, x, batch, cache)
         return None
+
+    @property
+    def narrows(self) -> bool:
+        """Whether ``forward_wanted`` can be called."""
+        return bool(getattr(self._run, "narrows", False))
+
+    def forward_wanted(self, x: torch.Tensor, batch, cache: LayerCache, wanted, normed: Optional[torch.Tensor] = None,
+                       then: Optional[Part] = None):
+        """``forward`` where nobody reads the stream behind this block but for the tokens of ``wanted``: ``(their rows of the stream, that norm
+        of them or None)``. What the block keeps for later steps it keeps of all tokens."""
+        settle(x, batch)
+        return self._run(self, x, batch, cache, normed=normed, then=then, wanted=wanted)

@@ -148,6 +148,34 @@ class Branches(Mixer):
             out.zero_()                  # (a fill kernel)
         self.forward(h, batch, cache, out)
 
+    def mix_wanted(self, h, batch, cache: LayerCache, out, wanted, *also) -> None:
+        """``mix`` for the tokens of ``wanted``, in their order: branches that run as one and offer ``attend_wanted`` read for those alone."""
+        ws, n = batch.workspace, h.shape[0]
+        if self.in_weight is None:
+            delta = ws.get("block.delta", (n, self.spec.dim), torch.float32)
+            self.mix(h, batch, cache, delta, False)
+            wanted.gather((delta, out), *also)
+            return
+        projected = ws.get("branches.in", (n, self.in_cols[-1]), self.dtype)
+        linear(h, self.in_weight, None, projected)
+        heads = ws.get("branches.heads", (n, self.out_cols[-1]), self.dtype)
+        few = ws.get("wanted.heads", (wanted.count, self.out_cols[-1]), self.dtype)
+        # (those that read for all tokens first: what they leave is picked out by the launch that picks the others' queries)
+        late = []
+        for i in sorted(range(len(self.branches)), key=lambda i: callable(getattr(self.branches[i], "attend_wanted", None))):
+            branch, columns = self.branches[i], slice(self.out_cols[i], self.out_cols[i + 1])
+            operands = (projected[:, self.in_cols[i]:self.in_cols[i + 1]], batch, self._cache_of(i, cache))
+            if callable(getattr(branch, "attend_wanted", None)):
+                branch.attend_wanted(*operands, wanted, *also, *late, out=few[:, columns])
+                also, late = (), []
+            else:
+                branch.attend(*operands, out=heads[:, columns])
+                late.append((heads[:, columns], few[:, columns]))
+        if also or late:
+            wanted.gather(*also, *late)
+        if wanted.count:
+            linear(few, self.proj_weight, None, out)
+
     def forward(self, h, batch, cache: LayerCache, residual) -> None:
         if self.in_weight is not None:
             self.mix(h, batch, cache, residual, True)
