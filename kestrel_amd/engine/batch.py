@@ -105,13 +105,14 @@ class WantedTokens:
     ``batch`` lists them as single tokens, in the order of the logits, that read their requests' caches and write nothing. Its columns, and whatever a
     part hands over on the way, are picked out of the step by ``gather``, the columns by its first call."""
 
-    # Most wanted tokens, and tokens of the step to each of them: attention over single tokens reads a request's keys once for each of them.
-    MOST, SHARE = 64, 2
+    # Most wanted tokens, and tokens of the step to each of them: attention over single tokens reads a request's keys once for each of them. And the fewest
+    # tokens of a step: up to 16 a layer is three launches that wait for its weights, whichever rows they are for.
+    MOST, SHARE, TOKENS = 64, 2, 17
 
     @classmethod
     def pays(cls, batch: "StepBatch") -> bool:
         wanted = int(batch.logit_rows.numel())
-        return not batch.decode_only and wanted <= cls.MOST and wanted * cls.SHARE <= batch.n_tokens
+        return not batch.decode_only and batch.n_tokens >= cls.TOKENS and wanted <= cls.MOST and wanted * cls.SHARE <= batch.n_tokens
 
     def __init__(self, batch: "StepBatch") -> None:
         self.rows = batch.logit_rows
