@@ -5,7 +5,7 @@
 //    order; the fallback of the bf16 path;
 // and, of aligned fp32 operands, the true 32-bit path,
 //  * up to 16 rows of a linear without a gate: a stream of weights (gemv_f32_kernel);
-//  * else K in steps of 32: the matrix pipes (gemm_f32_mfma_kernel);
+//  * else K in steps of 32: the matrix pipes, every number as three of bf16 (gemm_f32_split_kernel);
 //  * else wider FMA tiles, k in ascending order as the first (gemm_f32_kernel).
 // So a row's result does not depend on what else is in the batch, but for the step from 16 to 17 rows without a gate.
 #include "ka_common.h"
@@ -73,129 +73,200 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
     }
 }
 
-// Many rows in fp32 where K is a multiple of 32: true fp32 products and sums on the matrix pipes (v_mfma_f32_32x32x2_f32, twice
-// the rate of the vector unit without packed FMAs), operands straight from memory into swizzled LDS as in ka_dma_tiles.h (a
-// K-step of 32 numbers is the same 128 bytes a row, of 16 the same 64), two stages of STEP numbers.
+// Many rows in fp32 where K is a multiple of 32: products on the bf16 matrix pipes, which have sixteen times the rate of the fp32 ones. A number of 32 bits is
+// the sum of three bf16 numbers to its last bit (24 bits of mantissa, eight in each: what rounding to the nearest leaves is representable, so
+// both subtractions are exact), and w x = w1 x1 + (w1 x2 + w2 x1) + (w2 x2 + w1 x3 + w3 x1) + what is below 2^-25 of it: six products, each exact in the
+// pipe, summed in fp32.
 //
-// The order of a sum is fixed by K alone. Every sixteen k are summed from zero (of every eight in the order 0 4 1 5 2 6 3 7: a lane
-// holds four neighbours), these sums are added in order within a part, K being cut into F32_PARTS parts, and the parts' sums
-// are added in their order. The short chains cost 5 to 8 % (an addition on the vector unit per eight products) and take the
-// error of a sum from that of a chain of K / 4 terms to that of one of K / 64.
-// A part may be anybody's: KG = 1, the waves walk over the parts one after the other; KG = 4, a workgroup has four times the waves,
-// each quarter multiplies its own part and the sums meet in LDS. The second fills the chip where tiles are few (a prompt of some
-// hundred rows), and its bits are those of the first.
+// Operands go straight from memory into swizzled LDS as in ka_dma_tiles.h, two steps of 16 numbers at a time (whole lines), and are split by the wave that
+// multiplies them: 44 instructions per eight numbers a lane, laid between the products of the step before, which the compiler does only where each step is a
+// region of its own with an end that names the parts (157 rows of 2,048 x 8,192 by tiles of 64 x 64: 96 us without, 83 with). At one wave a SIMD an instruction
+// takes five cycles, so a step of 64 x 64 x 16 (24 products, some 225 other instructions) takes 1,400 where its products are 768: that is what bounds it. The
+// activations' parts by a launch of their own, in front, were no faster: 10 KB a step instead of 8.
 //
-// Measured, us, in the vector unit's kernel below -> here: 303 rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x 8,192 and 8,192 x
-// 2,048 254, 262, 276 and 1,006 -> 95, 43, 138 and 152; 2,048 rows 813, 267, 1,017 and 1,041 -> 484, 164, 666 and 649 (107 TFLOP/s of
-// the 157 that the pipes have). Error against 64 bits of such sums: 8.1e-7 -> 1.4e-7 (K = 8,192: 1.6e-6 -> 2.2e-7).
+// The order of a sum is fixed by K alone. K is cut into F32_PARTS parts, each summed by a wave of its own (so no wave waits for another before the
+// end): w1 x1 of 128 of K from zero, these sums in order, the five smaller products, whose roundings weigh 2^-8, in an accumulator beside them; the
+// parts' sums meet in LDS and are added in their order. All tiles give the same bits.
+//
+// What three bf16 numbers cannot say (infinities, numbers beyond bf16's largest) leaves an infinity or NaN in the sum: such an output is summed again by
+// plain FMA from memory. (Numbers below 2^-109 lose what is below 2^-133 of them.)
+//
+// Measured, us, fp32 products on the matrix pipes (v_mfma_f32_32x32x2_f32) -> here, 64 rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x
+// 8,192 and 8,192 x 2,048 28.6, 16.4, 27.8 and 52.2 -> 25.0, 15.8, 27.4 and 47.3; 282 rows 85, 38, 105 and 131 -> 66, 30, 90 and 92; 2,048 rows 446, 162, 591 and 611
+// -> 385, 134, 511 and 432. Error against 64 bits of such sums 1.35e-7 -> 8.7e-8, of K = 8,192 2.2e-7 -> 1.1e-7.
 constexpr int F32_PARTS = 4;
 constexpr int F32_STEP = 32;
+constexpr int F32_BLOCK = 8;       // steps of 16 that are summed from zero
 
-template <int WN, int WM, int GN, int GM, int KG, int STEP>
-__global__ void __launch_bounds__(KA_WAVE * GN * GM * KG)
-gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
-                     float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
-    static_assert(KG == 1 || KG == F32_PARTS, "the parts one after the other, or one a group of waves");
-    constexpr int WAVES = GN * GM, BN = 32 * WN * GN, BM = 32 * WM * GM;
+typedef __attribute__((ext_vector_type(2))) float gs_float2;
+typedef __attribute__((ext_vector_type(2))) __bf16 gs_bf16x2;
+
+// part[0] + part[1] + part[2] is the eight numbers of lo and hi to the last bit
+__device__ __forceinline__ void gs_split(const floatx4& lo, const floatx4& hi, bf16x8 (&part)[3]) {
+    uint4 out[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = i < 2 ? lo[2 * i] : hi[2 * i - 4], b = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector(gs_float2{a, b}, gs_bf16x2));
+            (i == 0 ? out[p].x : i == 1 ? out[p].y : i == 2 ? out[p].z : out[p].w) = pair;
+            if (p == 2) break;
+            a -= __uint_as_float(pair << 16);
+            b -= __uint_as_float(pair & 0xffff0000u);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) part[p] = __builtin_bit_cast(bf16x8, out[p]);
+}
+
+template <int WN, int WM, int NS>
+__global__ void __launch_bounds__(KA_WAVE * F32_PARTS, WN * WM > 1 ? 1 : 2)
+gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
+                      float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
+    constexpr int BN = 32 * WN, BM = 32 * WM, STEP = 16;
     constexpr int ROW = STEP * 4, CPR = ROW / 16, RPL = KA_WAVE / CPR, STAGE = (BN + BM) * ROW;
-    constexpr int W_LOADS = BN / RPL / WAVES, X_LOADS = BM / RPL / WAVES;
-    static_assert(W_LOADS * RPL * WAVES == BN && X_LOADS * RPL * WAVES == BM, "the tile does not divide over the waves' loads");
+    constexpr int W_LOADS = BN / RPL, X_LOADS = BM / RPL, LPW = W_LOADS + X_LOADS;
     extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
     const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8;
     const int logical = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
     if (logical >= total || (int)blockIdx.x / 8 >= per_xcd) return;
     const int n0 = logical / tiles_m * BN, m0 = logical % tiles_m * BM;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
-    const int group = wave / WAVES, part_wave = wave % WAVES;
-    const int wn = part_wave / GM, wm = part_wave % GM, li = lane % 32, lg = lane / 32;
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
+    const int li = lane % 32, lg = lane / 32;
     const float* wsrc[W_LOADS];
     const float* xsrc[X_LOADS];
+    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP * (F32_STEP / STEP), k_steps = K / STEP;
+    const int first = part * part_steps, steps = max(0, min(part_steps, k_steps - first));
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(part_wave * W_LOADS + i, lane);
-        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + kd_load_channel<CPR>(r, lane) / 2;      // (four numbers a piece)
+        const int r = kd_load_row<CPR>(i, lane);
+        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + kd_load_channel<CPR>(r, lane) / 2 + first * STEP;      // (four numbers a piece)
     }
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(part_wave * X_LOADS + i, lane);
-        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2;
+        const int r = kd_load_row<CPR>(i, lane);
+        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2 + first * STEP;
     }
-    unsigned char* mine = gf_lds + group * 2 * STAGE;
-    auto fetch = [&](int stage, int k) {
-        unsigned char* base = mine + stage * STAGE;
+    unsigned char* mine = gf_lds + part * NS * STAGE;
+    auto fetch = [&](int step) {
+        unsigned char* base = mine + step % NS * STAGE;
 #pragma unroll
         for (int i = 0; i < W_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + k), (GD_LDS void*)(base + (part_wave * W_LOADS + i) * RPL * ROW), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + step * STEP), (GD_LDS void*)(base + i * RPL * ROW), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < X_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + k), (GD_LDS void*)(base + BN * ROW + (part_wave * X_LOADS + i) * RPL * ROW), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + step * STEP), (GD_LDS void*)(base + BN * ROW + i * RPL * ROW), 16, 0, 0);
     };
     const int swz = kd_swizzle<CPR>(li);
-    floatx16 acc[WN][WM], sum[WN][WM];
-    auto clear = [](floatx16 (&x)[WN][WM]) {
+    floatx16 acc[WN][WM], few[WN][WM], low[WN][WM];
 #pragma unroll
-        for (int a = 0; a < WN; ++a)
+    for (int a = 0; a < WN; ++a)
 #pragma unroll
-            for (int b = 0; b < WM; ++b)
+        for (int b = 0; b < WM; ++b)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) x[a][b][v] = 0.f;
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = few[a][b][v] = low[a][b][v] = 0.f;
+    bf16x8 op[2][WN + WM][3];
+    // the operands of a step from LDS, split (the step's loads have landed; a wave reads what it asked for itself: no barrier)
+    auto operands = [&](auto slot_c, int step) {
+        constexpr int slot = decltype(slot_c)::value;
+        const unsigned char* base = mine + step % NS * STAGE;
+        floatx4 raw[WN + WM][2];
+#pragma unroll
+        for (int r = 0; r < WN + WM; ++r)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) raw[r][h] = *reinterpret_cast<const floatx4*>(base + (r * 32 + li) * ROW + ((h * 2 + lg) ^ swz) * 16);
+#pragma unroll
+        for (int r = 0; r < WN + WM; ++r) gs_split(raw[r][0], raw[r][1], op[slot][r]);
     };
-    clear(acc);
-    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP * (F32_STEP / STEP), k_steps = K / STEP;
-    // this wave's steps: all of K, or its group's part
-    const int first = KG == 1 ? 0 : group * part_steps;
-    const int steps = max(0, min(KG == 1 ? k_steps : part_steps, k_steps - first));
-    const int rounds = KG == 1 ? k_steps : min(part_steps, k_steps);           // (the same for every wave: barriers)
-    if (steps > 0) fetch(0, first * STEP);
-    int done = 0;                                                              // KG == 1: parts added into `sum`
-    for (int s = 0; s < rounds; ++s) {
-        gd_wait_loads<0>();                                                    // own loads of this step have landed
-        gd_wait_lds();                                                         // own reads of the step before are in registers
-        if constexpr (WAVES > 1) gd_barrier();                                 // (a wave that has its part of K to itself reads what it asked for)
-        if (s + 1 < steps) fetch((s + 1) & 1, (first + s + 1) * STEP);
-        if (s < steps) {
-            const unsigned char* base = mine + (s & 1) * STAGE;
-#pragma unroll
-            for (int g = 0; g < STEP / 16; ++g) {
-                floatx4 w[2][WN], x[2][WM];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int place = (((g * 2 + h) * 2 + lg) ^ swz) * 16;
-#pragma unroll
-                    for (int a = 0; a < WN; ++a) w[h][a] = *reinterpret_cast<const floatx4*>(base + ((wn * WN + a) * 32 + li) * ROW + place);
-#pragma unroll
-                    for (int b = 0; b < WM; ++b) x[h][b] = *reinterpret_cast<const floatx4*>(base + (BN + (wm * WM + b) * 32 + li) * ROW + place);
-                }
-#pragma unroll
-                for (int a = 0; a < WN; ++a)
-#pragma unroll
-                    for (int b = 0; b < WM; ++b) {
-                        floatx16 few = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) few = __builtin_amdgcn_mfma_f32_32x32x2f32(w[j / 4][a][j % 4], x[j / 4][b][j % 4], few, 0, 0, 0);
-                        acc[a][b] += few;
-                    }
+    // Step s, the place-th of four: its products, and between them the split of the next one's operands, which the matrix pipe does not need.
+    // STEADY: a step that has NS behind it.
+    auto step = [&](auto place_c, auto steady_c, int s) {
+        constexpr int place = decltype(place_c)::value, slot = place & 1;
+        constexpr bool STEADY = decltype(steady_c)::value;
+        if constexpr (slot == 1) {                                             // the last step of a pair
+            if constexpr (STEADY) gd_wait_loads<2 * LPW * (NS / 2 - 2)>();
+            else if (s + 1 < steps) gd_wait_younger<2 * LPW, NS / 2 - 2>(min(NS / 2 - 2, (steps - 1 - s) / 2 - 1));
+            gd_wait_lds();                                                     // own reads of the pair are in registers: its stages may be written
+            if (STEADY || s + NS < steps) {
+                fetch(s + NS - 1);
+                fetch(s + NS);
             }
         }
-        if (KG == 1 && (s + 1) % part_steps == 0 && s + 1 < rounds) {          // a part ends
+        operands(std::integral_constant<int, slot ^ 1>{}, s + 1);              // (behind the last step: memory that nobody uses)
+        auto add = [&](floatx16 (&sum)[WN][WM], int i, int j) {
 #pragma unroll
             for (int a = 0; a < WN; ++a)
 #pragma unroll
-                for (int b = 0; b < WM; ++b)
+                for (int b = 0; b < WM; ++b) sum[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[slot][a][i], op[slot][WN + b][j], sum[a][b], 0, 0, 0);
+        };
+        add(low, 0, 2);
+        add(low, 2, 0);
+        add(few, 0, 0);
+        add(low, 1, 1);
+        add(low, 0, 1);
+        add(low, 1, 0);
+        constexpr int PRODUCTS = 6 * WN * WM, EACH = (44 * (WN + WM) + PRODUCTS - 1) / PRODUCTS;
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * (WN + WM), 0);
+        gd_static_for<0, PRODUCTS>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, EACH, 0);
+        });
+        // (the split belongs here: the compiler would put it off to the step that uses it, in front of that step's products)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) sum[a][b][v] = done ? sum[a][b][v] + acc[a][b][v] : acc[a][b][v];
-            clear(acc);
-            ++done;
+        for (int r = 0; r < WN + WM; ++r)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(op[slot ^ 1][r][i]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto settle = [&] {
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b) {
+                acc[a][b] += few[a][b];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) few[a][b][v] = 0.f;
+            }
+    };
+    if (steps > 0) {
+#pragma unroll
+        for (int st = 0; st < NS; ++st)
+            if (st < steps) fetch(st);
+        gd_wait_younger<2 * LPW, NS / 2 - 1>(min(NS / 2, steps / 2) - 1);
+        operands(std::integral_constant<int, 0>{}, 0);
+        int s = 0;
+        auto block = [&](auto steady_c) {
+            step(std::integral_constant<int, 0>{}, steady_c, s);
+            step(std::integral_constant<int, 1>{}, steady_c, s + 1);
+            step(std::integral_constant<int, 2>{}, steady_c, s + 2);
+            step(std::integral_constant<int, 3>{}, steady_c, s + 3);
+            s += 4;
+            if (s % F32_BLOCK == 0) settle();
+        };
+        while (s + 3 + NS < steps) block(std::true_type{});
+        while (s + 3 < steps) block(std::false_type{});
+        if (s < steps) {                                                       // (an even number of steps)
+            step(std::integral_constant<int, 0>{}, std::false_type{}, s);
+            step(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
         }
+        settle();
     }
-    // acc[a][b][v] is out[m][n] with n = n0 + (wn WN + a) 32 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + (wm WM + b) 32 + li
+    // acc[a][b][v] is out[m][n] with n = n0 + a 32 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + b 32 + li
     const bool vectors = N % 4 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    auto store = [&](int a, int b, int q, const float (&y)[4]) {
-        const int m = m0 + (wm * WM + b) * 32 + li, n = n0 + (wn * WN + a) * 32 + q * 8 + lg * 4;
+    auto store = [&](int a, int b, int q, const floatx4& y) {
+        const int m = m0 + b * 32 + li, n = n0 + a * 32 + q * 8 + lg * 4;
         if (m >= M || n >= N) return;
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = y[j] + (bias && n + j < N ? bias[n + j] : 0.f);
+        for (int j = 0; j < 4; ++j) {
+            v[j] = y[j];
+            if (!(fabsf(v[j]) < INFINITY) && n + j < N) {                      // (see above)
+                v[j] = 0.f;
+                for (int k = 0; k < K; ++k) v[j] = fmaf(A[(size_t)m * lda + k], W[(size_t)(n + j) * ldw + k], v[j]);
+            }
+            v[j] += bias && n + j < N ? bias[n + j] : 0.f;
+        }
         if (ka_act_gated(act)) {
             ka_gated_store<false, 4>(out, KA_F32, ldo, m, n, N, v, act);
             return;
@@ -212,45 +283,35 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, long lda, const float* __restr
             for (int j = 0; j < 4 && n + j < N; ++j) op[j] = accumulate ? op[j] + v[j] : v[j];
         }
     };
-    if constexpr (KG == 1) {
-        gd_static_for<0, WN * WM * 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
-            float y[4];
+    // the parts' sums through LDS; every wave finishes a quarter of the tile's numbers
+    gd_wait_lds();
+    gd_barrier();
+    floatx4* sums = reinterpret_cast<floatx4*>(gf_lds);
+    gd_static_for<0, WN * WM * 4>([&](auto ic) {
+        constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
+        floatx4 y;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) y[j] = done ? sum[a][b][q * 4 + j] + acc[a][b][q * 4 + j] : acc[a][b][q * 4 + j];
-            store(a, b, q, y);
-        });
-    } else {
-        // the parts' sums through LDS; every group of waves finishes a quarter of the tile's numbers
-        gd_wait_lds();
-        gd_barrier();
-        float* sums = reinterpret_cast<float*>(gf_lds);
-        gd_static_for<0, WN * WM * 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
-            *reinterpret_cast<floatx4*>(sums + (((group * WAVES + part_wave) * WN * WM * 4 + i) * KA_WAVE + lane) * 4) =
-                floatx4{acc[a][b][q * 4], acc[a][b][q * 4 + 1], acc[a][b][q * 4 + 2], acc[a][b][q * 4 + 3]};
-        });
-        gd_wait_lds();
-        gd_barrier();
-        const int parts = (k_steps + part_steps - 1) / part_steps;             // (those that hold anything)
-        gd_static_for<0, WN * WM>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            const int at = i * 4 + group;
-            floatx4 y = *reinterpret_cast<const floatx4*>(sums + ((part_wave * WN * WM * 4 + at) * KA_WAVE + lane) * 4);
-            for (int p = 1; p < parts; ++p) y += *reinterpret_cast<const floatx4*>(sums + (((p * WAVES + part_wave) * WN * WM * 4 + at) * KA_WAVE + lane) * 4);
-            const float v[4] = {y[0], y[1], y[2], y[3]};
-            store(i / WM, i % WM, group, v);
-        });
+        for (int j = 0; j < 4; ++j) y[j] = acc[a][b][q * 4 + j] + low[a][b][q * 4 + j];
+        sums[(part * WN * WM * 4 + i) * KA_WAVE + lane] = y;
+    });
+    gd_wait_lds();
+    gd_barrier();
+    const int parts = (k_steps + part_steps - 1) / part_steps;                 // (those that hold anything)
+    for (int i = 0; i < WN * WM; ++i) {
+        const int at = i * 4 + part;
+        floatx4 y = sums[at * KA_WAVE + lane];
+        for (int p = 1; p < parts; ++p) y += sums[(p * WN * WM * 4 + at) * KA_WAVE + lane];
+        store(i / WM, i % WM, part, y);
     }
 }
 
-template <int WN, int WM, int GN, int GM, int KG, int STEP>
-static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
-                           int act, int accumulate, hipStream_t stream) {
-    constexpr int BN = 32 * WN * GN, BM = 32 * WM * GM, smem = KG * 2 * (BN + BM) * STEP * 4;
-    static_assert(KG == 1 || smem >= KG * GN * GM * WN * WM * 4 * KA_WAVE * 16, "the parts' sums fit");
+template <int WN, int WM, int NS>
+static int launch_f32_split(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+                            int act, int accumulate, hipStream_t stream) {
+    constexpr int BN = 32 * WN, BM = 32 * WM, smem = F32_PARTS * NS * (BN + BM) * 64;
+    static_assert(smem >= F32_PARTS * WN * WM * 4 * KA_WAVE * 16, "the parts' sums fit");
     static bool configured = false;
-    auto kernel = gemm_f32_mfma_kernel<WN, WM, GN, GM, KG, STEP>;
+    auto kernel = gemm_f32_split_kernel<WN, WM, NS>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         KA_CHECK(e == hipSuccess, "ka_linear_generic: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
@@ -259,45 +320,30 @@ static int launch_f32_mfma(const float* A, long lda, const float* W, long ldw, c
     const int tiles_n = ka_cdiv(N, BN), tiles_m = ka_cdiv(M, BM);
     const long blocks = ((long)tiles_n * tiles_m + 7) / 8 * 8;
     KA_CHECK(blocks < (1L << 31), "ka_linear_generic: too many tiles");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * GN * GM * KG), smem, stream, A, lda, W, ldw, bias, out, ldo, M, N, K, act,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * F32_PARTS), smem, stream, A, lda, W, ldw, bias, out, ldo, M, N, K, act,
                        accumulate, tiles_n, tiles_m);
     KA_LAUNCH_CHECK();
     return 0;
 }
 
-// The tile: the one that is done first by what was measured (us per 2,048 of K: a first part, and as much again for every round of one tile a CU). All give the
-// same bits. Fitted to every tile's times at 17 to 2,048 rows of 1,024 x 1,024, 2,048 x 2,048, 2,560 x 2,560, 6,144 x 2,048, 8,192 x 2,048, 2,048 x 8,192 and 10,240 x 2,560
-// (outputs x inputs), tiles a CU rounded up, us per 2,048 of K, average of all sizes:
-//              1     2     3     4     5     6     7     8    10    12
-//   64 x 128   98   157   231   309
-//   64 x 64    45    83   122   159   198   235   269
-//   64 x 32    28    49    70    92   112   132   153   174   216   258
-//   32 x 32    17    29    41    51    61    73    82    95   116   138
-// What it chooses is 0.2 % behind the fastest tile on the average and 3.5 % at most (1,024 x 1,024, 350 rows). By a rate for each tile alone, without the
-// first part, it was up to 20 % behind: tiles of 64 x 128 one a CU do not overlap a start with anything (2,048 x 2,048, 1,024 rows 105 us, now 90).
-// K-steps: of 32 where a workgroup has a CU to itself and where every wave waits for nobody (tiles of 32 x 32, a part of K a wave: no barrier; with one
-// a step 2,048 of 8,192 took 144 us at 304 rows, 133 without); of 16, half the LDS and so two or three workgroups a CU, where there are more tiles
-// of 64 x 32 or 64 x 64 than CUs (steps of 32 and 16, 64 x 64: 6,144 of 2,048, 304 rows 88.0 and 84.7, 450 rows 128.7 and 123.5; 64 x 32: 8,192 of 2,048,
-// 304 rows 122.7 and 112.9; one a CU: 64 x 64 of 2,048 x 8,192, 450 rows 161.5 and 163.3, 64 x 32 of 2,048 x 2,048, 64 rows 26.9 and 33.1).
-// Three and four stages of 16 were slower at every size.
+// The tile: the one that is done first by what was measured (us per 2,048 of K: a first part, and as much again for every round of one tile a CU); all give the
+// same bits. Tiles of 32 x 32 leave room for two workgroups a CU, or for eight stages instead of four where no CU has two and K is long (2,048 of 8,192, 17
+// and 96 rows: 49.2 and 48.7 us with four, 43.1 and 46.4 with eight; K of 2,048 the same). Measured, us per 2,048 of K, tiles a CU rounded up (17 to 2,048 rows
+// of 2,048 x 2,048, 6,144 x 2,048 and 8,192 x 2,048):
+//              1      2      3     4     7     8    12    16
+//   64 x 64    30     60     90   122         254   387   509
+//   64 x 32    22     38           78         161
+//   32 x 32    16     25     34    43    73    88
 static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                            int act, int accumulate, hipStream_t stream) {
     const int cus = ka_compute_units();
-    auto tiles = [&](int bn, int bm) { return (long)ka_cdiv(N, bn) * ka_cdiv(M, bm); };
-    auto us = [&](int bn, int bm, float first, float round) { return first + ka_cdiv(tiles(bn, bm), cus) * round; };
-    const float t128 = us(64, 128, 40.f, 62.f), t64 = us(64, 64, 3.5f, 39.5f), t32 = us(64, 32, 8.f, 21.f), t1 = us(32, 32, 6.f, 11.f);
-    const float best = fminf(fminf(t128, t64), fminf(t32, t1));
-#define KA_F32(...) return launch_f32_mfma<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
-    if (t128 <= best) KA_F32(1, 2, 2, 2, 1, 32);
-    if (t64 <= best) {
-        if (tiles(64, 64) > cus) KA_F32(1, 2, 2, 1, F32_PARTS, 16);
-        KA_F32(1, 2, 2, 1, F32_PARTS, 32);
-    }
-    if (t32 <= best) {
-        if (tiles(64, 32) > cus) KA_F32(1, 1, 2, 1, F32_PARTS, 16);
-        KA_F32(1, 1, 2, 1, F32_PARTS, 32);
-    }
-    KA_F32(1, 1, 1, 1, F32_PARTS, 32);
+    auto rounds = [&](int bn, int bm) { return (float)((((long)ka_cdiv(N, bn) * ka_cdiv(M, bm)) + cus - 1) / cus); };
+    const float t64 = 30.5f * rounds(64, 64), t32 = 1.f + 20.f * rounds(64, 32), t1 = 6.f + 9.6f * rounds(32, 32);
+#define KA_F32(...) return launch_f32_split<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
+    if (t64 <= t32 && t64 <= t1) KA_F32(2, 2, 4);
+    if (t32 <= t1) KA_F32(2, 1, 4);
+    if (rounds(32, 32) <= 1.f && K >= 4096) KA_F32(1, 1, 8);
+    KA_F32(1, 1, 4);
 #undef KA_F32
 }
 

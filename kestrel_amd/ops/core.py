@@ -1208,8 +1208,8 @@ def rope_cache(qkv: torch.Tensor, positions: torch.Tensor, slots: Optional[torch
 
 def linear_generic(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                    act: int = 0, accumulate: bool = False) -> None:
-    """``out = act(a @ weight.T + bias)`` or ``out += ...``, any sizes and type mix: 32-bit operands on the
-    fp32 matrix pipes, other mixes by plain fp32 FMA."""
+    """``out = act(a @ weight.T + bias)`` or ``out += ...``, any sizes and type mix: 32-bit operands of many
+    rows on the matrix pipes (each number as three of bf16, no bit lost), other mixes by plain fp32 FMA."""
     _dev(a, weight, bias, out)
     m, k = a.shape
     n = weight.shape[0]
