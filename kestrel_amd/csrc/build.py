@@ -31,7 +31,7 @@ ARCH = "gfx950"
 LIBRARIES: Dict[str, List[str]] = {
     "core": ["ka_error.hip", "elementwise.hip", "gemm_generic.hip", "gemv_pairs_f32.hip", "attention_generic.hip", "mixer_parts.hip", "sequence_parts.hip", "recurrent_parts.hip", "linear_attention.hip", "stream_parts.hip", "experts.hip",
              "sampling.hip", "peaks.hip"],
-    "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_few_bf16.hip", "gemm_phased_bf16.hip", "gemm_quad_bf16.hip", "gemm_quad_f32_bf16.hip", "gemv_bf16.hip", "gemv_share_bf16.hip", "gemv_share_long_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
+    "fast": ["ka_error.hip", "gemm_bf16.hip", "gemm_few_bf16.hip", "gemm_phased_bf16.hip", "gemm_quad_bf16.hip", "gemm_quad_f32_bf16.hip", "gemm_quad_pair_bf16.hip", "gemv_bf16.hip", "gemv_share_bf16.hip", "gemv_share_long_bf16.hip", "attention_bf16.hip", "attention_biased_bf16.hip", "heads_linear_bf16.hip", "matrix_memory_bf16.hip", "linear_attention_bf16.hip", "decayed_chunks_bf16.hip", "latent_expand_bf16.hip", "decode_beside.hip", "experts_bf16.hip",
              "gemm_library.hip"],
 }
 

@@ -532,19 +532,22 @@ int ka_few_rows_by_tiles(const KaFewRows& f, hipStream_t stream) {
 // The tile and the parts of K for `ka_linear_pair_tiles_bf16`.
 //  * Tiles of 128 x 128: as many parts as leave the fewest K-steps to a CU, a part more than another costing the finishing kernel one more read
 //    of the output (a K-step 0.55 us, eight of them a tile's start and end, 4 TB/s for the sums; 1.08 of that is measured on the average).
-//  * The phased tiles of 256 rows where their estimate says so (pair_lead) and their workgroups are one round of the chip: a K-step takes `step` us with few workgroups
-//    and `full` more with one on every CU (the clock gives way under load), a workgroup's start and end `edge` and `edge_full` more, a million sums
-//    `sums`. Fitted to 1,151 timings of 80 to 2,048 rows, widths of 512 to 4,096, K of 2,560 to 20,480 in all: off by 5 % on the average. Not where more
-//    than four tenths of a tile's rows are none, which streams weights: five stages of a small tile do that better (2,048, K = 4,096, 300 rows: 20.6
-//    and 23.7 us).
-// Measured with the norm behind, small tiles in the parts they would come in and the phased ones chosen (us): N = 2,048, K = 10,240: 768 rows 54.0 and 47.7,
-// 1,280 rows 84.4 and 66.0; 2,560, 12,800: 385 rows 49.6 and 47.9, 448 rows 52.5 and 49.1, 1,024 rows 108 and 77; 4,096, 12,288, 640 rows 97 and 80.
+//  * The phased tiles of 256 x 256, and those of four waves (gemm_quad_pair_bf16.hip), where their estimate says so and their workgroups are one round of the
+//    chip: a K-step takes `step` us with few workgroups and `full` more with one on every CU (the clock gives way under load), a workgroup's start and
+//    end `edge` and `edge_full` more, a million sums `sums`. Fitted to timings of 65 to 2,048 rows, widths of 512 to 4,096, K of 1,536 to 20,480 in all:
+//    off by 5 % on the average. The phased tiles give way only to an estimate 5 % below theirs: from some 1,300 rows on both take the same time, and theirs
+//    is the shorter chain of sums (2,048, K = 10,240: 1,536 rows 75.3 and 74.6 us, 2,048 rows 88.6 and 90.2; 2,560, 12,800, 1,536 rows 100.8 and 105.5). Not
+//    tiles of more than 128 rows where more than four tenths of them are none.
+// Measured with the norm behind, what was chosen without the tiles of four waves and with them (us): N = 2,048, K = 10,240: 96 rows 21.3 and 19.5, 282 rows 29.3 and 27.5,
+// 512 rows 38.1 and 34.0, 743 rows 48.8 and 44.4, 1,024 rows 58.2 and 51.9; 2,560, 12,800: 256 rows 36.0 and 35.0, 384 rows 47.2 and 45.4, 512 rows 52.2 and
+// 47.6; 1,024, 5,120, 1,940 rows 37.9 and 33.9; 4,096, 14,336, 199 rows 43.5 and 40.9; 3,072, 13,312, 540 rows 67.8 and 59.0. Of 45 sizes drawn over that range
+// 28 are faster, 17 go as before.
 struct PairChoice {
-    int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased; parts 0: none fits
+    int tile, parts;        // tile 0: 128 x 128 (pair_tiles_kernel); else a tile of ka_pair_phased or ka_pair_quad; parts 0: none fits
     double us;
 };
 
-// How far ahead of the small tiles' the estimate of phased tiles that take `us` has to be (0.99: 1 % behind will do). Both sides measured at 336 sizes where the estimates meet
+// How far ahead of the small tiles' the estimate of phased tiles of 256 x 256 that take `us` has to be (those of four waves: not at all) (0.99: 1 % behind will do). Both sides measured at 336 sizes where the estimates meet
 // (512 to 4,096 wide, K of 2,560 to 20,480, their ratio 0.93 to 1.03):
 //  * Short ones are up to 20 % slower, their start and end being more than the estimate has (1,024, 5,120, 769 rows 22.4 and 26.1 us; 2,048, 4,096, 771 rows 28.6 and
 //    30.3; 1,024, 8,192, 769 rows 28.7 and 31.1).
@@ -569,20 +572,21 @@ static PairChoice pair_tiles_choice(int M, int N, int steps, long partial_floats
         if (best.parts == 0 || us < best.us) best = {0, parts, us};
     }
     static const struct { int tile, rows_w, rows_x; double step, full, edge, edge_full, sums; } tiles[] = {
-        {3, 128, 256, 0.83, 0.19, 8.4, -7.2, 1.93}, {1, 256, 256, 1.05, 0.51, 11.9, -8.6, 1.43}};
+        {1, 256, 256, 1.05, 0.51, 11.9, -8.6, 1.43}, {8, 128, 128, 0.47, 0.10, 6.0, 0.0, 1.3},  {5, 160, 128, 0.50, 0.20, 8.0, 0.0, 1.3},
+        {10, 160, 192, 0.62, 0.24, 8.0, 0.0, 1.3},   {3, 128, 256, 0.66, 0.22, 8.0, 0.0, 1.3}, {12, 160, 256, 0.74, 0.33, 8.0, 0.0, 1.3}};
     PairChoice large = {0, 0, 0.0};
     for (const auto& t : tiles) {
-        if (!phased || M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L) continue;
+        if (!phased || (t.rows_x > PT_TILE && M * 10L < ka_cdiv(M, t.rows_x) * t.rows_x * 6L)) continue;
         const long each = (long)ka_cdiv(N, t.rows_w) * ka_cdiv(M, t.rows_x);
         for (int parts = 1; parts <= 8 && each * parts <= cus && (long)parts * M * N <= partial_floats; ++parts) {
             const int per = ka_cdiv(steps, parts), last = steps - (parts - 1) * per;
-            if (per < 4 || ka_cdiv(steps, per) != parts || last < 2) continue;
+            if (per < 4 || ka_cdiv(steps, per) != parts || last < 2 || (large_only && parts == 1 && t.tile != 1)) continue;
             const double load = (double)(each * parts) / cus * (each * parts) / cus;
             const double us = per * (t.step + t.full * load) + t.edge + t.edge_full * load + parts * (double)M * N * t.sums * 1e-6;
-            if (large.parts == 0 || us < large.us) large = {t.tile, parts, us};
+            if (large.parts == 0 || us < (large.tile == 1 && t.tile != 1 ? 0.95 : 1.0) * large.us) large = {t.tile, parts, us};
         }
     }
-    if (large.parts && (best.parts == 0 || (large_only ? 1.05 : pair_lead(M, large.us)) * large.us < best.us)) {
+    if (large.parts && (best.parts == 0 || (large_only ? 1.05 : large.tile == 1 ? pair_lead(M, large.us) : 1.0) * large.us < best.us)) {
         best = large;
         best.us *= 1.05;               // (what the vendor library is compared with)
     }
@@ -593,14 +597,14 @@ static bool pair_tiles_fit(int M, int N, int K1, int K2) {
     return M >= 1 && N >= 1 && N % 4 == 0 && K1 % PT_BK == 0 && K2 % PT_BK == 0 && K1 >= PT_BK && K2 >= PT_BK;
 }
 
-// Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles, whose offsets have to fit in 32 bits.
+// Parts and tile (parts + PT_TILE_CODE * tile), 0: not covered. phased 0: without the phased tiles and those of four waves, whose offsets have to fit in 32 bits.
 KA_API int ka_linear_pair_tiles_parts(int M, int N, int K1, int K2, long partial_floats, int phased) {
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
     const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, phased, false);
     return c.parts ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
-// The same for outputs of more small tiles than a CU's worth: tiles of 256 x 256 with K in parts where they are faster than two products of the vendor
+// The same for outputs of more small tiles than a CU's worth: large tiles with K in parts where they are faster than two products of the vendor
 // library and the norm behind them (its operations at 0.85 PFLOP/s, 8 us for two launches' starts and ends, 10 bytes an output at 4 TB/s). Measured,
 // us, library and tiles: N = 2,048, K = 10,240: 1,536 rows 91.5 and 74, 2,048 rows 105.5 and 88.5; 2,560, 12,800: 1,280 rows 131 and 89.5, 2,048 rows
 // 158 and 131; 2,560, 5,120: 2,048 rows 83 and 72; 4,096, 8,192: 2,048 rows 140 and 133; in one part 4,096 rows of the last 249 against 243.
@@ -608,7 +612,7 @@ KA_API int ka_linear_pair_large_parts(int M, int N, int K1, int K2, long partial
     if (!pair_tiles_fit(M, N, K1, K2)) return 0;
     const PairChoice c = pair_tiles_choice(M, N, (K1 + K2) / PT_BK, partial_floats, true, true);
     const double library = 2.0 * M * N * (double)(K1 + K2) / 0.85e9 + 8.0 + (double)M * N * 10.0 / 4.0e6;
-    return c.tile == 1 && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
+    return c.tile && c.parts > 1 && c.us < library ? c.parts + PT_TILE_CODE * c.tile : 0;
 }
 
 KA_API int ka_linear_pair_tiles_bf16(const void* A1, long lda1, int K1, const void* A2, long lda2, int K2, const void* W1, long ldw1,

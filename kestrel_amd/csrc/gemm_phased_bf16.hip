@@ -260,16 +260,12 @@ static int launch_pair(KaPairTiles p, int parts, hipStream_t stream) {
     return 0;
 }
 
-// tile: 256 x 256 (W x A rows) 1, 128 x 256 3. Every part needs two K-steps.
+// tile: 256 x 256 (W x A rows) 1, those of ka_pair_quad. Every part needs two K-steps.
 int ka_pair_phased(const KaPairTiles& p, int tile, int parts, hipStream_t stream) {
     const int steps = p.steps[0] + p.steps[1];
     KA_CHECK(parts >= 1 && p.per >= 2 && (parts - 1) * p.per < steps && parts * p.per >= steps && steps - (parts - 1) * p.per >= 2,
              "pair of linears: %d parts of %d K-steps, %d in all", parts, p.per, steps);
     for (int s = 0; s < 2; ++s)
         KA_CHECK((p.M - 1) * p.lda[s] + p.steps[s] * 64L < (1L << 31) && (p.N - 1) * p.ldw[s] + p.steps[s] * 64L < (1L << 31), "pair of linears: an operand of 4 GB");
-    switch (tile) {
-        case 1: return launch_pair<4, 4, 2, 2, 2, 4>(p, parts, stream);
-        case 3: return launch_pair<2, 2, 2, 2, 2, 4>(p, parts, stream);
-    }
-    KA_CHECK(false, "pair of linears: unknown tile %d", tile);
+    return tile == 1 ? launch_pair<4, 4, 2, 2, 2, 4>(p, parts, stream) : ka_pair_quad(p, tile, parts, stream);
 }

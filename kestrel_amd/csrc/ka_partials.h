@@ -44,6 +44,7 @@ __device__ __forceinline__ KaPairPlace ka_pair_place(const KaPairTiles& p, int b
     return {logical / tiles, tile / p.tiles_m, tile % p.tiles_m};
 }
 int ka_pair_phased(const KaPairTiles& p, int tile, int parts, hipStream_t stream);
+int ka_pair_quad(const KaPairTiles& p, int tile, int parts, hipStream_t stream);
 
 // out = act(sum of the parts + biases) (+ out): one thread per four neighbouring outputs
 static __global__ void __launch_bounds__(256)

@@ -163,7 +163,7 @@ PAIR_TILES_MAX = 160
 PAIR_TILES_NORMED = 128
 PAIR_TILES_ALONE = (32, 80)
 PAIR_TILES_LONG = 6144
-# A code of parts and tile: parts + PAIR_TILE_CODE * tile (0: 128 x 128; 1 and 3: the phased tiles).
+# A code of parts and tile: parts + PAIR_TILE_CODE * tile (0: 128 x 128; 1: the phased tiles of 256 x 256; others: those of four waves).
 PAIR_TILE_CODE = 100
 _library_space = {}
 SCRATCH_FLOATS = 8 << 20

@@ -134,3 +134,10 @@ def test_a_replayed_graph_repeats_the_eager_bits():
         torch.cuda.synchronize()
         assert all(torch.equal(x, y) for x, y in zip(*fields))
         run(*fields[0])
+
+
+# the tiles of four waves: a part of two K-steps (less than their stages), an odd number, more than the stages, parts of one linear alone, ragged rows and columns
+@pytest.mark.parametrize("tile", [5, 8, 10, 12])
+@pytest.mark.parametrize("m, n, k1, k2, parts", [(65, 132, 64, 64, 1), (257, 260, 192, 1024, 3), (300, 516, 512, 512, 2), (513, 128, 640, 320, 7), (256, 256, 1088, 64, 2)])
+def test_two_last_linears_by_four_waves(tile, m, n, k1, k2, parts):
+    test_two_last_linears_in_parts(tile, m, n, k1, k2, parts)
