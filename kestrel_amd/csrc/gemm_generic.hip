@@ -88,6 +88,10 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 // end): w1 x1 of 128 of K from zero, these sums in order, the five smaller products, whose roundings weigh 2^-8, in an accumulator beside them; the
 // parts' sums meet in LDS and are added in their order. All tiles give the same bits.
 //
+// Weights that are bf16 numbers, as checkpoints hold them, have one part, and three of the six products are zeros: a wave begins its part with the other three, looks
+// at the lower halves of the weights as it goes, and where it meets one that is not zero begins again with all six, to the same bits (282 rows as below:
+// 51, 26, 75 and 75 us; weights that need all six pay for the first steps, 67, 31, 95 and 93).
+//
 // What three bf16 numbers cannot say (infinities, numbers beyond bf16's largest) leaves an infinity or NaN in the sum: such an output is summed again by
 // plain FMA from memory. (Numbers below 2^-109 lose what is below 2^-133 of them.)
 //
@@ -160,16 +164,21 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
     };
     const int swz = kd_swizzle<CPR>(li);
     floatx16 acc[WN][WM], few[WN][WM], low[WN][WM];
+    auto clear = [&] {
 #pragma unroll
-    for (int a = 0; a < WN; ++a)
+        for (int a = 0; a < WN; ++a)
 #pragma unroll
-        for (int b = 0; b < WM; ++b)
+            for (int b = 0; b < WM; ++b)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = few[a][b][v] = low[a][b][v] = 0.f;
+                for (int v = 0; v < 16; ++v) acc[a][b][v] = few[a][b][v] = low[a][b][v] = 0.f;
+    };
+    clear();
     bf16x8 op[2][WN + WM][3];
     // the operands of a step from LDS, split (the step's loads have landed; a wave reads what it asked for itself: no barrier)
-    auto operands = [&](auto slot_c, int step) {
+    unsigned seen = 0;                                                         // bits of the weights that were read
+    auto operands = [&](auto slot_c, auto whole_c, int step) __attribute__((always_inline)) {
         constexpr int slot = decltype(slot_c)::value;
+        constexpr bool WHOLE = decltype(whole_c)::value;
         const unsigned char* base = mine + step % NS * STAGE;
         floatx4 raw[WN + WM][2];
 #pragma unroll
@@ -177,11 +186,25 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
 #pragma unroll
             for (int h = 0; h < 2; ++h) raw[r][h] = *reinterpret_cast<const floatx4*>(base + (r * 32 + li) * ROW + ((h * 2 + lg) ^ swz) * 16);
 #pragma unroll
-        for (int r = 0; r < WN + WM; ++r) gs_split(raw[r][0], raw[r][1], op[slot][r]);
+        for (int r = 0; r < WN + WM; ++r) {
+            if (WHOLE || r >= WN) {
+                gs_split(raw[r][0], raw[r][1], op[slot][r]);
+                continue;
+            }
+            uint4 upper;
+            const uint4 lo = __builtin_bit_cast(uint4, raw[r][0]), hi = __builtin_bit_cast(uint4, raw[r][1]);
+            upper.x = __builtin_amdgcn_perm(lo.y, lo.x, 0x07060302);
+            upper.y = __builtin_amdgcn_perm(lo.w, lo.z, 0x07060302);
+            upper.z = __builtin_amdgcn_perm(hi.y, hi.x, 0x07060302);
+            upper.w = __builtin_amdgcn_perm(hi.w, hi.z, 0x07060302);
+            op[slot][r][0] = __builtin_bit_cast(bf16x8, upper);
+            seen |= lo.x | lo.y | lo.z | lo.w | hi.x | hi.y | hi.z | hi.w;
+        }
     };
     // Step s, the place-th of four: its products, and between them the split of the next one's operands, which the matrix pipe does not need.
     // STEADY: a step that has NS behind it.
-    auto step = [&](auto place_c, auto steady_c, int s) {
+    auto step = [&](auto place_c, auto steady_c, auto whole_c, int s) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole_c)::value;
         constexpr int place = decltype(place_c)::value, slot = place & 1;
         constexpr bool STEADY = decltype(steady_c)::value;
         if constexpr (slot == 1) {                                             // the last step of a pair
@@ -193,7 +216,7 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
                 fetch(s + NS);
             }
         }
-        operands(std::integral_constant<int, slot ^ 1>{}, s + 1);              // (behind the last step: memory that nobody uses)
+        operands(std::integral_constant<int, slot ^ 1>{}, whole_c, s + 1);              // (behind the last step: memory that nobody uses)
         auto add = [&](floatx16 (&sum)[WN][WM], int i, int j) {
 #pragma unroll
             for (int a = 0; a < WN; ++a)
@@ -201,12 +224,12 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
                 for (int b = 0; b < WM; ++b) sum[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[slot][a][i], op[slot][WN + b][j], sum[a][b], 0, 0, 0);
         };
         add(low, 0, 2);
-        add(low, 2, 0);
+        if constexpr (WHOLE) add(low, 2, 0);
         add(few, 0, 0);
-        add(low, 1, 1);
+        if constexpr (WHOLE) add(low, 1, 1);
         add(low, 0, 1);
-        add(low, 1, 0);
-        constexpr int PRODUCTS = 6 * WN * WM, EACH = (44 * (WN + WM) + PRODUCTS - 1) / PRODUCTS;
+        if constexpr (WHOLE) add(low, 1, 0);
+        constexpr int PRODUCTS = (WHOLE ? 6 : 3) * WN * WM, EACH = ((WHOLE ? 44 : 8) * WN + 44 * WM + PRODUCTS - 1) / PRODUCTS;
         __builtin_amdgcn_sched_group_barrier(0x100, 2 * (WN + WM), 0);
         gd_static_for<0, PRODUCTS>([&](auto) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -216,7 +239,7 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
 #pragma unroll
         for (int r = 0; r < WN + WM; ++r)
 #pragma unroll
-            for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(op[slot ^ 1][r][i]));
+            for (int i = 0; i < (WHOLE || r >= WN ? 3 : 1); ++i) asm volatile("" : "+v"(op[slot ^ 1][r][i]));
         __builtin_amdgcn_sched_barrier(0);
     };
     auto settle = [&] {
@@ -229,28 +252,38 @@ gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __rest
                 for (int v = 0; v < 16; ++v) few[a][b][v] = 0.f;
             }
     };
-    if (steps > 0) {
+    // Whether every weight of the part was a bf16 number; a part that meets another ends early and is begun again with all six products.
+    auto multiply = [&](auto whole_c) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole_c)::value;
 #pragma unroll
         for (int st = 0; st < NS; ++st)
             if (st < steps) fetch(st);
         gd_wait_younger<2 * LPW, NS / 2 - 1>(min(NS / 2, steps / 2) - 1);
-        operands(std::integral_constant<int, 0>{}, 0);
+        operands(std::integral_constant<int, 0>{}, whole_c, 0);
         int s = 0;
-        auto block = [&](auto steady_c) {
-            step(std::integral_constant<int, 0>{}, steady_c, s);
-            step(std::integral_constant<int, 1>{}, steady_c, s + 1);
-            step(std::integral_constant<int, 2>{}, steady_c, s + 2);
-            step(std::integral_constant<int, 3>{}, steady_c, s + 3);
+        auto block = [&](auto steady_c) __attribute__((always_inline)) {
+            step(std::integral_constant<int, 0>{}, steady_c, whole_c, s);
+            step(std::integral_constant<int, 1>{}, steady_c, whole_c, s + 1);
+            step(std::integral_constant<int, 2>{}, steady_c, whole_c, s + 2);
+            step(std::integral_constant<int, 3>{}, steady_c, whole_c, s + 3);
             s += 4;
             if (s % F32_BLOCK == 0) settle();
         };
-        while (s + 3 + NS < steps) block(std::true_type{});
-        while (s + 3 < steps) block(std::false_type{});
-        if (s < steps) {                                                       // (an even number of steps)
-            step(std::integral_constant<int, 0>{}, std::false_type{}, s);
-            step(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
+        auto narrow = [&] { return WHOLE || __builtin_amdgcn_ballot_w64((seen & 0xffff) != 0) == 0; };
+        while (s + 3 + NS < steps && narrow()) block(std::true_type{});
+        while (s + 3 < steps && narrow()) block(std::false_type{});
+        if (s < steps && narrow()) {                                           // (an even number of steps)
+            step(std::integral_constant<int, 0>{}, std::false_type{}, whole_c, s);
+            step(std::integral_constant<int, 1>{}, std::false_type{}, whole_c, s + 1);
         }
         settle();
+        return narrow();
+    };
+    if (steps > 0 && !multiply(std::false_type{})) {
+        gd_wait_loads<0>();                                                    // (what was asked for ahead lands in stages that are written again)
+        gd_wait_lds();
+        clear();
+        multiply(std::true_type{});
     }
     // acc[a][b][v] is out[m][n] with n = n0 + a 32 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + b 32 + li
     const bool vectors = N % 4 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;

@@ -63,3 +63,19 @@ def test_scales_and_what_is_not_finite(scale):
     finite = exact.isfinite() & (exact.abs() < 3e38)
     assert bool((out.isnan() == exact.isnan()).all()) and bool((out.isinf() & (out > 0) == (exact == float("inf"))).all())
     assert bool(((out.double() - exact).abs() <= _bound(a, w) + 2.0 ** -126)[finite].all())
+
+
+@pytest.mark.parametrize("m, n, k", [(17, 70, 32), (40, 70, 64), (40, 70, 160), (65, 2050, 544), (300, 520, 2048), (130, 260, 4128)])
+@pytest.mark.parametrize("at", [0.0, 0.3, 1.0])
+def test_weights_of_bf16_numbers(m, n, k, at):
+    """Three products do where every weight of a part of K is a bf16 number: the same bits as six, which one weight of another kind asks for (``at``: where in K)."""
+    gen = torch.Generator(DEV).manual_seed(m + n + k)
+    a, w = torch.randn(m, k, generator=gen, device=DEV), torch.randn(n, k, generator=gen, device=DEV).bfloat16().float()
+    out, other = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    core.linear_generic(a, w, None, out)
+    assert bool(((out.double() - a.double() @ w.double().T).abs() <= _bound(a, w)).all())
+    w[n // 2, int(at * (k - 1))] += 2.0 ** -20
+    core.linear_generic(a, w, None, other)
+    rest = torch.arange(n, device=DEV) != n // 2
+    assert torch.equal(out[:, rest], other[:, rest])
+    assert bool(((other.double() - a.double() @ w.double().T).abs() <= _bound(a, w)).all())
