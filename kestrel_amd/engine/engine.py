@@ -12,6 +12,7 @@ this engine: prompts are token ids, an image is a block of given embeddings.
 from __future__ import annotations
 
 import asyncio
+import gc
 import logging
 import queue
 import threading
@@ -203,6 +204,8 @@ class InferenceEngine:
             # graphs, scratch memory and plans now, not in the middle of the first steps that need them
             done = self.runner.prepare(cfg.max_num_batched_tokens, wanted_rows=cfg.max_batch_size, tune_linears=cfg.tune_linears)
             sampler.reserve(cfg.max_batch_size)
+            # (what an engine before this one held in cycles of objects, device memory with it, goes back now rather than beside a request)
+            gc.collect()
             _LOGGER.info("warm-up: %d decode graphs and %d graphs of other steps captured in %.2f s, %d prompt steps in %.2f s, "
                          "%.0f MiB of kernel scratch",
                          int(done.get("graphs", 0)), int(done.get("step_graphs", 0)), done.get("capture_s", 0.0), int(done.get("prompt_steps", 0)),
