@@ -269,7 +269,8 @@ KA_API int ka_linears_first_f32(const float* x, long ldx, const float* gamma, co
     const char* who = "ka_linears_first_f32";
     KA_CHECK(M > 0 && N1 > 0 && N2 > 0 && K > 0 && ldx >= K && ldw1 >= K && ldw2 >= K && ldo1 >= N1 && ldo2 >= N2, "%s: M=%d N=%d, %d K=%d", who, M, N1, N2, K);
     KA_CHECK(ka_act_known(act1) && ka_act_known(act2), "%s: unknown activation %d or %d", who, act1, act2);
-    if (M > GP_ROWS || K % GP_STEP || K > 3072 || M * K > 16384 || ka_act_gated(act1) || ka_act_gated(act2)) return 0;
+    // (a workgroup normalises ITEMS fours a thread of a row, which has to be all of it: three up to six rows, two for seven and eight)
+    if (M > GP_ROWS || K % GP_STEP || K > (M <= 6 ? 3072 : 2048) || M * K > 16384 || ka_act_gated(act1) || ka_act_gated(act2)) return 0;
     if (!gp_vectors(x, ldx) || !gp_vectors(W1, ldw1) || !gp_vectors(W2, ldw2) || !gp_vectors(gamma, 0) || !gp_vectors(beta, 0)) return 0;
     if ((long)N1 + N2 >= (1L << 30)) return 0;
     GpFirst p = {x, ldx, gamma, beta, eps, {W1, W2}, {bias1, bias2}, {out1, out2}, {ldw1, ldw2}, {ldo1, ldo2}, {N1, N2}, {act1, act2}, M, K};
@@ -278,6 +279,7 @@ KA_API int ka_linears_first_f32(const float* x, long ldx, const float* gamma, co
     const int per_cu = M <= 3 && K > 1024 ? 3 : 2;
 #define KA_FIRST(MB, ITEMS)                                                                                                                                                       \
     {                                                                                                                                                                             \
+        KA_CHECK(M <= MB && K <= ITEMS * GP_THREADS * 4, "%s: %d rows of %d by a kernel of %d rows of %d", who, M, K, MB, ITEMS * GP_THREADS * 4);                                \
         static bool configured = false;                                                                                                                                           \
         if (!configured) {                                                                                                                                                        \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gp_first_kernel<MB, ITEMS>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);                  \
@@ -293,7 +295,7 @@ KA_API int ka_linears_first_f32(const float* x, long ldx, const float* gamma, co
     else if (M == 3) { KA_FIRST_ITEMS(3) }
     else if (M == 4) { KA_FIRST_ITEMS(4) }
     else if (M <= 6) { KA_FIRST_ITEMS(6) }
-    else KA_FIRST(8, 2)                  // (16,384 values at the most)
+    else KA_FIRST(8, 2)
 #undef KA_FIRST_ITEMS
 #undef KA_FIRST
     KA_LAUNCH_CHECK();
