@@ -282,7 +282,8 @@ KA_API int ka_linears_first_f32(const float* x, long ldx, const float* gamma, co
         KA_CHECK(M <= MB && K <= ITEMS * GP_THREADS * 4, "%s: %d rows of %d by a kernel of %d rows of %d", who, M, K, MB, ITEMS * GP_THREADS * 4);                                \
         static bool configured = false;                                                                                                                                           \
         if (!configured) {                                                                                                                                                        \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gp_first_kernel<MB, ITEMS>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);                  \
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gp_first_kernel<MB, ITEMS>), hipFuncAttributeMaxDynamicSharedMemorySize,              \
+                                               MB * ITEMS * GP_THREADS * 16);      /* the form's longest rows: 73,728 bytes of six */                                        \
             KA_CHECK(e == hipSuccess, "%s: cannot reserve LDS: %s", who, hipGetErrorString(e));                                                                                    \
             configured = true;                                                                                                                                                    \
         }                                                                                                                                                                         \
