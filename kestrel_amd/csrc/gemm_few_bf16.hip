@@ -133,7 +133,8 @@ few_whole_kernel(FwArgs p) {
         for (int a = 0; a < TW; ++a) sum[a] = (acc[0][0][a] + acc[0][1][a]) + sum[a];
     }
     // A wave's sums leave through LDS as rows (written once per value where they are computed, every activation was code TW x 4 times over).
-    gd_barrier();                                                       // the last K-step has been read by everybody
+    gd_wait_lds();
+    gd_barrier();                                                       // the last K-step is in everybody's registers
     constexpr int PITCH = T::BN + 4;
     static_assert(GX * 16 * PITCH * 4 <= T::SMEM, "the sums of all waves");
     float* const rows = reinterpret_cast<float*>(fw_lds) + wave * 16 * PITCH;
