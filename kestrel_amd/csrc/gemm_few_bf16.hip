@@ -227,6 +227,15 @@ static int launch_whole_rows(const FwArgs& p, int tw, int order, hipStream_t str
     KA_CHECK(false, "linear of few rows: unknown tile %d", tw);
 }
 
+// The tile for one linear (N2 = 0) or two of M rows, in sixteens of weight rows; 0: not by these tiles.
+KA_API int ka_few_rows_whole_tile(int M, int N1, int N2, int K, int halves) {
+    if (M < 17 || M > 64 || N1 < 1 || N2 < 0 || K < 64 || K % (halves ? 64 : 512)) return 0;
+    FwArgs p = {};
+    p.M = M; p.K = K; p.a.N = N1; p.b.N = N2;
+    p.b.W = N2 ? reinterpret_cast<const bf16_t*>(&p) : nullptr;          // (asked for as "there is one" alone)
+    return few_whole_tile(p, halves ? FW_HALVES : FW_EIGHTHS);
+}
+
 // `halves`: the sums of the kernel with parts of K, for a K in one part; else those of the persistent kernel. 0: done; 1: not covered, nothing was run; -1: an error.
 int ka_few_rows_whole(const SkinnyArgs& args, bool halves, hipStream_t stream) {
     const int K = args.K[0];

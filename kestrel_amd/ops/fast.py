@@ -51,6 +51,7 @@ _SIGNATURES = {
         _c_void_p, _c_long, _c_int, _c_int,                                                # A, lda, M, K
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int,                 # W, ldw, bias, out, ldo, N, act of either linear
         _c_void_p, _c_long, _c_void_p, _c_void_p, _c_long, _c_int, _c_int, _c_int, _c_void_p],   # ..., tile, stream
+    "ka_few_rows_whole_tile": [_c_int, _c_int, _c_int, _c_int, _c_int],                    # M, N1, N2, K, halves
     "ka_linear_quad_tile": [_c_int, _c_int, _c_int],
     "ka_linear_quad_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     "ka_linear_library_bf16": [_c_void_p, _c_long, _c_void_p, _c_long, _c_void_p, _c_void_p, _c_int, _c_long, _c_int,

@@ -10,6 +10,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
+def _tile(m, n, k, halves, n2=0):
+    """The tile by which a linear goes, in sixteens of weight rows; 0: by the kernels whose bits these are."""
+    from kestrel_amd.ops import fast
+
+    return fast.lib().ka_few_rows_whole_tile(m, n, n2, k, int(halves))
+
+
 def _near(got, want, dtype):
     """fp32: sums of at most 8,192 products in chains of MFMAs, as ``test_few_rows_tiles_gpu.py``; bf16: half a unit in the last place, 2^-9 of the value."""
     limit = 2.0 ** -20 if dtype == torch.float32 else 2.0 ** -8
@@ -23,6 +30,7 @@ def _near(got, want, dtype):
 def test_rows_have_the_bits_of_sixteen_rows_alone(m, n, k):
     from kestrel_amd.ops import fast
 
+    assert _tile(m, n, k, False) == {3072: 1, 4100: 2, 8196: 3, 10240: 3, 12292: 4, 16384: 4}[n]
     gen = torch.Generator().manual_seed(m + n + k)
     a, w = torch.randn(m, k, generator=gen).bfloat16().to(DEV), torch.randn(n, k, generator=gen).bfloat16().to(DEV)
     bias = torch.randn(n, generator=gen).to(DEV)
@@ -42,6 +50,7 @@ def test_rows_have_the_bits_of_sixteen_rows_alone(m, n, k):
 def test_five_sixteens():
     from kestrel_amd.ops import fast
 
+    assert _tile(50, 17924, 2560, False) == 5
     gen = torch.Generator().manual_seed(5)
     a, w = torch.randn(50, 2560, generator=gen).bfloat16().to(DEV), torch.randn(17924, 2560, generator=gen).bfloat16().to(DEV)
     out, alone = torch.empty(50, 17924, device=DEV), torch.empty(16, 17924, device=DEV)
@@ -56,6 +65,7 @@ def test_one_part_has_the_bits_of_the_kernel_with_parts(m, n, k):
     """Three to seven sixteens of weight rows a tile; K of fewer steps than there are stages; into the old values, whatever K."""
     from kestrel_amd.ops import fast
 
+    assert _tile(m, n, k, True) == {8196: 3, 10752: 3, 12292: 4, 18564: 5, 20484: 3, 28672: 4, 51204: 7}[n]
     gen = torch.Generator().manual_seed(m + n + k)
     a, w = torch.randn(m, k, generator=gen).bfloat16().to(DEV), torch.randn(n, k, generator=gen).bfloat16().to(DEV)
     bias, start = torch.randn(n, generator=gen).to(DEV), torch.randn(m + 1, n, generator=gen).to(DEV)
@@ -73,12 +83,20 @@ def test_one_part_has_the_bits_of_the_kernel_with_parts(m, n, k):
     _near(results[0], start[:m].double() + bias.double() + a.double() @ w.double().T, torch.float32)
 
 
+# (outputs too few or too many for one tile a CU, either side of 48 rows; K in no rounds of the eight sums, or in no whole steps; rows that other kernels take)
+@pytest.mark.parametrize("m, n, k, halves", [(48, 3068, 2048, False), (48, 16388, 1536, False), (48, 10244, 2048, False), (49, 1020, 512, False), (49, 16388, 2048, False),
+                                             (64, 20484, 2560, False), (64, 8192, 2112, False), (64, 8192, 2080, True), (16, 8192, 2048, False), (65, 8192, 2048, False)])
+def test_what_other_kernels_take(m, n, k, halves):
+    assert _tile(m, n, k, halves) == 0
+
+
 @pytest.mark.parametrize("m, ns, k", [(20, (2048, 3072), 1024), (64, (6144, 8192), 2048), (40, (8200, 9000), 4096)])
 def test_two_outputs_in_bf16(m, ns, k):
     """Two linears of the same rows, the second with an activation, into columns of wider rows; against either alone."""
     from kestrel_amd.ops import fast
     from kestrel_amd.ops.linear import ACT_GATED, activation_code
 
+    assert _tile(m, ns[0], k, k > 2560, ns[1]) == {1024: 2, 2048: 4, 4096: 5}[k]
     gen = torch.Generator().manual_seed(m + sum(ns) + k)
     a = torch.randn(m, k, generator=gen).bfloat16().to(DEV)
     ws = [(torch.randn(n, k, generator=gen) * k ** -0.5).bfloat16().to(DEV) for n in ns]
