@@ -488,7 +488,8 @@ class ModelRunner:
             cu_q.append(pad_tokens)
             kv_len.append(0)
             row_slot.append(-1)
-            logit_rows.extend([0] * (pad_rows - n_wanted))
+            # (places that nobody wants: a token that sees no keys where there is one, since the last layer reads a wanted token's keys)
+            logit_rows.extend([n_live if fill else 0] * (pad_rows - n_wanted))
             logit_slot.extend([-1] * (pad_rows - n_wanted))
             given_rows = given_rows + [-1] * (pad_tokens - len(given_rows))
             pad_rows += 1                                          # (the last row is one of the step's rows)

@@ -180,3 +180,17 @@ def test_what_does_not_fit_a_captured_layout_is_launched():
     assert runner.mixed_graph_replays == 1 and sorted(runner._mixed) == [(32, 8)]
     expected = plain.forward(helpers.flat_config(name), helpers.stored_weights(helpers.model_dir(name)), req.ids, None)
     helpers.assert_close(torch.cat([logits, last]), expected[list(range(20)) + [39]], dtype, "launched, then replayed")
+
+
+@pytest.mark.parametrize("tokens, place", [(20, 20), (31, 31), (32, 0)])
+def test_places_that_nobody_wants_see_no_keys(tokens, place):
+    """A replayed step has as many wanted places as its graph has rows: those that nobody asked for are what fills the step up, which reads no keys, and token 0 only where nothing does."""
+    from kestrel_amd.engine.step import StepEntry
+
+    runner = _runner("D", torch.float32, max_requests=8)
+    slot = runner.admit()
+    ids = helpers.random_ids(7, tokens, helpers.flat_config("D")["vocab_size"])
+    batch = runner.build_batch([StepEntry(slot, ids, want=[3, tokens - 1])], pad_rows=8, pad_tokens=32, fixed_pages=runner._pages_cap)
+    assert batch.logit_rows.tolist() == [3, tokens - 1] + [place] * 6
+    assert batch.logit_slot.tolist() == [slot, slot] + [-1] * 6
+    assert place == 0 or (batch.kv_hi[place:].tolist() == [0] * (32 - tokens) and all(s < 0 for s in batch.groups[0].slots[place:].tolist()))
