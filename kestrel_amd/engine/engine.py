@@ -180,6 +180,9 @@ class InferenceEngine:
             raise ValueError("RuntimeConfig.model_path must name a folder with config.json and model.safetensors")
         device = cfg.resolved_device()
         torch.cuda.set_device(device)
+        # What an engine before this one held in cycles of objects goes back now, device memory with it: neither counted against this one's pool nor freed beside a request.
+        gc.collect()
+        torch.cuda.empty_cache()
         started = time.perf_counter()
         net = load_model(cfg.model_path, cfg.dtype, device, cfg.model)
         self.plan = net.plan
@@ -204,8 +207,6 @@ class InferenceEngine:
             # graphs, scratch memory and plans now, not in the middle of the first steps that need them
             done = self.runner.prepare(cfg.max_num_batched_tokens, wanted_rows=cfg.max_batch_size, tune_linears=cfg.tune_linears)
             sampler.reserve(cfg.max_batch_size)
-            # (what an engine before this one held in cycles of objects, device memory with it, goes back now rather than beside a request)
-            gc.collect()
             _LOGGER.info("warm-up: %d decode graphs and %d graphs of other steps captured in %.2f s, %d prompt steps in %.2f s, "
                          "%.0f MiB of kernel scratch",
                          int(done.get("graphs", 0)), int(done.get("step_graphs", 0)), done.get("capture_s", 0.0), int(done.get("prompt_steps", 0)),

@@ -398,3 +398,35 @@ def test_configurations_drawn_at_random(seed, dtype, tmp_path):
     got = helpers.replay(runner, reqs, steps, poison=True)
     for tag, req in reqs.items():
         helpers.assert_close(got[tag], plain.forward(cfg, weights, req.ids, req.prefix), dtype, f"{cfg} request {tag}")
+
+
+@pytest.mark.parametrize("warmup", [False, True])
+def test_what_an_engine_before_left_in_cycles_is_free_for_the_pool(monkeypatch, warmup):
+    """A start collects cycles of objects before it asks how much memory is free."""
+    import gc
+    import weakref
+
+    from kestrel_amd import InferenceEngine, RuntimeConfig
+    from kestrel_amd.engine import engine as module
+
+    class Cycle:
+        pass
+
+    seen, real = [], module.pool_pages
+    monkeypatch.setattr(module, "pool_pages", lambda cfg, size, longest, free: seen.append(free) or real(cfg, size, longest, free))
+    gc.collect()
+    torch.cuda.empty_cache()
+    before, _total = torch.cuda.mem_get_info()
+    gc.disable()
+    try:
+        old = Cycle()
+        old.itself, old.pool = old, torch.empty(8 << 30, dtype=torch.uint8, device="cuda:0")
+        gone = weakref.ref(old)
+        del old
+        assert gone() is not None
+        engine = InferenceEngine.create_sync(RuntimeConfig(model_path=helpers.model_dir("A"), device="cuda:0", dtype=torch.bfloat16, kv_cache_pages=16, max_batch_size=2, warmup=warmup,
+                                                           enable_graphs=False))
+        engine.shutdown_sync()
+    finally:
+        gc.enable()
+    assert gone() is None and seen[0] > before - (4 << 30)
