@@ -5,7 +5,7 @@
 //    order; the fallback of the bf16 path;
 // and, of aligned fp32 operands, the true 32-bit path,
 //  * up to 16 rows of a linear without a gate: a stream of weights (gemv_f32_kernel);
-//  * else K in steps of 32: the matrix pipes, every number as three of bf16 (gemm_f32_split_kernel);
+//  * else K in steps of 32: the matrix pipes, in 32 bits, or the activations as three of bf16 where weights are bf16 numbers (gemm_f32_tiles_kernel);
 //  * else wider FMA tiles, k in ascending order as the first (gemm_f32_kernel).
 // So a row's result does not depend on what else is in the batch, but for the step from 16 to 17 rows without a gate.
 #include "ka_common.h"
@@ -73,41 +73,48 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
     }
 }
 
-// Many rows in fp32 where K is a multiple of 32: products on the bf16 matrix pipes, which have sixteen times the rate of the fp32 ones. A number of 32 bits is
-// the sum of three bf16 numbers to its last bit (24 bits of mantissa, eight in each: what rounding to the nearest leaves is representable, so
-// both subtractions are exact), and w x = w1 x1 + (w1 x2 + w2 x1) + (w2 x2 + w1 x3 + w3 x1) + what is below 2^-25 of it: six products, each exact in the
-// pipe, summed in fp32.
+// Many rows in fp32 where K is a multiple of 32, on the matrix pipes: products of 32 bits (v_mfma_f32_32x32x2_f32), and for weights that are bf16 numbers, as checkpoints hold
+// them, products of the activations' three bf16 parts (v_mfma_f32_32x32x16_bf16, sixteen times the rate). A number of 32 bits is the sum of three bf16 numbers to its last bit:
+// 24 bits of mantissa, eight in each; what rounding to the nearest leaves is representable, so both subtractions are exact. Then w x = w x1 + w x2 + w x3, each exact in the
+// pipe: nothing is left out, and the sums are fp32 either way.
 //
-// Operands go straight from memory into swizzled LDS as in ka_dma_tiles.h, two steps of 16 numbers at a time (whole lines), and are split by the wave that
-// multiplies them: 44 instructions per eight numbers a lane, laid between the products of the step before, which the compiler does only where each step is a
-// region of its own with an end that names the parts (157 rows of 2,048 x 8,192 by tiles of 64 x 64: 96 us without, 83 with). At one wave a SIMD an instruction
-// takes five cycles, so a step of 64 x 64 x 16 (24 products, some 225 other instructions) takes 1,400 where its products are 768: that is what bounds it. The
-// activations' parts by a launch of their own, in front, were no faster: 10 KB a step instead of 8.
+// Which of the two a sum takes is decided per weight row, row of A and part of K, by those rows alone, so that every tile gives the same bits:
+//  * A weight whose lower half is not zero has no single bf16 part. Where every row of the tile shows one among its first sixteen numbers (weights of 32 bits do),
+//    nothing but products of 32 bits is run.
+//  * A number of A below 2^-109 may have bits below bf16's smallest: what is left for the third part then has a lower half.
+//  * Infinities, NaN and what lies beyond bf16's largest leave a sum that is not finite.
+// Where a tile meets one of these, the wave that does multiplies its part once more in 32 bits, and the sums that need it take that result (us, 282 rows, usual numbers, a NaN
+// in every row, numbers of 1e-36, and one weight row in 50 of 32 bits: 2,048 x 6,144 64, 108, 133 and 121; 8,192 x 2,048 87, 169, 203 and 160).
 //
-// The order of a sum is fixed by K alone. K is cut into F32_PARTS parts, each summed by a wave of its own (so no wave waits for another before the
-// end): w1 x1 of 128 of K from zero, these sums in order, the five smaller products, whose roundings weigh 2^-8, in an accumulator beside them; the
-// parts' sums meet in LDS and are added in their order. All tiles give the same bits.
+// Operands go straight from memory into swizzled LDS as in ka_dma_tiles.h, whole lines of 32 numbers, and are split by the wave that multiplies them, between the products of
+// the half step before, which the compiler does only where each half is a region of its own with an end that names the parts. Tiles of 32 x 32 alone, two workgroups a
+// CU: waves with 64 x 64 split half as often, but are one a SIMD, and the vector unit, which fetches their sums from the matrix pipe's registers, is what multiplies 32-bit
+// numbers (us, tiles of 32 and of 64, bf16 weights and those of 32 bits: 282 rows of 2,048 x 6,144 61 and 55, 80 and 94; 2,048 rows 347 and 307, 515 and 558; 2,048 rows of
+// 8,192 x 2,048 422 and 306, 644 and 661; 2,560 x 7,680, 64 rows 31 and 51, 33 and 61).
 //
-// Weights that are bf16 numbers, as checkpoints hold them, have one part, and three of the six products are zeros: a wave begins its part with the other three, looks
-// at the lower halves of the weights as it goes, and where it meets one that is not zero begins again with all six, to the same bits (282 rows as below:
-// 51, 26, 75 and 75 us; weights that need all six pay for the first steps, 67, 31, 95 and 93).
+// The order of a sum is fixed by K alone. K is cut into F32_PARTS parts, each summed by a wave of its own (so no wave waits for another before the end); the parts' sums meet in LDS
+// and are added in their order.
+//  * Products of 32 bits: every sixteen k are summed from zero (of every eight in the order 0 4 1 5 2 6 3 7: a lane holds four neighbours), these sums added in order. The short
+//    chains take the error of a sum from that of a chain of K / 4 terms to that of one of K / 64 (of every 32 from zero: 6 % faster, an error up to 9 % larger).
+//  * Three parts: w x1 of 128 of K from zero, these sums in order; w x2 and w x3, whose roundings weigh 2^-8, in an accumulator beside them.
 //
-// What three bf16 numbers cannot say (infinities, numbers beyond bf16's largest) leaves an infinity or NaN in the sum: such an output is summed again by
-// plain FMA from memory. (Numbers below 2^-109 lose what is below 2^-133 of them.)
-//
-// Measured, us, fp32 products on the matrix pipes (v_mfma_f32_32x32x2_f32) -> here, 64 rows through 2,048 x 6,144, 2,048 x 2,048, 2,048 x
-// 8,192 and 8,192 x 2,048 28.6, 16.4, 27.8 and 52.2 -> 25.0, 15.8, 27.4 and 47.3; 282 rows 85, 38, 105 and 131 -> 66, 30, 90 and 92; 2,048 rows 446, 162, 591 and 611
-// -> 385, 134, 511 and 432. Error against 64 bits of such sums 1.35e-7 -> 8.7e-8, of K = 8,192 2.2e-7 -> 1.1e-7.
+// Measured, us, outputs x inputs; all products in 32 bits by tiles of 32 x 32 to 64 x 128 -> here with weights of 32 bits and with bf16 numbers: 6,144 x 2,048, 17 rows 19.3 -> 17.6, 15.4; 64
+// rows 27.1 -> 28.0, 23.3; 282 rows 81.8 -> 80.3, 59.1; 2,048 rows 445 -> 521, 329. 2,048 x 8,192: 51.1 -> 46.7, 34.8; 51.7 -> 47.8, 38.5; 130 -> 128, 84.8; 614 -> 659, 425. Over 14
+// shapes (1,024 to 10,240 outputs, K of 1,024 to 10,240): 17 to 32 rows 0.96 and 0.85 of the time, 48 to 64 0.98 and 0.85, 80 to 160 0.98 and 0.80, 282 1.01 and 0.74, 512 1.05 and 0.77,
+// 2,048 1.12 and 0.77. Error against 64 bits of sums of 2,048 1.35e-7, with bf16 weights 8.7e-8; of 8,192 2.2e-7 and 1.1e-7.
 constexpr int F32_PARTS = 4;
 constexpr int F32_STEP = 32;
-constexpr int F32_BLOCK = 8;       // steps of 16 that are summed from zero
+constexpr int F32_TILE = 32;
+constexpr int F32_BLOCK = 4;       // steps whose main products are summed from zero
 
 typedef __attribute__((ext_vector_type(2))) float gs_float2;
 typedef __attribute__((ext_vector_type(2))) __bf16 gs_bf16x2;
 
-// part[0] + part[1] + part[2] is the eight numbers of lo and hi to the last bit
-__device__ __forceinline__ void gs_split(const floatx4& lo, const floatx4& hi, bf16x8 (&part)[3]) {
+// part[0] + part[1] + part[2] is the eight numbers of lo and hi to the last bit, or the lower half of what is returned is not zero: what is left for the third part is a bf16
+// number exactly where its lower half is zero.
+__device__ __forceinline__ unsigned gs_split(const floatx4& lo, const floatx4& hi, bf16x8 (&part)[3]) {
     uint4 out[3];
+    unsigned left = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float a = i < 2 ? lo[2 * i] : hi[2 * i - 4], b = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
@@ -115,269 +122,235 @@ __device__ __forceinline__ void gs_split(const floatx4& lo, const floatx4& hi, b
         for (int p = 0; p < 3; ++p) {
             const unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector(gs_float2{a, b}, gs_bf16x2));
             (i == 0 ? out[p].x : i == 1 ? out[p].y : i == 2 ? out[p].z : out[p].w) = pair;
-            if (p == 2) break;
+            if (p == 2) {
+                left |= __float_as_uint(a) | __float_as_uint(b);
+                break;
+            }
             a -= __uint_as_float(pair << 16);
             b -= __uint_as_float(pair & 0xffff0000u);
         }
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p) part[p] = __builtin_bit_cast(bf16x8, out[p]);
+    return left;
 }
 
-template <int WN, int WM, int NS>
-__global__ void __launch_bounds__(KA_WAVE * F32_PARTS, WN * WM > 1 ? 1 : 2)
-gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
+// NS: steps in LDS
+template <int NS>
+__global__ void __launch_bounds__(KA_WAVE * F32_PARTS, 2)
+gemm_f32_tiles_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const float* __restrict__ bias,
                       float* __restrict__ out, long ldo, int M, int N, int K, int act, int accumulate, int tiles_n, int tiles_m) {
-    constexpr int BN = 32 * WN, BM = 32 * WM, STEP = 16;
-    constexpr int ROW = STEP * 4, CPR = ROW / 16, RPL = KA_WAVE / CPR, STAGE = (BN + BM) * ROW;
-    constexpr int W_LOADS = BN / RPL, X_LOADS = BM / RPL, LPW = W_LOADS + X_LOADS;
+    constexpr int ROW = F32_STEP * 4, CPR = ROW / 16, RPL = KA_WAVE / CPR, STAGE = 2 * F32_TILE * ROW;      // a step: the rows of W, then of A
+    constexpr int LOADS = F32_TILE / RPL, LPW = 2 * LOADS;
     extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
     const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8;
     const int logical = blockIdx.x % 8 * per_xcd + blockIdx.x / 8;
     if (logical >= total || (int)blockIdx.x / 8 >= per_xcd) return;
-    const int n0 = logical / tiles_m * BN, m0 = logical % tiles_m * BM;
+    // Up to ten tiles of A's rows at a time, through all of W: what an XCD's 64 workgroups read at once is nearly a square (2,048 rows of 2,048 x 6,144, bf16 weights, 433 -> 329 us).
+    const int groups = (tiles_m + 9) / 10, height = (tiles_m + groups - 1) / groups, group = logical / (height * tiles_n);
+    const int here = min(height, tiles_m - group * height), within = logical - group * height * tiles_n;
+    const int n0 = within / here * F32_TILE, m0 = (group * height + within % here) * F32_TILE;
     const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / KA_WAVE), lane = threadIdx.x % KA_WAVE;
     const int li = lane % 32, lg = lane / 32;
-    const float* wsrc[W_LOADS];
-    const float* xsrc[X_LOADS];
-    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP * (F32_STEP / STEP), k_steps = K / STEP;
+    const int part_steps = ((K + F32_PARTS - 1) / F32_PARTS + F32_STEP - 1) / F32_STEP, k_steps = K / F32_STEP;
     const int first = part * part_steps, steps = max(0, min(part_steps, k_steps - first));
+    const float* wsrc[LOADS];
+    const float* xsrc[LOADS];
 #pragma unroll
-    for (int i = 0; i < W_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(i, lane);
-        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + kd_load_channel<CPR>(r, lane) / 2 + first * STEP;      // (four numbers a piece)
-    }
-#pragma unroll
-    for (int i = 0; i < X_LOADS; ++i) {
-        const int r = kd_load_row<CPR>(i, lane);
-        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + kd_load_channel<CPR>(r, lane) / 2 + first * STEP;
+    for (int i = 0; i < LOADS; ++i) {                                          // (four numbers a piece; rows past the end: the last one again, not stored)
+        const int r = kd_load_row<CPR>(i, lane), c = kd_load_channel<CPR>(r, lane) / 2 + first * F32_STEP;
+        wsrc[i] = W + (size_t)min(n0 + r, N - 1) * ldw + c;
+        xsrc[i] = A + (size_t)min(m0 + r, M - 1) * lda + c;
     }
     unsigned char* mine = gf_lds + part * NS * STAGE;
     auto fetch = [&](int step) {
         unsigned char* base = mine + step % NS * STAGE;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + step * STEP), (GD_LDS void*)(base + i * RPL * ROW), 16, 0, 0);
+        for (int i = 0; i < LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(wsrc[i] + step * F32_STEP), (GD_LDS void*)(base + i * RPL * ROW), 16, 0, 0);
 #pragma unroll
-        for (int i = 0; i < X_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + step * STEP), (GD_LDS void*)(base + BN * ROW + i * RPL * ROW), 16, 0, 0);
+        for (int i = 0; i < LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const GD_GLOBAL void*)(xsrc[i] + step * F32_STEP), (GD_LDS void*)(base + (LOADS + i) * RPL * ROW), 16, 0, 0);
+    };
+    // the first stages, and the first step's loads landed
+    auto begin = [&] {
+#pragma unroll
+        for (int st = 0; st < NS; ++st)
+            if (st < steps) fetch(st);
+        gd_wait_younger<LPW, NS - 1>(min(NS, steps) - 1);
     };
     const int swz = kd_swizzle<CPR>(li);
-    floatx16 acc[WN][WM], few[WN][WM], low[WN][WM];
-    auto clear = [&] {
-#pragma unroll
-        for (int a = 0; a < WN; ++a)
-#pragma unroll
-            for (int b = 0; b < WM; ++b)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[a][b][v] = few[a][b][v] = low[a][b][v] = 0.f;
+    // four numbers of half a step of this lane's row of W (0) or of A (1); h = 0, 1: the eight of its products
+    auto four = [&](int step, int half, int operand, int h) {
+        return *reinterpret_cast<const floatx4*>(mine + step % NS * STAGE + (operand * F32_TILE + li) * ROW + ((half * 4 + h * 2 + lg) ^ swz) * 16);
     };
-    clear();
-    bf16x8 op[2][WN + WM][3];
-    // the operands of a step from LDS, split (the step's loads have landed; a wave reads what it asked for itself: no barrier)
-    unsigned seen = 0;                                                         // bits of the weights that were read
-    auto operands = [&](auto slot_c, auto whole_c, int step) __attribute__((always_inline)) {
-        constexpr int slot = decltype(slot_c)::value;
-        constexpr bool WHOLE = decltype(whole_c)::value;
-        const unsigned char* base = mine + step % NS * STAGE;
-        floatx4 raw[WN + WM][2];
+    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    floatx16 acc = zero;
+    unsigned odd[2] = {0, 0};        // this lane's row of W, of A: the lower half is not zero where it has a number that the parts do not say
+    unsigned rows[2] = {0, 0};       // the same, a bit a row
+    auto gather = [&] {
 #pragma unroll
-        for (int r = 0; r < WN + WM; ++r)
+        for (int i = 0; i < 2; ++i) {
+            const unsigned long long hit = __builtin_amdgcn_ballot_w64((odd[i] & 0xffff) != 0);
+            rows[i] = (unsigned)hit | (unsigned)(hit >> 32);
+        }
+    };
+    bool again = false;              // products of 32 bits
+    if (steps > 0) {
+        begin();
 #pragma unroll
-            for (int h = 0; h < 2; ++h) raw[r][h] = *reinterpret_cast<const floatx4*>(base + (r * 32 + li) * ROW + ((h * 2 + lg) ^ swz) * 16);
-#pragma unroll
-        for (int r = 0; r < WN + WM; ++r) {
-            if (WHOLE || r >= WN) {
-                gs_split(raw[r][0], raw[r][1], op[slot][r]);
-                continue;
-            }
+        for (int h = 0; h < 2; ++h) {
+            const uint4 w = __builtin_bit_cast(uint4, four(0, 0, 0, h));
+            odd[0] |= w.x | w.y | w.z | w.w;
+        }
+        gather();
+        again = rows[0] == 0xffffffffu;
+    }
+    if (steps > 0 && !again) {
+        floatx16 few = zero, low = zero;
+        bf16x8 w[2], x[2][3];
+        // The operands of half a step from LDS (its loads have landed; a wave reads what it asked for itself: no barrier). counts: the half step is one of the part's.
+        auto operands = [&](auto half_c, int step, unsigned counts) __attribute__((always_inline)) {
+            constexpr int half = decltype(half_c)::value;
+            const floatx4 w_lo = four(step, half, 0, 0), w_hi = four(step, half, 0, 1), x_lo = four(step, half, 1, 0), x_hi = four(step, half, 1, 1);
+            const uint4 lo = __builtin_bit_cast(uint4, w_lo), hi = __builtin_bit_cast(uint4, w_hi);
             uint4 upper;
-            const uint4 lo = __builtin_bit_cast(uint4, raw[r][0]), hi = __builtin_bit_cast(uint4, raw[r][1]);
             upper.x = __builtin_amdgcn_perm(lo.y, lo.x, 0x07060302);
             upper.y = __builtin_amdgcn_perm(lo.w, lo.z, 0x07060302);
             upper.z = __builtin_amdgcn_perm(hi.y, hi.x, 0x07060302);
             upper.w = __builtin_amdgcn_perm(hi.w, hi.z, 0x07060302);
-            op[slot][r][0] = __builtin_bit_cast(bf16x8, upper);
-            seen |= lo.x | lo.y | lo.z | lo.w | hi.x | hi.y | hi.z | hi.w;
-        }
-    };
-    // Step s, the place-th of four: its products, and between them the split of the next one's operands, which the matrix pipe does not need.
-    // STEADY: a step that has NS behind it.
-    auto step = [&](auto place_c, auto steady_c, auto whole_c, int s) __attribute__((always_inline)) {
-        constexpr bool WHOLE = decltype(whole_c)::value;
-        constexpr int place = decltype(place_c)::value, slot = place & 1;
-        constexpr bool STEADY = decltype(steady_c)::value;
-        if constexpr (slot == 1) {                                             // the last step of a pair
-            if constexpr (STEADY) gd_wait_loads<2 * LPW * (NS / 2 - 2)>();
-            else if (s + 1 < steps) gd_wait_younger<2 * LPW, NS / 2 - 2>(min(NS / 2 - 2, (steps - 1 - s) / 2 - 1));
-            gd_wait_lds();                                                     // own reads of the pair are in registers: its stages may be written
-            if (STEADY || s + NS < steps) {
-                fetch(s + NS - 1);
-                fetch(s + NS);
-            }
-        }
-        operands(std::integral_constant<int, slot ^ 1>{}, whole_c, s + 1);              // (behind the last step: memory that nobody uses)
-        auto add = [&](floatx16 (&sum)[WN][WM], int i, int j) {
-#pragma unroll
-            for (int a = 0; a < WN; ++a)
-#pragma unroll
-                for (int b = 0; b < WM; ++b) sum[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[slot][a][i], op[slot][WN + b][j], sum[a][b], 0, 0, 0);
+            w[half] = __builtin_bit_cast(bf16x8, upper);
+            odd[0] |= (lo.x | lo.y | lo.z | lo.w | hi.x | hi.y | hi.z | hi.w) & counts;
+            odd[1] |= gs_split(x_lo, x_hi, x[half]) & counts;
         };
-        add(low, 0, 2);
-        if constexpr (WHOLE) add(low, 2, 0);
-        add(few, 0, 0);
-        if constexpr (WHOLE) add(low, 1, 1);
-        add(low, 0, 1);
-        if constexpr (WHOLE) add(low, 1, 0);
-        constexpr int PRODUCTS = (WHOLE ? 6 : 3) * WN * WM, EACH = ((WHOLE ? 44 : 8) * WN + 44 * WM + PRODUCTS - 1) / PRODUCTS;
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * (WN + WM), 0);
-        gd_static_for<0, PRODUCTS>([&](auto) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, EACH, 0);
-        });
-        // (the split belongs here: the compiler would put it off to the step that uses it, in front of that step's products)
-#pragma unroll
-        for (int r = 0; r < WN + WM; ++r)
-#pragma unroll
-            for (int i = 0; i < (WHOLE || r >= WN ? 3 : 1); ++i) asm volatile("" : "+v"(op[slot ^ 1][r][i]));
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    auto settle = [&] {
-#pragma unroll
-        for (int a = 0; a < WN; ++a)
-#pragma unroll
-            for (int b = 0; b < WM; ++b) {
-                acc[a][b] += few[a][b];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) few[a][b][v] = 0.f;
+        // Half a step: its products, and between them the split of the next one's operands, which the matrix pipe does not need. STEADY: a step that has NS behind it.
+        auto half_step = [&](auto half_c, auto steady_c, int s) __attribute__((always_inline)) {
+            constexpr int half = decltype(half_c)::value;
+            constexpr bool STEADY = decltype(steady_c)::value;
+            if constexpr (half == 1) {
+                if constexpr (STEADY) gd_wait_loads<LPW * (NS - 2)>();
+                else if (s + 1 < steps) gd_wait_younger<LPW, NS - 2>(min(NS - 2, steps - 2 - s));
+                gd_wait_lds();                                                 // own reads of the step are in registers: its stage may be written
+                if (STEADY || s + NS < steps) fetch(s + NS);
+                operands(std::integral_constant<int, 0>{}, s + 1, STEADY || s + 1 < steps ? ~0u : 0u);      // (behind the last step: memory that nobody uses)
+            } else {
+                operands(std::integral_constant<int, 1>{}, s, ~0u);
             }
-    };
-    // Whether every weight of the part was a bf16 number; a part that meets another ends early and is begun again with all six products.
-    auto multiply = [&](auto whole_c) __attribute__((always_inline)) {
-        constexpr bool WHOLE = decltype(whole_c)::value;
-#pragma unroll
-        for (int st = 0; st < NS; ++st)
-            if (st < steps) fetch(st);
-        gd_wait_younger<2 * LPW, NS / 2 - 1>(min(NS / 2, steps / 2) - 1);
-        operands(std::integral_constant<int, 0>{}, whole_c, 0);
+            low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[half], x[half][2], low, 0, 0, 0);
+            few = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[half], x[half][0], few, 0, 0, 0);
+            low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[half], x[half][1], low, 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            gd_static_for<0, 3>([&](auto) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 20, 0);
+            });
+            // (the split belongs here: the compiler would put it off to the half step that uses it, in front of that one's products)
+            asm volatile("" : "+v"(w[half ^ 1]), "+v"(x[half ^ 1][0]), "+v"(x[half ^ 1][1]), "+v"(x[half ^ 1][2]));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto settle = [&] {
+            acc += few;
+            few = zero;
+        };
+        operands(std::integral_constant<int, 0>{}, 0, ~0u);
         int s = 0;
-        auto block = [&](auto steady_c) __attribute__((always_inline)) {
-            step(std::integral_constant<int, 0>{}, steady_c, whole_c, s);
-            step(std::integral_constant<int, 1>{}, steady_c, whole_c, s + 1);
-            step(std::integral_constant<int, 2>{}, steady_c, whole_c, s + 2);
-            step(std::integral_constant<int, 3>{}, steady_c, whole_c, s + 3);
-            s += 4;
+        auto two_steps = [&](auto steady_c) __attribute__((always_inline)) {
+            half_step(std::integral_constant<int, 0>{}, steady_c, s);
+            half_step(std::integral_constant<int, 1>{}, steady_c, s);
+            half_step(std::integral_constant<int, 0>{}, steady_c, s + 1);
+            half_step(std::integral_constant<int, 1>{}, steady_c, s + 1);
+            s += 2;
             if (s % F32_BLOCK == 0) settle();
         };
-        auto narrow = [&] { return WHOLE || __builtin_amdgcn_ballot_w64((seen & 0xffff) != 0) == 0; };
-        while (s + 3 + NS < steps && narrow()) block(std::true_type{});
-        while (s + 3 < steps && narrow()) block(std::false_type{});
-        if (s < steps && narrow()) {                                           // (an even number of steps)
-            step(std::integral_constant<int, 0>{}, std::false_type{}, whole_c, s);
-            step(std::integral_constant<int, 1>{}, std::false_type{}, whole_c, s + 1);
+        while (s + 1 + NS < steps) two_steps(std::true_type{});
+        while (s + 1 < steps) two_steps(std::false_type{});
+        if (s < steps) {
+            half_step(std::integral_constant<int, 0>{}, std::false_type{}, s);
+            half_step(std::integral_constant<int, 1>{}, std::false_type{}, s);
         }
         settle();
-        return narrow();
-    };
-    if (steps > 0 && !multiply(std::false_type{})) {
-        gd_wait_loads<0>();                                                    // (what was asked for ahead lands in stages that are written again)
-        gd_wait_lds();
-        clear();
-        multiply(std::true_type{});
+        acc += low;
+        gather();
+        bool beyond = false;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) beyond |= !(fabsf(acc[v]) < INFINITY);
+        again = rows[0] != 0 || rows[1] != 0 || __builtin_amdgcn_ballot_w64(beyond) != 0;
+        if (again) {
+            gd_wait_lds();
+            begin();
+        }
     }
-    // acc[a][b][v] is out[m][n] with n = n0 + a 32 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + b 32 + li
-    const bool vectors = N % 4 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    auto store = [&](int a, int b, int q, const floatx4& y) {
-        const int m = m0 + b * 32 + li, n = n0 + a * 32 + q * 8 + lg * 4;
-        if (m >= M || n >= N) return;
-        float v[4];
+    if (again) {
+        floatx16 sum = zero;
+        for (int s = 0; s < steps; ++s) {
+            if (s > 0) gd_wait_younger<LPW, NS - 1>(min(NS, steps - s) - 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[j] = y[j];
-            if (!(fabsf(v[j]) < INFINITY) && n + j < N) {                      // (see above)
-                v[j] = 0.f;
-                for (int k = 0; k < K; ++k) v[j] = fmaf(A[(size_t)m * lda + k], W[(size_t)(n + j) * ldw + k], v[j]);
+            for (int half = 0; half < 2; ++half) {
+                const floatx4 w[2] = {four(s, half, 0, 0), four(s, half, 0, 1)}, x[2] = {four(s, half, 1, 0), four(s, half, 1, 1)};
+                floatx16 y = zero;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) y = __builtin_amdgcn_mfma_f32_32x32x2f32(w[j / 4][j % 4], x[j / 4][j % 4], y, 0, 0, 0);
+                sum += y;
             }
-            v[j] += bias && n + j < N ? bias[n + j] : 0.f;
+            gd_wait_lds();                                                     // own reads of the step are in registers: its stage may be written
+            if (s + NS < steps) fetch(s + NS);
         }
-        if (ka_act_gated(act)) {
-            ka_gated_store<false, 4>(out, KA_F32, ldo, m, n, N, v, act);
-            return;
-        }
-        if (act)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = ka_activate(act, v[j]);
-        float* op = out + (size_t)m * ldo + n;
-        if (vectors) {
-            floatx4 r = {v[0], v[1], v[2], v[3]};
-            if (accumulate) r = *reinterpret_cast<const floatx4*>(op) + r;
-            *reinterpret_cast<floatx4*>(op) = r;
-        } else {
-            for (int j = 0; j < 4 && n + j < N; ++j) op[j] = accumulate ? op[j] + v[j] : v[j];
-        }
-    };
-    // the parts' sums through LDS; every wave finishes a quarter of the tile's numbers
+        for (int v = 0; v < 16; ++v)
+            if ((rows[0] >> (v / 4 * 8 + lg * 4 + v % 4) | rows[1] >> li) & 1 || !(fabsf(acc[v]) < INFINITY)) acc[v] = sum[v];
+    }
+    // acc[v] is out[m][n] with n = n0 + (v / 4) 8 + lg 4 + v % 4 and m = m0 + li. The parts' sums through LDS; every wave finishes a quarter of the tile's numbers.
     gd_wait_lds();
     gd_barrier();
     floatx4* sums = reinterpret_cast<floatx4*>(gf_lds);
-    gd_static_for<0, WN * WM * 4>([&](auto ic) {
-        constexpr int i = decltype(ic)::value, a = i / (4 * WM), b = i / 4 % WM, q = i % 4;
-        floatx4 y;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) y[j] = acc[a][b][q * 4 + j] + low[a][b][q * 4 + j];
-        sums[(part * WN * WM * 4 + i) * KA_WAVE + lane] = y;
-    });
+    for (int q = 0; q < 4; ++q) sums[(part * 4 + q) * KA_WAVE + lane] = floatx4{acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
     gd_wait_lds();
     gd_barrier();
     const int parts = (k_steps + part_steps - 1) / part_steps;                 // (those that hold anything)
-    for (int i = 0; i < WN * WM; ++i) {
-        const int at = i * 4 + part;
-        floatx4 y = sums[at * KA_WAVE + lane];
-        for (int p = 1; p < parts; ++p) y += sums[(p * WN * WM * 4 + at) * KA_WAVE + lane];
-        store(i / WM, i % WM, part, y);
+    floatx4 y = sums[part * KA_WAVE + lane];
+    for (int p = 1; p < parts; ++p) y += sums[(p * 4 + part) * KA_WAVE + lane];
+    const int m = m0 + li, n = n0 + part * 8 + lg * 4;
+    if (m >= M || n >= N) return;
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = y[j] + (bias && n + j < N ? bias[n + j] : 0.f);
+    if (ka_act_gated(act)) {
+        ka_gated_store<false, 4>(out, KA_F32, ldo, m, n, N, v, act);
+        return;
+    }
+    if (act)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ka_activate(act, v[j]);
+    float* op = out + (size_t)m * ldo + n;
+    if (N % 4 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+        floatx4 r = {v[0], v[1], v[2], v[3]};
+        if (accumulate) r = *reinterpret_cast<const floatx4*>(op) + r;
+        *reinterpret_cast<floatx4*>(op) = r;
+    } else {
+        for (int j = 0; j < 4 && n + j < N; ++j) op[j] = accumulate ? op[j] + v[j] : v[j];
     }
 }
 
-template <int WN, int WM, int NS>
-static int launch_f32_split(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
+template <int NS>
+static int launch_f32_tiles(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
                             int act, int accumulate, hipStream_t stream) {
-    constexpr int BN = 32 * WN, BM = 32 * WM, smem = F32_PARTS * NS * (BN + BM) * 64;
-    static_assert(smem >= F32_PARTS * WN * WM * 4 * KA_WAVE * 16, "the parts' sums fit");
+    constexpr int smem = F32_PARTS * NS * 2 * F32_TILE * F32_STEP * 4;
+    static_assert(smem >= F32_PARTS * 4 * KA_WAVE * 16, "the parts' sums fit");
     static bool configured = false;
-    auto kernel = gemm_f32_split_kernel<WN, WM, NS>;
+    auto kernel = gemm_f32_tiles_kernel<NS>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         KA_CHECK(e == hipSuccess, "ka_linear_generic: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
         configured = true;
     }
-    const int tiles_n = ka_cdiv(N, BN), tiles_m = ka_cdiv(M, BM);
+    const int tiles_n = ka_cdiv(N, F32_TILE), tiles_m = ka_cdiv(M, F32_TILE);
     const long blocks = ((long)tiles_n * tiles_m + 7) / 8 * 8;
     KA_CHECK(blocks < (1L << 31), "ka_linear_generic: too many tiles");
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KA_WAVE * F32_PARTS), smem, stream, A, lda, W, ldw, bias, out, ldo, M, N, K, act,
                        accumulate, tiles_n, tiles_m);
     KA_LAUNCH_CHECK();
     return 0;
-}
-
-// The tile: the one that is done first by what was measured (us per 2,048 of K: a first part, and as much again for every round of one tile a CU); all give the
-// same bits. Tiles of 32 x 32 leave room for two workgroups a CU, or for eight stages instead of four where no CU has two and K is long (2,048 of 8,192, 17
-// and 96 rows: 49.2 and 48.7 us with four, 43.1 and 46.4 with eight; K of 2,048 the same). Measured, us per 2,048 of K, tiles a CU rounded up (17 to 2,048 rows
-// of 2,048 x 2,048, 6,144 x 2,048 and 8,192 x 2,048):
-//              1      2      3     4     7     8    12    16
-//   64 x 64    30     60     90   122         254   387   509
-//   64 x 32    22     38           78         161
-//   32 x 32    16     25     34    43    73    88
-static int launch_f32_best(const float* A, long lda, const float* W, long ldw, const float* bias, float* out, long ldo, int M, int N, int K,
-                           int act, int accumulate, hipStream_t stream) {
-    const int cus = ka_compute_units();
-    auto rounds = [&](int bn, int bm) { return (float)((((long)ka_cdiv(N, bn) * ka_cdiv(M, bm)) + cus - 1) / cus); };
-    const float t64 = 30.5f * rounds(64, 64), t32 = 1.f + 20.f * rounds(64, 32), t1 = 6.f + 9.6f * rounds(32, 32);
-#define KA_F32(...) return launch_f32_split<__VA_ARGS__>(A, lda, W, ldw, bias, out, ldo, M, N, K, act, accumulate, stream)
-    if (t64 <= t32 && t64 <= t1) KA_F32(2, 2, 4);
-    if (t32 <= t1) KA_F32(2, 1, 4);
-    if (rounds(32, 32) <= 1.f && K >= 4096) KA_F32(1, 1, 8);
-    KA_F32(1, 1, 4);
-#undef KA_F32
 }
 
 // Many rows in fp32 (prompts on the 32-bit path): the same sums, k in ascending order for every
@@ -601,7 +574,9 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
     // (a gated linear at any number of rows, since the weight-streaming kernel has no pairs: its sums then never depend on the rows
     // beside a row. 1 to 16 rows of 2,048 inputs, 16,384 outputs: 199 to 212 us by vector tiles, 28 here; 1,408: 180 to 188 and 16.5)
     if (vectors && (M > GV_ROWS || ka_act_gated(act)) && K % F32_STEP == 0) {
-        return launch_f32_best((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream);
+        // (a third step in LDS where no CU has two workgroups, which have room for two each: 17 rows of 2,048 x 6,144, bf16 weights, 17.3 and 13.9 us; 10,240 x 2,560, 320 workgroups, 33.6 and 36.0)
+        const bool alone = (long)ka_cdiv(M, F32_TILE) * ka_cdiv(N, F32_TILE) <= ka_compute_units();
+        return (alone ? launch_f32_tiles<3> : launch_f32_tiles<2>)((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream);
     }
     if (vectors && M > GV_ROWS && ka_cdiv(M, 64) <= 65535) {
         if ((long)ka_cdiv(N, GF) * ka_cdiv(M, GF) >= 512)

@@ -1209,7 +1209,8 @@ def rope_cache(qkv: torch.Tensor, positions: torch.Tensor, slots: Optional[torch
 def linear_generic(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                    act: int = 0, accumulate: bool = False) -> None:
     """``out = act(a @ weight.T + bias)`` or ``out += ...``, any sizes and type mix: 32-bit operands of many
-    rows on the matrix pipes (each number as three of bf16, no bit lost), other mixes by plain fp32 FMA."""
+    rows on the matrix pipes (in 32 bits; where weights are bf16 numbers, the activations as three bf16 numbers each, in 32
+    bits again where those do not say a number to its last bit), other mixes by plain fp32 FMA."""
     _dev(a, weight, bias, out)
     m, k = a.shape
     n = weight.shape[0]

@@ -54,7 +54,7 @@ def linear(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     """``out = act(a @ weight.T + bias)``, or ``out += a @ weight.T + bias`` into fp32 ``out``.
 
     bf16 x bf16 goes to the MFMA kernels (a weight-streaming one for few rows, a tiled
-    one otherwise); fp32 of many rows to the matrix pipes in three parts, every other mix of types to the plain fp32 FMA kernel.
+    one otherwise); fp32 of many rows to the matrix pipes, every other mix of types to the plain fp32 FMA kernel.
     """
     if a.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         from . import fast
