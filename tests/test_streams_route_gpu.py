@@ -61,3 +61,40 @@ def test_what_stays_with_two_launches():
         assert not core.streams_step_route(x, y, torch.ones(S, S, device=DEV), torch.ones(S, device=DEV), form, h, router, None, logits, outputs, None, 1, 0, 0, 1.0,
                                            chosen, weights)
         assert bool((x == 1.0).all()) and bool((h == 7.0).all())
+
+
+# (one row, either side of 16 and of the most rows that stream weights; rows of 2,048 and the next longer ones, of 2,560 and the next; a shared expert among the others, of its own, none)
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65])
+@pytest.mark.parametrize("dim, shared", [(2048, "joined"), (2048, "own"), (2048, None), (2112, "joined"), (2560, "joined"), (2624, "joined"), (4096, "own")])
+def test_where_the_choice_goes(n, dim, shared):
+    """A routed mixture behind streams: the choice in the step's launch or in its own, by rows, width and shared expert; the same experts either way, and the same streams but for roundings."""
+    from types import SimpleNamespace
+
+    from kestrel_amd.engine.batch import Workspace
+    from kestrel_amd.ops import core
+    from kestrel_amd.parts.experts import RoutedExperts
+    from kestrel_amd.parts.specs import RoutedExpertsSpec
+
+    gen = torch.Generator().manual_seed(n + dim)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    spec = RoutedExpertsSpec("routed_experts", dim, 6, 64, 2, scores="sigmoid", group_best=2, shared_hidden={"joined": 64, "own": 128, None: None}[shared], shared_gate=False)
+    part = RoutedExperts(spec)
+    weights = {name: (rnd(*p.shape) * (p.shape[-1] ** -0.5 if len(p.shape) > 1 else 0.1)).bfloat16() for name, p in part.params().items()}
+    part.bind(weights, torch.bfloat16, torch.device(DEV))
+    streams = SimpleNamespace(matrix=rnd(3, 3).to(DEV), out=rnd(3).to(DEV))
+    reading = (rnd(3).to(DEV), ("rms", rnd(dim).to(DEV), None, 1e-5))
+    x, y = rnd(n, 3, dim).to(DEV), rnd(n, dim).to(DEV)
+    results = []
+    for together in (True, False):
+        batch, rows, h = SimpleNamespace(workspace=Workspace(torch.device(DEV))), x.clone(), torch.full((n, dim), 7.0, dtype=torch.bfloat16, device=DEV)
+        took = together and part.choose_streams(rows, y, streams, reading, h, batch)
+        assert took == (together and n <= 64 and (dim == 2048 and shared != "own" or dim > 2560 and n > 16))
+        if not took:
+            assert torch.equal(rows, x) and bool((h == 7.0).all())
+            core.streams_step(rows, y, streams.matrix, streams.out, reading, h)
+        part.mix_streams(h, batch, rows, streams, None, None, chosen=took)
+        results.append((h, batch.workspace.get("experts.chosen", (n, 2 + part.joined), torch.int32).clone(), rows))
+    (h, chosen, rows), (want_h, want_chosen, want_rows) = results
+    assert torch.equal(h, want_h) and torch.equal(chosen.sort(dim=1).values, want_chosen.sort(dim=1).values)
+    # (the weights of a choice differ by the order of the router's sums, some 24 roundings of 2^-24; a sigmoid's slope is a quarter)
+    assert bool(((rows - want_rows).abs() <= 1e-4 * want_rows.abs().amax(dim=(1, 2), keepdim=True)).all())

@@ -3,13 +3,14 @@
 import pytest
 import torch
 
-from tests import bokorax_cases, gozatar_cases, helpers, vufolorn_cases
+from tests import bogivik_cases, bokorax_cases, gozatar_cases, helpers, vufolorn_cases
+from tests.plain import moondream_plain as plain
 
 pytestmark = pytest.mark.gpu
 
 CASES = [("moondream2", "C"), ("moondream2", "F")] + \
-    [(family, name) for family in ("bokorax", "gozatar", "vufolorn") for name in "PQRS"]
-FOLDERS = {"bokorax": bokorax_cases.folder_for, "gozatar": gozatar_cases.folder_for, "vufolorn": vufolorn_cases.folder_for}
+    [(family, name) for family in ("bogivik", "bokorax", "gozatar", "vufolorn") for name in "PQRS"]
+FOLDERS = {"bogivik": lambda name, dtype: bogivik_cases.model_dir(name), "bokorax": bokorax_cases.folder_for, "gozatar": gozatar_cases.folder_for, "vufolorn": vufolorn_cases.folder_for}
 
 # (request, tokens, wanted places) of every step: nothing wanted; the last places of portions, several of one and places inside; a decoded token
 # beside portions, more of them wanted than half (all tokens of the last layer, also without the rule); portions of 70 and 81 tokens, so
@@ -57,6 +58,31 @@ def test_last_layer_for_wanted_tokens(monkeypatch, family, name, dtype, graphs):
     atol, rtol, spread = helpers.tolerance(dtype)
     bound = atol + rtol * whole.abs() + (spread or 2e-5) * whole.std(dim=1, keepdim=True)
     assert bool(((narrow - whole).abs() <= 2 * bound).all()), f"off by {float(((narrow - whole).abs() / bound).max()):.3g} bounds"
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["eager", "graphs"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("name", ["C", "D", "E", "F"])
+def test_wanted_tokens_inside_a_block_that_sees_both_ways(name, dtype, graphs):
+    """Given embeddings in front: wanted tokens of them, which see keys behind their own, and of the text, alone and beside a request without any."""
+    from kestrel_amd.engine.loading import load_model, make_runner
+    from kestrel_amd.engine.step import StepEntry
+
+    cfg = helpers.flat_config(name)
+    runner = make_runner(load_model(helpers.model_dir(name), dtype, torch.device("cuda:0")), 16, 64, 4, enable_graphs=graphs)
+    helpers.poison_cache(runner)
+    weights = helpers.stored_weights(helpers.model_dir(name))
+    prefix = torch.randn(37, cfg["dim"], generator=torch.Generator().manual_seed(9))
+    ids = {tag: helpers.random_ids(i, 60, cfg["vocab_size"]) for i, tag in enumerate("ab")}
+    first, second = runner.admit(), runner.admit()
+    embeds = prefix.to("cuda:0")
+    inside = StepEntry(first, [-1] * 37 + ids["a"][:20], want=(0, 18, 36, 50), embeds=embeds, bidirectional=[(0, 37)])
+    steps = [[StepEntry(second, ids["b"][:25], want=(24,)), inside], [StepEntry(second, ids["b"][25:55], want=(3, 29)), StepEntry(first, ids["a"][20:30], want=(9,))]]
+    places = [[("b", 24), ("a", 0), ("a", 18), ("a", 36), ("a", 50)], [("b", 28), ("b", 54), ("a", 66)]]
+    want = {"a": plain.forward(cfg, weights, ids["a"][:30], prefix), "b": plain.forward(cfg, weights, ids["b"][:55], None)}
+    for entries, order in zip(steps, places):
+        logits = runner.step(entries)
+        helpers.assert_close(logits, torch.stack([want[tag][place] for tag, place in order]), dtype, f"tiny {name}")
 
 
 @pytest.mark.parametrize("m", [0, 1, 7, 64])
