@@ -9,7 +9,8 @@
 
 // The order of a sum is that of the kernel that streams weights through registers, whose bits these are:
 //  * FW_EIGHTHS, skinny_persistent_kernel: its wave w takes K-steps w, w + 8, ..., the first and second 32 channels of each apart; a sum starts with the bias and
-//    takes the waves' in turn. The eight waves' sums are registers of their own here (64 TW a lane), so that K is read in its order (in the waves' order, with
+//    takes the waves' in turn. The eight waves' sums are registers of their own here (64 TW a lane; with four and five sixteens
+//    all 512 are taken, and 16 and 20 spill), so that K is read in its order (in the waves' order, with
 //    one set of sums: 21.3 instead of 17.8 us, 64 rows, 14,336 of 2,048).
 //  * FW_HALVES, skinny_wide_kernel with K in one part: all K-steps, the first and second 32 channels apart; the bias behind.
 enum { FW_EIGHTHS = 0, FW_HALVES = 1 };

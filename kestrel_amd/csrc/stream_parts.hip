@@ -223,8 +223,8 @@ __global__ void __launch_bounds__(THREADS) streams_step_kernel(StreamArgs a, con
 // handful of workgroups that wait for memory, and the choice behind it a wave a row that waits again; here the router's weights (120 to 500 KB, from L2 for all rows
 // but the first) are asked for beside the streams, in registers, and h meets them out of LDS: a wave takes every (THREADS / 64)-th output.
 // A row's numbers depend on that row alone. One CU brings the weights at 30 to 40 GB/s beyond the first trip, so long rows gain only where the linear alone is slow
-// (us, 30 outputs of 2,048, one row: step, linear and choice 9.4, this 7.5; 62 of 4,096: 11.9 and 15.7, 40 rows 21.4 and 16.5). 1,024 threads leave 128 registers: two
-// outputs ahead spilled, 25.8 us.
+// (us, 30 outputs of 2,048, one row: step, linear and choice 9.4, this 7.5; 62 of 4,096: 11.9 and 15.7, 40 rows 21.4 and 16.5). 1,024 threads leave 128 registers,
+// which one output ahead takes up (eight values spill); with two ahead 25.8 us.
 struct StreamRoute {
     const bf16_t* router;       // [outputs, dim], rows ld apart
     long ld;
