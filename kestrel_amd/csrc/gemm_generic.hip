@@ -83,8 +83,8 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 //    nothing but products of 32 bits is run.
 //  * A number of A below 2^-109 may have bits below bf16's smallest: what is left for the third part then has a lower half.
 //  * Infinities, NaN and what lies beyond bf16's largest leave a sum that is not finite.
-// Where a tile meets one of these, the wave that does multiplies its part once more in 32 bits, and the sums that need it take that result (us, 282 rows, usual numbers, a NaN
-// in every row, numbers of 1e-36, and one weight row in 50 of 32 bits: 2,048 x 6,144 64, 108, 133 and 121; 8,192 x 2,048 87, 169, 203 and 160).
+// Where a tile meets one of these, the wave that does multiplies its part once more in 32 bits, and the sums that need it take that result (us, inputs x outputs here and below, 282 rows, usual numbers, a
+// NaN in every row, numbers of 1e-36, and one weight row in 50 of 32 bits: 2,048 x 6,144 64, 108, 133 and 121; 8,192 x 2,048 87, 169, 203 and 160).
 //
 // Operands go straight from memory into swizzled LDS as in ka_dma_tiles.h, whole lines of 32 numbers, and are split by the wave that multiplies them, between the products of
 // the half step before, which the compiler does only where each half is a region of its own with an end that names the parts. Tiles of 32 x 32 alone, two workgroups a
@@ -98,8 +98,8 @@ gemm_generic_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W
 //    chains take the error of a sum from that of a chain of K / 4 terms to that of one of K / 64 (of every 32 from zero: 6 % faster, an error up to 9 % larger).
 //  * Three parts: w x1 of 128 of K from zero, these sums in order; w x2 and w x3, whose roundings weigh 2^-8, in an accumulator beside them.
 //
-// Measured, us, outputs x inputs; all products in 32 bits by tiles of 32 x 32 to 64 x 128 -> here with weights of 32 bits and with bf16 numbers: 6,144 x 2,048, 17 rows 19.3 -> 17.6, 15.4; 64
-// rows 27.1 -> 28.0, 23.3; 282 rows 81.8 -> 80.3, 59.1; 2,048 rows 445 -> 521, 329. 2,048 x 8,192: 51.1 -> 46.7, 34.8; 51.7 -> 47.8, 38.5; 130 -> 128, 84.8; 614 -> 659, 425. Over 14
+// Measured, us; all products in 32 bits by tiles of 32 x 32 to 64 x 128 -> here with weights of 32 bits and with bf16 numbers: 2,048 x 6,144, 17 rows 19.3 -> 17.6, 15.4; 64
+// rows 27.1 -> 28.0, 23.3; 282 rows 81.8 -> 80.3, 59.1; 2,048 rows 445 -> 521, 329. 8,192 x 2,048: 51.1 -> 46.7, 34.8; 51.7 -> 47.8, 38.5; 130 -> 128, 84.8; 614 -> 659, 425. Over 14
 // shapes (1,024 to 10,240 outputs, K of 1,024 to 10,240): 17 to 32 rows 0.96 and 0.85 of the time, 48 to 64 0.98 and 0.85, 80 to 160 0.98 and 0.80, 282 1.01 and 0.74, 512 1.05 and 0.77,
 // 2,048 1.12 and 0.77. Error against 64 bits of sums of 2,048 1.35e-7, with bf16 weights 8.7e-8; of 8,192 2.2e-7 and 1.1e-7.
 constexpr int F32_PARTS = 4;
@@ -574,7 +574,7 @@ KA_API int ka_linear_generic(const void* A, int a_dtype, long lda, const void* W
     // (a gated linear at any number of rows, since the weight-streaming kernel has no pairs: its sums then never depend on the rows
     // beside a row. 1 to 16 rows of 2,048 inputs, 16,384 outputs: 199 to 212 us by vector tiles, 28 here; 1,408: 180 to 188 and 16.5)
     if (vectors && (M > GV_ROWS || ka_act_gated(act)) && K % F32_STEP == 0) {
-        // (a third step in LDS where no CU has two workgroups, which have room for two each: 17 rows of 2,048 x 6,144, bf16 weights, 17.3 and 13.9 us; 10,240 x 2,560, 320 workgroups, 33.6 and 36.0)
+        // (a third step in LDS where no CU has two workgroups, which have room for two each: 17 rows of 2,048 x 6,144, bf16 weights, 17.3 and 13.9 us; 2,560 x 10,240 of 32 bits, 320 workgroups, 33.6 and 36.0)
         const bool alone = (long)ka_cdiv(M, F32_TILE) * ka_cdiv(N, F32_TILE) <= ka_compute_units();
         return (alone ? launch_f32_tiles<3> : launch_f32_tiles<2>)((const float*)A, lda, (const float*)W, ldw, bias, (float*)out, ldo, M, N, K, act, accumulate, stream);
     }
